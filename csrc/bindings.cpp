@@ -32,6 +32,7 @@ void lsd_gemm_set_ring8_flags(int v);
 void lsd_gemm_set_ring8_pack(int v);
 void lsd_norm_set_wave_narrow_min(int v);
 void lsd_norm_set_wave_min(int v);
+int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits);
 int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
 void lsd_attn_set_max_wg(int v);
@@ -153,7 +154,7 @@ GemmParams base_params(const torch::Tensor& a, const torch::Tensor& w, int64_t t
   return p;
 }
 
-// Launch with split-K bookkeeping: the decode path needs persistent zeroed
+// Launch with split-K bookkeeping: splits over blocks need persistent zeroed
 // ticket counters (one per column tile) and an fp32 partial-tile workspace.
 void run_gemm(GemmParams& p, int epi, int64_t tiled, int64_t splits,
               const c10::optional<torch::Tensor>& counters, const torch::Tensor& like,
@@ -164,6 +165,7 @@ void run_gemm(GemmParams& p, int epi, int64_t tiled, int64_t splits,
   int* cnt = nullptr;
   float* ws = nullptr;
   torch::Tensor wsbuf;
+  const bool deep = lsd_gemm_on_deep(p.M, p.N, p.K, epi, (int)tiled, (int)splits);  // sums inside a block: no workspace
   if (tiled && splits > 1 && epi != EPI_SLAB) {
     // tiled split-K with an in-kernel combine: the 256-row decode kernel
     // (gemm_d256, kind 2 / 3) or the 8-wave 128x64 ring (kind 1) -- ticket
@@ -180,8 +182,10 @@ void run_gemm(GemmParams& p, int epi, int64_t tiled, int64_t splits,
                 what, ": counter buffer too small (", counters->numel(), " < ", tiles, ")");
     cnt = counters->data_ptr<int>();
     TORCH_CHECK(splits * tile_floats * 4 < (1L << 31), what, ": split workspace too large");
-    wsbuf = torch::empty({tiles * splits * tile_floats}, like.options().dtype(torch::kFloat32));
-    ws = wsbuf.data_ptr<float>();
+    if (!deep) {
+      wsbuf = torch::empty({tiles * splits * tile_floats}, like.options().dtype(torch::kFloat32));
+      ws = wsbuf.data_ptr<float>();
+    }
   }
   if (!tiled && epi != EPI_SLAB) {
     const int nw = lsd_gemm_sk_nw(p.M, epi);  // column tile = 64 * nw (partial last tile masked)
@@ -197,8 +201,10 @@ void run_gemm(GemmParams& p, int epi, int64_t tiled, int64_t splits,
       const long rows = lsd_gemm_sk_rows(p.M, p.N, (int)splits);  // rows per row block
       const long bytes = tiles * splits * rows * 64 * nw * 4;
       TORCH_CHECK(splits * rows * 64 * nw * 4 < (1L << 31), what, ": split workspace too large");
-      wsbuf = torch::empty({bytes / 4}, like.options().dtype(torch::kFloat32));
-      ws = wsbuf.data_ptr<float>();
+      if (!deep) {
+        wsbuf = torch::empty({bytes / 4}, like.options().dtype(torch::kFloat32));
+        ws = wsbuf.data_ptr<float>();
+      }
     }
   }
   p.stamps = g_stamps;

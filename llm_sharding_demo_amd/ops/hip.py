@@ -1015,7 +1015,8 @@ class HipBackend(Backend):
         return self.R.gemm_kw(M, N, K, self.concurrency, nw)
 
     def _resid_splits(self, M: int, N: int, K: int) -> int:
-        return self.R.resid_splits(M, N, K, self._decode, getattr(self, "concurrency", 1))
+        S = self.R.resid_splits(M, N, K, self._decode, getattr(self, "concurrency", 1))
+        return self.R.slab_splits(M, N, K, S) if self._tiled(M, N) or self.R.defer_resid else S
 
     @classmethod
     def decode_attn_splits(cls, B: int, nh: int, n_kv: int, hd: int, max_ctx: int) -> int:

@@ -259,6 +259,26 @@ class Routing:
             return max(1, min(8, max(4, K // 800), K // 64))
         return self.sk_splits(M, N, K, lanes)
 
+    @staticmethod
+    def slab_splits(M: int, N: int, K: int, S: int) -> int:
+        """K splits of a residual projection of 9 .. 128 rows that leaves slabs,
+        near the S of resid_splits: on the deep ring (gemm_deep.hip) a CU takes in
+        about 50 KB a us, so the blocks' share per CU counts, and a slab costs the
+        next norm 0.25 us (4096 x 4096 at 40 rows: 5 slabs on 320 blocks 10.9 us, 4
+        on 256 8.7; 4096 x 14336: 8 slabs 21.9, 4 21.3, and the norm 5.7 -> 4.9).
+        A split has at least four k-steps of 64: below, its launch is all latency, and
+        an unsplit sum goes to the residual in fp32."""
+        if S <= 1 or not 8 < M <= 128 or K % 64:
+            return S
+        rows = 128 if M > 96 else 96 if M > 64 else math.ceil(M / 16) * 16
+
+        def us(s: int) -> float:
+            share = min(math.ceil(math.ceil(N / bn) * s / 256) * (bn + rows) for bn in (64, 32))
+            return share * K / s * 2 / 50e3 + 0.25 * s
+
+        most = max(1, K // 256)
+        return min((min(s, most) for s in (S, 4, 6, 8)), key=us)
+
     def logits_kw(self, M: int, N: int, K: int, lanes: int = 1):
         """lm_head: the 128x128 LDS-tiled kernel at vocab width (fills the
         chip without split-K; 41.8 vs 64.2 us at 128 rows, GPT-2 XL)."""
@@ -367,7 +387,9 @@ class Routing:
 def route_table(model: str, rows, routing: Routing | None = None) -> dict:
     """{(gemm, rows, phase): route} of one model's projections: what
     `tests/test_routing.py` pins and `python -m llm_sharding_demo_amd.ops.routing`
-    prints.  route = kernel family + K splits, no extension calls."""
+    prints.  route = kernel family + K splits, no extension calls.  The split-K and
+    tiled families run up to 128 rows on the deep ring (gemm_deep.hip), unsplit where
+    the split would be combined, and with slab_splits slabs."""
     from ..config import get_model_config
 
     r = routing or Routing.from_env("")

@@ -45,6 +45,9 @@ struct RecurParams {
   void* out; long ldo; int out_cols;   // delta (raw null): normed and gated rows, zeros up to out_cols;
                                        // Mamba-2: y silu(z) rows
   int write_ring;                      // single-token portions: this kernel keeps the ring
+  // delta rule in chunks with factors of their own: chunks first .. first + chunks - 1 of
+  // every sequence, their factors at work[sequence][chunk][head]
+  void* work; int first, chunks;
 };
 
 // Recurrence whose forget gate f also decides what is written:

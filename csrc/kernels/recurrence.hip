@@ -317,19 +317,218 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(ConvParams c, SeqParams 
 //   S = diag(e^{G_15 - G_0}) S0 + K^T U,   K^_s = k_s e^{G_15 - G_s}
 // Every factor is at most e^80 in size; channels that decay by more than that
 // within a chunk are left out of the two products over d and added term by term
-// (e^{G_t - G_s} <= 1 always).  One block per (sequence, head).
+// (e^{G_t - G_s} <= 1 always).
+//
+// Only the products with S0 and U follow one another; K~, Q~, K^, the inverse and P are a
+// chunk's own.  What bounds a prompt is the chain of chunks (9.4 us each on one block per
+// sequence and head), so where those blocks leave the chip idle a chunk's factors are made by
+// a block of their own, all at once (delta_factors_kernel), and the chain keeps what is left
+// (delta_state_kernel: a block per 64 columns of a state).  One sequence of 1000 tokens, 16
+// heads of 128 x 128: 590 us -> 22 + 70 + 9 (factors, states, output norm).  Above 192
+// (sequence, head) pairs the fused delta_chunk_kernel is as fast and needs no workspace.
+constexpr int DELTA_CT = 16, DELTA_WAVES = 2;
+
+template <int DKS>
+struct DeltaShared {
+  static constexpr int CT = DELTA_CT, DP = DKS * 32, LDD = DP + 8, LDT = CT + 4;
+  alignas(16) bf16 kt_h[CT * LDD], kt_l[CT * LDD], qt_h[CT * LDD], qt_l[CT * LDD];
+  alignas(16) bf16 kc_h[CT * LDD], kc_l[CT * LDD];     // columns k_s e^{G_0 - G_s}
+  alignas(16) bf16 kh_h[CT * LDD], kh_l[CT * LDD];     // K^
+  alignas(16) float Gs[CT][DP], Ks[CT][DP], Qs[CT][DP];
+  alignas(16) float e0[DP], s0[DP], er[DP], tot[4][DP], dtb[DP];
+  alignas(16) bf16 tm_h[CT * LDT], tm_l[CT * LDT], pm_h[CT * LDT], pm_l[CT * LDT];
+  float betas[CT], red[4][CT];
+  int bad[DP], nbad;
+  // operand of row r: k-slots (g, j) <-> d = 32 ks + 4 g + j, 32 ks + 16 + 4 g + (j - 4)
+  static __device__ __forceinline__ bf16x8 opnd(const bf16* a, int ks) {
+    const bf16* at = a + (threadIdx.x & 15) * LDD + ks * 32 + 4 * (lane_id() >> 4);
+    return cat(ld4(at), ld4(at + 16));
+  }
+};
+
+// K~, Q~, K^ and the decays of a chunk of nt tokens, from the threads' rows (token tid / 16,
+// channels 8 (tid % 16) ..): query, key, decay logits, and beta's logit of token tid % 16.
+// `next` runs once the rows are used up; emit(channel, k, q, G) gets four channels before their
+// decay and the log decays G_t.  Ends with a barrier.
+template <int DKS, class F, class EmitF>
+__device__ __forceinline__ void delta_factors(DeltaShared<DKS>& sm, bf16x8 xq, bf16x8 xk, bf16x8 xl, float rb, int nt,
+                                              bool elive, float A, float gain, float inv_sqrt_d, F next, EmitF emit) {
+  constexpr int CT = DELTA_CT, DP = DKS * 32, LDD = DeltaShared<DKS>::LDD;
+  constexpr float RANGE = 80.f;
+  const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int et = tid >> 4, ed = (tid & 15) * 8;
+  const bool tlive = et < nt && elive;
+  float q8[8], k8[8], lg[8];
+  {
+    float nq = 0.f, nk = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q8[e] = elive ? bf2f(xq[e]) : 0.f;
+      k8[e] = elive ? bf2f(xk[e]) : 0.f;
+      nq = fmaf(q8[e], q8[e], nq);
+      nk = fmaf(k8[e], k8[e], nk);
+      lg[e] = tlive ? A * softplus_f(gain * bf2f(xl[e]) + sm.dtb[ed + e]) : 0.f;
+    }
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+      nq += wave_xchg_n(nq, off);
+      nk += wave_xchg_n(nk, off);
+    }
+    const float iq = tlive ? inv_sqrt_d * rsqrtf(nq + UNIT_EPS) : 0.f, ik = tlive ? rsqrtf(nk + UNIT_EPS) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q8[e] *= iq;
+      k8[e] *= ik;
+    }
+  }
+  // log decays summed over the tokens: within the wave's four by lanes, across waves by LDS
+  float pre[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    pre[e] = lg[e];
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+      const float u = __shfl_up(pre[e], off, 64);
+      if (lane >= off) pre[e] += u;
+    }
+  }
+  if (ed < DP) {
+    if (lane >= 48) {
+      *reinterpret_cast<f32x4*>(&sm.tot[w][ed]) = f32x4{pre[0], pre[1], pre[2], pre[3]};
+      *reinterpret_cast<f32x4*>(&sm.tot[w][ed + 4]) = f32x4{pre[4], pre[5], pre[6], pre[7]};
+    }
+    if (et == 0) {
+      *reinterpret_cast<f32x4*>(&sm.e0[ed]) = f32x4{lg[0], lg[1], lg[2], lg[3]};
+      *reinterpret_cast<f32x4*>(&sm.e0[ed + 4]) = f32x4{lg[4], lg[5], lg[6], lg[7]};
+    }
+  }
+  if (tid < CT) sm.betas[tid] = tid < nt ? sigmoid_x(gain * rb) : 0.f;
+  next();
+  if (tid == 0) sm.nbad = 0;
+  __syncthreads();
+  if (ed < DP) {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      asm volatile("" ::: "memory");  // four channels at a time
+      const int d0 = ed + 4 * hf;
+      const f32x4 g0 = *reinterpret_cast<const f32x4*>(&sm.e0[d0]);
+      f32x4 gt = {0.f, 0.f, 0.f, 0.f}, all = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(&sm.tot[q][d0]);
+        if (q < w) gt += v;  // wave-uniform
+        all += v;
+      }
+      f32x4 kt, qt, kc, kf;
+      bool wides = false;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = 4 * hf + i;
+        gt[i] += pre[e];
+        const float G0 = g0[i], Gt = gt[i], Gc = all[i];
+        const float E = exp_f(Gt - G0);
+        const bool wide = G0 - Gc > RANGE;
+        kt[i] = k8[e] * E;
+        qt[i] = q8[e] * E;
+        kc[i] = wide ? 0.f : k8[e] * exp_f(G0 - Gt);
+        kf[i] = k8[e] * exp_f(Gc - Gt);
+        wides |= wide;
+        if (et == 15) {
+          sm.s0[ed + e] = exp_f(G0);
+          sm.er[ed + e] = exp_f(Gc - G0);
+          if (wide) sm.bad[atomicAdd(&sm.nbad, 1)] = ed + e;
+        }
+      }
+      emit(d0, f32x4{k8[4 * hf], k8[4 * hf + 1], k8[4 * hf + 2], k8[4 * hf + 3]},
+           f32x4{q8[4 * hf], q8[4 * hf + 1], q8[4 * hf + 2], q8[4 * hf + 3]}, gt);
+      if (wides) {  // the same channels for every token
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sm.Gs[et][d0 + i] = gt[i];
+          sm.Ks[et][d0 + i] = k8[4 * hf + i];
+          sm.Qs[et][d0 + i] = q8[4 * hf + i];
+        }
+      }
+      auto put = [&](bf16* hp, bf16* lp, f32x4 v) {
+        const bf16x4 a = hi4(v);
+        st4(hp + et * LDD + d0, a);
+        st4(lp + et * LDD + d0, lo4(v, a));
+      };
+      put(sm.kt_h, sm.kt_l, kt);
+      put(sm.qt_h, sm.qt_l, qt);
+      put(sm.kc_h, sm.kc_l, kc);
+      put(sm.kh_h, sm.kh_l, kf);
+    }
+  }
+  __syncthreads();
+}
+
+// wave 0: diag(beta) on the right of (I + A)^-1, wave 1: P, in two terms each
+template <int DKS>
+__device__ __forceinline__ void delta_matrices(DeltaShared<DKS>& sm, int w) {
+  constexpr int CT = DELTA_CT, LDT = DeltaShared<DKS>::LDT;
+  const int lane = lane_id(), r = lane & 15, g = lane >> 4;
+  auto opnd = [&](const bf16* a, int ks) { return DeltaShared<DKS>::opnd(a, ks); };
+        const bf16 *ah = w == 0 ? sm.kt_h : sm.qt_h, *al = w == 0 ? sm.kt_l : sm.qt_l;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < DKS; ++ks) {
+          asm volatile("" ::: "memory");  // operands of one step at a time
+          acc = mfma3(opnd(ah, ks), opnd(al, ks), opnd(sm.kc_h, ks), opnd(sm.kc_l, ks), acc);
+        }
+        const int nb = sm.nbad;
+        for (int q = 0; q < nb; ++q) {
+          const int d = sm.bad[q];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = 4 * g + i;
+            if (r <= t) acc[i] += (w == 0 ? sm.Ks[t][d] : sm.Qs[t][d]) * sm.Ks[r][d] * exp_f(sm.Gs[t][d] - sm.Gs[r][d]);
+          }
+        }
+        if (w == 1) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = 4 * g + i;
+            const float v = r <= t ? acc[i] : 0.f;
+            const bf16 a = f2bf(v);
+            sm.pm_h[t * LDT + r] = a;
+            sm.pm_l[t * LDT + r] = f2bf(v - bf2f(a));
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] = r < 4 * g + i ? acc[i] * sm.betas[4 * g + i] : 0.f;
+          // column r of the inverse by forward substitution (each lane group alike);
+          // A_ts is register t % 4 of lane 16 (t / 4) + s
+          float inv[CT];
+#pragma unroll
+          for (int t = 0; t < CT; ++t) {
+            float v = t == r ? 1.f : 0.f;
+#pragma unroll
+            for (int s = 0; s < t; ++s) {
+              // (a bit cast of a vector's element would take element 0)
+              const int a = __builtin_amdgcn_readlane(__float_as_int(acc[t & 3]), 16 * (t >> 2) + s);
+              v = fmaf(-__int_as_float(a), inv[s], v);
+            }
+            inv[t] = v;
+          }
+          const float bt = sm.betas[r];
+          if (g == 0) {
+#pragma unroll
+            for (int t = 0; t < CT; ++t) {
+              const float v = inv[t] * bt;
+              const bf16 a = f2bf(v);
+              sm.tm_h[t * LDT + r] = a;
+              sm.tm_l[t * LDT + r] = f2bf(v - bf2f(a));
+            }
+          }
+        }
+}
+
+// One block per (sequence, head), the whole chunk in it.
 template <int DKS, int VTW>
 __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, const bf16* __restrict__ x, long ldx) {
-  constexpr int CT = 16, DP = DKS * 32, DT = DKS * 2, LDD = DP + 8, LDT = CT + 4;
-  constexpr float RANGE = 80.f;
-  __shared__ __attribute__((aligned(16))) bf16 kt_h[CT * LDD], kt_l[CT * LDD], qt_h[CT * LDD], qt_l[CT * LDD];
-  __shared__ __attribute__((aligned(16))) bf16 kc_h[CT * LDD], kc_l[CT * LDD];     // columns k_s e^{G_0 - G_s}
-  __shared__ __attribute__((aligned(16))) bf16 kh_h[CT * LDD], kh_l[CT * LDD];     // K^
-  __shared__ __attribute__((aligned(16))) float Gs[CT][DP], Ks[CT][DP], Qs[CT][DP];
-  __shared__ __attribute__((aligned(16))) float e0[DP], s0[DP], er[DP], tot[4][DP], dtb[DP];
-  __shared__ __attribute__((aligned(16))) bf16 tm_h[CT * LDT], tm_l[CT * LDT], pm_h[CT * LDT], pm_l[CT * LDT];
-  __shared__ float betas[CT], red[4][CT];
-  __shared__ int bad[DP], nbad;
+  constexpr int CT = DELTA_CT, DP = DKS * 32, DT = DKS * 2, LDD = DeltaShared<DKS>::LDD, LDT = DeltaShared<DKS>::LDT;
+  __shared__ DeltaShared<DKS> sm;
   const int h = blockIdx.x, b = blockIdx.y, D = p.D, V = p.V;
   const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -366,7 +565,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
   // element work: token tid / 16, channels 8 (tid % 16) ..
   const int et = tid >> 4, ed = (tid & 15) * 8;
   const bool elive = ed < D;  // D % 8 == 0
-  for (int d = tid; d < DP; d += 256) dtb[d] = d < D ? p.dt_bias[(long)h * D + d] : 0.f;
+  for (int d = tid; d < DP; d += 256) sm.dtb[d] = d < D ? p.dt_bias[(long)h * D + d] : 0.f;
   __syncthreads();
 
   // rows of the next chunk, in flight under this one
@@ -384,108 +583,9 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
   fetch(0);
   for (int t0 = 0; t0 < n; t0 += CT) {
     const int nt = min(CT, n - t0);
-    const bool tlive = et < nt && elive;
-    float q8[8], k8[8], lg[8];
-    {
-      float nq = 0.f, nk = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        q8[e] = elive ? bf2f(xq[e]) : 0.f;
-        k8[e] = elive ? bf2f(xk[e]) : 0.f;
-        nq = fmaf(q8[e], q8[e], nq);
-        nk = fmaf(k8[e], k8[e], nk);
-        lg[e] = tlive ? A * softplus_f(gain * bf2f(xl[e]) + dtb[ed + e]) : 0.f;
-      }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) {
-        nq += wave_xchg_n(nq, off);
-        nk += wave_xchg_n(nk, off);
-      }
-      const float iq = tlive ? inv_sqrt_d * rsqrtf(nq + UNIT_EPS) : 0.f, ik = tlive ? rsqrtf(nk + UNIT_EPS) : 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        q8[e] *= iq;
-        k8[e] *= ik;
-      }
-    }
-    // log decays summed over the tokens: within the wave's four by lanes, across waves by LDS
-    float pre[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      pre[e] = lg[e];
-#pragma unroll
-      for (int off = 16; off < 64; off <<= 1) {
-        const float u = __shfl_up(pre[e], off, 64);
-        if (lane >= off) pre[e] += u;
-      }
-    }
-    if (ed < DP) {
-      if (lane >= 48) {
-        *reinterpret_cast<f32x4*>(&tot[w][ed]) = f32x4{pre[0], pre[1], pre[2], pre[3]};
-        *reinterpret_cast<f32x4*>(&tot[w][ed + 4]) = f32x4{pre[4], pre[5], pre[6], pre[7]};
-      }
-      if (et == 0) {
-        *reinterpret_cast<f32x4*>(&e0[ed]) = f32x4{lg[0], lg[1], lg[2], lg[3]};
-        *reinterpret_cast<f32x4*>(&e0[ed + 4]) = f32x4{lg[4], lg[5], lg[6], lg[7]};
-      }
-    }
-    if (tid < CT) betas[tid] = tid < nt ? sigmoid_x(gain * rb) : 0.f;
-    if (t0 + CT < n) fetch(t0 + CT);
-    if (tid == 0) nbad = 0;
-    __syncthreads();
-    if (ed < DP) {
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        asm volatile("" ::: "memory");  // four channels at a time
-        const int d0 = ed + 4 * hf;
-        const f32x4 g0 = *reinterpret_cast<const f32x4*>(&e0[d0]);
-        f32x4 gt = {0.f, 0.f, 0.f, 0.f}, all = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(&tot[q][d0]);
-          if (q < w) gt += v;  // wave-uniform
-          all += v;
-        }
-        f32x4 kt, qt, kc, kf;
-        bool wides = false;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int e = 4 * hf + i;
-          gt[i] += pre[e];
-          const float G0 = g0[i], Gt = gt[i], Gc = all[i];
-          const float E = exp_f(Gt - G0);
-          const bool wide = G0 - Gc > RANGE;
-          kt[i] = k8[e] * E;
-          qt[i] = q8[e] * E;
-          kc[i] = wide ? 0.f : k8[e] * exp_f(G0 - Gt);
-          kf[i] = k8[e] * exp_f(Gc - Gt);
-          wides |= wide;
-          if (et == 15) {
-            s0[ed + e] = exp_f(G0);
-            er[ed + e] = exp_f(Gc - G0);
-            if (wide) bad[atomicAdd(&nbad, 1)] = ed + e;
-          }
-        }
-        if (wides) {  // the same channels for every token
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            Gs[et][d0 + i] = gt[i];
-            Ks[et][d0 + i] = k8[4 * hf + i];
-            Qs[et][d0 + i] = q8[4 * hf + i];
-          }
-        }
-        auto put = [&](bf16* hp, bf16* lp, f32x4 v) {
-          const bf16x4 a = hi4(v);
-          st4(hp + et * LDD + d0, a);
-          st4(lp + et * LDD + d0, lo4(v, a));
-        };
-        put(kt_h, kt_l, kt);
-        put(qt_h, qt_l, qt);
-        put(kc_h, kc_l, kc);
-        put(kh_h, kh_l, kf);
-      }
-    }
-    __syncthreads();
+    delta_factors<DKS>(sm, xq, xk, xl, rb, nt, elive, A, gain, inv_sqrt_d, [&]() {
+      if (t0 + CT < n) fetch(t0 + CT);
+    }, [](int, f32x4, f32x4, f32x4) {});
     // values and gates of the chunk in the accumulator layout (tokens 4 g + i, columns r)
     f32x4 vals[VTW], gates[VTW];
 #pragma unroll
@@ -499,74 +599,17 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
         vals[j][i] = live ? xv : 0.f;
         gates[j][i] = bf2f((gateb + (long)t0 * p.ldl)[tc * ldl + vc]);
       }
-    // operand of row r: k-slots (g, j) <-> d = 32 ks + 4 g + j, 32 ks + 16 + 4 g + (j - 4)
-    auto opnd = [&](const bf16* a, int ks) {
-      return cat(ld4(a + r * LDD + ks * 32 + 4 * g), ld4(a + r * LDD + ks * 32 + 16 + 4 * g));
-    };
-    if (w < 2) {  // wave 0: A and (I + A)^-1, wave 1: P
-      const bf16 *ah = w == 0 ? kt_h : qt_h, *al = w == 0 ? kt_l : qt_l;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < DKS; ++ks) {
-        asm volatile("" ::: "memory");  // operands of one step at a time
-        acc = mfma3(opnd(ah, ks), opnd(al, ks), opnd(kc_h, ks), opnd(kc_l, ks), acc);
-      }
-      const int nb = nbad;
-      for (int q = 0; q < nb; ++q) {
-        const int d = bad[q];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = 4 * g + i;
-          if (r <= t) acc[i] += (w == 0 ? Ks[t][d] : Qs[t][d]) * Ks[r][d] * exp_f(Gs[t][d] - Gs[r][d]);
-        }
-      }
-      if (w == 1) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int t = 4 * g + i;
-          const float v = r <= t ? acc[i] : 0.f;
-          const bf16 a = f2bf(v);
-          pm_h[t * LDT + r] = a;
-          pm_l[t * LDT + r] = f2bf(v - bf2f(a));
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = r < 4 * g + i ? acc[i] * betas[4 * g + i] : 0.f;
-        // column r of the inverse by forward substitution (each lane group alike);
-        // A_ts is register t % 4 of lane 16 (t / 4) + s
-        float inv[CT];
-#pragma unroll
-        for (int t = 0; t < CT; ++t) {
-          float v = t == r ? 1.f : 0.f;
-#pragma unroll
-          for (int s = 0; s < t; ++s) {
-            // (a bit cast of a vector's element would take element 0)
-            const int a = __builtin_amdgcn_readlane(__float_as_int(acc[t & 3]), 16 * (t >> 2) + s);
-            v = fmaf(-__int_as_float(a), inv[s], v);
-          }
-          inv[t] = v;
-        }
-        const float bt = betas[r];
-        if (g == 0) {
-#pragma unroll
-          for (int t = 0; t < CT; ++t) {
-            const float v = inv[t] * bt;
-            const bf16 a = f2bf(v);
-            tm_h[t * LDT + r] = a;
-            tm_l[t * LDT + r] = f2bf(v - bf2f(a));
-          }
-        }
-      }
-    }
+    auto opnd = [&](const bf16* a, int ks) { return DeltaShared<DKS>::opnd(a, ks); };
+    if (w < 2) delta_matrices<DKS>(sm, w);
     f32x4 ks_acc[VTW], o[VTW];
 #pragma unroll
     for (int j = 0; j < VTW; ++j) ks_acc[j] = o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < DKS; ++ks) {
       if constexpr (VTW > 1) asm volatile("" ::: "memory");  // operands of one step at a time
-      const f32x4 da = *reinterpret_cast<const f32x4*>(&s0[ks * 32 + 4 * g]);
-      const f32x4 db = *reinterpret_cast<const f32x4*>(&s0[ks * 32 + 16 + 4 * g]);
-      const bf16x8 kah = opnd(kt_h, ks), kal = opnd(kt_l, ks), qah = opnd(qt_h, ks), qal = opnd(qt_l, ks);
+      const f32x4 da = *reinterpret_cast<const f32x4*>(&sm.s0[ks * 32 + 4 * g]);
+      const f32x4 db = *reinterpret_cast<const f32x4*>(&sm.s0[ks * 32 + 16 + 4 * g]);
+      const bf16x8 kah = opnd(sm.kt_h, ks), kal = opnd(sm.kt_l, ks), qah = opnd(sm.qt_h, ks), qal = opnd(sm.qt_l, ks);
 #pragma unroll
       for (int j = 0; j < VTW; ++j) {
         S[2 * ks][j] *= da;
@@ -578,8 +621,8 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
       }
     }
     __syncthreads();
-    const bf16x4 th = ld4(tm_h + r * LDT + 4 * g), tl = ld4(tm_l + r * LDT + 4 * g);
-    const bf16x4 ph = ld4(pm_h + r * LDT + 4 * g), pl = ld4(pm_l + r * LDT + 4 * g);
+    const bf16x4 th = ld4(sm.tm_h + r * LDT + 4 * g), tl = ld4(sm.tm_l + r * LDT + 4 * g);
+    const bf16x4 ph = ld4(sm.pm_h + r * LDT + 4 * g), pl = ld4(sm.pm_l + r * LDT + 4 * g);
     bf16x4 uh[VTW], ul[VTW];
     f32x4 ss = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -598,13 +641,13 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
       float v = ss[i];
 #pragma unroll
       for (int off = 1; off < 16; off <<= 1) v += wave_xchg_n(v, off);
-      if (r == 0) red[w][4 * g + i] = v;
+      if (r == 0) sm.red[w][4 * g + i] = v;
     }
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const f32x4 dec = *reinterpret_cast<const f32x4*>(&er[dt * 16 + 4 * g]);
+      const f32x4 dec = *reinterpret_cast<const f32x4*>(&sm.er[dt * 16 + 4 * g]);
       const int at = (4 * g + (r >> 2)) * LDD + dt * 16 + 4 * (r & 3);
-      const bf16x4 ah = ds_read_tr(kh_h + at), al = ds_read_tr(kh_l + at);
+      const bf16x4 ah = ds_read_tr(sm.kh_h + at), al = ds_read_tr(sm.kh_l + at);
 #pragma unroll
       for (int j = 0; j < VTW; ++j) S[dt][j] = mfma3s(ah, al, uh[j], ul[j], S[dt][j] * dec);
     }
@@ -614,7 +657,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
     for (int i = 0; i < 4; ++i) {
       const int t = 4 * g + i;
       if (t >= nt) continue;
-      const float rs = rsqrtf((red[0][t] + red[1][t] + red[2][t] + red[3][t]) / V + p.eps);
+      const float rs = rsqrtf((sm.red[0][t] + sm.red[1][t] + sm.red[2][t] + sm.red[3][t]) / V + p.eps);
 #pragma unroll
       for (int j = 0; j < VTW; ++j) {
         const int v = (w * VTW + j) * 16 + r;
@@ -638,6 +681,227 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
         const int d = dt * 16 + g4 + i, v = (w * VTW + j) * 16 + r;
         if (d < D && v < p.Vp) Sg[d * p.Vp + v] = S[dt][j][i];
       }
+}
+
+// Bytes of a chunk's factors in the workspace: k_t e^{G_t}, q_t e^{G_t} and K^ as operand
+// fragments in two terms, the inverse and P likewise, e^{G_15}, and the values of 128 columns
+// as accumulator tiles.
+template <int DKS>
+struct DeltaItem {
+  static constexpr int KT = 0, QT = DKS * 2048, KH = DKS * 4096, TM = DKS * 6144, PM = TM + 1024, ER = PM + 1024,
+                       FACTORS = (ER + DKS * 128 + 1023) / 1024 * 1024, VALS = FACTORS, BYTES = VALS + 4096;
+};
+
+// The factors of one chunk: block (head, chunk, sequence).
+template <int DKS>
+__global__ __launch_bounds__(256, 2) void delta_factors_kernel(RecurParams p, const bf16* __restrict__ x, long ldx) {
+  using I = DeltaItem<DKS>;
+  constexpr int CT = DELTA_CT, DP = DKS * 32, DT = DKS * 2, LDD = DeltaShared<DKS>::LDD, LDT = DeltaShared<DKS>::LDT;
+  __shared__ DeltaShared<DKS> sm;
+  const int h = blockIdx.x, b = blockIdx.z, D = p.D, V = p.V;
+  const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int kh = h / (p.heads / p.groups), r0 = p.s.cu[b], n = p.s.cu[b + 1] - r0, t0 = (p.first + (int)blockIdx.y) * CT;
+  if (t0 >= n) return;
+  const int nt = min(CT, n - t0), et = tid >> 4, ed = (tid & 15) * 8;
+  const bool elive = ed < D;
+  const long row = r0 + t0 + min(et, nt - 1);
+  const int dc = elive ? ed : 0;
+  const bf16x8 xq = ld8(x + row * ldx + p.q_ch + kh * D + dc), xk = ld8(x + row * ldx + p.k_ch + kh * D + dc);
+  const bf16x8 xl = ld8(static_cast<const bf16*>(p.low) + row * p.ldl + (long)h * D + dc);
+  const float rb = bf2f(static_cast<const bf16*>(p.c.y)[(long)(r0 + t0 + min(tid & 15, nt - 1)) * p.c.ldy + p.gate_col + h]);
+  char* item = static_cast<char*>(p.work) + (((long)b * p.chunks + blockIdx.y) * p.heads + h) * I::BYTES;
+  // values: tile j of 16 columns, tokens 4 g + i of column r
+  for (int j = w; j * 16 < V; j += 4) {
+    const int v = j * 16 + r;
+    const bf16* xv = x + (r0 + t0) * ldx + p.v_ch + (long)h * V + min(v, V - 1);
+    bf16x4 t;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bf16 e = xv[min(4 * g + i, nt - 1) * ldx];
+      t[i] = 4 * g + i < nt && v < V ? e : f2bf(0.f);
+    }
+    st4(reinterpret_cast<bf16*>(item + I::VALS + j * 512) + lane * 4, t);
+  }
+  for (int d = tid; d < DP; d += 256) sm.dtb[d] = d < D ? p.dt_bias[(long)h * D + d] : 0.f;
+  __syncthreads();
+  // for the products with the state, k and q decay from the chunk's beginning: the state then
+  // enters them as it is
+  auto emit = [&](int d0, f32x4 k, f32x4 q, f32x4 G) {
+    const int ks = d0 / 32, dd = d0 % 32;
+    bf16* o = reinterpret_cast<bf16*>(item + ks * 2048) + ((dd % 16 / 4) * 16 + et) * 8 + dd / 16 * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float e = exp_f(G[i]);
+      k[i] *= e;
+      q[i] *= e;
+    }
+    const bf16x4 kh = hi4(k), qh = hi4(q);
+    st4(o + I::KT / 2, kh);
+    st4(o + I::KT / 2 + 512, lo4(k, kh));
+    st4(o + I::QT / 2, qh);
+    st4(o + I::QT / 2 + 512, lo4(q, qh));
+  };
+  delta_factors<DKS>(sm, xq, xk, xl, rb, nt, elive, p.A[h], p.c.gain, rsqrtf((float)D), []() {}, emit);
+  if (w < 2) delta_matrices<DKS>(sm, w);
+  for (int dt = w; dt < DT; dt += 4) {  // K^ with tokens along k
+    const int at = (4 * g + (r >> 2)) * LDD + dt * 16 + 4 * (r & 3);
+    st8(reinterpret_cast<bf16*>(item + I::KH + dt * 1024) + lane * 8, cat(ds_read_tr(sm.kh_h + at), ds_read_tr(sm.kh_l + at)));
+  }
+  for (int d = tid; d < DP; d += 256) reinterpret_cast<float*>(item + I::ER)[d] = sm.s0[d] * sm.er[d];
+  __syncthreads();
+  if (w < 2) {  // the inverse, P
+    const int at = r * LDT + 4 * g;
+    st8(reinterpret_cast<bf16*>(item + (w == 0 ? I::TM : I::PM)) + lane * 8,
+        cat(ld4((w == 0 ? sm.tm_h : sm.pm_h) + at), ld4((w == 0 ? sm.tm_l : sm.pm_l) + at)));
+  }
+}
+
+// LDS ring of delta_state_kernel: as many chunks as fit, and as the wait counter can tell apart.
+template <int DKS, int WAVES>
+struct DeltaRing {
+  static constexpr int VALS = WAVES * 512, SLOT = DeltaItem<DKS>::FACTORS + VALS, INS = SLOT / 1024,
+                       LPS = (INS + WAVES - 1) / WAVES, FIT = 160 * 1024 / SLOT, COUNT = (63 + 4 + 2 * LPS) / (LPS + 4),
+                       SLOTS = FIT < COUNT ? FIT : COUNT, BYTES = SLOTS * SLOT;
+};
+
+// The chain of chunks for 16 WAVES columns of a state: block (columns and head, sequence).
+// Factors come through the ring, SLOTS chunks ahead; outputs leave in fp32, normed and gated
+// by head_norm_gate.  A wave has its SIMD to itself and its chain is bound by the number of its
+// instructions: 416 a chunk, 1.1 us (566 and 1.5 us before the state enters its products as it
+// is, the accumulators stay in vector registers and the output's resource is scalar).
+template <int DKS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void delta_state_kernel(RecurParams p) {
+  using I = DeltaItem<DKS>;
+  using R = DeltaRing<DKS, WAVES>;
+  constexpr int CT = DELTA_CT, DT = DKS * 2, VALS = R::VALS, SLOT = R::SLOT, INS = R::INS, LPS = R::LPS, SLOTS = R::SLOTS;
+  typedef __attribute__((address_space(3))) void lds_void;
+  typedef __attribute__((address_space(1))) const void gbl_cvoid;
+  static_assert(LPS * (SLOTS - 2) + 4 * (SLOTS - 1) <= 63, "the wait counter holds 63 loads");
+  // (a dynamic array: with a static one of this size the compiler counts on a single wave per
+  // SIMD and moves the state between accumulation registers and the others, 150 instructions a chunk)
+  extern __shared__ __attribute__((aligned(16))) char ring[];
+  // the column blocks of a head lie p.heads apart: with a multiple of 8 heads in one XCD's L2
+  const int h = blockIdx.x % p.heads, vb = blockIdx.x / p.heads, b = blockIdx.y, D = p.D, V = p.V;
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int r0 = __builtin_amdgcn_readfirstlane(p.s.cu[b]), n = __builtin_amdgcn_readfirstlane(p.s.cu[b + 1]) - r0;
+  const int nc = min(p.chunks, (n + CT - 1) / CT - p.first);
+  if (nc <= 0) return;
+  const int v = (vb * WAVES + w) * 16 + r;
+  float* Sg = p.S + ((long)p.s.slots[b] * p.heads + h) * D * p.Vp;
+  const bool fresh = p.s.start[b] == 0 && p.first == 0;
+  f32x4 S[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = dt * 16 + 4 * g + i;
+      S[dt][i] = !fresh && d < D && v < V ? Sg[d * p.Vp + v] : 0.f;
+    }
+  const long pitch = (long)p.heads * I::BYTES;
+  const char* items = static_cast<const char*>(p.work) + ((long)b * p.chunks * p.heads + h) * I::BYTES;
+  const unsigned at = lane * 16;
+  auto issue = [&](int c) {  // past the end the last chunk again, so that the counts hold
+    const char* it = items + min(c, nc - 1) * pitch;
+    char* slot = ring + (c % SLOTS) * SLOT;
+#pragma unroll
+    for (int q = 0; q < LPS; ++q) {
+      const int k = min(w + q * WAVES, INS - 1);
+      const char* src = it + (k * 1024 + (k * 1024 >= I::FACTORS ? vb * VALS : 0));  // scalar
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(src + at), (lds_void*)(slot + k * 1024), 16, 0, 0);
+    }
+  };
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the state is there before loads are counted
+#pragma unroll
+  for (int c = 0; c < SLOTS; ++c) issue(c);
+  float* raw = p.raw + (long)(r0 + p.first * CT) * p.ldr + (long)h * V;
+  // A wave has its SIMD to itself, so nothing but its own order hides the reads of LDS: what
+  // a chunk's first products need is read under the previous chunk's last ones, the rest under
+  // the first products.
+  bf16x8 kt[DKS][2], qt[DKS][2];
+  auto factors = [&](int c) {
+    const char* f = ring + (c % SLOTS) * SLOT;
+#pragma unroll
+    for (int ks = 0; ks < DKS; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        kt[ks][t] = *reinterpret_cast<const bf16x8*>(f + I::KT + ks * 2048 + t * 1024 + lane * 16);
+        qt[ks][t] = *reinterpret_cast<const bf16x8*>(f + I::QT + ks * 2048 + t * 1024 + lane * 16);
+      }
+  };
+  auto first4 = [](bf16x8 a) { return bf16x4{a[0], a[1], a[2], a[3]}; };
+  constexpr auto vmcnt = [](int k) { return (k & 0xF) | ((k >> 4) << 14) | (0x7 << 4) | (0xF << 8); };
+  __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 1)));  // chunk 0 has landed
+  __builtin_amdgcn_s_barrier();
+  factors(0);
+  for (int c = 0; c < nc; ++c) {
+    const char* f = ring + (c % SLOTS) * SLOT;
+    bf16x8 kf[DT];
+    f32x4 er[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      kf[dt] = *reinterpret_cast<const bf16x8*>(f + I::KH + dt * 1024 + lane * 16);
+      er[dt] = *reinterpret_cast<const f32x4*>(f + I::ER + (dt * 16 + 4 * g) * 4);
+    }
+    const bf16x8 tm = *reinterpret_cast<const bf16x8*>(f + I::TM + lane * 16);
+    const bf16x8 pm = *reinterpret_cast<const bf16x8*>(f + I::PM + lane * 16);
+    const bf16x4 vv = *reinterpret_cast<const bf16x4*>(f + I::FACTORS + w * 512 + lane * 8);
+    __builtin_amdgcn_sched_barrier(0);
+    // four independent sums, so that no product waits for the one before it
+    f32x4 ka = {0.f, 0.f, 0.f, 0.f}, kb = ka, oa = ka, ob = ka;
+#pragma unroll
+    for (int ks = 0; ks < DKS; ++ks) {
+      bf16x8 sh, sl;
+      split8(S[2 * ks], S[2 * ks + 1], sh, sl);
+      ka = mfma16(kt[ks][0], sh, ka);
+      oa = mfma16(qt[ks][0], sh, oa);
+      kb = mfma16(kt[ks][1], sh, kb);
+      ob = mfma16(qt[ks][1], sh, ob);
+      ka = mfma16(kt[ks][0], sl, ka);
+      oa = mfma16(qt[ks][0], sl, oa);
+    }
+    // chunk c is read by everyone, chunk c + 1 has landed: behind its loads are those of
+    // SLOTS - 2 chunks and, once as many chunks have ended, four stores of each
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    if (c >= SLOTS - 1) __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 2) + 4 * (SLOTS - 1)));
+    else __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 2)));
+    __builtin_amdgcn_s_barrier();
+    issue(c + SLOTS);
+    factors(c + 1);  // past the end: chunk nc - 1 again
+    __builtin_amdgcn_sched_barrier(0);
+    // a 16-term product of two-term operands: [a hi | a lo] [b hi | b hi] in one, a hi b lo
+    const f32x4 xv = f32x4{bf2f(vv[0]), bf2f(vv[1]), bf2f(vv[2]), bf2f(vv[3])} - (ka + kb);
+    const bf16x4 xh = hi4(xv), xl = lo4(xv, xh);
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 u = mfma16(tm, cat(xh, xh), z) + mfma16k16(first4(tm), xl, z);
+    const bf16x4 uh = hi4(u), ul = lo4(u, uh);
+    const bf16x8 uu = cat(uh, uh);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) S[dt] = mfma16(kf[dt], uu, S[dt] * er[dt]);
+    oa = mfma16(pm, uu, oa);
+    ob = mfma16k16(first4(pm), ul, ob);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) S[dt] = mfma16k16(first4(kf[dt]), ul, S[dt]);
+    const f32x4 o = oa + ob;
+    // every wave issues four stores (counted above); what is out of range is dropped
+    const int nt = min(CT, n - (p.first + c) * CT);
+    const unsigned long at = reinterpret_cast<unsigned long>(raw + (long)c * CT * p.ldr);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at), hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<float*>((unsigned long)hi << 32 | lo), (short)0,
+        __builtin_amdgcn_readfirstlane(nt * (int)p.ldr * 4), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(o[i]), rs, v < V ? ((4 * g + i) * (int)p.ldr + v) * 4 : -4, 0, 0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // no load may reach LDS that is another block's by then
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d = dt * 16 + 4 * g + i;
+      if (d < D && v < p.Vp) Sg[d * p.Vp + v] = S[dt][i];
+    }
 }
 
 // Chunked Mamba-2 over x [rows][x | B | C] behind convolution and SiLU (bf16).
@@ -1067,6 +1331,31 @@ extern "C" hipError_t lsd_recur_chunk(const RecurParams* p, int delta, const bf1
   }
 #undef LSD_CK_D
 #undef LSD_CK
+  return hipGetLastError();
+}
+
+// Bytes of one (chunk, head) of the delta rule's factors, and the tokens of a chunk.
+extern "C" long lsd_delta_item(int D) {
+  return D <= 32 ? DeltaItem<1>::BYTES : D <= 64 ? DeltaItem<2>::BYTES : DeltaItem<4>::BYTES;
+}
+extern "C" int lsd_delta_chunk() { return DELTA_CT; }
+
+// Chunks first .. first + chunks - 1 of every sequence, their factors through p->work.
+extern "C" hipError_t lsd_delta_split(const RecurParams* p, const bf16* x, long ldx, hipStream_t st) {
+  if (p->s.B == 0 || p->chunks <= 0) return hipSuccess;
+  if (p->D > 128 || p->V > 128 || !p->raw || !p->work) return hipErrorInvalidValue;
+  const dim3 gf(p->heads, p->chunks, p->s.B), gs(p->heads * ((p->V + 16 * DELTA_WAVES - 1) / (16 * DELTA_WAVES)), p->s.B);
+#define LSD_DS(KS)                                                                                          \
+  constexpr int lds = DeltaRing<KS, DELTA_WAVES>::BYTES;                                                     \
+  static const hipError_t room = hipFuncSetAttribute(                                                        \
+      reinterpret_cast<const void*>(&delta_state_kernel<KS, DELTA_WAVES>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+  if (room != hipSuccess) return room;                                                                       \
+  hipLaunchKernelGGL((delta_factors_kernel<KS>), gf, dim3(256), 0, st, *p, x, ldx);                           \
+  hipLaunchKernelGGL((delta_state_kernel<KS, DELTA_WAVES>), gs, dim3(64 * DELTA_WAVES), lds, st, *p);
+  if (p->D <= 32) { LSD_DS(1) }
+  else if (p->D <= 64) { LSD_DS(2) }
+  else { LSD_DS(4) }
+#undef LSD_DS
   return hipGetLastError();
 }
 

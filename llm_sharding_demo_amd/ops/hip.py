@@ -815,7 +815,7 @@ class HipBackend(Backend):
             self.C.delta_seq(y[s], c0, c0 + m.conv_channels, low[s], n, mt.seq_slots, mt.q_start, mt.cu_q, m.heads,
                              m.kv_heads, m.dim, m.vdim, w("mixer.taps"), entry[1], entry[0], w("mixer.A"),
                              w("mixer.dt_bias"), w("mixer.norm"), gain, eps, out[s], mt.is_decode,
-                             self._chunked(mt) and self.C.chunk_ok(True, m.dim, m.vdim, m.kv_heads, m.heads))
+                             self._chunked(mt) and self.C.chunk_ok(True, m.dim, m.vdim, m.kv_heads, m.heads), mt.max_q)
 
     def _chunked(self, meta) -> bool:
         """Prompts of bf16 models run in chunks (very short portions token by token)."""

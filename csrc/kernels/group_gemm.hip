@@ -13,7 +13,8 @@
 //
 // bf16: MFMA 16x16x32, tiles staged HBM -> LDS by 16-byte LDS-DMA into a ring
 // of k-steps (the scheme of gemm_ring in gemm.hip), 4 waves as 2 x 2.
-// fp32: plain VALU tiles with fused multiply-adds, for models served in fp32.
+// fp32, for models served in it: MFMA 16x16x4 on fp32 operands, the same staging; VALU tiles
+// with fused multiply-adds where K has no whole steps of 32 or a row starts off 16 bytes.
 //
 // A few tokens (single-stream decode): weight streaming instead of tiles, one
 // wave per output column and (token, choice), no sorting by expert; the down
@@ -283,7 +284,161 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
   }
 }
 
-// fp32: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
+// fp32: 16 MT x 64 tiles, 32-deep k-steps (128-byte rows, the bf16 kernel's staging and swizzle);
+// wave w owns 16 columns of all rows and leaves out the 16-row tiles that hold none, so an
+// expert's last rows cost what they are.  A lane's 16-byte fragment feeds four MFMA 16x16x4,
+// whose k-slot g stands for k = 4 g + j in both operands.
+// Bound by the matrix cores, whose fp32 rate is a sixteenth of bf16's (154 TF/s), and, where
+// experts have some tens of rows, by their weights.  64 x 128 tiles were no faster.
+// 2260 rows over 32 experts of 2048 x 1024 and 565 through a shared one of 2048 (VALU tiles
+// before): up 631 -> 355 us, down 320 -> 187; 565 x 2048 x 2048 143 -> 65; 4096 x 4096 x 2048
+// at 114 TF/s.
+template <int MODE, int MT>
+__global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kernel(GgParams p) {
+  using namespace gg;
+  constexpr int TM = 16 * MT, TN = 64, BKF = 32, SLOTS = 3;
+  constexpr int A_BYTES = TM * 128, SLOT_BYTES = (TM + TN) * 128, LPS = TM / 32 + TN / 32, CLD = TN + 4;
+  constexpr int SMEM = SLOTS * SLOT_BYTES > TM * CLD * 4 ? SLOTS * SLOT_BYTES : TM * CLD * 4;
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
+  Tile t = locate<MODE, TM, TN>(p);
+  if (!t.live) return;
+  resolve<MODE, float>(p, t);
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
+
+  const float* ap[TM / 32];
+  const float* wp[TN / 32];
+#pragma unroll
+  for (int q = 0; q < TM / 32; ++q) {
+    const int row = (w * (TM / 32) + q) * 8 + (lane >> 3);
+    ap[q] = static_cast<const float*>(t.A) + a_row<MODE>(p, t, row) * t.lda + (((lane & 7) ^ ((row >> 1) & 7)) << 2);
+  }
+#pragma unroll
+  for (int q = 0; q < TN / 32; ++q) {
+    const int row = (w * (TN / 32) + q) * 8 + (lane >> 3);
+    wp[q] = static_cast<const float*>(t.W) + (long)min(t.n0 + row, t.N - 1) * t.ldw + (((lane & 7) ^ ((row >> 1) & 7)) << 2);
+  }
+  auto issue = [&](int kt, int slot) {
+    char* b = smem + slot * SLOT_BYTES;
+#pragma unroll
+    for (int q = 0; q < TM / 32; ++q)
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(ap[q] + (long)kt * BKF), (lds_void*)(b + (w * (TM / 32) + q) * 1024), 16,
+                                       0, 0);
+#pragma unroll
+    for (int q = 0; q < TN / 32; ++q)
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(wp[q] + (long)kt * BKF),
+                                       (lds_void*)(b + A_BYTES + (w * (TN / 32) + q) * 1024), 16, 0, 0);
+  };
+  auto frag = [&](const char* tile, int row, int chunk) {
+    return *reinterpret_cast<const f32x4*>(tile + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4));
+  };
+  f32x4 acc[2][MT];  // halves of the sums: a chain half as long rounds less
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[0][i] = acc[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __builtin_amdgcn_s_waitcnt(vmcnt(0));  // the routing loads are done before loads are counted
+  const int KT = t.K / BKF;
+#pragma unroll
+  for (int d = 0; d < SLOTS; ++d)
+    if (d < KT) issue(d, d);
+  // k-step kt has landed for all waves, whose reads of the one before are done
+  auto landed = [&](int kt) {
+    constexpr int NO_LDS = ~0xf00;  // and no LDS read under way
+    const int later = min(SLOTS - 1 - (kt > 0), KT - 1 - kt);
+    if (later == 2) __builtin_amdgcn_s_waitcnt(vmcnt(2 * LPS) & NO_LDS);
+    else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt(LPS) & NO_LDS);
+    else __builtin_amdgcn_s_waitcnt(vmcnt(0) & NO_LDS);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // L: row tiles that hold rows (a branch per tile would keep the fragments' loads apart).
+  // Half a step's fragments are read while the other half is multiplied
+  auto steps = [&](auto L) {
+    f32x4 wf[2], af[2][L];
+    auto read = [&](int slot, int kk) {
+      const char* ta = smem + slot * SLOT_BYTES;
+      wf[kk] = frag(ta + A_BYTES, w * 16 + r, kk * 4 + g);
+#pragma unroll
+      for (int i = 0; i < L; ++i) af[kk][i] = frag(ta, i * 16 + r, kk * 4 + g);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto products = [&](int kk) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < L; ++i)
+          acc[kk][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[kk][i][e], wf[kk][e], acc[kk][i], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    landed(0);
+    read(0, 0);
+    int slot = 0;
+    for (int kt = 0; kt < KT; ++kt) {
+      read(slot, 1);
+      products(0);
+      const int next = slot == SLOTS - 1 ? 0 : slot + 1;
+      if (kt + 1 < KT) {
+        landed(kt + 1);
+        if (kt + SLOTS < KT) issue(kt + SLOTS, slot);
+        read(next, 0);
+      }
+      products(1);
+      slot = next;
+    }
+  };
+  if constexpr (MT == 4) {
+    if (live == 4) steps(std::integral_constant<int, 4>{});
+    else if (live == 3) steps(std::integral_constant<int, 3>{});
+  }
+  if (live == 2) steps(std::integral_constant<int, 2>{});
+  else if (live == 1) steps(std::integral_constant<int, 1>{});
+  __syncthreads();
+  float* ct = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ct[(i * 16 + 4 * g + q) * CLD + w * 16 + r] = acc[0][i][q] + acc[1][i][q];
+  __syncthreads();
+  constexpr int CPR = TN / 4;
+  for (int c = threadIdx.x; c < min(TM, t.rows) * CPR; c += 256) {
+    const int row = c / CPR, ch = (c % CPR) * 4, n = t.n0 + ch, m = t.row0 + row;
+    if (n >= t.N) continue;
+    const float* src = ct + row * CLD + ch;
+    f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    if constexpr (MODE == GG_UP) {  // gate and up rows in 16-row blocks; N % 32 == 0
+      if (ch & 16) continue;
+      const f32x4 u = *reinterpret_cast<const f32x4*>(src + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = glu_exact(v[e], u[e], t.limit, p.alpha, p.up_one);
+      *reinterpret_cast<f32x4*>(static_cast<float*>(t.out) + (long)m * t.ldo + (n >> 5) * 16 + (n & 15)) = v;
+      continue;
+    }
+    long orow = m;
+    float wt = 1.f;
+    if constexpr (MODE == GG_DOWN) {
+      if (t.routed) {
+        const int ent = p.perm[m];
+        wt = p.wts[ent];
+        orow = (long)(ent % p.top) * p.T + ent / p.top;
+      } else if (p.wts_s) {
+        wt = p.wts_s[m];
+      }
+    }
+    float* o = static_cast<float*>(t.out) + orow * t.ldo + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // single stores: rows of any width
+      if (n + e >= t.N) break;
+      if constexpr (MODE == GG_DOWN) o[e] = v[e] * wt;
+      else if constexpr (MODE == GG_ADD) o[e] += v[e];
+      else if constexpr (MODE == GG_F32) {
+        const float gt = p.gate ? 1.f / (1.f + expf(-p.gate[m * p.ldg + t.group * p.o_gs + n + e])) : 1.f;
+        o[e] = (v[e] + (p.bias ? p.bias[n + e] : 0.f)) * gt;
+      }
+      else o[e] = v[e];
+    }
+  }
+}
+
+// Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
 template <int MODE>
 __global__ __launch_bounds__(256) void group_gemm_f32_kernel(GgParams p) {
   using namespace gg;
@@ -490,21 +645,40 @@ extern "C" hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStr
   }
 }
 
+template <int MODE, int MT>
+static hipError_t gg_f32_on(const GgParams& p, hipStream_t st) {
+  const long blocks = gg_blocks(p, MODE, 16 * MT, 64);
+  if (blocks) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+template <int MODE>
+static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
+  // the tiles' loads take whole 16 bytes and k-steps of 32
+  auto at = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
+  if (p.K % 32 || (p.Ns > 0 && p.Ks % 32) || (at(p.A) | at(p.W) | at(p.As) | at(p.Ws)) % 16) {
+    const long blocks = gg_blocks(p, MODE, 64, 64);
+    if (blocks) hipLaunchKernelGGL((group_gemm_f32_kernel<MODE>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+    return hipGetLastError();
+  }
+  if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
+    // half tiles where the fullest CU gets less work of them (N = K = 2048: 565 rows 67 against
+    // 80 us, 200 rows 32 against 46); at the same work the whole ones (1000 rows 84 against 91)
+    auto rounds = [&](int tm) { return (gg_blocks(p, MODE, tm, 64) + 255) / 256; };
+    if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, st);
+  }
+  return gg_f32_on<MODE, 4>(p, st);
+}
+
 // fp32 kernels: 64-row tiles
 extern "C" hipError_t lsd_group_gemm_f32(const GgParams* p, int mode, hipStream_t st) {
-  const dim3 grid((unsigned)gg_blocks(*p, mode, 64, 64));
-  if (grid.x == 0) return hipSuccess;
-#define LSD_GG_F32(MODE) \
-  case MODE: hipLaunchKernelGGL((group_gemm_f32_kernel<MODE>), grid, dim3(256), 0, st, *p); break;
   switch (mode) {
-    LSD_GG_F32(GG_UP)
-    LSD_GG_F32(GG_DOWN)
-    LSD_GG_F32(GG_F32)
-    LSD_GG_F32(GG_ADD)
+    case GG_UP: return gg_f32<GG_UP>(*p, st);
+    case GG_DOWN: return gg_f32<GG_DOWN>(*p, st);
+    case GG_F32: return gg_f32<GG_F32>(*p, st);
+    case GG_ADD: return gg_f32<GG_ADD>(*p, st);
     default: return hipErrorInvalidValue;
   }
-#undef LSD_GG_F32
-  return hipGetLastError();
 }
 
 // up: K input columns, F / Fs gated columns; down: K residual columns

@@ -1,0 +1,60 @@
+"""fp32 products and latent attention on matrix tiles against 64 bits.
+
+A sum of K products in fp32 is off by at most (K + 2) ulp of the sum of the
+products' sizes, in any order (ulp: 2^-24).
+"""
+
+import pytest
+import torch
+
+from . import timisun_oracle as orc
+from .test_timisun_gpu import C, latent_tokens, paged, rand  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+DEV, F64, ULP = "cuda:0", torch.float64, 2.0 ** -24
+
+
+@pytest.mark.parametrize("K", [16, 32, 48, 64, 96, 128, 160])
+@pytest.mark.parametrize("M,N", [(1, 1), (1, 65), (15, 64), (16, 63), (17, 130), (64, 3), (65, 129), (200, 32),
+                                 (1000, 4097), (513, 8100)])
+def test_linear_fp32_edges(C, M, N, K):  # noqa: F811
+    a, w, x, b = rand(M, K, seed=1), rand(N, K, seed=2), rand(M, N, seed=3), rand(N, seed=4)
+    want, size = a.to(F64) @ w.to(F64).T, a.to(F64).abs() @ w.to(F64).abs().T
+    got = C.linear_fp32(a.to(DEV), w.to(DEV), None, b.to(DEV)).cpu().to(F64)
+    assert bool(((got - want - b.to(F64)).abs() <= (K + 3) * ULP * (size + b.abs())).all())
+    if N % 4 == 0:
+        xd = x.to(DEV)
+        C.linear_fp32(a.to(DEV), w.to(DEV), xd)
+        assert bool(((xd.cpu().to(F64) - want - x.to(F64)).abs() <= (K + 3) * ULP * (size + x.abs())).all())
+
+
+def test_weights_off_16_bytes(C):  # noqa: F811
+    a, w = rand(70, 64, seed=1), rand(1, 80, 64, seed=2)
+    dev = torch.empty(80 * 64 + 1, device=DEV)[1:].view(1, 80, 64)
+    dev.copy_(w)
+    assert dev.data_ptr() % 16 == 4
+    want, size = a.to(F64) @ w[0].to(F64).T, a.to(F64).abs() @ w[0].to(F64).abs().T
+    for x in (w.to(DEV), dev):
+        got = C.batch_linear(a.to(DEV), x, 64).cpu().to(F64)
+        assert bool(((got - want).abs() <= 66 * ULP * size).all())
+
+
+@pytest.mark.parametrize("H", [1, 15, 16, 33])
+@pytest.mark.parametrize("rank,value", [(64, 64), (128, 40), (192, 192), (512, 448), (576, 512)])
+def test_latent_values_and_sinks_fp32(C, rank, value, H):  # noqa: F811
+    """Heads off the 16-head tile, fewer value than key columns, sinks; a stale
+    row behind the last key that is not a number."""
+    n, W, scale = 70, 45, rank ** -0.5
+    c, q, sink = rand(n, rank, seed=1), rand(n, H, rank, seed=2), rand(H, seed=3)
+    pool, table = paged(torch.cat([c, torch.full((1, rank), float("nan"))]), torch.float32, rank)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    cols = rank - 64 if value <= rank - 64 else rank
+    got = C.latent_decode(q.reshape(n, -1).to(DEV), pool, table, torch.ones(n, **i32), torch.arange(n, **i32), H, W,
+                          scale, 1, value, sink.to(DEV)).reshape(n, H, cols).cpu().to(F64)
+    s = torch.einsum("thr,kr->thk", q.to(F64), c.to(F64)) * scale
+    seen = torch.tensor([[orc.visible(p, k, W) for k in range(n)] for p in range(n)])
+    s = torch.cat([s.masked_fill(~seen[:, None], float("-inf")), sink.to(F64).expand(n, H)[..., None]], -1)
+    p = torch.softmax(s, -1)[..., :-1]
+    # a score is off by 4 ulp of its products' sizes at most (their roundings are
+    # independent: sqrt(rank) of the worst case), which weights share relatively
+    assert float((got - p @ c[:, :cols].to(F64)).pow(2).mean().sqrt()) < 2e-6

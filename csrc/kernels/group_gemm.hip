@@ -12,7 +12,11 @@
 //    of latent attention (attention_latent.hip).
 //
 // bf16: MFMA 16x16x32, tiles staged HBM -> LDS by 16-byte LDS-DMA into a ring
-// of k-steps (the scheme of gemm_ring in gemm.hip), 4 waves as 2 x 2.
+// of k-steps (the scheme of gemm_ring in gemm.hip), 4 waves as 2 x 2.  Decode is bound by the
+// stream of the experts' weights, prompts by the matrix cores; both lose what a block waits
+// before its first loads, so W starts without the routing, and the routing weights of a down
+// tile arrive under its products.  32 experts of 2048 x 1024 and a shared one of 2048, 4 a
+// token: 64 tokens up 58 -> 46 us (6.1 TB/s), down 37 -> 33; 16000 tokens down 587 -> 504.
 // fp32, for models served in it: MFMA 16x16x4 on fp32 operands, the same staging; VALU tiles
 // with fused multiply-adds where K has no whole steps of 32 or a row starts off 16 bytes.
 //
@@ -29,6 +33,16 @@ constexpr int BK = 64;
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void gbl_cvoid;
 constexpr int vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
+
+template <int V>
+struct Int {
+  static constexpr int v = V;
+};
+template <int N, class F>
+__device__ __forceinline__ void count_down(F f) {  // f(N - 1) .. f(0), compile-time
+  f(Int<N - 1>{});
+  if constexpr (N > 1) count_down<N - 1>(f);
+}
 
 // Where one row tile's operands are.
 struct Tile {
@@ -130,13 +144,13 @@ __device__ __forceinline__ float sigmoid_fast(float z) {
 }
 }  // namespace gg
 
-template <int MODE, int TM, int TN, int SLOTS>
+template <int MODE, int TM, int TN, int SLOTS, int AUX = 0>
 __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
   using namespace gg;
   constexpr int MI = TM / 32, JT = TN / 32;  // 16 x 16 tiles per wave (2 x 2 waves)
   constexpr int A_BYTES = TM * BK * 2, SLOT_BYTES = (TM + TN) * BK * 2;
   constexpr int LPS = TM / 32 + TN / 32;     // LDS-DMA instructions per thread per k-step
-  constexpr int D = SLOTS - 1;
+  constexpr int LPA = TM / 32, D = SLOTS - 1;
   constexpr int CLD = TN + 4;
   constexpr int SMEM = SLOTS * SLOT_BYTES > TM * CLD * 4 ? SLOTS * SLOT_BYTES : TM * CLD * 4;
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
@@ -149,71 +163,72 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
   const int lane = lane_id(), w = threadIdx.x >> 6;
   const int wm = w >> 1, wn = w & 1, r = lane & 15, g = lane >> 4;
 
-  // per-lane source addresses of this wave's LDS-DMA rows (16-byte chunks
-  // XOR-swizzled on the source side, as in gemm.hip stage_tile)
+  // The ring is filled as early as each operand's addresses are known: W first, A behind the
+  // row numbers it is gathered by.  Loads into registers between them only make the counted
+  // waits below wait for more.
+  const int KT = t.K / BK;
+// Few rows: each column tile starts its sums at another k (512 bytes on), so that the blocks
+  // under way do not all stand at the same place of rows that lie powers of two apart
+  const int rot = MODE == GG_UP && TM == 32 ? t.n0 / TN * 4 % KT : 0;
+  auto at_k = [&](int kt) { return (kt + rot >= KT ? kt + rot - KT : kt + rot) * BK; };
   const bf16* ap[TM / 32];
   const bf16* wp[TN / 32];
+  long arow[TM / 32];
 #pragma unroll
-  for (int q = 0; q < TM / 32; ++q) {
-    const int row = (w * (TM / 32) + q) * 8 + (lane >> 3);
-    ap[q] = static_cast<const bf16*>(t.A) + a_row<MODE>(p, t, row) * t.lda + (((lane & 7) ^ ((row >> 1) & 7)) << 3);
+  for (int q = 0; q < TM / 32; ++q) arow[q] = a_row<MODE>(p, t, (w * (TM / 32) + q) * 8 + (lane >> 3));
+  int ent = 0;  // GG_DOWN: the tile's row threadIdx.x
+  if constexpr (MODE == GG_DOWN) {
+    ent = t.row0 + min((int)threadIdx.x % TM, t.rows - 1);
+    if (t.routed) ent = p.perm[ent];
   }
+  // per-lane source addresses of this wave's LDS-DMA rows (16-byte chunks
+  // XOR-swizzled on the source side, as in gemm.hip stage_tile)
 #pragma unroll
   for (int q = 0; q < TN / 32; ++q) {
     const int row = (w * (TN / 32) + q) * 8 + (lane >> 3);
     wp[q] = static_cast<const bf16*>(t.W) + (long)min(t.n0 + row, t.N - 1) * t.ldw +
             (((lane & 7) ^ ((row >> 1) & 7)) << 3);
   }
-  auto issue = [&](int kt, int slot) {
+  auto issue_w = [&](int kt, int slot) {
+    char* b = smem + slot * SLOT_BYTES;
+#pragma unroll
+    for (int q = 0; q < TN / 32; ++q)
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(wp[q] + at_k(kt)),
+                                       (lds_void*)(b + A_BYTES + (w * (TN / 32) + q) * 1024), 16, 0, AUX);
+  };
+  auto issue_a = [&](int kt, int slot) {
     char* b = smem + slot * SLOT_BYTES;
 #pragma unroll
     for (int q = 0; q < TM / 32; ++q)
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(ap[q] + kt * BK), (lds_void*)(b + (w * (TM / 32) + q) * 1024), 16,
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(ap[q] + at_k(kt)), (lds_void*)(b + (w * (TM / 32) + q) * 1024), 16,
                                        0, 0);
-#pragma unroll
-    for (int q = 0; q < TN / 32; ++q)
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(wp[q] + kt * BK),
-                                       (lds_void*)(b + A_BYTES + (w * (TN / 32) + q) * 1024), 16, 0, 0);
   };
   auto frag = [&](const char* tile, int row, int chunk) {
     return *reinterpret_cast<const bf16x8*>(tile + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4));
   };
-
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < KT) issue_w(d, d);
+#pragma unroll
+  for (int q = 0; q < TM / 32; ++q) {
+    const int row = (w * (TM / 32) + q) * 8 + (lane >> 3);
+    ap[q] = static_cast<const bf16*>(t.A) + arow[q] * t.lda + (((lane & 7) ^ ((row >> 1) & 7)) << 3);
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < KT) issue_a(d, d);
+  float wt_row = 1.f;
   if constexpr (MODE == GG_DOWN) {
-    if (threadIdx.x < TM) {
-      const int m = t.row0 + min((int)threadIdx.x, t.rows - 1);
-      int row = m;
-      float wt = 1.f;
-      if (t.routed) {
-        const int ent = p.perm[m];
-        wt = p.wts[ent];
-        row = (ent % p.top) * p.T + ent / p.top;  // < top * T, checked on the host to fit
-      } else if (p.wts_s) {
-        wt = p.wts_s[m];
-      }
-      s_row[threadIdx.x] = row;
-      s_wt[threadIdx.x] = wt;
-    }
+    if (t.routed) wt_row = p.wts[ent];
+    else if (p.wts_s) wt_row = p.wts_s[ent];
   }
   f32x4 acc[MI][JT];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < JT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // the routing loads above are done before the counted waits start
-  __builtin_amdgcn_s_waitcnt(vmcnt(0));
-  const int KT = t.K / BK;
-#pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (d < KT) issue(d, d);
-  int slot = 0;
-  for (int kt = 0; kt < KT; ++kt) {
-    const int later = min(D - 1, KT - 1 - kt);  // k-steps after kt already issued
-    if (later >= 2) __builtin_amdgcn_s_waitcnt(vmcnt(2 * LPS));
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt(LPS));
-    else __builtin_amdgcn_s_waitcnt(vmcnt(0));
-    __builtin_amdgcn_s_barrier();
-    if (kt + D < KT) issue(kt + D, slot == 0 ? SLOTS - 1 : slot - 1);
+  int slot = 0, kt = 0;
+  auto step = [&]() {
     const char* ta = smem + slot * SLOT_BYTES;
     const char* tw = ta + A_BYTES;
 #pragma unroll
@@ -229,6 +244,49 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
         for (int j = 0; j < JT; ++j) acc[i][j] = mfma16(af[i], wf[j], acc[i][j]);
     }
     slot = slot == SLOTS - 1 ? 0 : slot + 1;
+  };
+  auto turn = [&](bool more) {
+    __builtin_amdgcn_s_barrier();  // every wave's part of k-step kt has landed; step kt - 1 is read
+    if (more) {
+      issue_a(kt + D, slot == 0 ? SLOTS - 1 : slot - 1);
+      issue_w(kt + D, slot == 0 ? SLOTS - 1 : slot - 1);
+    }
+    step();
+    ++kt;
+  };
+  if constexpr (D == 1) {
+    while (kt < KT) {
+      __builtin_amdgcn_s_waitcnt(vmcnt(0));
+      turn(kt + 1 < KT);
+    }
+  } else {
+    // The first waits: behind A of k-step kt are A of the filled steps after it and all of the
+    // steps issued since
+    count_down<D - 1>([&](auto ic) {
+      constexpr int d = decltype(ic)::v + 1;  // filled steps after kt
+      if (kt + D < KT) {
+        __builtin_amdgcn_s_waitcnt(vmcnt(LPA * d + LPS * (D - 1 - d)));
+        turn(true);
+      }
+    });
+    while (kt + D < KT) {
+      __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (D - 1)));
+      turn(true);
+    }
+    count_down<D>([&](auto ic) {  // the last D steps, nothing left to issue
+      constexpr int d = decltype(ic)::v;
+      if (KT - 1 - kt == d) {
+        if (KT >= 2 * D) __builtin_amdgcn_s_waitcnt(vmcnt(LPS * d));
+        else __builtin_amdgcn_s_waitcnt(vmcnt(LPA * d));  // filled ones: A alone is behind
+        turn(false);
+      }
+    });
+  }
+  if constexpr (MODE == GG_DOWN) {
+    if (threadIdx.x < TM) {
+      s_row[threadIdx.x] = t.routed ? (ent % p.top) * p.T + ent / p.top : ent;  // < top * T, checked on the host to fit
+      s_wt[threadIdx.x] = wt_row;
+    }
   }
   __syncthreads();
 
@@ -621,18 +679,23 @@ static long gg_blocks(const GgParams& p, int mode, int tm, int tn) {
   return (long)((p.M + tm - 1) / tm) * ((p.N + tn - 1) / tn) * p.groups;
 }
 
+template <int MODE, int TM, int TN, int SLOTS, int AUX = 0>
+static hipError_t gg_on(const GgParams& p, hipStream_t st) {
+  const long blocks = gg_blocks(p, MODE, TM, TN);
+  if (blocks) hipLaunchKernelGGL((group_gemm_kernel<MODE, TM, TN, SLOTS, AUX>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
 template <int MODE>
 static hipError_t gg_launch(const GgParams& p, int tm, hipStream_t st) {
-  const int tn = tm == 32 ? 64 : 128;
-  const dim3 grid((unsigned)gg_blocks(p, MODE, tm, tn));
-  if (grid.x == 0) return hipSuccess;
   switch (tm) {
-    case 32: hipLaunchKernelGGL((group_gemm_kernel<MODE, 32, 64, 4>), grid, dim3(256), 0, st, p); break;
-    case 64: hipLaunchKernelGGL((group_gemm_kernel<MODE, 64, 128, 3>), grid, dim3(256), 0, st, p); break;
-    case 128: hipLaunchKernelGGL((group_gemm_kernel<MODE, 128, 128, 2>), grid, dim3(256), 0, st, p); break;
+    // decode: the experts' weights pass once, so non-temporally (2048 x 2048 up, 64 tokens of 4
+    // in 32 experts 54 -> 49 us); the heads' do for every row tile
+    case 32: return gg_on<MODE, 32, 64, 4, MODE == GG_BATCH ? 0 : 2>(p, st);
+    case 64: return gg_on<MODE, 64, 128, 3>(p, st);
+    case 128: return gg_on<MODE, 128, 128, 2>(p, st);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 // tm: row-tile rows (32 / 64 / 128; the expert modes' table must use the same)

@@ -55,7 +55,7 @@ hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* 
                            float* part_o, float* part_ml, int B, int nh, int n_kv, int hd,
                            int max_seq, int splits, float scale_log2, hipStream_t st);
 hipError_t lsd_attn_prefill(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
-                            const int* tiles, int n_tiles, const int* seq_slots,
+                            const int* tiles, int n_tiles, int rows, const int* seq_slots,
                             const int* q_start, const int* cu_q, bf16* out, long ldo, int nh,
                             int n_kv, int hd, int max_seq, float scale_log2, hipStream_t st);
 hipError_t lsd_attn_oproj(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
@@ -611,13 +611,14 @@ void attn_oproj(torch::Tensor q, torch::Tensor kc, torch::Tensor vc, torch::Tens
 
 torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
                            torch::Tensor tiles, torch::Tensor seq_slots, torch::Tensor q_start,
-                           torch::Tensor cu_q, int64_t nh) {
+                           torch::Tensor cu_q, int64_t nh, int64_t rows) {
   need(q, torch::kBFloat16, "q");
   need_rows(q, "q");
   check_cache(kc, vc);
   const int n_kv = kc.size(1), hd = kc.size(3);
   TORCH_CHECK(q.size(1) == nh * hd && nh % n_kv == 0, "q must be [T, nh*hd]");
   TORCH_CHECK(hd == 64 || hd == 128, "head_dim must be 64 or 128");
+  TORCH_CHECK(rows == 64 || rows == 128, "query tiles of 64 or 128");
   need(tiles, torch::kInt32, "tiles");
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 2 && tiles.is_contiguous(), "tiles [n, 2]");
   need(seq_slots, torch::kInt32, "seq_slots");
@@ -627,7 +628,7 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   auto out = torch::empty_like(q);
   const float sl2 = 1.4426950408889634f / std::sqrt((float)hd);
   check_hip(lsd_attn_prefill(bptr(q), q.stride(0), bptr(kc), bptr(vc), tiles.data_ptr<int>(),
-                             tiles.size(0), seq_slots.data_ptr<int>(), q_start.data_ptr<int>(),
+                             tiles.size(0), (int)rows, seq_slots.data_ptr<int>(), q_start.data_ptr<int>(),
                              cu_q.data_ptr<int>(), bptr_mut(out), out.stride(0), nh, n_kv, hd,
                              kc.size(2), sl2, cur_stream()), "attn_prefill");
   return out;
@@ -790,7 +791,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm", &norm, py::arg("x"), py::arg("slab"), py::arg("pbias"), py::arg("w"), py::arg("b"), py::arg("eps"),
         py::arg("rms"), py::arg("rows"), py::arg("want_out"), py::arg("width") = 0, py::arg("woff") = 0.0);
   m.def("attn_decode", &attn_decode);
-  m.def("attn_prefill", &attn_prefill);
+  m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("tiles"),
+        py::arg("seq_slots"), py::arg("q_start"), py::arg("cu_q"), py::arg("nh"), py::arg("rows") = 64);
   m.def("attn_oproj", &attn_oproj);
   m.def("sample", &sample, py::arg("logits"), py::arg("V"), py::arg("temp"), py::arg("topk"),
         py::arg("greedy"), py::arg("seeds"), py::arg("step"), py::arg("segmax") = py::none());

@@ -796,6 +796,12 @@ class HipBackend(Backend):
         qt = 2 if self._query_tiles(meta, 128, device).shape[0] * heads >= self.R.paged_tile_min else 1
         return self._query_tiles(meta, 64 * qt, device), qt
 
+    def _plain_tiles(self, meta, heads: int, device):
+        """Query tiles of the prompt kernel and their queries."""
+        blocks = heads * sum(-(-n // 128) for n in meta.host_qlens)
+        rows = 128 if blocks >= self.R.attn_tile_min else 64
+        return self._query_tiles(meta, rows, device), rows
+
     @staticmethod
     def _query_tiles(meta, rows: int, device):
         """(sequence, first query) of every `rows`-query tile, kept on the batch."""
@@ -927,7 +933,7 @@ class HipBackend(Backend):
                 self._query_tiles(meta, rows, meta.cu_q.device)
             return
         if not mcfg.layers:
-            meta._tiles = prefill_tiles(meta).to(meta.cu_q.device)
+            self._plain_tiles(meta, mcfg.n_heads, meta.cu_q.device)
             return
         for heads in {l.mixer.heads for l in mcfg.layers if isinstance(l.mixer, LatentAttentionSpec)}:
             self._latent_tiles(meta, heads, 128, meta.cu_q.device)
@@ -1121,12 +1127,9 @@ class HipBackend(Backend):
         if meta.is_decode:
             splits = self.decode_attn_splits(meta.num_seqs, nh, n_kv, hd, meta.max_ctx)
             return self.C.attn_decode(q, cache_k, cache_v, meta.seq_slots, meta.token_pos, nh, splits)
-        tiles = getattr(meta, "_tiles", None)
-        if tiles is None:
-            tiles = prefill_tiles(meta).to(q.device)
-            meta._tiles = tiles
+        tiles, rows = self._plain_tiles(meta, nh, q.device)
         return self.C.attn_prefill(q, cache_k, cache_v, tiles, meta.seq_slots, meta.q_start,
-                                   meta.cu_q, nh)
+                                   meta.cu_q, nh, rows)
 
     def linear(self, a, w, b=None, act: str = "none", out=None, scale: float = 1.0):
         """act(a w^T + b) in bf16; out: the caller's rows; scale: common factor

@@ -141,6 +141,9 @@ class Routing:
     talk_target: int = 512
     # ... and prompt attention with few query tiles
     talk_prefill_target: int = 512
+    # prompt attention: query tiles of 128 (else 64) from attn_tile_min blocks (32 heads
+    # of 128: 2000 tokens, 512 blocks, 56 against 60 us; 500 tokens, 128 blocks, 15 against 12)
+    attn_tile_min: int = 512
     # attention over paged heads without mixing: query tiles of 128 (else 64) from
     # paged_tile_min blocks; decode waves a launch aims for, at least paged_split_keys
     # keys each

@@ -426,13 +426,14 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(const float* pa
 //  * K and V go to LDS by DMA, a tile ahead in the other of two buffers; their 16-byte chunks
 //    are permuted within a row so that both the row reads of K and the transposing reads
 //    of V, 8 rows by 32 bytes at a time, meet every bank once.
-//  * weights are taken relative to m, which follows the running maximum only when that is
-//    more than 2^6 ahead, so sums are rarely rescaled; only tiles on the diagonal are masked.
+//  * sums are rescaled only where a query's maximum moved, and only tiles on the diagonal are
+//    masked.  (A maximum that lags by up to 2^6 saves 3 % more, but the largest weight is
+//    then not exactly one: the error against 64 bits grows by as much.)
 //  * a kv head's blocks run side by side on one XCD, whose L2 then holds its keys, and the
 //    longest first: the last ones to end are short.
 // Before (one 16-query tile per wave, K and V through registers) -> now:
-//   32 heads over 8 of 128: 7937 tokens 1290 -> 555 us (931 TF/s), 8 x 500 80 -> 40, 500 17 -> 12
-//   25 heads of 64: 4 x 1000 tokens 72 -> 38 us, 20 x 200 27 -> 19
+//   32 heads over 8 of 128: 7937 tokens 1290 -> 570 us (900 TF/s), 8 x 500 80 -> 42, 500 16 -> 12
+//   25 heads of 64: 4 x 1000 tokens 72 -> 41 us, 20 x 200 27 -> 19
 typedef short short4v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x4 ds_read_tr(const bf16* lds_ptr) {
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
       tmax *= scale_log2;
       tmax = fmaxf(tmax, wave_xchg<16>(tmax));
       tmax = fmaxf(tmax, wave_xchg<32>(tmax));
-      if (__any(tmax > m[t] + 6.f)) {
+      if (__any(tmax > m[t])) {
         const float mn = fmaxf(m[t], tmax);
         const float alpha = __builtin_amdgcn_exp2f(m[t] - mn);
         m[t] = mn;

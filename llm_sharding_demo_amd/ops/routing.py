@@ -142,7 +142,7 @@ class Routing:
     # ... and prompt attention with few query tiles
     talk_prefill_target: int = 512
     # prompt attention: query tiles of 128 (else 64) from attn_tile_min blocks (32 heads
-    # of 128: 2000 tokens, 512 blocks, 56 against 60 us; 500 tokens, 128 blocks, 15 against 12)
+    # of 128: 2000 tokens, 512 blocks, 58 against 62 us; 500 tokens, 128 blocks, 16 against 12)
     attn_tile_min: int = 512
     # attention over paged heads without mixing: query tiles of 128 (else 64) from
     # paged_tile_min blocks; decode waves a launch aims for, at least paged_split_keys

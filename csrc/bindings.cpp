@@ -50,6 +50,7 @@ hipError_t lsd_embed(const int* ids, const int* pos, const bf16* wte, const bf16
 hipError_t lsd_norm(float* x, const void* slab, int slab_bf16, int splits, const bf16* pbias, const bf16* w,
                     const bf16* b, bf16* out, int T, int H, float eps, int rms, const int* rows,
                     int nrows, int Hn, float woff, hipStream_t st);
+int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits);
 hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                            const int* seq_slots, const int* qpos, bf16* out, long ldo,
                            float* part_o, float* part_ml, int B, int nh, int n_kv, int hd,
@@ -559,9 +560,10 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   torch::Tensor po, pml;
   float* pop = nullptr;
   float* pmlp = nullptr;
-  if (splits > 1) {
-    po = torch::empty({B, nh, splits, hd}, q.options().dtype(torch::kFloat32));
-    pml = torch::empty({B, nh, splits, 2}, q.options().dtype(torch::kFloat32));
+  const int64_t parts = splits * lsd_attn_decode_split(B, n_kv, (int)(nh / n_kv), hd, (int)splits);
+  if (parts > 1) {
+    po = torch::empty({B, nh, parts, hd}, q.options().dtype(torch::kFloat32));
+    pml = torch::empty({B, nh, parts, 2}, q.options().dtype(torch::kFloat32));
     pop = po.data_ptr<float>();
     pmlp = pml.data_ptr<float>();
   }

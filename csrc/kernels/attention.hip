@@ -396,24 +396,57 @@ __global__ __launch_bounds__(NWV * 64) void attn_oproj_kernel(
   }
 }
 
-// Merge split-K decode partials: one block per (sequence, head).
+// Merge split-K decode partials: one wave per (sequence, head).  What it costs is the round
+// trips to memory: the partials of 16 splits are requested together with all maxima and sums,
+// not split by split behind them (1 sequence, 16 splits, with the kernel in front: 17.8 -> 6.9 us).
 template <int HD>
 __global__ __launch_bounds__(64) void attn_decode_combine_kernel(const float* part_o,
                                                                  const float* part_ml, bf16* out,
                                                                  long ldo, int nh, int splits) {
-  const int b = blockIdx.x / nh, h = blockIdx.x % nh;
+  constexpr int DPL = HD / 64, AT_ONCE = 16, MAXL = 256 / 64;  // columns per lane; splits <= 256
+  __shared__ float ws[256];
+  const int b = blockIdx.x / nh, h = blockIdx.x % nh, lane = threadIdx.x;
   const long p0 = ((long)b * nh + h) * splits;
-  float mm = NEG;
-  for (int s = 0; s < splits; ++s) mm = fmaxf(mm, part_ml[(p0 + s) * 2]);
-  for (int d = threadIdx.x; d < HD; d += 64) {
-    float ll = 0.f, oo = 0.f;
-    for (int s = 0; s < splits; ++s) {
-      const float f = exp2f(part_ml[(p0 + s) * 2] - mm);
-      ll += part_ml[(p0 + s) * 2 + 1] * f;
-      oo += part_o[(p0 + s) * HD + d] * f;
-    }
-    out[(long)b * ldo + (long)h * HD + d] = f2bf(ll > 0.f ? oo / ll : 0.f);
+  const float* po = part_o + p0 * HD + lane * DPL;
+  float v[AT_ONCE][DPL];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i)
+#pragma unroll
+      for (int d = 0; d < DPL; ++d) v[i][d] = po[(long)min(s0 + i, splits - 1) * HD + d];
+  };
+  float m[MAXL], l[MAXL];
+#pragma unroll
+  for (int i = 0; i < MAXL; ++i) {
+    const int s = min(lane + i * 64, splits - 1);
+    m[i] = part_ml[(p0 + s) * 2];
+    l[i] = lane + i * 64 < splits ? part_ml[(p0 + s) * 2 + 1] : 0.f;
   }
+  load(0);
+  float mm = m[0];
+#pragma unroll
+  for (int i = 1; i < MAXL; ++i) mm = fmaxf(mm, m[i]);
+  mm = wave_max(mm);
+  float ll = 0.f;
+#pragma unroll
+  for (int i = 0; i < MAXL; ++i) {
+    const float f = exp2f(m[i] - mm);
+    ll += l[i] * f;
+    ws[lane + i * 64] = lane + i * 64 < splits ? f : 0.f;
+  }
+  ll = wave_sum(ll);
+  __syncthreads();
+  float oo[DPL] = {};
+  for (int s0 = 0; s0 < splits; s0 += AT_ONCE) {
+    if (s0) load(s0);
+#pragma unroll
+    for (int i = 0; i < AT_ONCE; ++i)
+#pragma unroll
+      for (int d = 0; d < DPL; ++d) oo[d] += v[i][d] * (s0 + i < splits ? ws[s0 + i] : 0.f);
+  }
+#pragma unroll
+  for (int d = 0; d < DPL; ++d)
+    out[(long)b * ldo + (long)h * HD + lane * DPL + d] = f2bf(ll > 0.f ? oo[d] / ll : 0.f);
 }
 
 // ---------------------------------------------------------------------------
@@ -611,8 +644,11 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
 // then staged through this wave's own LDS region for the fragment reads.
 // Waves are independent: no block barrier.  The math is ~2% of the HBM time
 // of the KV stream, so the kernel runs at the KV roofline.
-template <int HD, int G>
-__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
+//
+// NW waves per block.  SPLIT_P: the weights enter the second product as two bf16 terms (value,
+// remainder), for the calls whose weights the VALU kernel would hold in fp32.
+template <int HD, int G, int NW, bool SPLIT_P>
+__global__ __launch_bounds__(NW * 64) void attn_decode_mfma_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
     const int* __restrict__ seq_slots, const int* __restrict__ qpos, bf16* out, long ldo,
     float* part_o, float* part_ml, int n_kv, int max_seq, int splits, float scale_log2,
@@ -622,9 +658,9 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   constexpr int LDR = HD + 8;        // padded LDS row (elements): +16 B
   constexpr int CPR = HD / 8;        // 16-B chunks per key row
   constexpr int CH = KT * CPR / 64;  // chunks per lane per tile (per K and per V)
-  __shared__ __attribute__((aligned(16))) bf16 lds[4][2][KT * LDR];
+  __shared__ __attribute__((aligned(16))) bf16 lds[NW][2][KT * LDR];
   const int lane = lane_id(), w = threadIdx.x >> 6;
-  const int item = blockIdx.x * 4 + w;
+  const int item = blockIdx.x * NW + w;
   if (item >= n_items) return;  // waves are independent: no barriers below
   bf16* ks = lds[w][0];
   bf16* vs = lds[w][1];
@@ -713,11 +749,12 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     for (int di = 0; di < HD / 16; ++di) o[di] *= alpha;
     // O^T += V^T . P^T over the 32 keys: k-slot j of group g <-> key 4g + j
     // (j < 4), 16 + 4g + (j - 4) (j >= 4)
-    bf16x8 pf;
+    bf16x8 pf, pl;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      pf[j] = f2bf(sacc[0][j]);
-      pf[4 + j] = f2bf(sacc[1][j]);
+    for (int j = 0; j < 8; ++j) {
+      const float e = sacc[j >> 2][j & 3];
+      pf[j] = f2bf(e);
+      pl[j] = f2bf(e - bf2f(pf[j]));
     }
     const int r0 = 4 * g + (r >> 2);
 #pragma unroll
@@ -726,6 +763,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       const bf16x4 lo = ds_read_tr(vs + r0 * LDR + col);
       const bf16x4 hi = ds_read_tr(vs + (r0 + 16) * LDR + col);
       const bf16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (SPLIT_P) o[di] = mfma16(vf, pl, o[di]);
       o[di] = mfma16(vf, pf, o[di]);
     }
   }
@@ -767,9 +805,9 @@ extern "C" void lsd_attn_set_small_waves128(int v) { g_attn_small_waves128 = v; 
 // requests V with K (lsd_attn_set_large_waves: tuning / A/B)
 static int g_attn_large_waves64 = 4, g_attn_large_waves128 = 4;
 // grouped-query decode on MFMA (attn_decode_mfma_kernel) for HD = 128,
-// G in {2, 4, 8}, at least this many waves ((sequence, kv head) items x
-// context splits); 0 = off (lsd_attn_set_mfma_min).  ops/hip.py picks the
-// splits so that long contexts reach it with few sequences.
+// G in {2, 4, 8}: from this many waves ((sequence, kv head) items x context
+// splits) with bf16 weights, below with two terms; 0 = off
+// (lsd_attn_set_mfma_min).
 static int g_attn_mfma_min = 256;
 extern "C" void lsd_attn_set_mfma_min(int v) { g_attn_mfma_min = v; }
 extern "C" void lsd_attn_set_large_waves(int hd, int v) {
@@ -791,6 +829,20 @@ static hipError_t attn_decode_combine(const float* part_o, const float* part_ml,
   return hipGetLastError();
 }
 
+static bool attn_on_mfma(int G, int hd) {
+  return g_attn_mfma_min > 0 && hd == 128 && g_attn_max_wg == 0 && (G == 2 || G == 4 || G == 8);
+}
+
+// How many parts each of the caller's context splits is taken in (the partials are sized for
+// all): a wave needs about 1.1 us per 32 keys, so few waves take short ranges.  32 heads over
+// 8: 1 sequence of 912 keys, 4 splits -> 16: 13.0 -> 6.9 us; 8 of 2000, 4 -> 8: 22.3 -> 17.1; but
+// 40 of 780, 2 -> 4: 27.1 -> 32.0 (640 waves and more fill the chip).
+extern "C" int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits) {
+  if (!attn_on_mfma(G, hd)) return 1;
+  const long waves = (long)B * n_kv * splits, f = waves > 160 ? 640 / waves : 4;
+  return f < 1 ? 1 : (int)(f * splits <= 256 ? f : 256 / splits);
+}
+
 extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                                       const int* seq_slots, const int* qpos, bf16* out, long ldo,
                                       float* part_o, float* part_ml, int B, int nh, int n_kv,
@@ -800,22 +852,31 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
   const int G = nh / n_kv;
   const int n_items = B * n_kv;
   const int gx = g_attn_max_wg > 0 ? (n_items < g_attn_max_wg ? n_items : g_attn_max_wg) : n_items;
-  // fewer blocks than half the CUs: wider blocks (g_attn_small_waves waves),
-  // K and V of an item requested in one round of loads
-  if (g_attn_mfma_min > 0 && hd == 128 && g_attn_max_wg == 0 && (long)n_items * splits >= g_attn_mfma_min) {
-    const dim3 mgrid((n_items + 3) / 4, splits);
-#define LSD_DEC_MFMA(GV)                                                                        \
-  if (G == GV) {                                                                                \
-    hipLaunchKernelGGL((attn_decode_mfma_kernel<128, GV>), mgrid, dim3(256), 0, st, q, ldq, kc, \
-                       vc, seq_slots, qpos, out, ldo, part_o, part_ml, n_kv, max_seq, splits,   \
-                       scale_log2, n_items);                                                    \
-    return attn_decode_combine(part_o, part_ml, out, ldo, B, nh, hd, splits, st);              \
+  // grouped heads: on MFMA at any size (1 sequence of 912 keys with the merge 16.1 -> 6.9 us, 4 of
+  // them 17.0 -> 8.4, 1 of 100 11.7 -> 5.7 against the VALU kernel).  Below g_attn_mfma_min waves
+  // the weights keep a second term
+  if (attn_on_mfma(G, hd)) {
+    const int f = lsd_attn_decode_split(B, n_kv, G, hd, splits);
+    const bool few = (long)n_items * splits < g_attn_mfma_min;
+    splits *= f;
+#define LSD_DEC_MFMA(GV, NWV, SP)                                                                \
+  if (G == GV && few == SP && (n_items * splits <= 1024) == (NWV == 1)) {                        \
+    hipLaunchKernelGGL((attn_decode_mfma_kernel<128, GV, NWV, SP>), dim3((n_items + NWV - 1) / NWV, splits), \
+                       dim3(64 * NWV), 0, st, q, ldq, kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml, \
+                       n_kv, max_seq, splits, scale_log2, n_items);                              \
+    return attn_decode_combine(part_o, part_ml, out, ldo, B, nh, hd, splits, st);                \
   }
-    LSD_DEC_MFMA(2)
-    LSD_DEC_MFMA(4)
-    LSD_DEC_MFMA(8)
+#define LSD_DEC_MFMA_G(GV) \
+  LSD_DEC_MFMA(GV, 1, true) LSD_DEC_MFMA(GV, 1, false) LSD_DEC_MFMA(GV, 4, true) LSD_DEC_MFMA(GV, 4, false)
+    LSD_DEC_MFMA_G(2)
+    LSD_DEC_MFMA_G(4)
+    LSD_DEC_MFMA_G(8)
+#undef LSD_DEC_MFMA_G
 #undef LSD_DEC_MFMA
+    return hipErrorInvalidValue;
   }
+  // fewer blocks than half the CUs: wider blocks (g_attn_small_waves waves),
+  // K and V of an item requested in one round of loads.
   // full batches: 4 waves (unroll 4) by default; 8 waves, 4 waves with
   // unroll 2 (42) and 2 waves (2) for A/B (lsd_attn_set_large_waves)
   const int lw = hd == 64 ? g_attn_large_waves64 : g_attn_large_waves128;

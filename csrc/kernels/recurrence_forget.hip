@@ -22,7 +22,9 @@ namespace {
 __device__ __forceinline__ float write_gate(float z, float lower) { return (1.f - lower) / (1.f + expf(z)); }
 
 // One (sequence, head, LV * 4 columns of the state) per block; thread (dg, lv)
-// holds rows dg + i * 256 / LV of four columns.  Dynamic LDS: q, 1 - f [D].
+// holds rows dg + i * 256 / LV of four columns.  Dynamic LDS: q, 1 - f [D].  The state passes
+// the caches by, as recur_seq_kernel's (a step with four such layers of 64 sequences 1366 ->
+// 1287 us, of 24 1213 -> 1177).
 template <typename T, int LV, int NR>
 __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(ForgetParams p) {
   constexpr int VB = LV * 4, DG = 256 / LV;
@@ -42,7 +44,7 @@ __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(Forget
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (start > 0 && live && dg + i * DG < D) s[i] = *reinterpret_cast<const f32x4*>(Sg + (long)(dg + i * DG) * p.Vp);
+    if (start > 0 && live && dg + i * DG < D) s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sg + (long)(dg + i * DG) * p.Vp));
   }
   for (int t = 0; t < n; ++t) {
     const long row = r0 + t;
@@ -94,7 +96,7 @@ __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(Forget
   if (live) {
 #pragma unroll
     for (int i = 0; i < NR; ++i)
-      if (dg + i * DG < D) *reinterpret_cast<f32x4*>(Sg + (long)(dg + i * DG) * p.Vp) = s[i];
+      if (dg + i * DG < D) __builtin_nontemporal_store(s[i], reinterpret_cast<f32x4*>(Sg + (long)(dg + i * DG) * p.Vp));
   }
 }
 

@@ -46,7 +46,8 @@ struct RecurParams {
                                        // Mamba-2: y silu(z) rows
   int write_ring;                      // single-token portions: this kernel keeps the ring
   // delta rule in chunks with factors of their own: chunks first .. first + chunks - 1 of
-  // every sequence, their factors at work[sequence][chunk][head]
+  // every sequence, their factors at work[sequence][chunk][head].  Mamba-2 in segments: chunks
+  // of a segment, their states
   void* work; int first, chunks;
 };
 

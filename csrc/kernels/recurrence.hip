@@ -913,7 +913,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void delta_state_kernel(RecurParams 
 //   y = diag(e^{a}) C S + P x + D x,   P_ts = (C_t . B_s) e^{a_t - a_s} dt_s  (s <= t)
 //   S = e^{a_31} S + B^T diag(dt_s e^{a_31 - a_s}) x
 // Rows y silu(z) leave in bf16 (z: the first columns of the in-projection).  One block per (sequence, head), wave w owns columns of the state.
-template <int NKS, int VTW>
+//
+// Few sequences: one block's chunks are a chain of 3 us each on a quarter of the chip, so a
+// sequence's segments of p.chunks chunks run together.  SSD_LOCAL leaves the state that each but
+// the last ends with (the first from the sequence's, the others from zero) and its summed log
+// decay in p.work; SSD_FULL joins those before its own and goes through its chunks.
+//   work: [sequence][head][segment] states, the last place the sequence's own before the
+//   portion, which another segment may have overwritten by then; then as many decays
+// 1000 tokens of 64 heads of 64 x 128: 101 us in one segment, 13 + 28 in eight.
+enum SsdPass : int { SSD_WHOLE, SSD_LOCAL, SSD_FULL };
+template <int NKS, int VTW, int PASS>
 __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const bf16* __restrict__ x, long ldx) {
   constexpr int CT = 32, NP = NKS * 32, NT = NKS * 2, LDB = NP + 8, VP = VTW * 64, LDX = VP + 8;
   constexpr int NB = CT * NP / 1024, NX = CT * VP / 1024;  // groups of four elements per thread
@@ -922,9 +931,17 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
   const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int kg = h / (p.heads / p.groups);
-  const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b], n = p.s.cu[b + 1] - r0;
-  if (n <= 0) return;
+  const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b], rows = p.s.cu[b + 1] - r0;
+  const int seg = PASS == SSD_WHOLE ? 0 : blockIdx.z, segs = PASS == SSD_WHOLE ? 1 : gridDim.z;
+  const bool copies = PASS == SSD_LOCAL && seg == segs - 1;
+  const int begin = PASS == SSD_WHOLE || copies ? 0 : seg * p.chunks * CT;
+  // the segment's tokens: begin .. n - 1
+  const int n = seg == segs - 1 ? rows : min(rows, begin + p.chunks * CT);
+  if (begin >= rows) return;
   float* Sg = p.S + ((long)slot * p.heads + h) * N * p.Vp;
+  const long item = ((long)b * p.heads + h) * segs;
+  float* states = static_cast<float*>(p.work) + item * N * p.Vp;
+  float* decays = static_cast<float*>(p.work) + (long)gridDim.y * p.heads * segs * N * p.Vp + item;
   const float A = p.A[h], gain = p.c.gain, skip = p.skip[h], dtb = p.dt_bias[h];
   const bf16* y = static_cast<const bf16*>(p.c.y) + (long)r0 * p.c.ldy;
   const int ldxi = (int)ldx, ldy = (int)p.c.ldy, ldo = (int)p.ldo;  // offsets within a chunk are 32-bit
@@ -933,15 +950,40 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
   const bf16* xv = x + r0 * ldx + p.v_ch + (long)h * V;
 
   f32x4 S[NT][VTW];
+  auto each = [&](auto f) {
 #pragma unroll
-  for (int dt = 0; dt < NT; ++dt)
+    for (int dt = 0; dt < NT; ++dt)
 #pragma unroll
-    for (int j = 0; j < VTW; ++j)
+      for (int j = 0; j < VTW; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = dt * 16 + 4 * g + i, v = (w * VTW + j) * 16 + r;
-        S[dt][j][i] = start > 0 && d < N && v < V ? Sg[d * p.Vp + v] : 0.f;
-      }
+        for (int i = 0; i < 4; ++i) {
+          const int d = dt * 16 + 4 * g + i, v = (w * VTW + j) * 16 + r;
+          S[dt][j][i] = f(S[dt][j][i], dt, j, i, d < N && v < V);
+        }
+  };
+  // all loads of a state are under way together: none is made under a condition
+  auto state = [&](const float* from) {
+    f32x4 L[NT][VTW];
+#pragma unroll
+    for (int dt = 0; dt < NT; ++dt)
+#pragma unroll
+      for (int j = 0; j < VTW; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) L[dt][j][i] = from[min(dt * 16 + 4 * g + i, N - 1) * p.Vp + min((w * VTW + j) * 16 + r, V - 1)];
+    each([&](float x, int dt, int j, int i, bool in) { return in ? L[dt][j][i] + x : 0.f; });
+  };
+  each([&](float, int, int, int, bool) { return 0.f; });
+  if constexpr (PASS == SSD_FULL) {
+    if (seg > 0 || start > 0) state(states + (seg == 0 ? (long)(segs - 1) * N * p.Vp : 0));
+    for (int j = 1; j < seg; ++j) {
+      const float dec = exp_f(decays[j]);
+      each([&](float x, int, int, int, bool) { return x * dec; });
+      state(states + (long)j * N * p.Vp);
+    }
+  } else {
+    if (start > 0 && (seg == 0 || copies)) state(Sg);
+  }
+  float total = 0.f;  // summed log decay
   // rows of the next chunk, in flight under this one's products
   bf16x4 rb[NB], rc[NB], rx[NX];
   float rdt = 0.f;
@@ -953,9 +995,12 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
       // clamped to valid rows (their dt is zero) and columns (zeros)
       const int c = tid + q * 256, t = min(c / (NP / 4), n - 1 - t0), d = (c % (NP / 4)) * 4;
       const int at = t * ldxi + min(d, N - 4);
-      const bf16x4 vb = ld4(xb + (long)t0 * ldx + at), vc = ld4(xc + (long)t0 * ldx + at);
+      const bf16x4 vb = ld4(xb + (long)t0 * ldx + at);
       rb[q] = d < N ? vb : z;
-      rc[q] = d < N ? vc : z;
+      if constexpr (PASS != SSD_LOCAL) {
+        const bf16x4 vc = ld4(xc + (long)t0 * ldx + at);
+        rc[q] = d < N ? vc : z;
+      }
     }
 #pragma unroll
     for (int q = 0; q < NX; ++q) {
@@ -965,15 +1010,15 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
     }
     rdt = bf2f((y + (long)t0 * p.c.ldy + p.gate_col + h)[min(tl, n - 1 - t0) * ldy]);
   };
-  fetch(0);
-  for (int t0 = 0, buf = 0; t0 < n; t0 += CT, buf ^= 1) {
+  if (!copies) fetch(begin);
+  for (int t0 = begin, buf = 0; !copies && t0 < n; t0 += CT, buf ^= 1) {
     const int nt = min(CT, n - t0);
     const bf16 *B = bs[buf], *C = cs[buf], *X = xs[buf];
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       const int c = tid + q * 256, at = c / (NP / 4) * LDB + (c % (NP / 4)) * 4;
       st4(bs[buf] + at, rb[q]);
-      st4(cs[buf] + at, rc[q]);
+      if constexpr (PASS != SSD_LOCAL) st4(cs[buf] + at, rc[q]);
     }
 #pragma unroll
     for (int q = 0; q < NX; ++q) {
@@ -990,9 +1035,11 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
     }
     const float a_end = __shfl(a, 31, 64);
     const float wend = dt * exp_f(a_end - a);
+    total += a_end;
     __syncthreads();  // the rows are there; the buffers written next were last read before this
     if (t0 + CT < n) fetch(t0 + CT);
     float zg[2][VTW][4];  // the gate of the rows and columns this lane ends with
+    if constexpr (PASS != SSD_LOCAL)
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -1020,6 +1067,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
 #pragma unroll
       for (int j = 0; j < VTW; ++j) o[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    if constexpr (PASS != SSD_LOCAL)
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       const int at = r * LDB + ks * 32 + 4 * g;
@@ -1055,6 +1103,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
         for (int i = 0; i < 4; ++i) u[st][i] = bf2f(xf[j][st * 4 + i]) * wv[st][i];
       split8(u[0], u[1], uh[j], ul[j]);
     }
+    if constexpr (PASS != SSD_LOCAL)
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const float at = __shfl(a, mt * 16 + r, 64);
@@ -1087,6 +1136,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
         S[dt2][j] = mfma16(bf, ul[j], S[dt2][j]);
       }
     }
+    if constexpr (PASS == SSD_LOCAL) continue;
     bf16* out = static_cast<bf16*>(p.out) + (long)(r0 + t0) * p.ldo + (long)h * V;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
@@ -1099,6 +1149,13 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
             out[t * ldo + v] = f2bf((o[mt][j][i] + skip * bf2f(xf[j][mt * 4 + i])) * silu(gain * zg[mt][j][i]));
         }
   }
+  float* end = Sg;
+  if constexpr (PASS == SSD_LOCAL) {
+    end = states + (long)seg * N * p.Vp;
+    if (tid == 0 && !copies) decays[seg] = total;
+  } else if (n < rows) {
+    return;  // a later segment ends the portion
+  }
   int g4 = 4 * g;
   asm volatile("" : "+v"(g4));  // addresses are formed anew: none stays in a register through the loop
 #pragma unroll
@@ -1108,7 +1165,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(RecurParams p, const 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int d = dt * 16 + g4 + i, v = (w * VTW + j) * 16 + r;
-        if (d < N && v < p.Vp) Sg[d * p.Vp + v] = S[dt][j][i];
+        if (d < N && v < p.Vp) end[d * p.Vp + v] = S[dt][j][i];
       }
 }
 
@@ -1328,13 +1385,32 @@ extern "C" hipError_t lsd_recur_chunk(const RecurParams* p, int delta, const bf1
   else if (p->D <= 64) { LSD_CK(KERNEL, 2) }   \
   else if (p->D <= 128) { LSD_CK(KERNEL, 4) }  \
   else return hipErrorInvalidValue;
-  if (delta) {
-    LSD_CK_D(delta_chunk_kernel)
-  } else {
-    LSD_CK_D(ssd_chunk_kernel)
-  }
+  if (!delta) return hipErrorInvalidValue;
+  LSD_CK_D(delta_chunk_kernel)
 #undef LSD_CK_D
 #undef LSD_CK
+  return hipGetLastError();
+}
+
+// Segments of p->chunks chunks of every sequence run together, their states through p->work
+extern "C" hipError_t lsd_ssd_chunk(const RecurParams* p, int segs, const bf16* x, long ldx, hipStream_t st) {
+  if (p->s.B == 0) return hipSuccess;
+  if (p->D > 128 || p->V > 128 || segs < 1 || (segs > 1 && (!p->work || p->chunks < 1))) return hipErrorInvalidValue;
+  const dim3 grid(p->heads, p->s.B, segs);
+#define LSD_SSD(KS, VTW)                                                                                           \
+  if (segs == 1) {                                                                                                 \
+    hipLaunchKernelGGL((ssd_chunk_kernel<KS, VTW, SSD_WHOLE>), grid, dim3(256), 0, st, *p, x, ldx);                 \
+  } else {                                                                                                         \
+    hipLaunchKernelGGL((ssd_chunk_kernel<KS, VTW, SSD_LOCAL>), grid, dim3(256), 0, st, *p, x, ldx);                 \
+    hipLaunchKernelGGL((ssd_chunk_kernel<KS, VTW, SSD_FULL>), grid, dim3(256), 0, st, *p, x, ldx);                  \
+  }
+#define LSD_SSD_V(KS) \
+  if (p->V <= 64) { LSD_SSD(KS, 1) } else { LSD_SSD(KS, 2) }
+  if (p->D <= 32) { LSD_SSD_V(1) }
+  else if (p->D <= 64) { LSD_SSD_V(2) }
+  else { LSD_SSD_V(4) }
+#undef LSD_SSD_V
+#undef LSD_SSD
   return hipGetLastError();
 }
 

@@ -35,6 +35,7 @@ hipError_t lsd_conv_silu(const ConvParams* c, const SeqParams* s, int T, lsd_bf1
 long lsd_delta_item(int D);
 int lsd_delta_chunk();
 hipError_t lsd_delta_split(const RecurParams* p, const lsd_bf16_t* x, long ldx, hipStream_t st);
+hipError_t lsd_ssd_chunk(const RecurParams* p, int segs, const lsd_bf16_t* x, long ldx, hipStream_t st);
 hipError_t lsd_recur_chunk(const RecurParams* p, int delta, const lsd_bf16_t* x, long ldx, hipStream_t st);
 hipError_t lsd_conv_tail(const ConvParams* c, const SeqParams* s, int f32, hipStream_t st);
 hipError_t lsd_head_norm_gate(const MixOutParams* p, int f32, hipStream_t st);
@@ -151,12 +152,31 @@ void out_rows(P& p, const Tensor& out, const Tensor& y) {
 }
 
 // Rows of SiLU(convolution) (bf16) for the chunked forms, which then run.
-void run_chunks(const RecurParams& p, int delta, const Tensor& y) {
+void run_chunks(const RecurParams& p, const Tensor& y) {
   const int64_t T = y.size(0), ld = (p.c.channels + 7) / 8 * 8;
   auto x = torch::empty({T, ld}, y.options());
   auto* xp = reinterpret_cast<lsd_bf16_t*>(x.data_ptr());
   check_hip(lsd_conv_silu(&p.c, &p.s, T, xp, ld, cur_stream()), "conv_silu");
-  check_hip(lsd_recur_chunk(&p, delta, xp, ld, cur_stream()), "recur_chunk");
+  check_hip(lsd_recur_chunk(&p, 1, xp, ld, cur_stream()), "recur_chunk");
+}
+
+// Mamba-2: segs segments of each sequence together (0: where that is faster)
+void run_ssd(RecurParams p, const Tensor& y, int64_t max_rows, int64_t segs) {
+  const int64_t T = y.size(0), ld = (p.c.channels + 7) / 8 * 8, chunks = (max_rows + 31) / 32, blocks = (int64_t)p.s.B * p.heads;
+  // three chunks and more a segment, up to two blocks a CU.  Steps of 64 heads of 64 x 128, one
+  // segment against the rule's: 1 sequence of 150 tokens 1146 us (one), 300 1516 -> 1494, 1000 2545
+  // -> 2372, 4000 7497 -> 6656, 2 of 500 2297 -> 2254; 4 of 500 3611, with two segments 3625
+  if (segs == 0) segs = blocks > 128 ? 1 : std::clamp<int64_t>(std::min(512 / std::max<int64_t>(1, blocks), chunks / 3), 1, 8);
+  auto x = torch::empty({T, ld}, y.options());
+  auto* xp = reinterpret_cast<lsd_bf16_t*>(x.data_ptr());
+  check_hip(lsd_conv_silu(&p.c, &p.s, T, xp, ld, cur_stream()), "conv_silu");
+  Tensor work;
+  if (segs > 1) {
+    work = torch::empty({blocks * segs * ((int64_t)p.D * p.Vp + 1)}, y.options().dtype(torch::kFloat32));
+    p.work = work.data_ptr();
+    p.chunks = (int)((chunks + segs - 1) / segs);
+  }
+  check_hip(lsd_ssd_chunk(&p, (int)segs, xp, ld, cur_stream()), "ssd_chunk");
 }
 
 void norm_and_gate(const RecurParams& p, int64_t T, bool f32) {
@@ -219,7 +239,7 @@ void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_
     if (split == 1 || (split < 0 && (int64_t)p.s.B * heads <= 192))
       run_delta_split(p, y, max_rows > 0 ? std::min(max_rows, y.size(0)) : y.size(0));
     else
-      run_chunks(p, 1, y);
+      run_chunks(p, y);
     check_hip(lsd_conv_tail(&p.c, &p.s, f32, cur_stream()), "conv_tail");
     return;
   }
@@ -235,10 +255,12 @@ void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_
   if (!single) check_hip(lsd_conv_tail(&p.c, &p.s, f32, cur_stream()), "conv_tail");
 }
 
-// y [T, N]: z | x | B | C | dt.  `chunked`: prompts of bf16 models
+// y [T, N]: z | x | B | C | dt.  `chunked`: prompts of bf16 models; max_rows: rows of the longest
+// sequence (0: not known); segs: segments of each that run together (0: by size)
 void ssm_seq(Tensor y, Tensor slots, Tensor start, Tensor cu, int64_t heads, int64_t groups, int64_t N, int64_t V,
              int64_t norm_groups, Tensor taps, Tensor bias, Tensor ring, Tensor state, Tensor A, Tensor dt_bias,
-             Tensor skip, Tensor norm, double gain, double eps, Tensor out, bool single, bool chunked) {
+             Tensor skip, Tensor norm, double gain, double eps, Tensor out, bool single, bool chunked, int64_t max_rows,
+             int64_t segs) {
   const bool f32 = is_f32(y, "y");
   const int64_t inner = heads * V;
   RecurParams p{};
@@ -258,7 +280,8 @@ void ssm_seq(Tensor y, Tensor slots, Tensor start, Tensor cu, int64_t heads, int
   TORCH_CHECK(!single || p.s.B == y.size(0), "ssm_seq: one row per sequence");
   if (chunked) {
     TORCH_CHECK(!f32 && !single && lsd_chunk_ok(0, N, V, groups, heads), "ssm_seq: no chunked kernel");
-    run_chunks(p, 0, y);
+    TORCH_CHECK(max_rows >= 0 && segs >= 0 && segs <= 64 && p.s.B <= 65535, "ssm_seq: max_rows, segs");
+    run_ssd(p, y, max_rows > 0 ? std::min(max_rows, y.size(0)) : y.size(0), segs);
   } else {
     TORCH_CHECK(lsd_recur_block(N, V) > 0, "ssm_seq: no kernel for state size ", N);
     check_hip(lsd_recur_seq(&p, 0, f32, cur_stream()), "ssm_seq");
@@ -701,7 +724,8 @@ void lsd_register_mixers(pybind11::module& m) {
   m.def("ssm_seq", &ssm_seq, py::arg("y"), py::arg("slots"), py::arg("start"), py::arg("cu"), py::arg("heads"),
         py::arg("groups"), py::arg("state_dim"), py::arg("vdim"), py::arg("norm_groups"), py::arg("taps"), py::arg("bias"),
         py::arg("ring"), py::arg("state"), py::arg("A"), py::arg("dt_bias"), py::arg("skip"), py::arg("norm"),
-        py::arg("gain"), py::arg("eps"), py::arg("out"), py::arg("single"), py::arg("chunked") = false);
+        py::arg("gain"), py::arg("eps"), py::arg("out"), py::arg("single"), py::arg("chunked") = false,
+        py::arg("max_rows") = 0, py::arg("segs") = 0);
   m.def("forget_ok", [](int64_t D, int64_t V) { return lsd_forget_ok((int)D, (int)V) != 0; });
   m.def("forget_seq", &forget_seq, py::arg("y"), py::arg("slots"), py::arg("start"), py::arg("cu"), py::arg("heads"),
         py::arg("dim"), py::arg("vdim"), py::arg("bias"), py::arg("lower"), py::arg("norm"), py::arg("eps"),

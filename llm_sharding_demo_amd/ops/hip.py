@@ -832,7 +832,7 @@ class HipBackend(Backend):
             self.C.ssm_seq(y[s], mt.seq_slots, mt.q_start, mt.cu_q, m.heads, m.groups, m.state, m.vdim, m.norm_groups,
                            w("mixer.taps"), w("mixer.conv.b"), entry[1], entry[0], w("mixer.A"), w("mixer.dt_bias"),
                            w("mixer.D"), w("mixer.norm"), gain, eps, out[s], mt.is_decode,
-                           self._chunked(mt) and self.C.chunk_ok(False, m.state, m.vdim, m.groups, m.heads))
+                           self._chunked(mt) and self.C.chunk_ok(False, m.state, m.vdim, m.groups, m.heads), mt.max_q)
 
     def _tm(self, rows: float) -> int:
         return 64 if self.fp32 else self.R.group_tm(rows)

@@ -1022,6 +1022,8 @@ class HipBackend(Backend):
 
     def _resid_splits(self, M: int, N: int, K: int) -> int:
         S = self.R.resid_splits(M, N, K, self._decode, getattr(self, "concurrency", 1))
+        if not self._decode:
+            S = self.R.prompt_slabs(M, N, K, S)
         return self.R.slab_splits(M, N, K, S) if self._tiled(M, N) or self.R.defer_resid else S
 
     @classmethod

@@ -282,6 +282,28 @@ class Routing:
         most = max(1, K // 256)
         return min((min(s, most) for s in (S, 4, 6, 8)), key=us)
 
+    @staticmethod
+    def prompt_slabs(M: int, N: int, K: int, S: int) -> int:
+        """K splits of a prompt's residual projection whose rule leaves S > 1
+        slabs: as many as let the 256 x 256 kernel (from 160 blocks on) fill one
+        round of the CUs, where that beats S on the 128-row rings, slabs written
+        and read included.  1000 rows with their norm: 2048 x 5632 2 splits 42.5 us,
+        8 34.6; 2048 x 2048 2 21.0 (kept), 8 23.9; 1600 x 6400 3 39.0, 8 32.5; 500 rows
+        have too few tiles."""
+        if S <= 1 or M < 256 or K % 64:
+            return S
+        big, ring = math.ceil(M / 256) * math.ceil(N / 256), math.ceil(M / 128) * math.ceil(N / 128)
+        if big * S >= 160:
+            return S
+        slab = M * N * 4 / 5.2e6
+
+        def us(s: int) -> float:
+            if big * s >= 160:
+                return math.ceil(big * s / 256) * (K / s * 0.021 + 10) + s * slab
+            return max(1.0, ring * s / 256) * K / s * 0.0115 + 4 + s * slab
+
+        return min([S] + [s for s in range(S + 1, 9) if 160 <= big * s <= 256 and K >= 512 * s], key=us)
+
     def logits_kw(self, M: int, N: int, K: int, lanes: int = 1):
         """lm_head: the 128x128 LDS-tiled kernel at vocab width (fills the
         chip without split-K; 41.8 vs 64.2 us at 128 rows, GPT-2 XL)."""
@@ -392,7 +414,7 @@ def route_table(model: str, rows, routing: Routing | None = None) -> dict:
     `tests/test_routing.py` pins and `python -m llm_sharding_demo_amd.ops.routing`
     prints.  route = kernel family + K splits, no extension calls.  The split-K and
     tiled families run up to 128 rows on the deep ring (gemm_deep.hip), unsplit where
-    the split would be combined, and with slab_splits slabs."""
+    the split would be combined, and with slab_splits slabs; prompts with prompt_slabs."""
     from ..config import get_model_config
 
     r = routing or Routing.from_env("")

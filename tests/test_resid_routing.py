@@ -35,6 +35,16 @@ def test_resid_rule_prefill_chunks_keep_prefill_rule():
     assert dec == 6 and pre == max(1, min(-(-256 // 52), 6400 // 64 // 2))
 
 
+def test_prompt_slabs():
+    """More slabs only for prompts that leave some anyway and have tiles enough."""
+    from llm_sharding_demo_amd.ops.routing import Routing
+
+    for M, N, K, S, want in [(1000, 2048, 5632, 2, 8), (1000, 2048, 2048, 2, 2), (1000, 1600, 6400, 3, 8),
+                             (500, 2048, 5632, 4, 4), (512, 1600, 6400, 5, 5), (3000, 2048, 5632, 1, 1),
+                             (200, 2048, 5632, 8, 8), (1000, 2048, 96, 2, 2), (700, 4096, 14336, 2, 5)]:
+        assert Routing.prompt_slabs(M, N, K, S) == want, (M, N, K)
+
+
 def test_gemv_ok_matches_dispatch():
     """lsd_gemv_ok must accept exactly the (epilogue, norm) pairs lsd_gemv
     instantiates: BF16+LN etc. read 'not ok' so the caller

@@ -122,10 +122,10 @@ def rope_spec_table(rope: RopeSpec, max_pos: int, device) -> torch.Tensor:
     return torch.stack([ang.cos(), ang.sin()], -1).float().contiguous().to(device)
 
 
-def prefill_tiles(meta) -> torch.Tensor:
-    """(sequence, query offset) of every 64-query tile of a packed batch."""
+def prefill_tiles(meta, rows: int = 64) -> torch.Tensor:
+    """(sequence, query offset) of every tile of `rows` queries of a packed batch."""
     qlens = meta.host_qlens
-    tiles = [(i, off) for i, n in enumerate(qlens) for off in range(0, n, 64)]
+    tiles = [(i, off) for i, n in enumerate(qlens) for off in range(0, n, rows)]
     return torch.tensor(tiles, dtype=torch.int32).reshape(-1, 2)
 
 
@@ -797,10 +797,13 @@ class HipBackend(Backend):
         return self._query_tiles(meta, 64 * qt, device), qt
 
     def _plain_tiles(self, meta, heads: int, device):
-        """Query tiles of the prompt kernel and their queries."""
-        blocks = heads * sum(-(-n // 128) for n in meta.host_qlens)
-        rows = 128 if blocks >= self.R.attn_tile_min else 64
-        return self._query_tiles(meta, rows, device), rows
+        """Query tiles of the prompt kernel and their queries, kept on the batch."""
+        kept = meta.__dict__.get("_tiles")
+        if kept is None or kept[0] != heads:
+            blocks = heads * sum([(n + 127) // 128 for n in meta.host_qlens])
+            rows = 128 if blocks >= self.R.attn_tile_min else 64
+            kept = meta._tiles = heads, prefill_tiles(meta, rows).to(device), rows
+        return kept[1:]
 
     @staticmethod
     def _query_tiles(meta, rows: int, device):
@@ -1021,10 +1024,21 @@ class HipBackend(Backend):
         return self.R.gemm_kw(M, N, K, self.concurrency, nw)
 
     def _resid_splits(self, M: int, N: int, K: int) -> int:
-        S = self.R.resid_splits(M, N, K, self._decode, getattr(self, "concurrency", 1))
-        if not self._decode:
-            S = self.R.prompt_slabs(M, N, K, S)
-        return self.R.slab_splits(M, N, K, S) if self._tiled(M, N) or self.R.defer_resid else S
+        # kept with the routing: the rules cost the host some 10 us, and an eagerly issued
+        # prompt asks twice a layer
+        plans = self.R.__dict__.setdefault("_resid_plans", {})
+        key = M, N, K, self._decode, getattr(self, "concurrency", 1)
+        S = plans.get(key)
+        if S is None:
+            S = self.R.resid_splits(*key)
+            if not self._decode:
+                S = self.R.prompt_slabs(M, N, K, S)
+            if self._tiled(M, N) or self.R.defer_resid:
+                S = self.R.slab_splits(M, N, K, S)
+            if len(plans) >= 4096:
+                plans.clear()
+            plans[key] = S
+        return S
 
     @classmethod
     def decode_attn_splits(cls, B: int, nh: int, n_kv: int, hd: int, max_ctx: int) -> int:

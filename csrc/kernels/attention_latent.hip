@@ -25,8 +25,9 @@
 //    in turn, each with a private LDS tile, merged at the end, or (wide rows)
 //    share a tile and divide the value columns; long ranges are split over
 //    blocks (latent_combine).
-//  * plain: one (token, head) per block on the VALU -- fp32 models, and ranks
-//    without an MFMA instantiation.
+//  * plain: fp32 models, 16 heads of a token per block on fp32 MFMA; one (token, head)
+//    per block on the VALU for fp32 ranks above 576 and bf16 ranks without an MFMA
+//    instantiation.
 //
 // The MFMA kernels swap the operands (S^T = K Q^T) as attention.hip does, so a
 // lane holds one query's scores and P^T needs no LDS trip.  The softmax weights

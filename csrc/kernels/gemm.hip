@@ -5,7 +5,7 @@
 // `server.py:102`).  Weights are stored [N][K] (K-contiguous) so a
 // 16x16x32 B-operand fragment is one 16-byte load.
 //
-// The kernels (decode microbatches of up to 128 rows: gemm_deep.hip):
+// The kernels (decode microbatches of up to 128 or 256 rows: gemm_deep.hip):
 //  * gemm_sk      -- decode microbatches whose K has no whole 64-wide steps.  Weight-bandwidth bound:
 //    W streamed HBM -> VGPRs (read once, no LDS round trip), the small A
 //    operand staged through LDS with full-line LDS-DMA, split-K across
@@ -1822,14 +1822,14 @@ static hipError_t launch_tiled(const GemmParams& p, int* cnt, float* ws, hipStre
 
 using namespace lsd;
 
-extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi);  // gemm_deep.hip
+extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits);  // gemm_deep.hip
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st);
 
-// Kinds 0 and 1 of up to 128 rows run on the deep ring (gemm_deep.hip), which is faster at
-// every shape (its head has both times); the split-K kernel takes what has no whole k-steps
-// of 64, the ring and tiled kernels what has more rows.
+// Kinds 0 and 1 of up to 128 rows, and up to 256 of few blocks, run on the deep ring
+// (gemm_deep.hip), which is faster there at every shape (its head has both times); the split-K
+// kernel takes what has no whole k-steps of 64, the ring and tiled kernels what has more rows.
 extern "C" int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits) {
-  return kind <= 1 && lsd_gemm_deep_ok(M, N, K, epi) && (epi != EPI_SLAB || splits <= K / 64);
+  return kind <= 1 && lsd_gemm_deep_ok(M, N, K, epi, splits);
 }
 
 extern "C" void lsd_gemm_set_big_min(int v) { g_big_min_blocks = v; }

@@ -1,4 +1,4 @@
-// Decode GEMM of 9 .. 128 rows:  C[M,N] = A[M,K] . W[N,K]^T  (+ epilogue)
+// Decode GEMM of 9 .. 256 rows:  C[M,N] = A[M,K] . W[N,K]^T  (+ epilogue)
 //
 // What bounds it is the stream of W out of HBM, which is read once, and the rate at which
 // a CU takes LDS-DMA in (about 50 GB/s: W and A together).  So:
@@ -9,7 +9,8 @@
 //    With two, W arrives at half the rate.  Wide tiles of up to 64 rows load W non-temporally
 //    (28672 x 4096 at 40 rows 49.5 -> 44.0 us, 4096 x 14336 23.0 -> 21.3); narrow ones, whose
 //    weights are small, and more rows are 0 to 20 % slower that way.
-//  * a block holds all rows, so W is read once, and its width (64, 32 or 16 columns) follows
+//  * a block holds all rows (up to 128; more are two blocks beside each other, the second of
+//    which finds W in L2), so W is read once, and its width (64, 32 or 16 columns) follows
 //    from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
 //    32-wide parts among them (WK) and are summed through LDS.  No K splits over blocks, no
 //    tickets and no workspace, except where the caller takes the partial sums as slabs.
@@ -40,8 +41,8 @@ __device__ __forceinline__ void count_down(F f) {  // f(N - 1) .. f(0), compile-
 }  // namespace
 
 // WM x WN waves of MTW x NTW 16 x 16 tiles, times WK waves on different 32-wide parts of a
-// k-step of BK; SLOTS k-steps in LDS; AUX: cache policy of W.
-template <int WM, int WN, int WK, int MTW, int NTW, int BK, int SLOTS, int AUX, int EPI>
+// k-step of BK; SLOTS k-steps in LDS; AUX: cache policy of W; TWO: two row blocks.
+template <int WM, int WN, int WK, int MTW, int NTW, int BK, int SLOTS, int AUX, int EPI, bool TWO = false>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams p, int tiles_n) {
   constexpr int WAVES = WM * WN * WK, BM = 16 * WM * MTW, BN = 16 * WN * NTW;
   constexpr int RB = BK * 2, CPR = RB / 16, RPI = 64 / CPR;  // bytes and 16-byte chunks of a row, rows per instruction
@@ -56,7 +57,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
   const int r = lane & 15, g = lane >> 4;
   const int wk = w % WK, wn = (w / WK) % WN, wm = w / (WK * WN);
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int split = bid / tiles_n, n0 = (bid - split * tiles_n) * BN;
+  const int m0 = TWO ? (bid & 1) * BM : 0, nb = TWO ? bid >> 1 : bid;  // (row blocks side by side share W)
+  const int split = nb / tiles_n, n0 = (nb - split * tiles_n) * BN;
   const int KT = p.K / BK;
   const int kb = (int)((long)KT * split / p.splits), ke = (int)((long)KT * (split + 1) / p.splits);
 
@@ -71,7 +73,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
   for (int q = 0; q < LA; ++q) {
     const int ins = min(w + q * WAVES, IA - 1), row = ins * RPI + lane / CPR;
     dsta[q] = ins * 1024;
-    srca[q] = p.A + (long)min(row, p.M - 1) * p.lda + (((lane % CPR) ^ swz(row)) << 3);
+    srca[q] = p.A + (long)min(m0 + row, p.M - 1) * p.lda + (((lane % CPR) ^ swz(row)) << 3);
   }
 #pragma unroll
   for (int q = 0; q < LW; ++q) {
@@ -154,9 +156,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
     }
   };
   for (int c = threadIdx.x; c < BM * (BN / 8); c += 64 * WAVES) {
-    const int m = c / (BN / 8), ch = c % (BN / 8), n = n0 + ch * 8;
+    const int row = c / (BN / 8), ch = c % (BN / 8), m = m0 + row, n = n0 + ch * 8;
     if (m >= p.M || n >= p.N) continue;
-    const float* s = ct + m * CLD + ch * 8;
+    const float* s = ct + row * CLD + ch * 8;
     float v[8];
     eight(s, v);
     if constexpr (EPI == EPI_SILU_MUL) {
@@ -177,13 +179,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
 // the least of ceil(blocks / CUs) (columns + rows) is the fastest one: measured at 64 rows,
 // 4800 x 1600 on 75 blocks of 64 columns 11.9 us, on 150 of 32 8.8; 2624 x 2048 on 82 of 32 8.8,
 // on 164 of 16 7.5; 8512 x 2048 on 133 of 64 13.0, on 266 of 32 15.6.
+static int deep_rows(int M) {  // of a block
+  return M > 192 ? 128 : M > 128 ? 96 : M > 96 ? 128 : M > 64 ? 96 : (M + 15) / 16 * 16;
+}
 static int deep_cols(int M, int N, int K, int splits, int epi) {
-  const int rows = M > 96 ? 128 : M > 64 ? 96 : (M + 15) / 16 * 16;
+  const int rows = deep_rows(M), mbs = (M + rows - 1) / rows;
   int best = 0;
   long least = 0;
   for (int bn = 64; bn >= 16; bn /= 2) {
     if (bn == 16 && (M > 64 || epi == EPI_SILU_MUL || K % 128 != 0 || K / 128 < splits)) break;
-    const long blocks = (long)((N + bn - 1) / bn) * splits, cost = (blocks + 255) / 256 * (bn + rows);
+    const long blocks = (long)((N + bn - 1) / bn) * splits * mbs, cost = (blocks + 255) / 256 * (bn + rows);
     if (best == 0 || cost < least) { best = bn; least = cost; }
   }
   return best;
@@ -204,14 +209,14 @@ static hipError_t deep_rows64(const GemmParams& p, int bn, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int EPI, int MTW>
+template <int EPI, int MTW, bool TWO>
 static hipError_t deep_rows128(const GemmParams& p, int bn, hipStream_t st) {
   const int tn = (p.N + bn - 1) / bn;
-  const dim3 grid((unsigned)(tn * p.splits)), block(512);
+  const dim3 grid((unsigned)(tn * p.splits * (TWO ? 2 : 1))), block(512);
   if (bn == 64)
-    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 2, 64, MTW == 3 ? 4 : 3, 0, EPI>), grid, block, 0, st, p, tn);
+    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 2, 64, MTW == 3 ? 4 : 3, 0, EPI, TWO>), grid, block, 0, st, p, tn);
   else
-    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 1, 64, MTW == 3 ? 5 : 4, 0, EPI>), grid, block, 0, st, p, tn);
+    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 1, 64, MTW == 3 ? 5 : 4, 0, EPI, TWO>), grid, block, 0, st, p, tn);
   return hipGetLastError();
 }
 
@@ -222,24 +227,33 @@ static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
   if (p.M <= 32) return deep_rows64<EPI, 2>(p, bn, st);
   if (p.M <= 48) return deep_rows64<EPI, 3>(p, bn, st);
   if (p.M <= 64) return deep_rows64<EPI, 4>(p, bn, st);
-  return p.M <= 96 ? deep_rows128<EPI, 3>(p, bn, st) : deep_rows128<EPI, 4>(p, bn, st);
+  if (p.M <= 96) return deep_rows128<EPI, 3, false>(p, bn, st);
+  if (p.M <= 128) return deep_rows128<EPI, 4, false>(p, bn, st);
+  return p.M <= 192 ? deep_rows128<EPI, 3, true>(p, bn, st) : deep_rows128<EPI, 4, true>(p, bn, st);
 }
 
 }  // namespace lsd
 
 using namespace lsd;
 
-// 1 .. 128 rows, whole k-steps; gate / up pairs lie in one tile.  splits > 1 only as slabs:
-// the other epilogues run unsplit, whatever the caller asked for.
-extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi) {
-  return M >= 1 && M <= 128 && K >= 64 && K % 64 == 0 && N % (epi == EPI_SILU_MUL ? 32 : 16) == 0;
+// 1 .. 256 rows, whole k-steps; gate / up pairs lie in one tile.  splits > 1 only as slabs:
+// the other epilogues run unsplit, whatever the caller asked for.  More than 128 rows are two
+// row blocks, which is faster than the larger tiles up to two blocks a CU: whole steps of 48
+// layers of 1600, 160 sequences 4472 -> 4117 us, 256 5426 -> 5326; 12 layers of 2048, 140 sequences
+// 1285 -> 1198.  Not with more: 4096 x 14336 at 256 rows in 8 slabs, 1024 blocks, 47.5 -> 57.2 us.
+extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits) {
+  if (M < 1 || M > 256 || K < 64 || K % 64 != 0 || N % (epi == EPI_SILU_MUL ? 32 : 16) != 0) return 0;
+  if (epi != EPI_SLAB) splits = 1;
+  if (splits < 1 || splits > K / 64) return 0;
+  if (M <= 128) return 1;
+  const int bn = deep_cols(M, N, K, splits, epi);
+  return (long)((N + bn - 1) / bn) * splits * 2 <= 512;
 }
 
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st) {
-  if (!lsd_gemm_deep_ok(p->M, p->N, p->K, epi)) return hipErrorInvalidValue;
+  if (!lsd_gemm_deep_ok(p->M, p->N, p->K, epi, p->splits)) return hipErrorInvalidValue;
   GemmParams q = *p;
   if (epi != EPI_SLAB) q.splits = 1;
-  if (q.splits < 1 || q.splits > q.K / 64) return hipErrorInvalidValue;
   switch (epi) {
 #define LSD_DEEP(E) \
   case E: return deep_launch<E>(q, st);

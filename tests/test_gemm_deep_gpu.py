@@ -1,4 +1,4 @@
-"""Decode GEMM of up to 128 rows (csrc/kernels/gemm_deep.hip) against float64: every row class
+"""Decode GEMM of up to 256 rows (csrc/kernels/gemm_deep.hip) against float64: every row class
 and tile width, partial tiles of rows and columns, K down to one k-step and one k-step a split.
 
 Bound per element: sums of K products in fp32 in any order are at most K 2^-24 sum |a w| off;
@@ -38,7 +38,7 @@ def check(got, want, a, w, rounded=True, more=0.0):
 
 
 # columns: 16-wide tiles with a ragged end, 32- and 64-wide ones, K with and without 128-wide steps
-@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129, 192, 193, 256])
 @pytest.mark.parametrize("N,K", [(64, 64), (1616, 128), (4160, 192), (2624, 1024), (10304, 320), (20000, 128)])
 def test_epilogues(C, CNT, M, N, K):
     a, w, b = data(M, N, K)
@@ -62,7 +62,7 @@ def test_epilogues(C, CNT, M, N, K):
     assert int(CNT.abs().sum()) == 0
 
 
-@pytest.mark.parametrize("M", [9, 40, 64, 96, 128])
+@pytest.mark.parametrize("M", [9, 40, 64, 96, 128, 150, 193])
 @pytest.mark.parametrize("N,K,S", [(64, 64, 1), (1664, 128, 2), (2048, 1024, 4), (4096, 1024, 8), (768, 768, 6), (768, 768, 12)])
 def test_slabs(C, CNT, M, N, K, S):
     a, w, _ = data(M, N, K)
@@ -77,7 +77,7 @@ def test_slabs(C, CNT, M, N, K, S):
     check(slab.double().sum(0), a.double() @ w.double().T, a, w, rounded=False)
 
 
-@pytest.mark.parametrize("M", [9, 33, 64, 96, 128])
+@pytest.mark.parametrize("M", [9, 33, 64, 96, 128, 129, 256])
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("heads,kv,hd,K", [(4, 2, 64, 128), (25, 25, 64, 320), (32, 8, 128, 256)])
 def test_qkv(C, CNT, M, rope, heads, kv, hd, K):

@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256) void latent_plain_f32_kernel(LatentAttnParams 
       nx[c] = *reinterpret_cast<const f32x4*>(cache + ((long)table[key / PAGE] * PAGE + key % PAGE) * R + at % (R / 4) * 4);
     }
   };
-  fetch(lo);
+  if (lo <= pos) fetch(lo);  // (no key, as behind position -1: there is no row to read)
   for (int k0 = lo; k0 <= pos; k0 += KT) {
 #pragma unroll
     for (int c = 0; c < NL; ++c) {

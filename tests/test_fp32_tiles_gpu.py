@@ -58,3 +58,17 @@ def test_latent_values_and_sinks_fp32(C, rank, value, H):  # noqa: F811
     # a score is off by 4 ulp of its products' sizes at most (their roundings are
     # independent: sqrt(rank) of the worst case), which weights share relatively
     assert float((got - p @ c[:, :cols].to(F64)).pow(2).mean().sqrt()) < 2e-6
+
+
+@pytest.mark.parametrize("H,rank", [(1, 64), (16, 512), (33, 576)])
+def test_latent_without_keys_fp32(C, H, rank):  # noqa: F811
+    """A row at position -1 has no key and reads none: its sink takes all the weight."""
+    n = 3
+    c, q, sink = rand(n, rank, seed=1), rand(2, H, rank, seed=2), rand(H, seed=3)
+    pool, table = paged(c, torch.float32, rank)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    got = C.latent_decode(q.reshape(2, -1).to(DEV), pool, table, torch.ones(2, **i32), torch.tensor([-1, n - 1], **i32), H,
+                          1 << 30, rank ** -0.5, 1, rank, sink.to(DEV)).reshape(2, H, -1).cpu().to(F64)
+    assert not got[0].any()
+    s = torch.cat([q[1].to(F64) @ c.to(F64).T * rank ** -0.5, sink.to(F64)[:, None]], -1)
+    assert float((got[1] - (torch.softmax(s, -1)[:, :-1] @ c.to(F64))[:, : got.shape[2]]).abs().max()) < 1e-5

@@ -1424,10 +1424,11 @@ extern "C" int lsd_delta_chunk() { return DELTA_CT; }
 extern "C" hipError_t lsd_delta_split(const RecurParams* p, const bf16* x, long ldx, hipStream_t st) {
   if (p->s.B == 0 || p->chunks <= 0) return hipSuccess;
   if (p->D > 128 || p->V > 128 || !p->raw || !p->work) return hipErrorInvalidValue;
+  // (the attribute is the current device's, of which a process may use several: set at each call)
   const dim3 gf(p->heads, p->chunks, p->s.B), gs(p->heads * ((p->V + 16 * DELTA_WAVES - 1) / (16 * DELTA_WAVES)), p->s.B);
 #define LSD_DS(KS)                                                                                          \
   constexpr int lds = DeltaRing<KS, DELTA_WAVES>::BYTES;                                                     \
-  static const hipError_t room = hipFuncSetAttribute(                                                        \
+  const hipError_t room = hipFuncSetAttribute(                                                               \
       reinterpret_cast<const void*>(&delta_state_kernel<KS, DELTA_WAVES>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
   if (room != hipSuccess) return room;                                                                       \
   hipLaunchKernelGGL((delta_factors_kernel<KS>), gf, dim3(256), 0, st, *p, x, ldx);                           \

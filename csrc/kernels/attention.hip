@@ -398,7 +398,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_oproj_kernel(
 
 // Merge split-K decode partials: one wave per (sequence, head).  What it costs is the round
 // trips to memory: the partials of 16 splits are requested together with all maxima and sums,
-// not split by split behind them (1 sequence, 16 splits, with the kernel in front: 17.8 -> 6.9 us).
+// not split by split behind them (1 sequence, 16 splits, with the kernel in front: 17.8 -> 7.2 us).
 template <int HD>
 __global__ __launch_bounds__(64) void attn_decode_combine_kernel(const float* part_o,
                                                                  const float* part_ml, bf16* out,
@@ -645,8 +645,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
 // Waves are independent: no block barrier.  The math is ~2% of the HBM time
 // of the KV stream, so the kernel runs at the KV roofline.
 //
-// NW waves per block.  SPLIT_P: the weights enter the second product as two bf16 terms (value,
-// remainder), for the calls whose weights the VALU kernel would hold in fp32.
+// NW waves per block.  SPLIT_P: the weights enter the second product as three bf16 terms, which
+// hold all 24 bits of them, for the calls whose weights the VALU kernel would hold in fp32.
 template <int HD, int G, int NW, bool SPLIT_P>
 __global__ __launch_bounds__(NW * 64) void attn_decode_mfma_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ kc, const bf16* __restrict__ vc,
@@ -749,12 +749,14 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_mfma_kernel(
     for (int di = 0; di < HD / 16; ++di) o[di] *= alpha;
     // O^T += V^T . P^T over the 32 keys: k-slot j of group g <-> key 4g + j
     // (j < 4), 16 + 4g + (j - 4) (j >= 4)
-    bf16x8 pf, pl;
+    bf16x8 pf, pm, pl;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float e = sacc[j >> 2][j & 3];
       pf[j] = f2bf(e);
-      pl[j] = f2bf(e - bf2f(pf[j]));
+      const float e2 = e - bf2f(pf[j]);
+      pm[j] = f2bf(e2);
+      pl[j] = f2bf(e2 - bf2f(pm[j]));
     }
     const int r0 = 4 * g + (r >> 2);
 #pragma unroll
@@ -763,7 +765,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_mfma_kernel(
       const bf16x4 lo = ds_read_tr(vs + r0 * LDR + col);
       const bf16x4 hi = ds_read_tr(vs + (r0 + 16) * LDR + col);
       const bf16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      if constexpr (SPLIT_P) o[di] = mfma16(vf, pl, o[di]);
+      if constexpr (SPLIT_P) o[di] = mfma16(vf, pm, mfma16(vf, pl, o[di]));
       o[di] = mfma16(vf, pf, o[di]);
     }
   }
@@ -806,7 +808,7 @@ extern "C" void lsd_attn_set_small_waves128(int v) { g_attn_small_waves128 = v; 
 static int g_attn_large_waves64 = 4, g_attn_large_waves128 = 4;
 // grouped-query decode on MFMA (attn_decode_mfma_kernel) for HD = 128,
 // G in {2, 4, 8}: from this many waves ((sequence, kv head) items x context
-// splits) with bf16 weights, below with two terms; 0 = off
+// splits) with bf16 weights, below with three terms; 0 = off
 // (lsd_attn_set_mfma_min).
 static int g_attn_mfma_min = 256;
 extern "C" void lsd_attn_set_mfma_min(int v) { g_attn_mfma_min = v; }
@@ -835,8 +837,8 @@ static bool attn_on_mfma(int G, int hd) {
 
 // How many parts each of the caller's context splits is taken in (the partials are sized for
 // all): a wave needs about 1.1 us per 32 keys, so few waves take short ranges.  32 heads over
-// 8: 1 sequence of 912 keys, 4 splits -> 16: 13.0 -> 6.9 us; 8 of 2000, 4 -> 8: 22.3 -> 17.1; but
-// 40 of 780, 2 -> 4: 27.1 -> 32.0 (640 waves and more fill the chip).
+// 8: 1 sequence of 912 keys, 4 splits -> 16: 13.0 -> 6.9 us; 8 of 2000, 4 -> 8: 22.3 -> 17.1 (weights
+// in two terms; three add 3 %); but 40 of 780, 2 -> 4: 27.1 -> 32.0 (640 waves and more fill the chip).
 extern "C" int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits) {
   if (!attn_on_mfma(G, hd)) return 1;
   const long waves = (long)B * n_kv * splits, f = waves > 160 ? 640 / waves : 4;
@@ -852,9 +854,9 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
   const int G = nh / n_kv;
   const int n_items = B * n_kv;
   const int gx = g_attn_max_wg > 0 ? (n_items < g_attn_max_wg ? n_items : g_attn_max_wg) : n_items;
-  // grouped heads: on MFMA at any size (1 sequence of 912 keys with the merge 16.1 -> 6.9 us, 4 of
-  // them 17.0 -> 8.4, 1 of 100 11.7 -> 5.7 against the VALU kernel).  Below g_attn_mfma_min waves
-  // the weights keep a second term
+  // grouped heads: on MFMA at any size (1 sequence of 912 keys with the merge 15.7 -> 7.2 us, 4 of
+  // them 16.6 -> 8.8, 1 of 100 11.5 -> 5.8 against the VALU kernel).  Below g_attn_mfma_min waves
+  // the weights keep all their bits, in three terms (two of 16 bits together: 7.0, 8.5 and 5.7 us)
   if (attn_on_mfma(G, hd)) {
     const int f = lsd_attn_decode_split(B, n_kv, G, hd, splits);
     const bool few = (long)n_items * splits < g_attn_mfma_min;

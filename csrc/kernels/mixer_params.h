@@ -46,8 +46,8 @@ struct RecurParams {
                                        // Mamba-2: y silu(z) rows
   int write_ring;                      // single-token portions: this kernel keeps the ring
   // delta rule in chunks with factors of their own: chunks first .. first + chunks - 1 of
-  // every sequence, their factors at work[sequence][chunk][head].  Mamba-2 in segments: chunks
-  // of a segment, their states
+  // every sequence, their factors at work[sequence][chunk][head]; without: chunks first and on.
+  // Mamba-2 in segments: chunks of a segment, their states
   void* work; int first, chunks;
 };
 

@@ -528,7 +528,7 @@ __device__ __forceinline__ void delta_matrices(DeltaShared<DKS>& sm, int w) {
         }
 }
 
-// One block per (sequence, head), the whole chunk in it.
+// One block per (sequence, head), the whole chunk in it: chunks p.first and on.
 template <int DKS, int VTW>
 __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, const bf16* __restrict__ x, long ldx) {
   constexpr int CT = DELTA_CT, DP = DKS * 32, DT = DKS * 2, LDD = DeltaShared<DKS>::LDD, LDT = DeltaShared<DKS>::LDT;
@@ -538,7 +538,8 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
   const int r = lane & 15, g = lane >> 4;
   const int kh = h / (p.heads / p.groups);
   const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b], n = p.s.cu[b + 1] - r0;
-  if (n <= 0) return;
+  const int begin = p.first * CT;
+  if (n <= begin) return;
   float* Sg = p.S + ((long)slot * p.heads + h) * D * p.Vp;
   const float A = p.A[h], gain = p.c.gain;
   // uniform bases of the sequence's rows; offsets within a chunk are 32-bit
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int d = dt * 16 + 4 * g + i, v = (w * VTW + j) * 16 + r;
-        S[dt][j][i] = start > 0 && d < D && v < V ? Sg[d * p.Vp + v] : 0.f;
+        S[dt][j][i] = (start > 0 || begin > 0) && d < D && v < V ? Sg[d * p.Vp + v] : 0.f;
       }
   const float inv_sqrt_d = rsqrtf((float)D);
   float nrm[VTW];
@@ -584,8 +585,8 @@ __global__ __launch_bounds__(256, 2) void delta_chunk_kernel(RecurParams p, cons
     xl = ld8(lowb + (long)t0 * p.ldl + ol);
     rb = bf2f((yb + (long)t0 * p.c.ldy)[min(tid & 15, n - 1 - t0) * ldy]);
   };
-  fetch(0);
-  for (int t0 = 0; t0 < n; t0 += CT) {
+  fetch(begin);
+  for (int t0 = begin; t0 < n; t0 += CT) {
     const int nt = min(CT, n - t0);
     delta_factors<DKS>(sm, xq, xk, xl, rb, nt, elive, A, gain, inv_sqrt_d, [&]() {
       if (t0 + CT < n) fetch(t0 + CT);

@@ -188,7 +188,10 @@ void norm_and_gate(const RecurParams& p, int64_t T, bool f32) {
 }
 
 // Delta rule of few sequences: factors of many chunks at once, in portions of at most
-// 256 MB of them (9000 tokens of 16 heads of 128 x 128), then the chain.
+// 256 MB of them (528 chunks, 8448 tokens, of 16 heads of 128 x 128), then the chain.  max_rows
+// sizes the launches alone: a sequence that is longer goes on in the form without factors,
+// whose blocks find nothing to do otherwise (8 sequences of 150 tokens 91 -> 93 us; one sequence
+// is all rows, whatever is said).
 void run_delta_split(RecurParams p, const Tensor& y, int64_t max_rows) {
   const int64_t T = y.size(0), ld = (p.c.channels + 7) / 8 * 8, ct = lsd_delta_chunk();
   auto x = torch::empty({T, ld}, y.options());
@@ -205,12 +208,16 @@ void run_delta_split(RecurParams p, const Tensor& y, int64_t max_rows) {
     check_hip(lsd_delta_split(&p, xp, ld, cur_stream()), "delta_split");
   }
   norm_and_gate(p, T, false);
+  if (p.s.B > 1) {
+    p.first = (int)all; p.raw = nullptr;
+    check_hip(lsd_recur_chunk(&p, 1, xp, ld, cur_stream()), "recur_chunk");
+  }
 }
 
 // y [T, N] rows of q | k | v conv channels from column c0 and beta's logits from
 // gate_col; low [T, >= heads D at 0, heads V at gate_off].  Token by
-// token, or (chunked) prompts of bf16 models; max_rows: rows of the longest sequence (0:
-// not known).  split: factors of their own, -1 where that is faster -- with the convolution, 16
+// token, or (chunked) prompts of bf16 models; max_rows: rows of the longest sequence, to size
+// launches by (0: not known).  split: factors of their own, -1 where that is faster -- with the convolution, 16
 // heads of 128 x 128 and 1000 tokens each: 4 sequences 709 -> 232 us, 8 616 -> 403, 12 842 -> 681,
 // 16 750 -> 842; one of 20 tokens 42 -> 35, of 4000 2170 -> 404, of 16000 11690 -> 1600
 void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_off, Tensor slots, Tensor start,
@@ -237,7 +244,7 @@ void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_
     TORCH_CHECK(!f32 && !single && lsd_chunk_ok(1, D, V, groups, heads), "delta_seq: no chunked kernel");
     TORCH_CHECK(max_rows >= 0 && split >= -1 && split <= 1 && p.s.B <= 65535, "delta_seq: max_rows, split");
     if (split == 1 || (split < 0 && (int64_t)p.s.B * heads <= 192))
-      run_delta_split(p, y, max_rows > 0 ? std::min(max_rows, y.size(0)) : y.size(0));
+      run_delta_split(p, y, max_rows > 0 && p.s.B > 1 ? std::min(max_rows, y.size(0)) : y.size(0));
     else
       run_chunks(p, y);
     check_hip(lsd_conv_tail(&p.c, &p.s, f32, cur_stream()), "conv_tail");

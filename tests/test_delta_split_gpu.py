@@ -58,3 +58,14 @@ def test_long_sequences_in_portions(C):
     a, b = (run(C, s, lens, [0] * 8, 32, 32, 128, 128, max_rows=520) for s in (0, 1))
     assert bool(((a[0] - b[0]).abs() <= 2.0 ** -7 * (a[0].abs() + a[0].pow(2).mean().sqrt())).all())
     assert bool(((a[1] - b[1]).abs() <= 1e-4 * a[1].abs().amax()).all())
+
+
+@pytest.mark.parametrize("lens,starts,hint", [([100, 37, 16], [0, 9, 0], 16), ([100, 37, 16], [0, 9, 0], 40),
+                                              ([48, 33, 1], [4, 0, 0], 1), ([70], [0], 5)])
+def test_longer_than_said(C, lens, starts, hint):
+    """max_rows sizes launches: rows behind it are not left out, whatever it says."""
+    a, b = (run(C, s, lens, starts, 2, 1, 128, 128, max_rows=m) for s, m in ((0, 0), (1, hint)))
+    assert not b[0].isnan().any()
+    assert bool(((a[0] - b[0]).abs() <= 2.0 ** -7 * (a[0].abs() + a[0].pow(2).mean().sqrt())).all())
+    assert bool(((a[1] - b[1]).abs() <= 1e-4 * a[1].abs().amax()).all())
+    assert torch.equal(a[2], b[2])

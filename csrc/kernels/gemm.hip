@@ -1825,9 +1825,9 @@ using namespace lsd;
 extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits);  // gemm_deep.hip
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st);
 
-// Kinds 0 and 1 of up to 128 rows, and up to 256 of few blocks, run on the deep ring
-// (gemm_deep.hip), which is faster there at every shape (its head has both times); the split-K
-// kernel takes what has no whole k-steps of 64, the ring and tiled kernels what has more rows.
+// Kinds 0 and 1 of up to 48 rows, and up to 256 of few blocks, run on the deep ring where K has
+// whole k-steps of 64 (gemm_deep.hip has the line and both sides' times); the split-K kernel,
+// the rings and the tiled kernels take the rest.
 extern "C" int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits) {
   return kind <= 1 && lsd_gemm_deep_ok(M, N, K, epi, splits);
 }

@@ -237,17 +237,22 @@ static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
 using namespace lsd;
 
 // 1 .. 256 rows, whole k-steps; gate / up pairs lie in one tile.  splits > 1 only as slabs:
-// the other epilogues run unsplit, whatever the caller asked for.  More than 128 rows are two
-// row blocks, which is faster than the larger tiles up to two blocks a CU: whole steps of 48
-// layers of 1600, 160 sequences 4472 -> 4117 us, 256 5426 -> 5326; 12 layers of 2048, 140 sequences
-// 1285 -> 1198.  Not with more: 4096 x 14336 at 256 rows in 8 slabs, 1024 blocks, 47.5 -> 57.2 us.
+// the other epilogues run unsplit, whatever the caller asked for.  More than 48 rows only up to
+// two blocks a CU (49 .. 64 rows two and a half): behind that the 128 x 128 tiles, which read A half
+// as often, are as fast or faster.  Vocabulary-wide, deep ring against those tiles:
+//   50304 x 1600  64 rows 40.3 against 37.0 us, 96 50 against 41, 128 56 against 44 (48 rows 38 and 37)
+//   128256 x 4096  64 rows 220 against 203, 128 260 against 208 (40 rows both 190)
+//   40960 x 1600  64 rows 31.5 against 35, 80 36 against 37, 128 44 against 42
+// More than 128 rows are two row blocks: whole steps of 48 layers of 1600, 160 sequences
+// 4472 -> 4117 us, 256 5426 -> 5326; 12 layers of 2048, 140 sequences 1285 -> 1198; not with more
+// blocks: 4096 x 14336 at 256 rows in 8 slabs, 1024 of them, 47.5 -> 57.2 us.
 extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits) {
   if (M < 1 || M > 256 || K < 64 || K % 64 != 0 || N % (epi == EPI_SILU_MUL ? 32 : 16) != 0) return 0;
   if (epi != EPI_SLAB) splits = 1;
   if (splits < 1 || splits > K / 64) return 0;
-  if (M <= 128) return 1;
+  if (M <= 48) return 1;
   const int bn = deep_cols(M, N, K, splits, epi);
-  return (long)((N + bn - 1) / bn) * splits * 2 <= 512;
+  return (long)((N + bn - 1) / bn) * splits * (M > 128 ? 2 : 1) <= (M > 64 ? 512 : 640);
 }
 
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st) {

@@ -60,3 +60,22 @@ def test_gemv_ok_matches_dispatch():
         for norm in (0, 1, 2):
             ok = bool(_C.gemv_ok(1, 1600, epi, norm))
             assert ok == ((epi, norm) in dispatched), (epi, norm)
+
+
+def test_deep_ring_leaves_wide_outputs_to_the_tiles():
+    """The deep ring (gemm_deep.hip) holds all rows of a block: with more than 48 rows, outputs
+    of more blocks than run together (vocabularies) are faster on the 128 x 128 tiles."""
+    import pytest
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+    EPI_F32, EPI_SLAB = 3, 5
+
+    for M, N, K, epi, splits, want in [
+            (9, 50304, 1600, EPI_F32, 1, True), (48, 128256, 4096, EPI_F32, 1, True), (49, 50304, 1600, EPI_F32, 1, False),
+            (64, 40960, 1600, EPI_F32, 1, True), (64, 128256, 4096, EPI_F32, 1, False), (65, 32768, 2048, EPI_F32, 1, True),
+            (65, 32832, 2048, EPI_F32, 1, False), (128, 50304, 768, EPI_F32, 1, False), (256, 50304, 768, EPI_F32, 1, False),
+            (40, 1600, 1632, EPI_F32, 1, False), (128, 4096, 14336, EPI_SLAB, 8, True), (257, 1600, 1600, EPI_F32, 1, False)]:
+        assert _C.gemm_on_deep(M, N, K, epi, 1, splits) == want, (M, N, K)
+    assert not _C.gemm_on_deep(40, 4096, 4096, EPI_F32, 2, 1)  # the all-rows kernel

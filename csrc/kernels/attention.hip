@@ -840,19 +840,32 @@ static bool attn_on_mfma(int G, int hd) {
 }
 
 // How many parts each of the caller's context splits is taken in (the partials are sized for
-// all): a wave needs about 1.1 us per 32 keys, so few waves take short ranges.  32 heads over
+// all): few waves take short ranges.  A wave needs about 1.2 us per 32 keys; a merge, where the
+// caller's splits have none, 2.4 us and what its (sequence, head) pairs add.  32 heads over
 // 8: 1 sequence of 912 keys, 4 splits -> 16: 13.0 -> 6.9 us; 8 of 2000, 4 -> 8: 22.3 -> 17.1 (weights
 // in two terms; three add 3 %); but 40 of 780, 2 -> 4: 27.1 -> 32.0 (640 waves and more fill the chip).
-extern "C" int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits) {
+// One launch against two parts and their merge: 32 sequences of 20 keys 3.8 against 7.1 us, of
+// 130 8.2 against 10.4, of 260 14 against 13.2; four parts: 1 sequence of 60 keys 4.8 against
+// 5.8, of 100 7.3 against 6.0.  keys: the longest context, 0 where the caller does not know it.
+extern "C" int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits, int keys) {
   if (!attn_on_mfma(G, hd)) return 1;
-  const long waves = (long)B * n_kv * splits, f = waves > 160 ? 640 / waves : 4;
-  return f < 1 ? 1 : (int)(f * splits <= 256 ? f : 256 / splits);
+  const long waves = (long)B * n_kv * splits;
+  const int most = waves > 160 ? (int)(640 / waves) : 4;
+  int best = 1;
+  long least = 0;
+  for (int f = 1; f == 1 || (f <= most && f * splits <= 256); ++f) {
+    const long tiles = ((long)keys + 32 * splits * f - 1) / (32 * splits * f);
+    const long cost = 120 * tiles + (splits * f > 1 ? 240 + (long)B * n_kv * G / 5 : 0);  // 1/100 us
+    if (f == 1 || cost < least) { best = f; least = cost; }
+  }
+  return best;
 }
 
+// parts: lsd_attn_decode_split's; part_o and part_ml hold splits x parts
 extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                                       const int* seq_slots, const int* qpos, bf16* out, long ldo,
                                       float* part_o, float* part_ml, int B, int nh, int n_kv,
-                                      int hd, int max_seq, int splits, float scale_log2,
+                                      int hd, int max_seq, int splits, int parts, float scale_log2,
                                       hipStream_t st) {
   if (B == 0) return hipSuccess;
   const int G = nh / n_kv;
@@ -861,10 +874,11 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
   // grouped heads: on MFMA at any size (1 sequence of 912 keys with the merge 15.7 -> 7.2 us, 4 of
   // them 16.6 -> 8.8, 1 of 100 11.5 -> 5.8 against the VALU kernel).  Below g_attn_mfma_min waves
   // the weights keep all their bits, in three terms (two of 16 bits together: 7.0, 8.5 and 5.7 us)
+  // (16 heads over 8, 24 sequences of 130 keys: 8.2 -> 9.4 us, where the VALU kernel is ahead; of
+  // 60 and of 260 5.6 -> 5.3 and 13.8 -> 12.1)
   if (attn_on_mfma(G, hd)) {
-    const int f = lsd_attn_decode_split(B, n_kv, G, hd, splits);
     const bool few = (long)n_items * splits < g_attn_mfma_min;
-    splits *= f;
+    splits *= parts;
 #define LSD_DEC_MFMA(GV, NWV, SP)                                                                \
   if (G == GV && few == SP && (n_items * splits <= 1024) == (NWV == 1)) {                        \
     hipLaunchKernelGGL((attn_decode_mfma_kernel<128, GV, NWV, SP>), dim3((n_items + NWV - 1) / NWV, splits), \

@@ -1142,7 +1142,7 @@ class HipBackend(Backend):
         nh = q.shape[1] // hd
         if meta.is_decode:
             splits = self.decode_attn_splits(meta.num_seqs, nh, n_kv, hd, meta.max_ctx)
-            return self.C.attn_decode(q, cache_k, cache_v, meta.seq_slots, meta.token_pos, nh, splits)
+            return self.C.attn_decode(q, cache_k, cache_v, meta.seq_slots, meta.token_pos, nh, splits, meta.max_ctx)
         tiles, rows = self._plain_tiles(meta, nh, q.device)
         return self.C.attn_prefill(q, cache_k, cache_v, tiles, meta.seq_slots, meta.q_start,
                                    meta.cu_q, nh, rows)

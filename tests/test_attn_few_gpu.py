@@ -13,7 +13,8 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("nh,n_kv", [(4, 2), (32, 8), (8, 1)])
 @pytest.mark.parametrize("splits", [1, 3, 4, 32, 200])
 @pytest.mark.parametrize("last", [0, 30, 31, 32, 128, 911])
-def test_few_sequences(B, nh, n_kv, splits, last):
+@pytest.mark.parametrize("keys", [0, 912])  # (known: ranges are taken in parts)
+def test_few_sequences(B, nh, n_kv, splits, last, keys):
     from llm_sharding_demo_amd import _C as C
 
     hd, S = 128, 920
@@ -25,7 +26,7 @@ def test_few_sequences(B, nh, n_kv, splits, last):
         kc[s, :, p + 1:], vc[s, :, p + 1:] = float("nan"), float("nan")
     i32 = dict(dtype=torch.int32, device=DEV)
     args = (q.to(DEV), kc.to(DEV), vc.to(DEV), torch.tensor(slots, **i32), torch.tensor(pos, **i32), nh, splits)
-    got = C.attn_decode(*args).cpu().double().reshape(B, nh, hd)
+    got = C.attn_decode(*args, keys).cpu().double().reshape(B, nh, hd)
     C.attn_set_mfma_min(0)
     try:
         valu = C.attn_decode(*args).cpu().double().reshape(B, nh, hd)

@@ -79,3 +79,20 @@ def test_deep_ring_leaves_wide_outputs_to_the_tiles():
             (40, 1600, 1632, EPI_F32, 1, False), (128, 4096, 14336, EPI_SLAB, 8, True), (257, 1600, 1600, EPI_F32, 1, False)]:
         assert _C.gemm_on_deep(M, N, K, epi, 1, splits) == want, (M, N, K)
     assert not _C.gemm_on_deep(40, 4096, 4096, EPI_F32, 2, 1)  # the all-rows kernel
+
+
+def test_decode_attention_parts_by_context():
+    """Few waves take their ranges of keys in parts, unless the merge costs more than
+    they save: one unsplit launch for short contexts, no parts of less than a tile."""
+    import pytest
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+
+    for B, n_kv, splits, keys, want in [(32, 8, 1, 20, 1), (32, 8, 1, 130, 1), (32, 8, 1, 260, 2), (16, 8, 1, 60, 1),
+                                        (1, 8, 1, 20, 1), (1, 8, 1, 60, 1), (1, 8, 1, 100, 4), (1, 8, 4, 912, 4),
+                                        (1, 8, 4, 100, 1), (40, 8, 2, 780, 1), (1, 8, 200, 8000, 1), (1, 8, 4, 0, 1),
+                                        (1, 1, 100, 8000, 2), (0, 8, 1, 100, 4)]:
+        assert _C.attn_decode_split(B, n_kv, 4, 128, splits, keys) == want, (B, splits, keys)
+    assert _C.attn_decode_split(1, 8, 3, 128, 1, 900) == 1 and _C.attn_decode_split(1, 8, 4, 64, 1, 900) == 1

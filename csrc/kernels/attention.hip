@@ -397,14 +397,17 @@ __global__ __launch_bounds__(NWV * 64) void attn_oproj_kernel(
 }
 
 // Merge split-K decode partials: one wave per (sequence, head).  What it costs is the round
-// trips to memory: the partials of 16 splits are requested together with all maxima and sums,
+// trips to memory: the partials of AT_ONCE splits are requested together with all maxima and sums,
 // not split by split behind them (1 sequence, 16 splits, with the kernel in front: 17.8 -> 7.2 us).
-template <int HD>
+// MAXL: splits / 64, rounded up.  Requests beyond the last split are not free: 16 of them for two
+// splits cost more than two loads in turn (4 sequences of 260 keys, 12 heads of 64: 6.9 -> 7.2 us; with
+// 4 at once 6.9), so up to 4 splits take the short form.
+template <int HD, int AT_ONCE, int MAXL>
 __global__ __launch_bounds__(64) void attn_decode_combine_kernel(const float* part_o,
                                                                  const float* part_ml, bf16* out,
                                                                  long ldo, int nh, int splits) {
-  constexpr int DPL = HD / 64, AT_ONCE = 16, MAXL = 256 / 64;  // columns per lane; splits <= 256
-  __shared__ float ws[256];
+  constexpr int DPL = HD / 64;  // columns per lane
+  __shared__ float ws[64 * MAXL];
   const int b = blockIdx.x / nh, h = blockIdx.x % nh, lane = threadIdx.x;
   const long p0 = ((long)b * nh + h) * splits;
   const float* po = part_o + p0 * HD + lane * DPL;
@@ -825,12 +828,17 @@ extern "C" void lsd_attn_set_large_waves(int hd, int v) {
 static hipError_t attn_decode_combine(const float* part_o, const float* part_ml, bf16* out, long ldo,
                                       int B, int nh, int hd, int splits, hipStream_t st) {
   if (splits > 1) {
-    if (hd == 64)
-      hipLaunchKernelGGL((attn_decode_combine_kernel<64>), dim3(B * nh), dim3(64), 0, st, part_o,
-                         part_ml, out, ldo, nh, splits);
-    else
-      hipLaunchKernelGGL((attn_decode_combine_kernel<128>), dim3(B * nh), dim3(64), 0, st, part_o,
-                         part_ml, out, ldo, nh, splits);
+#define LSD_COMBINE(HDV, AT, ML)                                                                  \
+  hipLaunchKernelGGL((attn_decode_combine_kernel<HDV, AT, ML>), dim3(B * nh), dim3(64), 0, st,     \
+                     part_o, part_ml, out, ldo, nh, splits)
+#define LSD_COMBINE_HD(HDV)                                      \
+  if (splits <= 4) LSD_COMBINE(HDV, 4, 1);                       \
+  else if (splits <= 64) LSD_COMBINE(HDV, 16, 1);                \
+  else LSD_COMBINE(HDV, 16, 4);
+    if (splits > 256) return hipErrorInvalidValue;
+    if (hd == 64) { LSD_COMBINE_HD(64) } else { LSD_COMBINE_HD(128) }
+#undef LSD_COMBINE_HD
+#undef LSD_COMBINE
   }
   return hipGetLastError();
 }

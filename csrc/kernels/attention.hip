@@ -888,14 +888,14 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
     const bool few = (long)n_items * splits < g_attn_mfma_min;
     splits *= parts;
 #define LSD_DEC_MFMA(GV, NWV, SP)                                                                \
-  if (G == GV && few == SP && (n_items * splits <= 1024) == (NWV == 1)) {                        \
+  if (G == GV && few == SP && (few || n_items * splits <= 1024) == (NWV == 1)) {                 \
     hipLaunchKernelGGL((attn_decode_mfma_kernel<128, GV, NWV, SP>), dim3((n_items + NWV - 1) / NWV, splits), \
                        dim3(64 * NWV), 0, st, q, ldq, kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml, \
                        n_kv, max_seq, splits, scale_log2, n_items);                              \
     return attn_decode_combine(part_o, part_ml, out, ldo, B, nh, hd, splits, st);                \
   }
 #define LSD_DEC_MFMA_G(GV) \
-  LSD_DEC_MFMA(GV, 1, true) LSD_DEC_MFMA(GV, 1, false) LSD_DEC_MFMA(GV, 4, true) LSD_DEC_MFMA(GV, 4, false)
+  LSD_DEC_MFMA(GV, 1, true) LSD_DEC_MFMA(GV, 1, false) LSD_DEC_MFMA(GV, 4, false)
     LSD_DEC_MFMA_G(2)
     LSD_DEC_MFMA_G(4)
     LSD_DEC_MFMA_G(8)

@@ -53,6 +53,20 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// s_waitcnt immediate for vmcnt(n) alone (gfx9 layout: vmcnt[3:0] | vmcnt[5:4] << 14)
+constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
+
+// f(Int<N - 1>) .. f(Int<0>): counted waits need their counts at compile time
+template <int V>
+struct Int {
+  static constexpr int v = V;
+};
+template <int N, class F>
+__device__ __forceinline__ void count_down(F f) {
+  f(Int<N - 1>{});
+  if constexpr (N > 1) count_down<N - 1>(f);
+}
+
 template <typename T>
 __device__ __forceinline__ T shfl_xor(T v, int m) { return __shfl_xor(v, m, 64); }
 

@@ -28,16 +28,6 @@ namespace {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void gbl_cvoid;
 constexpr int NT_LOAD = 2;  // cache policy of an LDS-DMA: non-temporal
-
-template <int V>
-struct Int {
-  static constexpr int v = V;
-};
-template <int N, class F>
-__device__ __forceinline__ void count_down(F f) {  // f(N - 1) .. f(0), compile-time
-  f(Int<N - 1>{});
-  if constexpr (N > 1) count_down<N - 1>(f);
-}
 }  // namespace
 
 // WM x WN waves of MTW x NTW 16 x 16 tiles, times WK waves on different 32-wide parts of a

@@ -136,9 +136,6 @@ __device__ __forceinline__ void epilogue4(const GemmParams& p, int row0, int n, 
 //   epi8_pre  -- bias, residual x, QKV position / slot      (independent loads)
 //   epi8_pre2 -- QKV RoPE (cos, sin) of that position        (dependent loads)
 //   epi8_post -- the math and the stores
-// s_waitcnt immediate for vmcnt(n) alone (gfx9 layout: vmcnt[3:0] | vmcnt[5:4] << 14)
-constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
 struct Epi8Pre {
   bf16x8 b;
   f32x4 x0, x1, cs0, cs1;

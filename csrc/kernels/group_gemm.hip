@@ -32,17 +32,6 @@ namespace gg {
 constexpr int BK = 64;
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void gbl_cvoid;
-constexpr int vmcnt(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
-template <int V>
-struct Int {
-  static constexpr int v = V;
-};
-template <int N, class F>
-__device__ __forceinline__ void count_down(F f) {  // f(N - 1) .. f(0), compile-time
-  f(Int<N - 1>{});
-  if constexpr (N > 1) count_down<N - 1>(f);
-}
 
 // Where one row tile's operands are.
 struct Tile {
@@ -256,7 +245,7 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
   };
   if constexpr (D == 1) {
     while (kt < KT) {
-      __builtin_amdgcn_s_waitcnt(vmcnt(0));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
       turn(kt + 1 < KT);
     }
   } else {
@@ -265,19 +254,19 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
     count_down<D - 1>([&](auto ic) {
       constexpr int d = decltype(ic)::v + 1;  // filled steps after kt
       if (kt + D < KT) {
-        __builtin_amdgcn_s_waitcnt(vmcnt(LPA * d + LPS * (D - 1 - d)));
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPA * d + LPS * (D - 1 - d)));
         turn(true);
       }
     });
     while (kt + D < KT) {
-      __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (D - 1)));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (D - 1)));
       turn(true);
     }
     count_down<D>([&](auto ic) {  // the last D steps, nothing left to issue
       constexpr int d = decltype(ic)::v;
       if (KT - 1 - kt == d) {
-        if (KT >= 2 * D) __builtin_amdgcn_s_waitcnt(vmcnt(LPS * d));
-        else __builtin_amdgcn_s_waitcnt(vmcnt(LPA * d));  // filled ones: A alone is behind
+        if (KT >= 2 * D) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * d));
+        else __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPA * d));  // filled ones: A alone is behind
         turn(false);
       }
     });
@@ -393,7 +382,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   f32x4 acc[2][MT];  // halves of the sums: a chain half as long rounds less
 #pragma unroll
   for (int i = 0; i < MT; ++i) acc[0][i] = acc[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  __builtin_amdgcn_s_waitcnt(vmcnt(0));  // the routing loads are done before loads are counted
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the routing loads are done before loads are counted
   const int KT = t.K / BKF;
 #pragma unroll
   for (int d = 0; d < SLOTS; ++d)
@@ -402,9 +391,9 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   auto landed = [&](int kt) {
     constexpr int NO_LDS = ~0xf00;  // and no LDS read under way
     const int later = min(SLOTS - 1 - (kt > 0), KT - 1 - kt);
-    if (later == 2) __builtin_amdgcn_s_waitcnt(vmcnt(2 * LPS) & NO_LDS);
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt(LPS) & NO_LDS);
-    else __builtin_amdgcn_s_waitcnt(vmcnt(0) & NO_LDS);
+    if (later == 2) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * LPS) & NO_LDS);
+    else if (later == 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS) & NO_LDS);
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0) & NO_LDS);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };

@@ -835,8 +835,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void delta_state_kernel(RecurParams 
       }
   };
   auto first4 = [](bf16x8 a) { return bf16x4{a[0], a[1], a[2], a[3]}; };
-  constexpr auto vmcnt = [](int k) { return (k & 0xF) | ((k >> 4) << 14) | (0x7 << 4) | (0xF << 8); };
-  __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 1)));  // chunk 0 has landed
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 1)));  // chunk 0 has landed
   __builtin_amdgcn_s_barrier();
   factors(0);
   for (int c = 0; c < nc; ++c) {
@@ -868,8 +867,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void delta_state_kernel(RecurParams 
     // chunk c is read by everyone, chunk c + 1 has landed: behind its loads are those of
     // SLOTS - 2 chunks and, once as many chunks have ended, four stores of each
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    if (c >= SLOTS - 1) __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 2) + 4 * (SLOTS - 1)));
-    else __builtin_amdgcn_s_waitcnt(vmcnt(LPS * (SLOTS - 2)));
+    if (c >= SLOTS - 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 2) + 4 * (SLOTS - 1)));
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 2)));
     __builtin_amdgcn_s_barrier();
     issue(c + SLOTS);
     factors(c + 1);  // past the end: chunk nc - 1 again

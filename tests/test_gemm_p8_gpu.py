@@ -25,9 +25,12 @@ def near(got, want, slack):
     return bool(((got - want).abs() <= slack + step * want.abs()).all())
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 64, 64), (256, 256, 128), (257, 288, 192), (300, 1600, 64), (511, 544, 448)])
+# (256 rows: the deep ring)
+@pytest.mark.parametrize("M,N,K", [(256, 64, 64), (256, 256, 128), (257, 288, 192), (300, 1600, 64), (511, 544, 448),
+                                   (512, 64, 64), (512, 256, 128)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_epilogues(C, M, N, K, bias):
+    assert C.gemm_on_deep(M, N, K, 0, 1, 1) == (M <= 256)
     g = torch.Generator().manual_seed(M + N)
     a, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
     b = torch.randn(N, generator=g).bfloat16() if bias else None

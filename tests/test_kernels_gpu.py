@@ -155,9 +155,9 @@ def _fp32_slabs(C):
     C.gemm_set_slab_bf16(int(prev))
 
 
-# 8-wave decode ring (256 / 130 rows), split-K decode kernel (64 rows, deferred) and the
-# 256x256 prefill-class kernel (1024 rows x 6 splits = 168 tiles)
-@pytest.mark.parametrize("tiled,M,splits", [(True, 256, 3), (True, 256, 5), (True, 130, 3), (False, 64, 5),
+# deep ring (64 to 256 rows), 8-wave ring (300 rows) and the 256x256 prefill-class kernel
+# (1024 rows x 6 splits = 168 tiles)
+@pytest.mark.parametrize("tiled,M,splits", [(True, 256, 3), (True, 256, 5), (True, 130, 3), (False, 64, 5), (True, 300, 5),
                                             (True, 1024, 6), (True, 1024, 1), (True, 3000, 1)])
 def test_linear_residual_bf16_slabs(C, CNT, tiled, M, splits):
     """bf16 partial slabs: each split's partial rounded once to bf16 (a bf16
@@ -182,13 +182,15 @@ def test_linear_residual_bf16_slabs(C, CNT, tiled, M, splits):
 @pytest.mark.parametrize("M", [1, 5, 16, 33, 64, 65, 100, 128, 200])
 @pytest.mark.parametrize("act", ["none", "gelu", "silu_mul"])
 @pytest.mark.parametrize("splits", [1, 3, 7])
-def test_linear(C, CNT, M, act, splits):
+@pytest.mark.parametrize("K", [640, 672])  # whole 64-wide steps: deep ring; others: split-K kernel
+def test_linear(C, CNT, M, act, splits, K):
     from llm_sharding_demo_amd.ops.hip import interleave_gate_up
 
-    N, K = 384, 640
+    N = 384
     a, w, bias = bf(M, K, seed=5), bf(N, K, scale=0.05, seed=6), bf(N, scale=0.1, seed=7)
-    tiled = M > 128
+    tiled = M > 128 and K % 64 == 0
     sp = 1 if tiled else splits
+    assert C.gemm_on_deep(M, N, K, 0, int(tiled), sp) == (K % 64 == 0)
     if act == "silu_mul":
         N = 256
         w = w[:N].contiguous()
@@ -205,10 +207,12 @@ def test_linear(C, CNT, M, act, splits):
 
 @pytest.mark.parametrize("M,splits", [(3, 1), (16, 4), (64, 5), (64, 16), (100, 1), (128, 5), (130, 3)])
 @pytest.mark.parametrize("defer", [False, True])
-def test_linear_residual_and_f32(C, CNT, M, splits, defer):
-    N, K = 256, 1024
+@pytest.mark.parametrize("K", [1024, 1056])  # deep ring, split-K kernel
+def test_linear_residual_and_f32(C, CNT, M, splits, defer, K):
+    N = 256
     a, w, bias = bf(M, K, seed=8), bf(N, K, scale=0.05, seed=9), bf(N, scale=0.1, seed=10)
-    tiled = M > 128
+    tiled = M > 128 and K % 64 == 0
+    assert C.gemm_on_deep(M, N, K, 4, int(tiled), splits) == (K % 64 == 0)
     x = torch.randn(M, N, device=DEV)
     x_ref = x + ref.linear(a, w, bias)
     slab = C.linear_residual(a, w, bias, x, splits, tiled, CNT, defer)
@@ -217,15 +221,18 @@ def test_linear_residual_and_f32(C, CNT, M, splits, defer):
         C.norm(x, slab, bias, None, None, 0.0, True, None, False)
     close(x, x_ref, 2e-3, 1e-3)
     close(C.linear_f32(a, w, tiled, 1 if tiled else splits, CNT), ref.linear(a, w), 2e-3, 1e-3)
+    assert int(CNT.abs().sum()) == 0
 
 
 @pytest.mark.parametrize("M", [1, 40, 128])
-def test_decode_gemm_wide_partial_tiles(C, CNT, M):
+@pytest.mark.parametrize("K", [512, 544])  # deep ring, split-K kernel
+def test_decode_gemm_wide_partial_tiles(C, CNT, M, K):
     """128-column decode tiles (NW = 2) with a masked partial last tile
     (N = 320 = 2.5 tiles): plain, GELU, split-K residual and fp32 epilogues."""
     C.gemm_set_nw2_rows(0)
     try:
-        N, K = 320, 512
+        N = 320
+        assert C.gemm_on_deep(M, N, K, 1, 0, 3) == (K % 64 == 0)
         a, w, bias = bf(M, K, seed=40), bf(N, K, scale=0.05, seed=41), bf(N, scale=0.1, seed=42)
         assert C.gemm_sk_nw(M, 0) == 2
         for sp in (1, 3):
@@ -242,12 +249,14 @@ def test_decode_gemm_wide_partial_tiles(C, CNT, M):
 
 @pytest.mark.parametrize("M", [129, 200, 256])
 @pytest.mark.parametrize("splits", [1, 3])
-def test_decode_gemm_two_row_blocks(C, CNT, M, splits):
+@pytest.mark.parametrize("K", [640, 672])  # deep ring, split-K kernel
+def test_decode_gemm_two_row_blocks(C, CNT, M, splits, K):
     """Decode GEMM above 128 rows runs as >= 2 row blocks of <= 128 (grid z)
     sharing each W tile: plain / GELU / SiLU-mul / fp32 / residual epilogues."""
     from llm_sharding_demo_amd.ops.hip import interleave_gate_up
 
-    N, K = 384, 640
+    N = 384
+    assert C.gemm_on_deep(M, N, K, 0, 0, splits) == (K % 64 == 0)
     a, w, bias = bf(M, K, seed=50), bf(N, K, scale=0.05, seed=51), bf(N, scale=0.1, seed=52)
     assert C.gemm_sk_rblocks(M, N, splits) >= 2
     close(C.linear(a, w, bias, 0, False, splits, CNT), ref.linear(a, w, bias), 3e-2)
@@ -266,11 +275,15 @@ def test_decode_gemm_two_row_blocks(C, CNT, M, splits):
     assert int(CNT.abs().sum()) == 0
 
 
-def test_split_k_deterministic(C, CNT):
-    a, w = bf(64, 1600, seed=30), bf(4800, 1600, scale=0.03, seed=31)
+@pytest.mark.parametrize("K", [1600, 1632])  # deep ring, split-K kernel
+def test_split_k_deterministic(C, CNT, K):
+    assert C.gemm_on_deep(64, 4800, K, 0, 0, 7) == (K % 64 == 0)
+    a, w = bf(64, K, seed=30), bf(4800, K, scale=0.03, seed=31)
     y1 = C.linear(a, w, None, 0, False, 7, CNT)
     for _ in range(5):
         assert torch.equal(C.linear(a, w, None, 0, False, 7, CNT), y1)
+    close(y1, ref.linear(a, w), 3e-2)
+    assert int(CNT.abs().sum()) == 0
 
 
 def test_gemm_large_prefill_shape(C, CNT):
@@ -293,15 +306,17 @@ def RING(C, request):
     C.gemm_set_ring_tn(128)
 
 
-@pytest.mark.parametrize("M", [100, 256, 300])
+@pytest.mark.parametrize("M", [100, 256, 257, 300, 384])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 640])
 def test_ring_gemm_epilogues(RING, CNT, M, K):
-    """Ring 128x128 kernel: every epilogue, M/N tails, 1, 2, 3, 4 and 10
-    k-steps (fewer than, equal to and more than the ring), split-K slabs."""
+    """Ring 128x128 kernel (above 256 rows; below, the deep ring): every epilogue,
+    M/N tails, 1, 2, 3, 4 and 10 k-steps (fewer than, equal to and more than the
+    ring), split-K slabs."""
     from llm_sharding_demo_amd.ops.hip import interleave_gate_up
 
     C = RING
     N = 352  # 2.75 tiles of 128 columns, 5.5 of 64: a partial last tile either way
+    assert C.gemm_on_deep(M, N, K, 0, 1, 1) == (M <= 256)
     a, w, bias = bf(M, K, seed=60), bf(N, K, scale=0.05, seed=61), bf(N, scale=0.1, seed=62)
     y_ref = ref.linear(a, w, bias)
     close(C.linear(a, w, bias, 0, True, 1, CNT), y_ref, 3e-2)
@@ -322,11 +337,12 @@ def test_ring_gemm_epilogues(RING, CNT, M, K):
         close(x, x_ref, 2e-3, 1e-3)
 
 
-@pytest.mark.parametrize("M", [129, 200, 256, 300])
+@pytest.mark.parametrize("M", [129, 200, 256, 257, 300, 384])
 @pytest.mark.parametrize("K", [64, 192, 640])
 def test_ring_gemm_96_row_tiles(C, CNT, M, K):
-    """Ring kernel with 96-row tiles (3 MFMA row tiles per wave): every
-    epilogue, partial row / column tiles, k-steps fewer than and beyond the ring."""
+    """Ring kernel with 96-row tiles (3 MFMA row tiles per wave; above 256 rows,
+    below the deep ring): every epilogue, partial row / column tiles, k-steps fewer
+    than and beyond the ring."""
     from llm_sharding_demo_amd.ops.hip import interleave_gate_up
 
     C.gemm_set_tiled3_max(1 << 30)
@@ -369,18 +385,21 @@ def RING8(C, request):
     C.gemm_set_ring_tn(128)
 
 
-@pytest.mark.parametrize("M", [100, 200, 256])
+@pytest.mark.parametrize("M", [100, 200, 256, 257, 300, 513])
 @pytest.mark.parametrize("K,splits", [(64, 1), (192, 1), (640, 1), (640, 2), (1600, 1), (1600, 3), (1600, 4)])
 def test_ring8_gemm_epilogues(RING8, CNT, M, K, splits):
-    """8-wave decode ring: every epilogue, M / N tails, 1 to 25 k-steps,
-    in-kernel split-K combine (8 computing waves) bit-stable across launches
-    that reuse the re-armed ticket counters, residual slabs folded by the norm."""
+    """8-wave decode ring (above 256 rows; below, the deep ring): every epilogue,
+    M / N tails, 1 to 25 k-steps, in-kernel split-K combine (8 computing waves)
+    bit-stable across launches that reuse the re-armed ticket counters, residual
+    slabs folded by the norm."""
     from llm_sharding_demo_amd.ops.hip import interleave_gate_up
 
     C, var = RING8
     if splits > 1 and var != 2:
         pytest.skip("the split-K combine is built for the 8-computing-wave layout")
     N = 352  # 5.5 tiles of 64 columns: a partial last tile
+    deep = C.gemm_on_deep(M, N, K, 0, 1, splits)
+    assert deep == (M <= 256) and (deep or var == 1 or C.gemm_ring8_tiles(M, N, K, splits) > 0)
     a, w, bias = bf(M, K, seed=90), bf(N, K, scale=0.05, seed=91), bf(N, scale=0.1, seed=92)
     y_ref = ref.linear(a, w, bias)
     y1 = C.linear(a, w, bias, 0, True, splits, CNT)
@@ -397,6 +416,21 @@ def test_ring8_gemm_epilogues(RING8, CNT, M, K, splits):
     if splits > 1:
         C.norm(x, slab, bias, None, None, 0.0, True, None, False)
     close(x, x_ref, 2e-3, 1e-3)
+    assert int(CNT.abs().sum()) == 0  # every ticket re-armed
+
+
+def test_ring8_wide_outputs(RING8, CNT):
+    """129 to 256 rows with more blocks than the deep ring takes."""
+    C, var = RING8
+    M, N, K = 200, 16464, 192
+    a, w = bf(M, K, seed=93), bf(N, K, scale=0.05, seed=94)
+    assert not C.gemm_on_deep(M, N, K, 3, 1, 1)
+    y = ref.linear(a, w)
+    close(C.linear_f32(a, w, True, 1, CNT), y, 2e-3, 1e-3)
+    x = torch.randn(M, N, device=DEV)
+    want = x + y
+    C.linear_residual(a, w, None, x, 1, True, CNT, False)
+    close(x, want, 2e-3, 1e-3)
 
 
 @pytest.fixture(params=[(2, 3), (3, 3), (2, 2), (2, 4), (3, 2)])
@@ -521,14 +555,15 @@ def _cache(slots, n_kv, S, hd):
 
 
 @pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("mode", ["decode1", "decode4", "tiled", "big", "d256", "d256s3", "d256rb"])
+@pytest.mark.parametrize("mode", ["decode1", "decode4", "splitk1", "splitk4", "tiled", "big", "d256", "d256s3", "d256rb"])
 def test_qkv_kv_append(C, CNT, rope, mode):
     from llm_sharding_demo_amd.ops.hip import rope_pair_permutation, rope_table
 
-    nh, n_kv, hd, H = 4, 2, 64, 256
+    nh, n_kv, hd = 4, 2, 64
+    H = 288 if mode.startswith("splitk") else 256  # whole 64-wide steps: deep ring; others: split-K kernel
     qs, kvs = nh * hd, n_kv * hd
     tiled = mode in ("tiled", "big", "d256", "d256s3", "d256rb")
-    splits = 4 if mode == "decode4" else (3 if mode == "d256s3" else (2 if mode == "d256rb" else 1))
+    splits = 4 if mode in ("decode4", "splitk4") else (3 if mode == "d256s3" else (2 if mode == "d256rb" else 1))
     # decode: 10 tokens of 2 sequences; tiled: 2 sequences of 150 tokens;
     # d256: 200 decode-like rows (100 + 100) on the 256-row kernel (kind 2);
     # d256rb: 400 rows in two 256-row blocks, split-K combine
@@ -537,6 +572,7 @@ def test_qkv_kv_append(C, CNT, rope, mode):
     if mode.startswith("d256"):
         tiled = 2
     T, slots, S = n0 + n1, 3, 320
+    assert C.gemm_on_deep(T, qs + 2 * kvs, H, 6, int(tiled), splits) == mode.startswith("decode")
     a, w, bias = bf(T, H, seed=13), bf(qs + 2 * kvs, H, scale=0.05, seed=14), bf(qs + 2 * kvs, scale=0.1, seed=15)
     tslot = torch.tensor([0] * n0 + [2] * n1, dtype=torch.int32, device=DEV)
     tpos = torch.tensor(list(range(n0)) + list(range(5, 5 + n1)), dtype=torch.int32, device=DEV)
@@ -568,6 +604,7 @@ def test_qkv_kv_append(C, CNT, rope, mode):
     close(q, q_ref, 3e-2)
     close(kc, kr, 3e-2)
     close(vc, vr, 3e-2)
+    assert int(CNT.abs().sum()) == 0
 
 
 @pytest.mark.parametrize("hd,nh,n_kv", [(64, 4, 4), (64, 8, 2), (128, 8, 2), (128, 32, 8)])

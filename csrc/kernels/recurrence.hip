@@ -327,7 +327,7 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(ConvParams c, SeqParams 
 // chunk's own.  What bounds a prompt is the chain of chunks (9.4 us each on one block per
 // sequence and head), so where those blocks leave the chip idle a chunk's factors are made by
 // a block of their own, all at once (delta_factors_kernel), and the chain keeps what is left
-// (delta_state_kernel: a block per 64 columns of a state).  One sequence of 1000 tokens, 16
+// (delta_state_kernel: a block per 32 columns of a state).  One sequence of 1000 tokens, 16
 // heads of 128 x 128: 590 us -> 22 + 70 + 9 (factors, states, output norm).  Above 192
 // (sequence, head) pairs the fused delta_chunk_kernel is as fast and needs no workspace.
 constexpr int DELTA_CT = 16, DELTA_WAVES = 2;

@@ -187,8 +187,13 @@ void norm_and_gate(const RecurParams& p, int64_t T, bool f32) {
   check_hip(lsd_head_norm_gate(&o, f32, cur_stream()), "head_norm_gate");
 }
 
-// Delta rule of few sequences: factors of many chunks at once, in portions of at most
-// 256 MB of them (528 chunks, 8448 tokens, of 16 heads of 128 x 128), then the chain.  max_rows
+// Chunks whose factors are made at once: at most 256 MB of them (528 chunks, 8448 tokens, of
+// one sequence with 16 heads of 128 x 128).
+int64_t delta_portion(int64_t D, int64_t heads, int64_t B) {
+  return std::clamp<int64_t>((256L << 20) / std::max<int64_t>(1, lsd_delta_item((int)D) * heads * B), 1, 65535);
+}
+
+// Delta rule of few sequences: factors of many chunks at once, then the chain.  max_rows
 // sizes the launches alone: a sequence that is longer goes on in the form without factors,
 // whose blocks find nothing to do otherwise (8 sequences of 150 tokens 91 -> 93 us; one sequence
 // is all rows, whatever is said).
@@ -198,7 +203,7 @@ void run_delta_split(RecurParams p, const Tensor& y, int64_t max_rows) {
   auto* xp = reinterpret_cast<lsd_bf16_t*>(x.data_ptr());
   check_hip(lsd_conv_silu(&p.c, &p.s, T, xp, ld, cur_stream()), "conv_silu");
   const int64_t all = (max_rows + ct - 1) / ct, per_chunk = lsd_delta_item(p.D) * p.heads * p.s.B;
-  const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>({all, (256L << 20) / std::max<int64_t>(1, per_chunk), 65535}));
+  const int64_t chunks = std::max<int64_t>(1, std::min(all, delta_portion(p.D, p.heads, p.s.B)));
   auto work = torch::empty({chunks * per_chunk}, y.options().dtype(torch::kUInt8));
   auto raw = torch::empty({T, (int64_t)p.heads * p.V}, y.options().dtype(torch::kFloat32));
   p.raw = raw.data_ptr<float>(); p.ldr = (int64_t)p.heads * p.V;
@@ -728,6 +733,7 @@ void lsd_register_mixers(pybind11::module& m) {
         py::arg("vdim"), py::arg("taps"), py::arg("ring"), py::arg("state"), py::arg("A"), py::arg("dt_bias"),
         py::arg("norm"), py::arg("gain"), py::arg("eps"), py::arg("out"), py::arg("single"), py::arg("chunked") = false,
         py::arg("max_rows") = 0, py::arg("split") = -1);
+  m.def("delta_portion_rows", [](int64_t D, int64_t heads, int64_t B) { return delta_portion(D, heads, B) * lsd_delta_chunk(); });
   m.def("ssm_seq", &ssm_seq, py::arg("y"), py::arg("slots"), py::arg("start"), py::arg("cu"), py::arg("heads"),
         py::arg("groups"), py::arg("state_dim"), py::arg("vdim"), py::arg("norm_groups"), py::arg("taps"), py::arg("bias"),
         py::arg("ring"), py::arg("state"), py::arg("A"), py::arg("dt_bias"), py::arg("skip"), py::arg("norm"),

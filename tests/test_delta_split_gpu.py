@@ -5,6 +5,8 @@ and of the row's root mean square, which the norm divides by) and states by fp32
 import pytest
 import torch
 
+from .test_vizalix_gpu import BF, DeltaCase, cuda, i32, portions, up
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -29,7 +31,6 @@ def run(C, split, lens, starts, H, G, D, V, n=4, strong=0.0, max_rows=0):
         dtb += strong * (torch.rand(H * D, generator=g, device=DEV) < 0.2)
     ring = rnd(len(lens), n, ch).bfloat16()
     state = rnd(len(lens), H, D, pad(V, 4)) * 0.1
-    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
     cu = [0]
     for k in lens:
         cu.append(cu[-1] + k)
@@ -53,11 +54,37 @@ def test_forms_agree(C, H, G, D, V, lens, starts, strong):
 
 
 def test_long_sequences_in_portions(C):
-    """256 (sequence, head) pairs: 31 chunks' factors fit the workspace at a time."""
-    lens = [520, 3, 500, 496, 1, 16, 40, 17]
-    a, b = (run(C, s, lens, [0] * 8, 32, 32, 128, 128, max_rows=520) for s in (0, 1))
+    """256 (sequence, head) pairs: some chunks' factors fit the workspace at a time.  Sequences
+    that end in the first, second and third portion, at its edge and behind cached tokens."""
+    p = C.delta_portion_rows(128, 32, 8)
+    lens = [2 * p + 5, 3, p, p + 1, 1, 16, p + 170, 17]
+    assert max(lens) > 2 * p
+    a, b = (run(C, s, lens, [0, 0, 5, 0, 9, 0, 130, 0], 32, 32, 128, 128, max_rows=max(lens)) for s in (0, 1))
     assert bool(((a[0] - b[0]).abs() <= 2.0 ** -7 * (a[0].abs() + a[0].pow(2).mean().sqrt())).all())
     assert bool(((a[1] - b[1]).abs() <= 1e-4 * a[1].abs().amax()).all())
+
+
+@pytest.mark.parametrize("H,G,D,V", [(4, 2, 24, 20), (2, 1, 128, 128), (3, 3, 64, 100)])
+@pytest.mark.parametrize("sizes", [[225], [129, 96], [33, 1, 191]])
+@pytest.mark.parametrize("decay,strong", [(1.0, 0.0), (0.01, 0.0), (30.0, 0.0), (1.0, 12.0)])
+def test_against_64_bits(C, H, G, D, V, sizes, decay, strong):
+    """Factors of their own (decays from the chunk's beginning) are no further from 64 bits
+    than those of the form that keeps a chunk in one block: root mean squares within 2 %."""
+    c = DeltaCase(C, H, G, D, V, 4, 225, BF, decay=decay, strong=strong)
+    taps, A, dtb, norm = c.par
+    off = []
+    for split in (0, 1):
+        c.state.fill_(float("nan"))
+        outs = []
+        for a, b in portions(225, sizes):
+            out = torch.full((b - a, up(H * V, 64)), float("nan"), dtype=BF, device=DEV)
+            C.delta_seq(cuda(c.y[a:b]), c.c0, c.c0 + c.ch, cuda(c.low[a:b]), c.nl, i32([1]), i32([a]), i32([0, b - a]), H, G,
+                        D, V, taps, c.ring, c.state, A, dtb, norm, c.gain, c.eps, out, False, True, b - a, split)
+            outs.append(out[:, : H * V])
+        off.append([float(((got.double().cpu() - want).pow(2).mean() / want.pow(2).mean()).sqrt())
+                    for got, want in ((torch.cat(outs), c.want), (c.state[1, ..., :V], c.S))])
+    (out0, state0), (out1, state1) = off
+    assert out1 < 1.02 * out0 and state1 < 1.02 * state0, off
 
 
 @pytest.mark.parametrize("lens,starts,hint", [([100, 37, 16], [0, 9, 0], 16), ([100, 37, 16], [0, 9, 0], 40),

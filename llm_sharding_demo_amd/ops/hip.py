@@ -1030,11 +1030,7 @@ class HipBackend(Backend):
         key = M, N, K, self._decode, getattr(self, "concurrency", 1)
         S = plans.get(key)
         if S is None:
-            S = self.R.resid_splits(*key)
-            if not self._decode:
-                S = self.R.prompt_slabs(M, N, K, S)
-            if self._tiled(M, N) or self.R.defer_resid:
-                S = self.R.slab_splits(M, N, K, S)
+            S = self.R.residual_splits(*key)
             if len(plans) >= 4096:
                 plans.clear()
             plans[key] = S

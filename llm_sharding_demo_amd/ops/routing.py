@@ -56,6 +56,9 @@ class Routing:
     attn_large_waves: int = 4
     attn_max_wg: int = 0       # cap the attention grid (A/B; 0 = none)
     # -- decode GEMMs ------------------------------------------------------
+    # Of up to 256 rows most run on the deep ring whatever family is chosen here (on_deep);
+    # the fields below then matter for what it leaves: K off 64, wide outputs, the 256-row
+    # kernel, more rows.  Their figures compare the kernels behind it.
     # split-K (last-arriver) kernel up to sk_max_m rows; tiled above
     # tiled_all_m rows at any width, above tiled_min_m rows when >=
     # tiled_min_n wide (GPT-2 XL 2 x 256: split-K 41.2k, all tiled 46.3k tok/s;
@@ -262,6 +265,37 @@ class Routing:
             return max(1, min(8, max(4, K // 800), K // 64))
         return self.sk_splits(M, N, K, lanes)
 
+    def residual_splits(self, M: int, N: int, K: int, decode: bool = True, lanes: int = 1) -> int:
+        """K splits a residual projection is launched with: the rule above, and
+        what the kernels behind it make of slabs."""
+        S = self.resid_splits(M, N, K, decode, lanes)
+        if not decode:
+            S = self.prompt_slabs(M, N, K, S)
+        if self.tiled(M, N) or self.defer_resid:
+            S = self.slab_splits(M, N, K, S)
+        return S
+
+    @staticmethod
+    def on_deep(M: int, N: int, K: int, splits: int = 1, pairs: bool = False) -> bool:
+        """Whether a split-K or tiled launch runs on the deep ring (mirrors
+        lsd_gemm_deep_ok() in gemm_deep.hip).  splits: slabs (other sums run
+        unsplit); pairs: gate / up rows."""
+        if not 1 <= M <= 256 or K < 64 or K % 64 or N % (32 if pairs else 16) or splits > K // 64:
+            return False
+        if M <= 48:
+            return True
+        rows = 128 if M > 192 else 96 if M > 128 else 128 if M > 96 else 96 if M > 64 else 64
+        two = math.ceil(M / rows)
+        best = least = 0
+        for bn in (64, 32, 16):
+            if bn == 16 and (M > 64 or pairs or K % 128 or K // 128 < splits):
+                break
+            blocks = math.ceil(N / bn) * splits * two
+            cost = math.ceil(blocks / 256) * (bn + rows)
+            if not best or cost < least:
+                best, least = blocks, cost
+        return best <= (512 if M > 64 else 640)
+
     @staticmethod
     def slab_splits(M: int, N: int, K: int, S: int) -> int:
         """K splits of a residual projection of 9 .. 128 rows that leaves slabs,
@@ -412,9 +446,9 @@ class Routing:
 def route_table(model: str, rows, routing: Routing | None = None) -> dict:
     """{(gemm, rows, phase): route} of one model's projections: what
     `tests/test_routing.py` pins and `python -m llm_sharding_demo_amd.ops.routing`
-    prints.  route = kernel family + K splits, no extension calls.  The split-K and
-    tiled families run up to 128 rows on the deep ring (gemm_deep.hip), unsplit where
-    the split would be combined, and with slab_splits slabs; prompts with prompt_slabs."""
+    prints.  route = kernel family + K splits, no extension calls.  "deep": the deep ring,
+    which takes split-K and tiled launches of up to 256 rows (on_deep) and sums what is
+    not left as slabs unsplit."""
     from ..config import get_model_config
 
     r = routing or Routing.from_env("")
@@ -431,15 +465,20 @@ def route_table(model: str, rows, routing: Routing | None = None) -> dict:
                 if M <= r.gemv_max_m and decode:
                     route = "gemv"
                 elif kind == "resid":
-                    s = r.resid_splits(M, N, K, decode, lanes)
+                    s = r.residual_splits(M, N, K, decode, lanes)
                     t = r.tiled(M, N)
+                    slabs = s if t or r.defer_resid else 1
                     route = f"{'tiled' if t else 'splitk-slab' if r.defer_resid and s > 1 else 'splitk'}/s{s}"
+                    if r.on_deep(M, N, K, slabs):
+                        route = f"deep/s{slabs}"
                 else:
                     if kind == "logits":
                         t, s = r.logits_kw(M, N, K, lanes)
                     else:
                         t, s = r.gemm_kw(M, N, K, lanes, 2 if (g == "up" and mc.arch == "llama") else 1)
                     route = {False: "splitk", True: "tiled", 2: "d256-64", 3: "d256-128"}[t] + f"/s{s}"
+                    if t in (False, True) and r.on_deep(M, N, K, 1, g == "up" and mc.arch == "llama"):
+                        route = "deep/s1"
                 if r.blaslt and ((g == "up" and (r.blaslt_gelu(M, decode) and mc.arch == "gpt2"
                                                  or mc.arch == "llama" and r.blaslt_silu(M, N, decode)))
                                  or (g == "qkv" and r.blaslt_qkv(M, K, decode))

@@ -46,7 +46,7 @@ def test_blaslt_oracle_routes_when_asked():
     assert t["gpt2-xl|prefill|65536|o"].startswith("tiled")   # K 1600 stays hand-written
     assert t["llama-3-8b|decode|512|qkv"] == "hipblaslt"
     assert t["llama-3-8b|decode|128|up"] == "hipblaslt"
-    assert t["gpt2-xl|decode|256|up"].startswith("tiled")
+    assert t["gpt2-xl|decode|256|up"].startswith("deep")
 
 
 def test_single_stream_on_gemv_and_key_shapes():
@@ -54,9 +54,28 @@ def test_single_stream_on_gemv_and_key_shapes():
     for m in ["gpt2", "gpt2-xl", "llama-3-8b"]:
         for g in ["qkv", "o", "up", "down", "lm_head"]:
             assert t[f"{m}|decode|1|{g}"] == "gemv"
-    assert t["gpt2-xl|decode|256|qkv"] == "tiled/s1"           # 8-wave LDS ring
-    assert t["gpt2-xl|decode|256|down"] == "tiled/s5"          # residual slabs folded by the norm
+    assert t["gpt2-xl|decode|256|qkv"] == "deep/s1"            # deep LDS ring
+    assert t["gpt2-xl|decode|256|down"] == "deep/s5"           # residual slabs folded by the norm
+    assert t["gpt2-xl|decode|128|lm_head"] == "tiled/s1"       # too wide for it
+    assert t["llama-3-8b|prefill|512|down"] == "tiled/s8"      # slabs that fill a round of 256x256 tiles
     assert t["llama-3-8b|decode|256|up"].startswith("d256")    # all-rows kernel for long K
+
+
+def test_deep_ring_rule_is_the_kernels():
+    """The table's copy of the rule against the launch's."""
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+    EPI_BF16, EPI_SILU, EPI_SLAB = 0, 2, 5
+    for M in (0, 1, 9, 16, 40, 48, 49, 64, 65, 96, 97, 128, 129, 150, 192, 193, 256, 257):
+        for N in (16, 64, 1600, 2624, 4800, 8512, 11264, 16384, 28672, 32768, 32784, 40960, 40976, 50304, 128256):
+            for K in (32, 64, 96, 128, 320, 768, 1600, 4096, 14336):
+                at = (M, N, K)
+                assert Routing.on_deep(*at) == _C.gemm_on_deep(*at, EPI_BF16, 1, 1) == _C.gemm_on_deep(*at, EPI_BF16, 0, 4), at
+                assert Routing.on_deep(*at, pairs=True) == _C.gemm_on_deep(*at, EPI_SILU, 1, 1), at
+                for S in (1, 2, 4, 5, 8, 12):
+                    assert Routing.on_deep(*at, S) == _C.gemm_on_deep(*at, EPI_SLAB, 0, S), (at, S)
 
 
 def test_routing_env_override():

@@ -991,7 +991,8 @@ extern "C" hipError_t lsd_latent_plain(const LatentAttnParams* p, int f32, hipSt
   const size_t lds = (p->rank_pad + 256) * sizeof(float);
 #define LSD_PL(T, OPT) hipLaunchKernelGGL((latent_plain_kernel<T, OPT>), grid, dim3(256), lds, st, *p)
   const int opt = (p->v_pad + 255) / 256;
-  // fp32 rows in whole 256-byte pieces, up to what 160 KB of LDS hold 32 of
+  // fp32 rows in whole 256-byte pieces, up to the 512 + 64 columns of the widest latent in use: there
+  // a block takes 86 KB of LDS, a lane 144 registers for queries, sums and the next keys
   if (f32 && p->rank_pad % 64 == 0 && p->rank_pad <= 576 && reinterpret_cast<uintptr_t>(p->cache) % 16 == 0) {
     const dim3 g16(p->B, (p->H + 15) / 16);
     switch (p->rank_pad / 64) {

@@ -5,7 +5,7 @@
 // `server.py:102`).  Weights are stored [N][K] (K-contiguous) so a
 // 16x16x32 B-operand fragment is one 16-byte load.
 //
-// The kernels (decode microbatches of up to 128 or 256 rows: gemm_deep.hip):
+// The kernels (most launches of up to 256 rows: gemm_deep.hip, which has the line):
 //  * gemm_sk      -- decode microbatches whose K has no whole 64-wide steps.  Weight-bandwidth bound:
 //    W streamed HBM -> VGPRs (read once, no LDS round trip), the small A
 //    operand staged through LDS with full-line LDS-DMA, split-K across
@@ -16,9 +16,9 @@
 //    global_load_lds (LDS-DMA), XOR-swizzled on the source address so the
 //    ds_read_b128 fragment reads are bank-conflict free, double buffered,
 //    XCD-aware tile order.
-//  * gemm_ring    -- the tiled kernel's grids of <= 256 workgroups (decode
-//    microbatches of 129-256 rows): 128x64 (or 128x128) tiles, a 3-slot LDS
-//    ring with two k-steps in flight, 1 block/CU.
+//  * gemm_ring    -- the tiled kernel's grids of <= 512 tiles of 128x64 (256 of
+//    128x128) above 256 rows, and below where the deep ring is not taken: a
+//    3-slot LDS ring with two k-steps in flight, 1 block/CU.
 //  * gemm_big     -- large prefill GEMMs: 256x256 tiles, 8 waves, 4-slot ring.
 //
 // Epilogues (fused, no extra pass): bias, gelu_new, silu(gate)*up, fp32

@@ -64,7 +64,9 @@ __device__ __forceinline__ float conv_at(const ConvParams& c, int ch, long row, 
 // Bound in decode by the state, read and written once a step: it passes the caches by, which
 // keep the weights of the step instead, and the SSM's registers fit four blocks a CU.  96
 // sequences: 64 heads of 64 x 128 91 -> 85 us, 16 of 128 x 128 60 -> 56, and the step that
-// holds three layers of each 1131 -> 1052; 16 sequences 567 -> 523.
+// holds three layers of each 1131 -> 1052; 16 sequences 567 -> 523.  No fewer sequences need the
+// caches: between two steps 4 GB of weights pass them.  Through and by the caches, 1 sequence
+// 430 and 426 us a step, 2 454 and 449, 4 478 and 467, 8 505 and 490.
 template <typename T, bool DELTA, int LV, int NR>
 __global__ __launch_bounds__(256, NR > 8 ? 2 : DELTA ? 3 : 4) void recur_seq_kernel(RecurParams p) {
   constexpr int VB = LV * 4, DG = 256 / LV;

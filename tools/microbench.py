@@ -537,7 +537,8 @@ def bench_llama_sk(M=256):
 
 
 def stamps_gemm(M, N, K, splits, act=0, label=""):
-    """Per-workgroup phase timeline of one decode-GEMM launch (diagnostic)."""
+    """Per-workgroup phase timeline of one launch of the split-K kernel (K an odd
+    multiple of 32; diagnostic)."""
     w = torch.randn(N, K, device=DEV).bfloat16()
     a = torch.randn(M, K, device=DEV).bfloat16()
     cnt = torch.zeros(1 << 16, dtype=torch.int32, device=DEV)
@@ -576,10 +577,10 @@ def main():
     which = sys.argv[1:] or ["gemm", "attn", "norm", "sample"]
     if "stamps" in which:
         for M, S in ((16, 1), (16, 4), (64, 1), (64, 4), (64, 8)):
-            stamps_gemm(M, 4800, 1600, S, label="_qkv")
+            stamps_gemm(M, 4800, 1632, S, label="_qkv")
         for M, S in ((64, 1), (64, 6), (64, 16)):
-            stamps_gemm(M, 1600, 1600, S, label="_proj")
-        stamps_gemm(64, 50304, 1600, 1, label="_lmhead")
+            stamps_gemm(M, 1600, 1632, S, label="_proj")
+        stamps_gemm(64, 50304, 1632, 1, label="_lmhead")
     H, F, V = 1600, 6400, 50304
     from llm_sharding_demo_amd.ops.hip import HipBackend
     R0 = HipBackend.R

@@ -193,6 +193,16 @@ int64_t delta_portion(int64_t D, int64_t heads, int64_t B) {
   return std::clamp<int64_t>((256L << 20) / std::max<int64_t>(1, lsd_delta_item((int)D) * heads * B), 1, 65535);
 }
 
+// Factors of their own: where the blocks of the fused form, one per sequence and head, leave the chip
+// idle and the longest sequence has chunks enough to pay for two launches more and the way
+// through memory.  With the convolution, heads of 128 x 128, fused against split: 64 pairs 8 tokens
+// 36 and 38 us, 20 46 and 40; 128 pairs 20 tokens 48 and 51, 64 71 and 62; 192 pairs 64 tokens 76 and
+// 79, 100 99 and 100, 150 127 and 121, 300 217 and 208.
+bool delta_split(int64_t heads, int64_t B, int64_t rows) {
+  const int64_t pairs = heads * B, chunks = (rows + lsd_delta_chunk() - 1) / lsd_delta_chunk();
+  return pairs <= 192 && chunks >= std::max<int64_t>(2, pairs / 32);
+}
+
 // Delta rule of few sequences: factors of many chunks at once, then the chain.  max_rows
 // sizes the launches alone: a sequence that is longer goes on in the form without factors,
 // whose blocks find nothing to do otherwise (8 sequences of 150 tokens 91 -> 93 us; one sequence
@@ -222,9 +232,9 @@ void run_delta_split(RecurParams p, const Tensor& y, int64_t max_rows) {
 // y [T, N] rows of q | k | v conv channels from column c0 and beta's logits from
 // gate_col; low [T, >= heads D at 0, heads V at gate_off].  Token by
 // token, or (chunked) prompts of bf16 models; max_rows: rows of the longest sequence, to size
-// launches by (0: not known).  split: factors of their own, -1 where that is faster -- with the convolution, 16
-// heads of 128 x 128 and 1000 tokens each: 4 sequences 709 -> 232 us, 8 616 -> 403, 12 842 -> 681,
-// 16 750 -> 842; one of 20 tokens 42 -> 35, of 4000 2170 -> 404, of 16000 11690 -> 1600
+// launches by (0: not known).  split: factors of their own, -1 by delta_split -- 16 heads of
+// 1000 tokens each: 4 sequences 611 -> 214 us, 8 689 -> 406, 12 703 -> 632, 16 723 -> 817; one of 20
+// tokens 41 -> 33, of 4000 2334 -> 397, of 16000 11690 -> 1600
 void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_off, Tensor slots, Tensor start,
                Tensor cu, int64_t heads, int64_t groups, int64_t D, int64_t V, Tensor taps, Tensor ring, Tensor state,
                Tensor A, Tensor dt_bias, Tensor norm, double gain, double eps, Tensor out, bool single, bool chunked,
@@ -248,8 +258,9 @@ void delta_seq(Tensor y, int64_t c0, int64_t gate_col, Tensor low, int64_t gate_
   if (chunked) {
     TORCH_CHECK(!f32 && !single && lsd_chunk_ok(1, D, V, groups, heads), "delta_seq: no chunked kernel");
     TORCH_CHECK(max_rows >= 0 && split >= -1 && split <= 1 && p.s.B <= 65535, "delta_seq: max_rows, split");
-    if (split == 1 || (split < 0 && (int64_t)p.s.B * heads <= 192))
-      run_delta_split(p, y, max_rows > 0 && p.s.B > 1 ? std::min(max_rows, y.size(0)) : y.size(0));
+    const int64_t rows = max_rows > 0 && p.s.B > 1 ? std::min(max_rows, y.size(0)) : y.size(0);
+    if (split == 1 || (split < 0 && delta_split(heads, p.s.B, rows)))
+      run_delta_split(p, y, rows);
     else
       run_chunks(p, y);
     check_hip(lsd_conv_tail(&p.c, &p.s, f32, cur_stream()), "conv_tail");
@@ -733,6 +744,7 @@ void lsd_register_mixers(pybind11::module& m) {
         py::arg("vdim"), py::arg("taps"), py::arg("ring"), py::arg("state"), py::arg("A"), py::arg("dt_bias"),
         py::arg("norm"), py::arg("gain"), py::arg("eps"), py::arg("out"), py::arg("single"), py::arg("chunked") = false,
         py::arg("max_rows") = 0, py::arg("split") = -1);
+  m.def("delta_split", &delta_split, py::arg("heads"), py::arg("seqs"), py::arg("rows"));
   m.def("delta_portion_rows", [](int64_t D, int64_t heads, int64_t B) { return delta_portion(D, heads, B) * lsd_delta_chunk(); });
   m.def("ssm_seq", &ssm_seq, py::arg("y"), py::arg("slots"), py::arg("start"), py::arg("cu"), py::arg("heads"),
         py::arg("groups"), py::arg("state_dim"), py::arg("vdim"), py::arg("norm_groups"), py::arg("taps"), py::arg("bias"),

@@ -96,3 +96,17 @@ def test_decode_attention_parts_by_context():
                                         (1, 1, 100, 8000, 2), (0, 8, 1, 100, 4)]:
         assert _C.attn_decode_split(B, n_kv, 4, 128, splits, keys) == want, (B, splits, keys)
     assert _C.attn_decode_split(1, 8, 3, 128, 1, 900) == 1 and _C.attn_decode_split(1, 8, 4, 64, 1, 900) == 1
+
+
+def test_delta_rule_splits_by_length():
+    """Factors of their own only where the longest sequence has chunks enough for them."""
+    import pytest
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+
+    for heads, seqs, rows, want in [(16, 1, 16, False), (16, 1, 17, True), (4, 40, 5, False), (16, 4, 20, True),
+                                    (16, 8, 20, False), (16, 8, 64, True), (16, 12, 64, False), (16, 12, 100, True),
+                                    (16, 13, 4000, False), (16, 1, 0, False)]:
+        assert _C.delta_split(heads, seqs, rows) == want, (heads, seqs, rows)

@@ -1105,59 +1105,33 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(GemmParams p, int tiles_m
 // rows mh * 128 + wr * 64 + [0, 64), columns nh * 128 + wc * 32 + [0, 32).
 // Each K-tile is four phases, one output quadrant (A half mh, B half nh) of
 // 16 MFMAs each, in the order (0,0) (0,1) (1,1) (1,0):
-//   phase  reads (ds_read_b128)       stages (glds, 2 per thread)  waits
-//   q0     A0 frags (8) + B0 frags (4)  B1 of tile t+1
-//   q1     B1 frags (4)                 A1 of tile t+1               A1(t)
-//   q2     A1 frags (8)                 A0 of tile t+2
-//   q3     --  (B0 frags kept)          B0 of tile t+2               A0/B0/B1(t+1)
-// so every half-tile is restaged >= 2 phases after its last read (A0 read
-// q0 -> restaged q2, B0 q0 -> q3, B1 q1 -> q0 next, A1 q2 -> q1 next) and is
-// issued 5-6 phases before it is read; the counted vmcnt waits (q1: 4
-// later halves in flight, q3: 3) always sit one phase before the first read
-// of what they retire.  Phase body: reads, stage, wait, s_barrier,
-// lgkmcnt(0), 16 MFMAs, s_barrier.  The two wave rows run staggered by one
-// barrier (wr = 1 takes an extra barrier up front, wr = 0 one at the end), so
-// on every SIMD one wave issues its LDS reads and DMA while the other runs
-// MFMAs (guide §5 "The 256^2 8-phase template").  All LDS is one array;
-// the epilogue reuses it as the fp32 C tile.
+//   phase  reads (ds_read_b128)       stages (2 DMA a thread each)   retires
+//   q0     A0(t) (8)                                                 B1(t)
+//   q1     B1(t) (4)                  A1(t+1), B0(t+2)               A1(t)
+//   q2     A1(t) (8)                                                 B0(t+1)
+//   q3     B0(t+1) (4)                A0(t+2), B1(t+2)               A0(t+1)
+// What bounds it is LDS: a K-tile's fragments (192 KB) and its DMA (64 KB) take as many
+// cycles at 128 B each as its MFMAs, so reads and DMA are spread so that every phase has the
+// same, 256 beside 256 cycles of MFMAs.  With B0(t) beside A0(t) in q0, 384 cycles there and 64 in
+// q3, and with the addresses computed in the loop, before:
+//   8192 x 8192 x 8192          798 -> 725 us (1377 -> 1516 TF/s)
+//   7937 x 28672 x 4096, SiLU  1464 -> 1380     7937 x 4096 x 14336, residual  740 -> 689
+//   16128 x 4800 x 1600         215 -> 209      12000 x 11264 x 2048, SiLU     510 -> 480
+// (one DMA half a phase instead of two in every other: 1.5 % slower).  B0 of the next tile goes
+// to the registers that B1 leaves, which is why tiles are unrolled in pairs.
+// A half-tile is restaged >= 2 phases after its last read and staged 4-5 phases before it
+// is read; the counted waits sit one phase before the first read of what they retire.
+// Phase body: reads, stage, wait, s_barrier, 16 MFMAs as their fragments arrive, s_barrier.
+// The two wave rows run staggered by one barrier (wr = 1 takes an extra barrier up front,
+// wr = 0 one at the end), so on every SIMD one wave issues its LDS reads and DMA while the
+// other runs MFMAs.  All LDS is one array; the epilogue reuses it as the C tile.
 constexpr int P8_HALF = 128 * 64 * 2;  // 16 KiB
 constexpr int P8_BUF = 4 * P8_HALF;    // A0 A1 B0 B1
 constexpr int P8_SMEM = 2 * P8_BUF;    // 128 KiB (== 256 x 128 fp32 C half-tile)
 
-template <bool BUF = false>
-__device__ __forceinline__ void p8_stage(char* lds, const bf16* src, long ld, int row0, int row_max,
-                                         int k0) {
-  const int lane = lane_id(), w = threadIdx.x >> 6;
-  if constexpr (BUF) {
-    // buffer_load ... lds: a wave-uniform resource at (row0, k0) and 32-bit lane offsets
-    // (one address VGPR per lane instead of a 64-bit global address)
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(src + (long)row0 * ld + k0), 0, 0x7fffffff, 0x00020000);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int inst = w * 2 + q;
-      const int row = inst * 8 + (lane >> 3);
-      const int lch = (lane & 7) ^ ((row >> 1) & 7);
-      const int off = ((min(row0 + row, row_max) - row0) * (int)ld + lch * 8) * 2;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(lds + inst * 1024), 16, off, 0, 0, 0);
-    }
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int inst = w * 2 + q;  // 16 x 1 KiB = 128 rows of 128 B
-    const int row = inst * 8 + (lane >> 3);
-    const int lch = (lane & 7) ^ ((row >> 1) & 7);
-    const bf16* gp = src + (long)min(row0 + row, row_max) * ld + k0 + lch * 8;
-    __builtin_amdgcn_global_load_lds((gbl_cvoid*)gp, (lds_void*)(lds + inst * 1024), 16, 0, 0);
-  }
-}
-
 // VAR 4 (default, gemm_set_big_kind 4): stage with buffer_load ... lds (wave-uniform
-// resource, 32-bit lane offsets) instead of global_load_lds with 64-bit lane addresses;
-// VAR 0 = kind 1.  Issuing each phase's DMA before its fragment reads, B fragments first
-// and a peeled k-loop were measured and removed (profiles/r3_p8_buffer_lds.log,
-// r3_rejected_p8_peeled_loop.log).
+// resource, 32-bit lane offsets, the K offset in a scalar) instead of global_load_lds with
+// 64-bit lane addresses; VAR 0 = kind 1.
 template <int EPI, int VAR = 0>
 __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m, int tiles_n, int G) {
   __shared__ __attribute__((aligned(16))) char smem[P8_SMEM];
@@ -1173,7 +1147,7 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
   const int kb = (int)((long)KT * split / p.splits);
   const int T = (int)((long)KT * (split + 1) / p.splits) - kb;  // K-tiles of this split
 
-  const int lane = lane_id(), w = threadIdx.x >> 6;
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = w >> 2, wc = w & 3;
   const int r = lane & 15, g = lane >> 4;
 
@@ -1184,41 +1158,57 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // half h of K-tile t: 0 = A0, 1 = A1, 2 = B0, 3 = B1
-  auto stage = [&](int t, int h) {
-    char* dst = smem + (t & 1) * P8_BUF + h * P8_HALF;
-    const int k0 = (kb + t) * 64;
-    if (h < 2) p8_stage<(VAR & 4) != 0>(dst, p.A, p.lda, m0 + h * 128, p.M - 1, k0);
-    else p8_stage<(VAR & 4) != 0>(dst, p.W, p.ldw, n0 + (h - 2) * 128, p.N - 1, k0);
+  // half h of a K-tile: 0 = A0, 1 = A1, 2 = B0, 3 = B1; this thread's two 16-byte pieces of it
+  // (rows behind the last one read that one again), bytes from the half's first row at K-tile 0
+  const bf16* base[4];
+  int off[4][2];
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const int row0 = (h < 2 ? m0 : n0) + (h & 1) * 128, last = (h < 2 ? p.M : p.N) - 1;
+    const long ld = h < 2 ? p.lda : p.ldw;
+    base[h] = (h < 2 ? p.A : p.W) + (long)row0 * ld + (long)kb * 64;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int row = (w * 2 + q) * 8 + (lane >> 3);
+      off[h][q] = ((min(row0 + row, last) - row0) * (int)ld + (((lane & 7) ^ ((row >> 1) & 7)) << 3)) * 2;
+    }
+  }
+  // (behind the last K-tile: the same loads of nothing, so the waits count alike)
+  auto stage = [&](int t, int buf, int h) {
+    char* dst = smem + buf * P8_BUF + h * P8_HALF + w * 2048;
+    if constexpr ((VAR & 4) != 0) {
+      const __amdgpu_buffer_rsrc_t rs =
+          __builtin_amdgcn_make_buffer_rsrc((void*)base[h], 0, t < T ? 0x7fffffff : 0, 0x00020000);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(dst + q * 1024), 16, off[h][q], t < T ? t * 128 : 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        __builtin_amdgcn_global_load_lds((gbl_cvoid*)(reinterpret_cast<const char*>(base[h]) + (long)min(t, T - 1) * 128 + off[h][q]),
+                                         (lds_void*)(dst + q * 1024), 16, 0, 0);
+    }
   };
   bf16x8 af[4][2], b0[2][2], b1[2][2];
-  auto read_a = [&](int t, int mh) {
-    const char* src = smem + (t & 1) * P8_BUF + mh * P8_HALF;
+  auto read_a = [&](int buf, int mh) {
+    const char* src = smem + buf * P8_BUF + mh * P8_HALF;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) af[i][kk] = lds_frag(src, wr * 64 + i * 16 + r, kk * 4 + g);
+      for (int i = 0; i < 4; ++i) af[i][kk] = lds_frag(src, wr * 64 + i * 16 + r, kk * 4 + g);
   };
-  auto read_b = [&](int t, int nh, bf16x8 (&bf)[2][2]) {
-    const char* src = smem + (t & 1) * P8_BUF + (2 + nh) * P8_HALF;
+  auto read_b = [&](int buf, int nh, bf16x8 (&bf)[2][2]) {
+    const char* src = smem + buf * P8_BUF + (2 + nh) * P8_HALF;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) bf[j][kk] = lds_frag(src, wc * 32 + j * 16 + r, kk * 4 + g);
+      for (int j = 0; j < 2; ++j) bf[j][kk] = lds_frag(src, wc * 32 + j * 16 + r, kk * 4 + g);
   };
-#ifdef LSD_P8_PROF
-  // diagnostic build only (LSD_HIPCC_FLAGS=-DLSD_P8_PROF): wave 0's cycles in
-  // the loop, in the counted vmcnt waits and in the two barriers of a phase
-  long long pf_t0 = 0, pf_vm = 0, pf_b1 = 0, pf_b2 = 0, pf_c = 0;
-#define P8_T() __builtin_amdgcn_s_memtime()
-#define P8_ACC(acc, stmt) { pf_c = P8_T(); stmt; acc += P8_T() - pf_c; }
-#else
-#define P8_ACC(acc, stmt) stmt;
-#endif
-  auto mma = [&](int mh, int nh, bf16x8 (&bf)[2][2]) {
-    P8_ACC(pf_b1, __builtin_amdgcn_s_barrier())
-    __builtin_amdgcn_s_waitcnt(LGKM0);
+  // vm: loads that may stay in flight
+  auto mma = [&](auto vm, int mh, int nh, bf16x8 (&bf)[2][2]) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(decltype(vm)::v));
     __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
@@ -1228,69 +1218,48 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
         for (int j = 0; j < 2; ++j)
           acc[mh * 4 + i][nh * 2 + j] = mfma16(bf[j][kk], af[i][kk], acc[mh * 4 + i][nh * 2 + j]);
     __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_s_waitcnt(LGKM0);  // q3's reads, which its MFMAs do not use
     __builtin_amdgcn_sched_barrier(0);
-    P8_ACC(pf_b2, __builtin_amdgcn_s_barrier())
+    __builtin_amdgcn_s_barrier();
+  };
+  // K-tile t in buffer `buf`; bx holds B0(t), by is free
+  auto tile = [&](int t, int buf, bf16x8 (&bx)[2][2], bf16x8 (&by)[2][2]) {
+    read_a(buf, 0);
+    mma(Int<8>{}, 0, 0, bx);
+    read_b(buf, 1, by);
+    stage(t + 1, buf ^ 1, 1);
+    stage(t + 2, buf, 2);
+    mma(Int<10>{}, 0, 1, by);
+    read_a(buf, 1);
+    mma(Int<8>{}, 1, 1, by);
+    read_b(buf ^ 1, 0, by);
+    stage(t + 2, buf, 0);
+    stage(t + 2, buf, 3);
+    mma(Int<10>{}, 1, 0, bx);
   };
 
   if (T > 0) {
-    // prologue: all of tile 0, then A0 / B0 of tile 1; tile 0 published
-    stage(0, 0);
-    stage(0, 2);
-    stage(0, 3);
-    stage(0, 1);
-    if (T > 1) {
-      stage(1, 0);
-      stage(1, 2);
-      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    // prologue: tile 0 and all of tile 1 but A1, in the order of the waits
+    stage(0, 0, 2);
+    stage(0, 0, 0);
+    stage(0, 0, 3);
+    stage(0, 0, 1);
+    stage(1, 1, 2);
+    stage(1, 1, 0);
+    stage(1, 1, 3);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(10));
     __builtin_amdgcn_s_barrier();
     LSD_STAMP(1)
     if (wr == 1) __builtin_amdgcn_s_barrier();  // stagger the wave rows by one barrier
-
-#ifdef LSD_P8_PROF
-    pf_t0 = P8_T();
-#endif
-    for (int t = 0; t < T; ++t) {
-      const bool n1 = t + 1 < T, n2 = t + 2 < T;
-      // q0: (A0, B0)
-      read_a(t, 0);
-      read_b(t, 0, b0);
-      if (n1) stage(t + 1, 3);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0, 0, b0);
-      // q1: (A0, B1); retire A1(t): 4 later halves in flight when t + 1 exists
-      read_b(t, 1, b1);
-      if (n1) stage(t + 1, 1);
-      P8_ACC(pf_vm, if (n1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-                    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory"))
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0, 1, b1);
-      // q2: (A1, B1)
-      read_a(t, 1);
-      if (n2) stage(t + 2, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1, 1, b1);
-      // q3: (A1, B0); retire A0 / B0 / B1 of t + 1 (A1(t+1), A0 / B0(t+2) stay in flight)
-      if (n2) stage(t + 2, 2);
-      P8_ACC(pf_vm, if (n2) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-                    else if (n1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory"))
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1, 0, b0);
+    read_b(0, 0, b0);
+    int t = 0;
+    for (; t + 1 < T; t += 2) {
+      tile(t, 0, b0, b1);
+      tile(t + 1, 1, b1, b0);
     }
+    if (t < T) tile(t, 0, b0, b1);
     if (wr == 0) __builtin_amdgcn_s_barrier();  // balance the stagger
-#ifdef LSD_P8_PROF
-    if (p.stamps && threadIdx.x == 0) {
-      long long* ps = p.stamps + (long)blockIdx.x * 8;
-      ps[4] = P8_T() - pf_t0;
-      ps[5] = pf_vm;
-      ps[6] = pf_b1;
-      ps[7] = pf_b2;
-    }
-#endif
   }
-#undef P8_ACC
   LSD_STAMP(2)
 
   // Epilogue.  A tile's is not hidden (one block per CU), so the math is done on the

@@ -56,3 +56,24 @@ def test_epilogues(C, M, N, K, bias):
     slab = C.linear_residual(*at, None, xd, 1, 1, None, True)
     slab = slab[0] if slab.dim() == 3 else slab
     assert near(slab, acc, off)
+
+
+# 1 .. 8 K-tiles a split, which ends in front of columns that are 2^30 times as large: nothing
+# that is staged behind a split's last tile may reach its sum
+@pytest.mark.parametrize("kind", [4, 1])
+@pytest.mark.parametrize("tiles", range(1, 9))
+def test_k_tiles(C, kind, tiles):
+    M, N, K = 300, 288, 128 * tiles
+    g = torch.Generator().manual_seed(tiles)
+    a, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    a[:, K // 2:] *= 2.0 ** 30
+    C.gemm_set_big_kind(kind)
+    try:
+        slabs = C.linear_residual(a.to(DEV), w.to(DEV), None, torch.zeros(M, N, device=DEV), 2, 1, None, False)
+    finally:
+        C.gemm_set_big_kind(4)
+    assert slabs.shape[0] == 2
+    for h, got in enumerate(slabs):
+        part = slice(h * K // 2, (h + 1) * K // 2)
+        x, y = a[:, part].to(F64), w[:, part].to(F64)
+        assert near(got.float(), x @ y.T, (K + 3) * 2.0 ** -24 * (x.abs() @ y.abs().T))

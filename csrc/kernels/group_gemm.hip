@@ -337,9 +337,9 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
 // whose k-slot g stands for k = 4 g + j in both operands.
 // Bound by the matrix cores, whose fp32 rate is a sixteenth of bf16's (154 TF/s), and, where
 // experts have some tens of rows, by their weights.  64 x 128 tiles were no faster.
-// 2260 rows over 32 experts of 2048 x 1024 and 565 through a shared one of 2048 (VALU tiles
-// before): up 631 -> 355 us, down 320 -> 187; 565 x 2048 x 2048 143 -> 65; 4096 x 4096 x 2048
-// at 114 TF/s.
+// Loads by lds_dma16 (global_load_lds before): 2260 rows over 32 experts of 2048 x 1024 and
+// 565 through a shared one of 2048 up 325 -> 295 us, down 169 -> 160; 565 x 2048 x 2048 63 -> 54;
+// 8192 x 8192 x 2048 118 -> 133 TF/s.
 template <int MODE, int MT>
 __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kernel(GgParams p) {
   using namespace gg;
@@ -353,28 +353,27 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
 
-  const float* ap[TM / 32];
-  const float* wp[TN / 32];
+  // rows from the tile's first one, gathered ones from the first of all (fit: gg_f32)
+  const long r0 = MODE == GG_UP && t.routed ? 0 : t.row0;
+  const float* ab = static_cast<const float*>(t.A) + r0 * t.lda;
+  const float* wb = static_cast<const float*>(t.W) + (long)t.n0 * t.ldw;
+  unsigned ao[TM / 32], wo[TN / 32];  // bytes
 #pragma unroll
   for (int q = 0; q < TM / 32; ++q) {
     const int row = (w * (TM / 32) + q) * 8 + (lane >> 3);
-    ap[q] = static_cast<const float*>(t.A) + a_row<MODE>(p, t, row) * t.lda + (((lane & 7) ^ ((row >> 1) & 7)) << 2);
+    ao[q] = (unsigned)((a_row<MODE>(p, t, row) - r0) * t.lda * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
 #pragma unroll
   for (int q = 0; q < TN / 32; ++q) {
     const int row = (w * (TN / 32) + q) * 8 + (lane >> 3);
-    wp[q] = static_cast<const float*>(t.W) + (long)min(t.n0 + row, t.N - 1) * t.ldw + (((lane & 7) ^ ((row >> 1) & 7)) << 2);
+    wo[q] = (unsigned)(min(row, t.N - 1 - t.n0) * t.ldw * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
   auto issue = [&](int kt, int slot) {
     char* b = smem + slot * SLOT_BYTES;
 #pragma unroll
-    for (int q = 0; q < TM / 32; ++q)
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(ap[q] + (long)kt * BKF), (lds_void*)(b + (w * (TM / 32) + q) * 1024), 16,
-                                       0, 0);
+    for (int q = 0; q < TM / 32; ++q) lds_dma16(ab, b + (w * (TM / 32) + q) * 1024, ao[q], kt * BKF * 4);
 #pragma unroll
-    for (int q = 0; q < TN / 32; ++q)
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(wp[q] + (long)kt * BKF),
-                                       (lds_void*)(b + A_BYTES + (w * (TN / 32) + q) * 1024), 16, 0, 0);
+    for (int q = 0; q < TN / 32; ++q) lds_dma16(wb, b + A_BYTES + (w * (TN / 32) + q) * 1024, wo[q], kt * BKF * 4);
   };
   auto frag = [&](const char* tile, int row, int chunk) {
     return *reinterpret_cast<const f32x4*>(tile + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4));
@@ -485,7 +484,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   }
 }
 
-// Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
+// Rows without whole k-steps of 32, off 16 bytes or 4 GB apart: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
 template <int MODE>
 __global__ __launch_bounds__(256) void group_gemm_f32_kernel(GgParams p) {
   using namespace gg;
@@ -706,9 +705,13 @@ static hipError_t gg_f32_on(const GgParams& p, hipStream_t st) {
 
 template <int MODE>
 static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
-  // the tiles' loads take whole 16 bytes and k-steps of 32
+  // the tiles' loads take whole 16 bytes and k-steps of 32, and count bytes from a tile's first
+  // row, or from the first of the rows it gathers, in 32 bits
   auto at = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
-  if (p.K % 32 || (p.Ns > 0 && p.Ks % 32) || (at(p.A) | at(p.W) | at(p.As) | at(p.Ws)) % 16) {
+  auto far = [](long rows, long ld, int K) { return (rows * ld + K) * 4 >= 1L << 32; };
+  if (p.K % 32 || (p.Ns > 0 && p.Ks % 32) || (at(p.A) | at(p.W) | at(p.As) | at(p.Ws)) % 16 ||
+      far(MODE == GG_UP ? p.T : 64, p.lda, p.K) || far(64, p.ldw, p.K) ||
+      (p.Ns > 0 && (far(64, p.ldas, p.Ks) || far(64, p.ldws, p.Ks)))) {
     const long blocks = gg_blocks(p, MODE, 64, 64);
     if (blocks) hipLaunchKernelGGL((group_gemm_f32_kernel<MODE>), dim3((unsigned)blocks), dim3(256), 0, st, p);
     return hipGetLastError();

@@ -72,3 +72,16 @@ def test_latent_without_keys_fp32(C, H, rank):  # noqa: F811
     assert not got[0].any()
     s = torch.cat([q[1].to(F64) @ c.to(F64).T * rank ** -0.5, sink.to(F64)[:, None]], -1)
     assert float((got[1] - (torch.softmax(s, -1)[:, :-1] @ c.to(F64))[:, : got.shape[2]]).abs().max()) < 1e-5
+
+
+# rows that a tile of 64 reaches in 32 bits, and the next wider ones
+@pytest.mark.parametrize("K,step", [(64, (1 << 24) - 4), (64, 1 << 24)])
+@pytest.mark.parametrize("far", ["a", "w"])
+def test_rows_far_apart(C, K, step, far):  # noqa: F811
+    n = 65
+    a, w = rand(n, K, seed=1), rand(n, K, seed=2)
+    room = torch.empty(n * step, device=DEV).as_strided((n, K), (step, 1))
+    room.copy_(a if far == "a" else w)
+    got = C.linear_fp32(*((room, w.to(DEV)) if far == "a" else (a.to(DEV), room))).cpu().to(F64)
+    size = a.to(F64).abs() @ w.to(F64).abs().T
+    assert bool(((got - a.to(F64) @ w.to(F64).T).abs() <= (K + 2) * ULP * size).all())

@@ -87,10 +87,13 @@ int g_group_rows = 8;  // row tiles per group of the expert tile order above 204
 
 void run(GgParams& p, int mode, int tm, bool f32, const char* what) {
   const int tiles_s = std::max(1, (p.T + tm - 1) / tm);
-  // Groups of like size: an XCD takes a part of one, and with a last group of few tiles half of
-  // the XCDs have nothing to do (565 tokens in fp32, 9 tiles as 8 + 1: up 365 -> 325 us, down 191 -> 170)
-  const int groups_s = p.T <= 2048 ? 1 : (tiles_s + g_group_rows - 1) / g_group_rows;
-  p.gr_s = (tiles_s + groups_s - 1) / groups_s;
+  // An XCD takes a part of one group, so no group may have many fewer tiles than the others (565
+  // tokens in fp32, 9 tiles as 8 + 1: up 365 us, in one group 325; down 191 and 170). Groups beyond
+  // g_group_rows cost less (2000 tokens, 16 tiles as 8 + 8: up 150 us, in one group 154).
+  int n = (tiles_s + g_group_rows - 1) / g_group_rows;
+  auto per = [&] { return (tiles_s + n - 1) / n; };
+  while (n > 1 && (per() * n - tiles_s) * 16 > tiles_s) --n;
+  p.gr_s = per();
   p.gr = p.T <= 2048 ? std::max(1, p.n_tiles) : g_group_rows;
   check_hip(f32 ? lsd_group_gemm_f32(&p, mode, cur_stream()) : lsd_group_gemm(&p, mode, tm, cur_stream()), what);
 }

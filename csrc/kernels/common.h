@@ -59,11 +59,12 @@ constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4
 // LDS-DMA of 16 bytes a lane (64 in a row of LDS) from base + off + soff, base and soff the
 // same in the whole wave.  Against global_load_lds, whose addresses are 64 bits a lane, it takes
 // fewer issue cycles beside the products of its wave: 8192 x 8192 x 2048 in fp32 119 -> 139 TF/s
-// (138 without any loads).  off + soff + 16 < 2^32.
+// (138 without any loads).  off + soff + 16 < 2^32; AUX: cache policy.
+template <int AUX = 0>
 __device__ __forceinline__ void lds_dma16(const void* base, void* lds, unsigned off, int soff) {
   typedef __attribute__((address_space(3))) void lds_void;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xffffffff, 0x00020000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 16, off, soff, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)lds, 16, off, soff, 0, AUX);
 }
 
 // f(Int<N - 1>) .. f(Int<0>): counted waits need their counts at compile time

@@ -352,11 +352,13 @@ typedef __attribute__((address_space(1))) const void gbl_cvoid;
 // same XOR is applied on the read (guide §5.4 rule 21).
 // kStageBL: the 4- and 8-wave decode / tiled stagers (stage_tile, stage8) issue buffer_load ...
 // lds from a wave-uniform resource at (row0, k0) with 32-bit lane offsets instead of
-// global_load_lds with 64-bit lane addresses (-DLSD_GLDS_GLOBAL restores the latter for A/B).
+// global_load_lds with 64-bit lane addresses, which take issue cycles from the products (-DLSD_GLDS_GLOBAL
+// restores the latter for A/B): 400 x 50304 x 1600 88.7 -> 82.1 us, 1000 x 6528 x 2048 36.0 -> 33.9,
+// 300 x 2048 x 7680 99.7 -> 79.8, 300 x 4800 x 1600 20.4 -> 20.0.
 #ifdef LSD_GLDS_GLOBAL
 constexpr bool kStageBL = false;
 #else
-constexpr bool kStageBL = false;
+constexpr bool kStageBL = true;
 #endif
 
 template <int ROWS = TBM, bool BL = kStageBL>

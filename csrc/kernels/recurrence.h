@@ -37,13 +37,13 @@ __device__ __forceinline__ float softplus_f(float z) {
   const float e = exp_f(-fabsf(z));
   return fmaxf(z, 0.f) + log1p_series(e * __builtin_amdgcn_rcpf(2.f + e));
 }
-// Sum over the threads of equal (tid % LV): every thread gets its column group's total.
-template <int LV>
+// Sum over the threads of equal (tid % LV) of W waves: every thread gets its column group's total.
+template <int LV, int W = 4>
 __device__ __forceinline__ f32x4 column_sum(f32x4 v, float (*red)[LV * 4]) {
 #pragma unroll
   for (int off = LV; off < 64; off <<= 1)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] += shfl_xor(v[i], off);
+    for (int i = 0; i < 4; ++i) v[i] += wave_xor_n(v[i], off);
   const int lane = lane_id(), w = threadIdx.x >> 6;
   __syncthreads();
   if (lane < LV) *reinterpret_cast<f32x4*>(&red[w][lane * 4]) = v;
@@ -51,7 +51,7 @@ __device__ __forceinline__ f32x4 column_sum(f32x4 v, float (*red)[LV * 4]) {
   const int lv = threadIdx.x % LV;
   f32x4 t = *reinterpret_cast<f32x4*>(&red[0][lv * 4]);
 #pragma unroll
-  for (int i = 1; i < 4; ++i) t += *reinterpret_cast<f32x4*>(&red[i][lv * 4]);
+  for (int i = 1; i < W; ++i) t += *reinterpret_cast<f32x4*>(&red[i][lv * 4]);
   return t;
 }
 

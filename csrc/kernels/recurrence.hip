@@ -3,8 +3,8 @@
 //
 //  * recur_seq: token by token, state in registers.  One launch does the
 //    convolution, SiLU, unit norms, decay, state update and read-out, and for
-//    the delta rule the output norm and gate.  Decode steps, and prompts of
-//    models served in fp32.
+//    the delta rule the output norm and gate.  Decode steps (recur_tile for
+//    common sizes), and prompts of models served in fp32.
 //  * conv_silu, delta_chunk, ssd_chunk: prompts of bf16 models.  Chunks of 16
 //    (delta rule) or 32 tokens (Mamba-2) become matrix products around a state
 //    that stays in the accumulators of four waves, each owning columns of it; the
@@ -61,12 +61,10 @@ __device__ __forceinline__ float conv_at(const ConvParams& c, int ch, long row, 
 
 // One (sequence, head, LV * 4 columns of the state) per block; thread (dg, lv)
 // holds rows dg + i * 256 / LV of four columns.  Dynamic LDS: q, k, decays [D].
-// Bound in decode by the state, read and written once a step: it passes the caches by, which
-// keep the weights of the step instead, and the SSM's registers fit four blocks a CU.  96
-// sequences: 64 heads of 64 x 128 91 -> 85 us, 16 of 128 x 128 60 -> 56, and the step that
-// holds three layers of each 1131 -> 1052; 16 sequences 567 -> 523.  No fewer sequences need the
-// caches: between two steps 4 GB of weights pass them.  Through and by the caches, 1 sequence
-// 430 and 426 us a step, 2 454 and 449, 4 478 and 467, 8 505 and 490.
+// Decode steps of common sizes run on recur_tile_kernel; this form takes any sizes and tap counts and
+// portions of several tokens.  Bound by the state, read and written once a launch: it passes the
+// caches by, which keep the weights of the step instead (through and by the caches, steps of three
+// such layers each, 96 sequences 1131 and 1052 us, 16 567 and 523, 8 505 and 490, 1 430 and 426).
 template <typename T, bool DELTA, int LV, int NR>
 __global__ __launch_bounds__(256, NR > 8 ? 2 : DELTA ? 3 : 4) void recur_seq_kernel(RecurParams p) {
   constexpr int VB = LV * 4, DG = 256 / LV;
@@ -224,6 +222,182 @@ __global__ __launch_bounds__(256, NR > 8 ? 2 : DELTA ? 3 : 4) void recur_seq_ker
 #pragma unroll
     for (int i = 0; i < NR; ++i)
       if (dg + i * DG < D) __builtin_nontemporal_store(s[i], reinterpret_cast<f32x4*>(Sg + (long)(dg + i * DG) * p.Vp));
+  }
+}
+
+__device__ __forceinline__ f32x4 four(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ f32x4 four(const bf16* p) {
+  const bf16x4 v = ld4(p);
+  return f32x4{bf2f(v[0]), bf2f(v[1]), bf2f(v[2]), bf2f(v[3])};
+}
+__device__ __forceinline__ f32x2 two(const float* p) { return *reinterpret_cast<const f32x2*>(p); }
+__device__ __forceinline__ f32x2 two(const bf16* p) {
+  const bf16x2 v = *reinterpret_cast<const bf16x2*>(p);
+  return f32x2{bf2f(v[0]), bf2f(v[1])};
+}
+__device__ __forceinline__ void put_two(float* p, f32x2 v) { *reinterpret_cast<f32x2*>(p) = v; }
+__device__ __forceinline__ void put_two(bf16* p, f32x2 v) { *reinterpret_cast<bf16x2*>(p) = pack2(v[0], v[1]); }
+__device__ __forceinline__ void put_four(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+__device__ __forceinline__ void put_four(bf16* p, f32x4 v) { st4(p, pack4(v)); }
+
+// A decode step where a block's threads hold whole rows and columns of the state (D = NR DG, V a
+// multiple of VB), four taps, and everything in fours lies on its vectors (recur_tiles).
+// The general form spends 800 vector and 500 scalar instructions a wave on addresses, masks and a
+// convolution by all threads, in 128 registers (183 for 128 x 128), and loads the gates one by one
+// behind its last sum.  Here a thread convolves two channels, all loads set out at once, as
+// vectors, and q, k and decays lie in LDS in the order in which a thread reads them; with eight rows
+// a thread at most (NT threads) 72 to 77 registers leave room for three quarters of the waves.
+// General form -> here, the state at 5.0 to 5.5 TB/s (read and written alone: 6.3):
+//   16 heads of 128 x 128  1 sequence 11.2 -> 6.0 us, 16 13.3 -> 9.5, 96 50.7 -> 40.0, 160 80.0 -> 66.4
+//   64 heads of 64 x 128   1 sequence 10.0 -> 6.9 us, 16 17.7 -> 15.0, 96 80.2 -> 75.2, 160 125 -> 121
+// (between other launches of a step, 96 sequences: 55 -> 41 and 87 -> 70).
+template <typename T, bool DELTA, int LV, int NR, int NT>
+__global__ __launch_bounds__(NT, 6) void recur_tile_kernel(RecurParams p) {
+  constexpr int VB = LV * 4, DG = NT / LV, D = NR * DG, W = NT / 64, PAIRS = (2 * D + VB) / 2;
+  static_assert(PAIRS + D / 4 <= NT || !DELTA, "decays on threads of their own");
+  static_assert(PAIRS < NT && D % 64 == 0 && NR % 4 == 0, "sizes");
+  // [key row d at (d % DG) NR + d / DG]
+  __shared__ __attribute__((aligned(16))) float qs[D], ks[D], gs[DELTA ? D : 4], vs[VB], red[W][LV * 4];
+  __shared__ float sc[2];
+  auto at = [](int d) { return d % DG * NR + d / DG; };
+  const int tid = threadIdx.x;
+  const int nvb = p.V / VB;
+  const int h = blockIdx.x / nvb, v0 = (blockIdx.x - h * nvb) * VB, b = blockIdx.y;
+  const int rep = p.heads / p.groups, kh = h / rep;
+  const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b];
+  if (p.s.cu[b + 1] == r0) return;
+  const int lv = tid % LV, dg = tid / LV, col = v0 + lv * 4;
+  float* Sg = p.S + ((long)slot * p.heads + h) * D * p.V + v0;  // (scalar; a lane adds own)
+  const unsigned own = dg * p.V + lv * 4;
+  f32x4 s[NR];
+  if (start > 0) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sg + (long)i * DG * p.V + own));
+  } else {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // this thread's two channels
+  const int part = tid * 2 < D ? 0 : tid * 2 < 2 * D ? 1 : 2, c0 = tid * 2 - part * D;
+  const int ch = part == 0 ? p.q_ch + kh * D + c0 : part == 1 ? p.k_ch + kh * D + c0 : p.v_ch + h * p.V + v0 + c0;
+  const bool keeps = p.write_ring && (part == 2 || (h - kh * rep == 0 && v0 == 0));
+  T* ring = static_cast<T*>(p.c.ring) + (long)slot * 4 * p.c.channels;
+  f32x4 norm = {};
+  if (DELTA && !p.raw && dg == 0) norm = four(p.norm + col);
+
+  const long row = r0;
+  const int pos = start;
+  const T* y = static_cast<const T*>(p.c.y) + row * p.c.ldy;
+  f32x4 gate = {};
+  if (DELTA ? !p.raw && dg == 0 : dg == 0)
+    gate = DELTA ? four(static_cast<const T*>(p.low) + row * p.ldl + p.gate_off + (long)h * p.V + col)
+                 : four(y + (long)h * p.V + col);
+  if (tid < PAIRS) {
+    f32x2 x[4], bias = {};
+    const f32x4 w[2] = {four(p.c.w + ch * 4), four(p.c.w + ch * 4 + 4)};
+    if (p.c.bias) bias = two(p.c.bias + ch);
+    const T* now = y + p.c.c0;
+#pragma unroll
+    for (int back = 0; back < 4; ++back) {
+      const bool live = back <= pos;
+      x[back] = two((back == 0 || !live ? now : ring + (long)((pos - back) & 3) * p.c.channels) + ch);
+      if (!live) x[back] = f32x2{0.f, 0.f};
+    }
+    if (keeps) put_two(ring + (long)(pos & 3) * p.c.channels + ch, x[0]);  // (as it was read)
+    float* dst = part == 2 ? vs + c0 : part == 0 ? qs : ks;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      float a = 0.f;
+#pragma unroll
+      for (int back = 3; back >= 0; --back) a = fmaf(w[e][3 - back], x[back][e], a);
+      a *= p.c.gain;
+      dst[part == 2 ? e : at(c0 + e)] = silu_x(p.c.bias ? a + bias[e] : a);
+    }
+  }
+  if (DELTA && tid >= NT - D / 4) {
+    const int d = (tid - (NT - D / 4)) * 4;
+    const f32x4 low = four(static_cast<const T*>(p.low) + row * p.ldl + (long)h * D + d), db = four(p.dt_bias + (long)h * D + d);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) gs[at(d + e)] = expf(p.A[h] * softplus_x(p.c.gain * low[e] + db[e]));
+  }
+  if (tid == NT - 1) {
+    const float gl = p.c.gain * to_f(y[p.gate_col + h]);
+    if constexpr (DELTA) {
+      sc[0] = sigmoid_x(gl);
+    } else {
+      const float dt = softplus_x(gl + p.dt_bias[h]);
+      sc[0] = dt;
+      sc[1] = expf(p.A[h] * dt);
+    }
+  }
+  __syncthreads();
+  const f32x4 v = four(vs + lv * 4);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  auto rows = [&](auto f) {  // f(i, q, k, decay)
+#pragma unroll
+    for (int i4 = 0; i4 < NR; i4 += 4) {
+      const f32x4 q = four(qs + dg * NR + i4), k = four(ks + dg * NR + i4), g = DELTA ? four(gs + dg * NR + i4) : f32x4{};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f(i4 + i, q[i], k[i], g[i]);
+    }
+  };
+  if constexpr (DELTA) {
+    float nq = 0.f, nk = 0.f;
+#pragma unroll
+    for (int d = 0; d < D; d += 64) {
+      const int j = at(d + lane_id());
+      nq += qs[j] * qs[j];
+      nk += ks[j] * ks[j];
+    }
+    const float iq = rsqrtf((float)D) / sqrtf(wave_sum(nq) + UNIT_EPS), ik = 1.f / sqrtf(wave_sum(nk) + UNIT_EPS);
+    f32x4 pr = {0.f, 0.f, 0.f, 0.f};
+    rows([&](int i, float, float k, float g) {
+      s[i] *= g;
+      pr += s[i] * (k * ik);
+    });
+    pr = column_sum<LV, W>(pr, red);
+    const f32x4 u = sc[0] * (v - pr);
+    rows([&](int i, float q, float k, float) {
+      s[i] += u * (k * ik);
+      o += s[i] * (q * iq);
+    });
+  } else {
+    const float a = sc[1];
+    const f32x4 u = v * sc[0];
+    rows([&](int i, float q, float k, float) {
+      s[i] = s[i] * a + u * k;
+      o += s[i] * q;
+    });
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) __builtin_nontemporal_store(s[i], reinterpret_cast<f32x4*>(Sg + (long)i * DG * p.V + own));
+  o = column_sum<LV, W>(o, red);
+  if constexpr (!DELTA) {  // y silu(z): the group norm follows
+    if (dg == 0) {
+      o += v * p.skip[h];
+      f32x4 r;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r[i] = o[i] * silu_x(p.c.gain * gate[i]);
+      put_four(static_cast<T*>(p.out) + row * p.ldo + (long)h * p.V + col, r);
+    }
+  } else if (p.raw) {
+    if (dg == 0) put_four(p.raw + row * p.ldr + (long)h * p.V + col, o);
+  } else {  // one block holds all of V: norm and gate here
+    if (tid < 64) {
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ss += dg == 0 ? o[i] * o[i] : 0.f;
+      const float rs = 1.f / sqrtf(wave_sum(ss) / p.V + p.eps);
+      if (dg == 0) {
+        f32x4 r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = o[i] * rs * norm[i] * sigmoid_x(p.c.gain * gate[i]);
+        put_four(static_cast<T*>(p.out) + row * p.ldo + (long)h * p.V + col, r);
+      }
+    }
+    if (h == p.heads - 1)
+      for (int c = p.heads * p.V + tid; c < p.out_cols; c += NT) from_f(static_cast<T*>(p.out) + row * p.ldo + c, 0.f);
   }
 }
 
@@ -1316,6 +1490,18 @@ extern "C" int lsd_recur_block(int D, int V) {
   return (D + 1024 / vb - 1) / (1024 / vb) <= 16 ? vb : 0;
 }
 
+// Whether a step's vectors of four lie on their sizes (recur_tile_kernel).
+static bool recur_tiles(const RecurParams& p, int delta, int f32, int vb) {
+  const uintptr_t four = f32 ? 15 : 7;
+  auto at = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
+  const int off = p.c.channels | p.c.c0 | p.q_ch | p.k_ch | p.v_ch | p.D | p.V | (int)(p.c.ldy & 3) | (int)(p.ldo & 3);
+  if (!p.write_ring || p.c.taps != 4 || p.V % vb || off % 4 || (at(p.c.y) | at(p.c.ring) | at(p.out)) & four) return false;
+  if ((at(p.c.w) | at(p.c.bias) | at(p.S)) & 15) return false;
+  if (!delta) return true;
+  return !((at(p.dt_bias) | at(p.norm) | at(p.raw)) & 15) && !(at(p.low) & four) && p.gate_off % 4 == 0 && p.ldl % 4 == 0 &&
+         p.ldr % 4 == 0;
+}
+
 extern "C" hipError_t lsd_recur_seq(const RecurParams* p, int delta, int f32, hipStream_t st) {
   if (p->s.B == 0) return hipSuccess;
   const int vb = lsd_recur_block(p->D, p->V);
@@ -1324,6 +1510,19 @@ extern "C" hipError_t lsd_recur_seq(const RecurParams* p, int delta, int f32, hi
   if (delta && !p->raw && nvb != 1) return hipErrorInvalidValue;
   const dim3 grid(p->heads * nvb, p->s.B);
   const size_t lds = 3 * p->D * sizeof(float);
+  if (recur_tiles(*p, delta, f32, vb)) {
+#define LSD_RT(T, DELTA, LV, NR, NT)                                                                    \
+  if (delta == DELTA && vb == 4 * LV && p->D == NR * (NT / LV)) {                                       \
+    hipLaunchKernelGGL((recur_tile_kernel<T, DELTA, LV, NR, NT>), grid, dim3(NT), 0, st, *p);           \
+    return hipGetLastError();                                                                           \
+  }
+#define LSD_RT_T(T)                                                                                     \
+  LSD_RT(T, true, 32, 8, 512) LSD_RT(T, false, 32, 8, 512) LSD_RT(T, true, 32, 8, 256) LSD_RT(T, false, 32, 8, 256) \
+  LSD_RT(T, true, 16, 8, 256) LSD_RT(T, false, 16, 8, 256) LSD_RT(T, true, 16, 4, 256) LSD_RT(T, false, 16, 4, 256)
+    if (f32) { LSD_RT_T(float) } else { LSD_RT_T(bf16) }
+#undef LSD_RT_T
+#undef LSD_RT
+  }
 #define LSD_RS(T, DELTA, LV, NR) \
   hipLaunchKernelGGL((recur_seq_kernel<T, DELTA, LV, NR>), grid, dim3(256), lds, st, *p)
 #define LSD_RS_N(T, DELTA, LV)                  \

@@ -22,14 +22,14 @@ namespace {
 __device__ __forceinline__ float write_gate(float z, float lower) { return (1.f - lower) / (1.f + expf(z)); }
 
 // One (sequence, head, LV * 4 columns of the state) per block; thread (dg, lv)
-// holds rows dg + i * 256 / LV of four columns.  Dynamic LDS: q, 1 - f [D].  The state passes
+// holds rows dg + i * NT / LV of four columns.  Dynamic LDS: q, 1 - f [D].  The state passes
 // the caches by, as recur_seq_kernel's (a step with four such layers of 64 sequences 1366 ->
 // 1287 us, of 24 1213 -> 1177; of 1, 4 and 8 the same either way: 645, 874 and 1045).
-template <typename T, int LV, int NR>
-__global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(ForgetParams p) {
-  constexpr int VB = LV * 4, DG = 256 / LV;
+template <typename T, int LV, int NR, int NT = 256>
+__global__ __launch_bounds__(NT, NR > 8 ? 4 : 6) void forget_seq_kernel(ForgetParams p) {
+  constexpr int VB = LV * 4, DG = NT / LV;
   extern __shared__ float dyn[];
-  __shared__ __attribute__((aligned(16))) float red[4][LV * 4];
+  __shared__ __attribute__((aligned(16))) float red[NT / 64][LV * 4];
   __shared__ __attribute__((aligned(16))) float vs[VB];
   const int D = p.D, tid = threadIdx.x;
   float *qs = dyn, *ks = dyn + D;
@@ -39,17 +39,19 @@ __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(Forget
   if (n <= 0) return;
   const int lv = tid % LV, dg = tid / LV, col = v0 + lv * 4;
   const bool live = col < p.Vp;
-  float* Sg = p.S + ((long)slot * p.heads + h) * D * p.Vp + col;
+  float* Sg = p.S + ((long)slot * p.heads + h) * D * p.Vp + v0;  // (scalar; a lane adds own)
+  const unsigned own = dg * p.Vp + lv * 4;
   f32x4 s[NR];
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (start > 0 && live && dg + i * DG < D) s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sg + (long)(dg + i * DG) * p.Vp));
+    if (start > 0 && live && dg + i * DG < D) 
+      s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sg + (long)i * DG * p.Vp + own));
   }
   for (int t = 0; t < n; ++t) {
     const long row = r0 + t;
     const T* y = static_cast<const T*>(p.y) + row * p.ldy;
-    for (int c = tid; c < 2 * D + VB; c += 256) {
+    for (int c = tid; c < 2 * D + VB; c += NT) {
       if (c < D) {
         qs[c] = silu_x(to_f(y[h * D + c]));
       } else if (c < 2 * D) {
@@ -71,7 +73,7 @@ __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(Forget
         o += s[i] * qs[d];
       }
     }
-    o = column_sum<LV>(o, red);  // its barriers also free q, 1 - f and v
+    o = column_sum<LV, NT / 64>(o, red);  // its barriers also free q, 1 - f and v
     if (p.raw) {
       if (dg == 0 && live) {
 #pragma unroll
@@ -90,13 +92,13 @@ __global__ __launch_bounds__(256, NR <= 8 ? 3 : 2) void forget_seq_kernel(Forget
           if (col + i < p.V) from_f(out + (long)h * p.V + col + i, o[i] * rs * p.norm[col + i]);
       }
       if (h == p.heads - 1)
-        for (int c = p.heads * p.V + tid; c < p.out_cols; c += 256) from_f(out + c, 0.f);
+        for (int c = p.heads * p.V + tid; c < p.out_cols; c += NT) from_f(out + c, 0.f);
     }
   }
   if (live) {
 #pragma unroll
     for (int i = 0; i < NR; ++i)
-      if (dg + i * DG < D) __builtin_nontemporal_store(s[i], reinterpret_cast<f32x4*>(Sg + (long)(dg + i * DG) * p.Vp));
+      if (dg + i * DG < D) __builtin_nontemporal_store(s[i], reinterpret_cast<f32x4*>(Sg + (long)i * DG * p.Vp + own));
   }
 }
 
@@ -483,13 +485,21 @@ extern "C" hipError_t lsd_forget_seq(const ForgetParams* p, int vb, int f32, hip
   if (!p->raw && nvb != 1) return hipErrorInvalidValue;
   const dim3 grid(p->heads * nvb, p->s.B);
   const size_t lds = 2 * p->D * sizeof(float);
-#define LSD_FS(T, LV, NR) hipLaunchKernelGGL((forget_seq_kernel<T, LV, NR>), grid, dim3(256), lds, st, *p)
-#define LSD_FS_N(T, LV)                \
-  if (nr <= 1) LSD_FS(T, LV, 1);       \
-  else if (nr <= 2) LSD_FS(T, LV, 2);  \
-  else if (nr <= 4) LSD_FS(T, LV, 4);  \
-  else if (nr <= 8) LSD_FS(T, LV, 8);  \
-  else LSD_FS(T, LV, 16);
+  // 16 rows a thread, four blocks a CU, or eight of twice the threads, three a CU: the latter start
+  // and end sooner (heads of 128 x 128, 16 a sequence: 1 sequence 7.8 -> 5.7 us, 24 11.1 -> 10.1, 96 41.1
+  // -> 39.0, 160 65.8 -> 62.6) unless that takes a round more (64 sequences 23.4 -> 27.0)
+  const long blocks = (long)grid.x * grid.y;
+  const bool wide = (blocks + 767) / 768 <= (blocks + 1023) / 1024;
+#define LSD_FS_NT(T, LV, NR, NT) hipLaunchKernelGGL((forget_seq_kernel<T, LV, NR, NT>), grid, dim3(NT), lds, st, *p)
+#define LSD_FS(T, LV, NR)                                               \
+  if (NR > 8 && wide) LSD_FS_NT(T, LV, (NR > 8 ? NR / 2 : NR), 512);    \
+  else LSD_FS_NT(T, LV, NR, 256)
+#define LSD_FS_N(T, LV)                    \
+  if (nr <= 1) { LSD_FS(T, LV, 1); }       \
+  else if (nr <= 2) { LSD_FS(T, LV, 2); }  \
+  else if (nr <= 4) { LSD_FS(T, LV, 4); }  \
+  else if (nr <= 8) { LSD_FS(T, LV, 8); }  \
+  else { LSD_FS(T, LV, 16); }
 #define LSD_FS_V(T)                    \
   switch (vb) {                        \
     case 4: LSD_FS_N(T, 1) break;      \
@@ -507,6 +517,7 @@ extern "C" hipError_t lsd_forget_seq(const ForgetParams* p, int vb, int f32, hip
 #undef LSD_FS_V
 #undef LSD_FS_N
 #undef LSD_FS
+#undef LSD_FS_NT
   return hipGetLastError();
 }
 

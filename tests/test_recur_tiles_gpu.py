@@ -48,3 +48,26 @@ def test_delta_off_vectors(C, c0, dt):  # noqa: F811
     y[:, c0: c0 + cols] = c.y[:, c.c0: c.c0 + cols]
     c.y, c.c0 = y, c.c0 + at
     check(c, 128, dt)
+
+
+# 16 heads: one round of blocks of 512 threads (48 sequences), of 256 (49 .. 64), then two of 512
+@DTYPES
+@pytest.mark.parametrize("B", [1, 48, 49, 64, 65])
+def test_forget_rounds(C, B, dt):  # noqa: F811
+    H, D, V, eps = 16, 128, 128, 1e-5
+    g = torch.Generator().manual_seed(B)
+    y = torch.randn(B, H * (2 * D + V), generator=g).to(dt)
+    bias, lower, norm = torch.randn(H * D, generator=g), torch.rand(H * D, generator=g), 1 + 0.2 * torch.randn(V, generator=g)
+    S = torch.randn(B, H, D, V, generator=g)
+    i32 = dict(dtype=torch.int32, device="cuda")
+    state, out = S.cuda(), torch.empty(B, H * V, dtype=dt, device="cuda")
+    C.forget_seq(y.cuda(), torch.arange(B, **i32), torch.full((B,), 9, **i32), torch.arange(B + 1, **i32), H, D, V, bias.cuda(),
+                 lower.cuda(), norm.cuda(), eps, state, out, False, 1)
+    q, z, v = y.double().split([H * D, H * D, H * V], 1)
+    write = ((1 - lower.double()) * torch.sigmoid(-z - bias.double())).reshape(B, H, D, 1)
+    want = S.double() * (1 - write) + write * v.reshape(B, H, 1, V)
+    assert err(state, want) < 2e-6  # three roundings a number, and expf in the gate
+    q = q * torch.sigmoid(q)
+    o = (want * q.reshape(B, H, D, 1)).sum(2)
+    o = o / torch.sqrt(o.pow(2).mean(-1, keepdim=True) + eps) * norm.double()
+    assert err(out.reshape(B, H, V), o) < (8e-3 if dt == BF else 1e-5)

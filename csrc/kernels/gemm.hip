@@ -1591,7 +1591,18 @@ __global__ __launch_bounds__(512) void gemm_d256_kernel(GemmParams p, int* __res
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-static int g_big_min_blocks = 160;  // lsd_gemm_set_big_min(): tuning / tests
+static int g_big_min_blocks = 160;  // lsd_gemm_set_big_min(): tuning / tests (1 << 16 and more: never)
+// Whether a tiled launch runs on 256 x 256 tiles, one block a CU: from g_big_min_blocks of them on, or
+// where the 128 x 128 tiles, two blocks a CU, take more than one round.  A round of either, with
+// the operands of 2048 columns: 1000 rows of 6144 (384 tiles, 96) 31.7 us and 38.5, of 8576 (536, 136) 53.0
+// and 40.1, of 11264 (704, 176) 54.4 and 41.6; 800 of 8576 (469, 136) 33.7 and 40.6; 2000 of 4096 (512, 128)
+// 34.9 and 40.4; 1300 of 6144 (528, 144) 53.1 and 41.3, with K = 4096 97.4 and 73.2, with 1600 43.4 and 34.4.
+static bool big_tiles(int M, int N, int K, int S) {
+  if (M < GBM || K % 64 != 0) return false;
+  const long big = (long)((M + GBM - 1) / GBM) * ((N + GBN - 1) / GBN) * S;
+  const long small = (long)((M + TBM - 1) / TBM) * ((N + TBM - 1) / TBM) * S;
+  return big >= g_big_min_blocks || (g_big_min_blocks < 1 << 16 && small > 512);
+}
 // lsd_gemm_set_big_group(): tile_order() group (0 = M-fastest).  4: XL prefill
 // GEMMs 10-25 % faster than M-fastest, 8 equal, 16+ slower
 // (profiles/r2_prefill_tile_order.log)
@@ -1707,10 +1718,8 @@ static hipError_t launch_d256(const GemmParams& p, int kind, int* cnt, float* ws
 
 template <int EPI>
 static hipError_t launch_tiled(const GemmParams& p, int* cnt, float* ws, hipStream_t st) {
-  // 256x256 pipelined kernel once the problem fills the chip with 1-block/CU
-  // tiles; the 128x128 kernel (2 blocks/CU) for smaller M / N.
   const int bm = (p.M + GBM - 1) / GBM, bn = (p.N + GBN - 1) / GBN;
-  if (p.M >= GBM && p.K % 64 == 0 && bm * bn * p.splits >= g_big_min_blocks) {
+  if (big_tiles(p.M, p.N, p.K, p.splits)) {
     if (g_big_kind == 1)
       hipLaunchKernelGGL((gemm_p8_kernel<EPI, 0>), dim3(bm * bn * p.splits), dim3(512), 0, st, p, bm, bn,
                          g_big_group);
@@ -1823,8 +1832,7 @@ extern "C" int lsd_gemm_d256_bn(int kind, int M, int N, int K) { return d256_bn(
 // (mirrors launch_tiled), else 0: the split workspace / counters are sized from it
 extern "C" int lsd_gemm_ring8_tiles(int M, int N, int K, int S) {
   if (g_ring8 != 2) return 0;
-  const int bm = (M + GBM - 1) / GBM, bn = (N + GBN - 1) / GBN;
-  if (M >= GBM && K % 64 == 0 && bm * bn * S >= g_big_min_blocks) return 0;
+  if (big_tiles(M, N, K, S)) return 0;
   if (!(g_ring_tn == 64 || g_ring_tn == 32 || g_ring_tn == 0)) return 0;
   const int tm = (M + TBM - 1) / TBM, tn64 = (N + 63) / 64;
   const bool narrow = g_ring_tn == 32 || (g_ring_tn == 0 && tm * tn64 * S < g_ring_fill);

@@ -108,7 +108,8 @@ class Routing:
     # the 256x256 kernel: 120 vs 145 us; profiles/r6_llama512_gemm.log)
     d256_rb_max_m: int = 512
     d256_rb_max_n: int = 8192
-    # the 256x256 pipelined kernel (gemm_p8) once a tiled launch has this
+    # the 256x256 pipelined kernel (gemm_p8) where the 128x128 tiles take more than a round of
+    # two a CU (big_tiles in gemm.hip), or once a tiled launch has this
     # many 256x256 tiles; the 128x128 kernels below (launch_tiled in gemm.hip)
     big_min_blocks: int = 160
     # -- grouped GEMMs (experts, per-head latent projections) ----------------

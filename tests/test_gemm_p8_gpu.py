@@ -77,3 +77,22 @@ def test_k_tiles(C, kind, tiles):
         part = slice(h * K // 2, (h + 1) * K // 2)
         x, y = a[:, part].to(F64), w[:, part].to(F64)
         assert near(got.float(), x @ y.T, (K + 3) * 2.0 ** -24 * (x.abs() @ y.abs().T))
+
+
+# 512 and 520 tiles of 128 x 128: one round of two a CU, and 132 tiles of 256 x 256
+@pytest.mark.parametrize("N", [8192, 8320])
+def test_more_than_a_round(C, N):
+    M, K = 1000, 192
+    g = torch.Generator().manual_seed(N)
+    a, w = torch.randn(M, K, generator=g).bfloat16(), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16()
+    acc = a.to(F64) @ w.to(F64).T
+    off = (K + 3) * 2.0 ** -24 * (a.to(F64).abs() @ w.to(F64).abs().T)
+    C.gemm_set_big_min(160)
+    try:
+        assert near(C.linear(a.to(DEV), w.to(DEV), None, 0, 1, 1, None), acc, off)
+        x = torch.randn(M, N, generator=g)
+        xd = x.to(DEV)
+        C.linear_residual(a.to(DEV), w.to(DEV), None, xd, 1, 1, None, False)
+    finally:
+        C.gemm_set_big_min(1)
+    assert bool(((xd.cpu().to(F64) - x.to(F64) - acc).abs() <= off + 2.0 ** -22 * (acc.abs() + x.abs())).all())

@@ -32,6 +32,7 @@ void lsd_gemm_set_ring8_flags(int v);
 void lsd_gemm_set_ring8_pack(int v);
 void lsd_norm_set_wave_narrow_min(int v);
 void lsd_norm_set_wave_min(int v);
+int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits);
 int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits);
 int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
@@ -851,6 +852,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   // gemm_d256 (launch kind 2 / 3: all <= 256 rows in one tile, 64 / 128 columns): ring depth
   m.def("gemm_set_d256_slots", [](int64_t v) { lsd_gemm_set_d256_slots((int)v); });
   m.def("gemm_set_ring8", [](int64_t v) { lsd_gemm_set_ring8((int)v); });
+  m.def("gemm_deep_shape", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t splits) {
+    const int s = lsd_gemm_deep_shape((int)M, (int)N, (int)K, (int)epi, (int)splits);
+    return std::make_pair(s / 1024, s % 1024); });
   m.def("gemm_on_deep", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t kind, int64_t splits) {
     return lsd_gemm_on_deep((int)M, (int)N, (int)K, (int)epi, (int)kind, (int)splits) != 0; });
   m.def("gemm_ring8_tiles", [](int64_t M, int64_t N, int64_t K, int64_t S) {

@@ -9,9 +9,9 @@
 //    With two, W arrives at half the rate.  Wide tiles of up to 64 rows load W non-temporally
 //    (28672 x 4096 at 40 rows 49.5 -> 44.0 us, 4096 x 14336 23.0 -> 21.3); narrow ones, whose
 //    weights are small, and more rows are 0 to 20 % slower that way.
-//  * a block holds all rows (up to 128; more are two blocks beside each other, the second of
-//    which finds W in L2), so W is read once, and its width (64, 32 or 16 columns) follows
-//    from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
+//  * a block holds all of up to 48 rows; more are also divided among blocks beside each other,
+//    which find W in L2, where that brings a CU fewer bytes.  Its width (96 to 16 columns)
+//    follows from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
 //    32-wide parts among them (WK) and are summed through LDS.  No K splits over blocks, no
 //    tickets and no workspace, except where the caller takes the partial sums as slabs.
 //
@@ -19,7 +19,7 @@
 //   28672 x 4096 gate/up, 40 rows   65.9 -> 44.0 us     4096 x 14336 slabs, 40 rows  28.8 -> 21.3
 //   6144 x 4096 QKV, 40 rows        18.7 -> 14.4        4096 x 4096 slabs, 40 rows   15.0 -> 8.7
 //   6144 x 2048, 24 rows            12.2 -> 7.6         2624 x 2048 fp32, 64 rows    13.1 -> 7.5
-//   11264 x 2048 gate/up, 96 rows   19.8 -> 17.7        4800 x 1600 QKV, 128 rows    13.6 -> 12.0
+//   11264 x 2048 gate/up, 96 rows   19.8 -> 16.8        4800 x 1600 QKV, 128 rows    13.6 -> 9.4
 #include "gemm_epilogue.h"
 
 namespace lsd {
@@ -31,9 +31,9 @@ constexpr int NT_LOAD = 2;  // cache policy of an LDS-DMA: non-temporal
 }  // namespace
 
 // WM x WN waves of MTW x NTW 16 x 16 tiles, times WK waves on different 32-wide parts of a
-// k-step of BK; SLOTS k-steps in LDS; AUX: cache policy of W; TWO: two row blocks.
-template <int WM, int WN, int WK, int MTW, int NTW, int BK, int SLOTS, int AUX, int EPI, bool TWO = false>
-__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams p, int tiles_n) {
+// k-step of BK; SLOTS k-steps in LDS; AUX: cache policy of W.
+template <int WM, int WN, int WK, int MTW, int NTW, int BK, int SLOTS, int AUX, int EPI>
+__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams p, int tiles_n, int row_blocks) {
   constexpr int WAVES = WM * WN * WK, BM = 16 * WM * MTW, BN = 16 * WN * NTW;
   constexpr int RB = BK * 2, CPR = RB / 16, RPI = 64 / CPR;  // bytes and 16-byte chunks of a row, rows per instruction
   constexpr int A_BYTES = BM * RB, SLOT = (BM + BN) * RB;
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
   const int r = lane & 15, g = lane >> 4;
   const int wk = w % WK, wn = (w / WK) % WN, wm = w / (WK * WN);
   const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int m0 = TWO ? (bid & 1) * BM : 0, nb = TWO ? bid >> 1 : bid;  // (row blocks side by side share W)
+  const int nb = row_blocks == 1 ? bid : bid / row_blocks, m0 = (bid - nb * row_blocks) * BM;  // (row blocks side by side share W)
   const int split = nb / tiles_n, n0 = (nb - split * tiles_n) * BN;
   const int KT = p.K / BK;
   const int kb = (int)((long)KT * split / p.splits), ke = (int)((long)KT * (split + 1) / p.splits);
@@ -165,11 +165,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
   }
 }
 
-// Columns of a block.  A CU takes in its blocks' rows of W and A at one rate, so the width with
-// the least of ceil(blocks / CUs) (columns + rows) is the fastest one: measured at 64 rows,
+// A block's rows and columns.  A CU takes in its blocks' rows of W and A at one rate, so the
+// shape with the least of ceil(blocks / CUs) (columns + rows) is the fastest one: measured at 64 rows,
 // 4800 x 1600 on 75 blocks of 64 columns 11.9 us, on 150 of 32 8.8; 2624 x 2048 on 82 of 32 8.8,
 // on 164 of 16 7.5; 8512 x 2048 on 133 of 64 13.0, on 266 of 32 15.6.
-static int deep_rows(int M) {  // of a block
+struct DeepShape {
+  int rows, cols;
+};
+// All rows in a block (up to 128; more are two blocks side by side): whether a call is taken at all
+// goes by these.
+static int deep_rows(int M) {
   return M > 192 ? 128 : M > 128 ? 96 : M > 96 ? 128 : M > 64 ? 96 : (M + 15) / 16 * 16;
 }
 static int deep_cols(int M, int N, int K, int splits, int epi) {
@@ -183,43 +188,76 @@ static int deep_cols(int M, int N, int K, int splits, int epi) {
   }
   return best;
 }
-
-template <int EPI, int MT>
-static hipError_t deep_rows64(const GemmParams& p, int bn, hipStream_t st) {
-  // slots: two blocks per CU
-  constexpr int S64 = MT == 1 ? 8 : MT == 2 ? 6 : 5, S32 = MT == 4 ? 6 : 8, S16 = MT == 1 ? 8 : MT == 2 ? 6 : MT == 3 ? 5 : 4;
-  const int tn = (p.N + bn - 1) / bn;
-  const dim3 grid((unsigned)(tn * p.splits)), block(256);
-  if (bn == 64)
-    hipLaunchKernelGGL((gemm_deep_kernel<1, 4, 1, MT, 1, 64, S64, NT_LOAD, EPI>), grid, block, 0, st, p, tn);
-  else if (bn == 32)
-    hipLaunchKernelGGL((gemm_deep_kernel<1, 2, 2, MT, 1, 64, S32, 0, EPI>), grid, block, 0, st, p, tn);
-  else if constexpr (EPI != EPI_SILU_MUL)
-    hipLaunchKernelGGL((gemm_deep_kernel<1, 1, 4, MT, 1, 128, S16, 0, EPI>), grid, block, 0, st, p, tn);
-  return hipGetLastError();
-}
-
-template <int EPI, int MTW, bool TWO>
-static hipError_t deep_rows128(const GemmParams& p, int bn, hipStream_t st) {
-  const int tn = (p.N + bn - 1) / bn;
-  const dim3 grid((unsigned)(tn * p.splits * (TWO ? 2 : 1))), block(512);
-  if (bn == 64)
-    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 2, 64, MTW == 3 ? 4 : 3, 0, EPI, TWO>), grid, block, 0, st, p, tn);
-  else
-    hipLaunchKernelGGL((gemm_deep_kernel<2, 2, 2, MTW, 1, 64, MTW == 3 ? 5 : 4, 0, EPI, TWO>), grid, block, 0, st, p, tn);
-  return hipGetLastError();
+// More than 48 rows also in blocks of fewer rows, whose neighbours find W in L2 (48 x 96 only up to two
+// of them: 140 rows of 11264 x 2048 24.2 us, so 25.4).  All rows in a block -> here:
+//   64 rows   2624 x 2048 8.3 -> 7.6 us (32 x 32)
+//   96 rows   3072 x 2048 12.3 -> 8.9 (48 x 32), 6464 13.2 -> 11.7 (48 x 64), 8512 14.9 -> 13.4 (48 x 80)
+//   128 rows  4800 x 1600 11.8 -> 9.4 (48 x 64), 6144 x 4096 24.9 -> 21.9 (48 x 80)
+//   256 rows  4800 x 1600 14.1 -> 11.9 (64 x 80), 11264 x 2048 gate/up 30.8 -> 27.3 (64 x 96)
+// and over 176 products of 50 to 256 rows 7 % on average; behind, by 0.2 us, 768 x 3072 in 8 slabs of
+// 128 rows (4.7 us).
+static DeepShape deep_shape(int M, int N, int K, int splits, int epi) {
+  DeepShape best{deep_rows(M), deep_cols(M, N, K, splits, epi)};
+  if (M <= 48) return best;
+  auto cost = [&](DeepShape s) {
+    const long blocks = (long)((N + s.cols - 1) / s.cols) * splits * ((M + s.rows - 1) / s.rows);
+    return (blocks + 255) / 256 * (s.rows + s.cols);
+  };
+  long least = cost(best);
+  auto offer = [&](DeepShape s) {
+    if (epi == EPI_SILU_MUL && s.cols % 32 != 0) return;
+    if (cost(s) < least) { best = s; least = cost(s); }
+  };
+  if (M <= 64) {
+    offer({32, 32});
+  } else {
+    for (int cols : {32, 64, 80, 96})
+      if (cols < 96 || M <= 96) offer({48, cols});
+    for (int cols : {64, 80, 96}) offer({64, cols});
+  }
+  return best;
 }
 
 template <int EPI>
 static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
-  const int bn = deep_cols(p.M, p.N, p.K, p.splits, EPI);
-  if (p.M <= 16) return deep_rows64<EPI, 1>(p, bn, st);
-  if (p.M <= 32) return deep_rows64<EPI, 2>(p, bn, st);
-  if (p.M <= 48) return deep_rows64<EPI, 3>(p, bn, st);
-  if (p.M <= 64) return deep_rows64<EPI, 4>(p, bn, st);
-  if (p.M <= 96) return deep_rows128<EPI, 3, false>(p, bn, st);
-  if (p.M <= 128) return deep_rows128<EPI, 4, false>(p, bn, st);
-  return p.M <= 192 ? deep_rows128<EPI, 3, true>(p, bn, st) : deep_rows128<EPI, 4, true>(p, bn, st);
+  const DeepShape s = deep_shape(p.M, p.N, p.K, p.splits, EPI);
+  const int tn = (p.N + s.cols - 1) / s.cols, mbs = (p.M + s.rows - 1) / s.rows;
+#define LSD_DEEP_K(ROWS, COLS, WM, WN, WK, BK, SLOTS, AUX)                                                            \
+  if (s.rows == ROWS && s.cols == COLS) {                                                                             \
+    hipLaunchKernelGGL((gemm_deep_kernel<WM, WN, WK, ROWS / (16 * WM), COLS / (16 * WN), BK, SLOTS, AUX, EPI>),       \
+                       dim3((unsigned)(tn * p.splits * mbs)), dim3(64 * WM * WN * WK), 0, st, p, tn, mbs);            \
+    return hipGetLastError();                                                                                         \
+  }
+  // slots: two blocks per CU
+  if (mbs == 1) {
+    LSD_DEEP_K(16, 64, 1, 4, 1, 64, 8, NT_LOAD)
+    LSD_DEEP_K(32, 64, 1, 4, 1, 64, 6, NT_LOAD)
+    LSD_DEEP_K(48, 64, 1, 4, 1, 64, 5, NT_LOAD)
+    LSD_DEEP_K(64, 64, 1, 4, 1, 64, 5, NT_LOAD)
+  } else {
+    LSD_DEEP_K(48, 64, 1, 4, 2, 64, 5, 0)
+    LSD_DEEP_K(64, 64, 4, 1, 2, 64, 5, 0)
+  }
+  LSD_DEEP_K(16, 32, 1, 2, 2, 64, 8, 0)
+  LSD_DEEP_K(32, 32, 1, 2, 2, 64, 8, 0)
+  LSD_DEEP_K(48, 32, 1, 2, 2, 64, 8, 0)
+  LSD_DEEP_K(64, 32, 1, 2, 2, 64, 6, 0)
+  if constexpr (EPI != EPI_SILU_MUL) {
+    LSD_DEEP_K(16, 16, 1, 1, 4, 128, 8, 0)
+    LSD_DEEP_K(32, 16, 1, 1, 4, 128, 6, 0)
+    LSD_DEEP_K(48, 16, 1, 1, 4, 128, 5, 0)
+    LSD_DEEP_K(64, 16, 1, 1, 4, 128, 4, 0)
+    LSD_DEEP_K(48, 80, 3, 1, 2, 64, 5, 0)
+    LSD_DEEP_K(64, 80, 4, 1, 2, 64, 4, 0)
+  }
+  LSD_DEEP_K(48, 96, 3, 2, 2, 64, 4, 0)
+  LSD_DEEP_K(64, 96, 2, 2, 2, 64, 4, 0)
+  LSD_DEEP_K(96, 64, 2, 2, 2, 64, 4, 0)
+  LSD_DEEP_K(96, 32, 2, 2, 2, 64, 5, 0)
+  LSD_DEEP_K(128, 64, 2, 2, 2, 64, 3, 0)
+  LSD_DEEP_K(128, 32, 2, 2, 2, 64, 4, 0)
+#undef LSD_DEEP_K
+  return hipErrorInvalidValue;
 }
 
 }  // namespace lsd
@@ -243,6 +281,12 @@ extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits) {
   if (M <= 48) return 1;
   const int bn = deep_cols(M, N, K, splits, epi);
   return (long)((N + bn - 1) / bn) * splits * (M > 128 ? 2 : 1) <= (M > 64 ? 512 : 640);
+}
+
+// rows * 1024 + columns of a block, for a call that is taken
+extern "C" int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits) {
+  const DeepShape s = deep_shape(M, N, K, epi == EPI_SLAB ? splits : 1, epi);
+  return s.rows * 1024 + s.cols;
 }
 
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st) {

@@ -72,9 +72,14 @@ __device__ __forceinline__ void lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ bf16x4 hi4(f32x4 v) { return pack4(v); }
+// (as two words: narrowed element by element, what only the 16-term product reads took three
+// instructions for a pair)
+__device__ __forceinline__ bf16x4 hi4(f32x4 v) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(bf16x4, u2{__builtin_bit_cast(unsigned, pack2(v[0], v[1])), __builtin_bit_cast(unsigned, pack2(v[2], v[3]))});
+}
 __device__ __forceinline__ bf16x4 lo4(f32x4 v, bf16x4 h) {
-  return pack4(f32x4{v[0] - bf2f(h[0]), v[1] - bf2f(h[1]), v[2] - bf2f(h[2]), v[3] - bf2f(h[3])});
+  return hi4(f32x4{v[0] - bf2f(h[0]), v[1] - bf2f(h[1]), v[2] - bf2f(h[2]), v[3] - bf2f(h[3])});
 }
 __device__ __forceinline__ bf16x8 cat(bf16x4 a, bf16x4 b) { return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]}; }
 // two bf16 terms of eight values (two accumulator tiles: k-slots 4 g + j and 16 + 4 g + j)

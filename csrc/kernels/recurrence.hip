@@ -513,10 +513,10 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(ConvParams c, SeqParams 
 // chunk's own.  What bounds a prompt is the chain of chunks (9.4 us each on one block per
 // sequence and head), so where those blocks leave the chip idle a chunk's factors are made by
 // a block of their own, all at once (delta_factors_kernel), and the chain keeps what is left
-// (delta_state_kernel: a block per 32 columns of a state).  One sequence of 1000 tokens, 16
-// heads of 128 x 128: 590 us -> 22 + 70 + 9 (factors, states, output norm).  Above 192
+// (delta_state_kernel: a block per 16 or 32 columns of a state).  One sequence of 1000 tokens, 16
+// heads of 128 x 128: 590 us -> 23 + 45 + 9 (factors, states, output norm).  Above 192
 // (sequence, head) pairs the fused delta_chunk_kernel is as fast and needs no workspace.
-constexpr int DELTA_CT = 16, DELTA_WAVES = 2;
+constexpr int DELTA_CT = 16;
 
 template <int DKS>
 struct DeltaShared {
@@ -948,148 +948,190 @@ __global__ __launch_bounds__(256, 2) void delta_factors_kernel(RecurParams p, co
   }
 }
 
-// LDS ring of delta_state_kernel: as many chunks as fit, and as the wait counter can tell apart.
+// LDS of delta_state_kernel: a ring of as many chunks as fit, and as the wait counter can tell
+// apart, and the waves' sums on their way to each other, of two chunks.
 template <int DKS, int WAVES>
 struct DeltaRing {
-  static constexpr int VALS = WAVES * 512, SLOT = DeltaItem<DKS>::FACTORS + VALS, INS = SLOT / 1024,
-                       LPS = (INS + WAVES - 1) / WAVES, FIT = 160 * 1024 / SLOT, COUNT = (63 + 4 + 2 * LPS) / (LPS + 4),
-                       SLOTS = FIT < COUNT ? FIT : COUNT, BYTES = SLOTS * SLOT;
+  static constexpr int SLOT = DeltaItem<DKS>::FACTORS + 1024, INS = SLOT / 1024, ALL = WAVES * DKS,
+                       LPS = (INS + ALL - 1) / ALL, ST = 4 / DKS, SUMS = DKS > 1 ? 2 * ALL * 2048 : 0,
+                       FIT = (160 * 1024 - SUMS) / SLOT, COUNT = (63 + ST + 2 * LPS) / (LPS + ST),
+                       SLOTS = FIT < COUNT ? FIT : COUNT, BYTES = SLOTS * SLOT + SUMS;
 };
 
 // The chain of chunks for 16 WAVES columns of a state: block (columns and head, sequence).
 // Factors come through the ring, SLOTS chunks ahead; outputs leave in fp32, normed and gated
-// by head_norm_gate.  A wave has its SIMD to itself and its chain is bound by the number of its
-// instructions: 416 a chunk, 1.1 us (566 and 1.5 us before the state enters its products as it
-// is, the accumulators stay in vector registers and the output's resource is scalar).
+// by head_norm_gate.
+//
+// A wave issues an instruction in four cycles and more, and its chain is bound by their number:
+// 416 a chunk and 1.1 us where one wave holds all rows of its columns.  So DKS waves hold 32 rows
+// each and exchange their sums over the rows through LDS, beside the barrier that the ring has
+// anyhow; each makes U for itself, and a chunk's outputs leave under the next one's products.
+// 220 instructions a chunk with buffer loads into the ring (a global load into LDS also counts
+// as an access of LDS, so that the next wait was for all of them) and low terms narrowed in
+// pairs; 1000 tokens, 16 heads of 128 x 128: 70.8 -> 45.2 us.
 template <int DKS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, 2) void delta_state_kernel(RecurParams p) {
+__global__ __launch_bounds__(64 * WAVES * DKS, 2) void delta_state_kernel(RecurParams p) {
   using I = DeltaItem<DKS>;
   using R = DeltaRing<DKS, WAVES>;
-  constexpr int CT = DELTA_CT, DT = DKS * 2, VALS = R::VALS, SLOT = R::SLOT, INS = R::INS, LPS = R::LPS, SLOTS = R::SLOTS;
-  typedef __attribute__((address_space(3))) void lds_void;
-  typedef __attribute__((address_space(1))) const void gbl_cvoid;
-  static_assert(LPS * (SLOTS - 2) + 4 * (SLOTS - 1) <= 63, "the wait counter holds 63 loads");
+  constexpr int CT = DELTA_CT, SLOT = R::SLOT, INS = R::INS, LPS = R::LPS, SLOTS = R::SLOTS, ST = R::ST;
+  static_assert(LPS * (SLOTS - 2) + ST * (SLOTS - 1) <= 63, "the wait counter holds 63 loads");
+  static_assert(WAVES <= 2, "a slot holds the values of two tiles");
   // (a dynamic array: with a static one of this size the compiler counts on a single wave per
   // SIMD and moves the state between accumulation registers and the others, 150 instructions a chunk)
   extern __shared__ __attribute__((aligned(16))) char ring[];
   // the column blocks of a head lie p.heads apart: with a multiple of 8 heads in one XCD's L2
   const int h = blockIdx.x % p.heads, vb = blockIdx.x / p.heads, b = blockIdx.y, D = p.D, V = p.V;
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int wc = w % WAVES, wr = w / WAVES, tile = vb * WAVES + wc;
   const int r0 = __builtin_amdgcn_readfirstlane(p.s.cu[b]), n = __builtin_amdgcn_readfirstlane(p.s.cu[b + 1]) - r0;
   const int nc = min(p.chunks, (n + CT - 1) / CT - p.first);
   if (nc <= 0) return;
-  const int v = (vb * WAVES + w) * 16 + r;
+  const int v = tile * 16 + r;
   float* Sg = p.S + ((long)p.s.slots[b] * p.heads + h) * D * p.Vp;
   const bool fresh = p.s.start[b] == 0 && p.first == 0;
-  f32x4 S[DT];
+  f32x4 S[2];  // rows 32 wr ..
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int d = dt * 16 + 4 * g + i;
+      const int d = wr * 32 + dt * 16 + 4 * g + i;
       S[dt][i] = !fresh && d < D && v < V ? Sg[d * p.Vp + v] : 0.f;
     }
-  const long pitch = (long)p.heads * I::BYTES;
+  // (factors of more than one chunk are 256 MB at most, and outputs a quarter of that)
+  const int pitch = (int)(p.heads * (long)I::BYTES);
   const char* items = static_cast<const char*>(p.work) + ((long)b * p.chunks * p.heads + h) * I::BYTES;
-  const unsigned at = lane * 16;
-  auto issue = [&](int c) {  // past the end the last chunk again, so that the counts hold
-    const char* it = items + min(c, nc - 1) * pitch;
-    char* slot = ring + (c % SLOTS) * SLOT;
+  auto issue = [&](int c, char* slot) {  // past the end the last chunk again, so that the counts hold
+    const int it = min(c, nc - 1) * pitch;
 #pragma unroll
     for (int q = 0; q < LPS; ++q) {
-      const int k = min(w + q * WAVES, INS - 1);
-      const char* src = it + (k * 1024 + (k * 1024 >= I::FACTORS ? vb * VALS : 0));  // scalar
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(src + at), (lds_void*)(slot + k * 1024), 16, 0, 0);
+      const int k = min(w + q * R::ALL, INS - 1);
+      lds_dma16(items, slot + k * 1024, lane * 16, it + k * 1024 + (k * 1024 >= I::FACTORS ? (vb * WAVES & ~1) * 512 : 0));
     }
+  };
+  // outputs: a wave's share of the tokens, 4 / DKS of each four; what is out of range is dropped
+  const unsigned long raw = reinterpret_cast<unsigned long>(p.raw + (long)(r0 + p.first * CT) * p.ldr + (long)h * V);
+  const unsigned raw_lo = __builtin_amdgcn_readfirstlane((unsigned)raw), raw_hi = __builtin_amdgcn_readfirstlane((unsigned)(raw >> 32));
+  const int step = CT * (int)p.ldr * 4;
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<float*>((unsigned long)raw_hi << 32 | raw_lo), (short)0,
+      __builtin_amdgcn_readfirstlane(min(nc * CT, n - p.first * CT) * (int)p.ldr * 4), 0x00020000);
+  int so = 0;
+  bool some = false;
+  auto store = [&](int i, float o) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(o), rs, some && v < V ? ((4 * g + wr * ST + i) * (int)p.ldr + v) * 4 : -4, so, 0);
   };
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the state is there before loads are counted
 #pragma unroll
-  for (int c = 0; c < SLOTS; ++c) issue(c);
-  float* raw = p.raw + (long)(r0 + p.first * CT) * p.ldr + (long)h * V;
-  // A wave has its SIMD to itself, so nothing but its own order hides the reads of LDS: what
-  // a chunk's first products need is read under the previous chunk's last ones, the rest under
-  // the first products.
-  bf16x8 kt[DKS][2], qt[DKS][2];
-  auto factors = [&](int c) {
-    const char* f = ring + (c % SLOTS) * SLOT;
+  for (int c = 0; c < SLOTS; ++c) {  // (stores of nothing: then every wait in the loop has the same count)
 #pragma unroll
-    for (int ks = 0; ks < DKS; ++ks)
+    for (int i = 0; i < ST; ++i) store(i, 0.f);
+    issue(c, ring + c * SLOT);
+  }
+  // Nothing but a wave's own order hides the reads of LDS: what a chunk's first products need is
+  // read under the previous chunk's last ones, the rest under the first products.
+  bf16x8 kt[2], qt[2];
+  const int rows = wr * 2048 + lane * 16;
+  auto factors = [&](const char* f) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        kt[ks][t] = *reinterpret_cast<const bf16x8*>(f + I::KT + ks * 2048 + t * 1024 + lane * 16);
-        qt[ks][t] = *reinterpret_cast<const bf16x8*>(f + I::QT + ks * 2048 + t * 1024 + lane * 16);
-      }
+    for (int t = 0; t < 2; ++t) {
+      kt[t] = *reinterpret_cast<const bf16x8*>(f + rows + I::KT + t * 1024);
+      qt[t] = *reinterpret_cast<const bf16x8*>(f + rows + I::QT + t * 1024);
+    }
   };
   auto first4 = [](bf16x8 a) { return bf16x4{a[0], a[1], a[2], a[3]}; };
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 1)));  // chunk 0 has landed
   __builtin_amdgcn_s_barrier();
-  factors(0);
+  char* f = ring;
+  // sums over the rows of each wave of these columns: of the values' products, then of the outputs'
+  float* sums = reinterpret_cast<float*>(ring + SLOTS * SLOT) + wc * DKS * 512 + lane * 4;
+  factors(f);
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+  f32x4 pa = z, pb = z;  // P U of the chunk before
+  float op[DKS][ST] = {};
+  auto output = [&]() {
+    const f32x4 pu = pa + pb;
+#pragma unroll
+    for (int i = 0; i < ST; ++i) {
+      float o;
+      if constexpr (DKS == 1) o = pu[i];
+      if constexpr (DKS == 2) o = wr ? pu[2 + i] : pu[i];
+      if constexpr (DKS == 4) o = wr & 2 ? (wr & 1 ? pu[3] : pu[2]) : (wr & 1 ? pu[1] : pu[0]);
+#pragma unroll
+      for (int k = 0; k < DKS; ++k) o += op[k][i];
+      store(i, o);
+    }
+  };
   for (int c = 0; c < nc; ++c) {
-    const char* f = ring + (c % SLOTS) * SLOT;
-    bf16x8 kf[DT];
-    f32x4 er[DT];
+    bf16x8 kf[2];
+    f32x4 er[2];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) {
-      kf[dt] = *reinterpret_cast<const bf16x8*>(f + I::KH + dt * 1024 + lane * 16);
-      er[dt] = *reinterpret_cast<const f32x4*>(f + I::ER + (dt * 16 + 4 * g) * 4);
+    for (int dt = 0; dt < 2; ++dt) {
+      kf[dt] = *reinterpret_cast<const bf16x8*>(f + rows + I::KH + dt * 1024);
+      er[dt] = *reinterpret_cast<const f32x4*>(f + I::ER + (wr * 32 + dt * 16 + 4 * g) * 4);
     }
-    const bf16x8 tm = *reinterpret_cast<const bf16x8*>(f + I::TM + lane * 16);
-    const bf16x8 pm = *reinterpret_cast<const bf16x8*>(f + I::PM + lane * 16);
-    const bf16x4 vv = *reinterpret_cast<const bf16x4*>(f + I::FACTORS + w * 512 + lane * 8);
+    const bf16x8 tm = *reinterpret_cast<const bf16x8*>(f + lane * 16 + I::TM);
+    const bf16x8 pm = *reinterpret_cast<const bf16x8*>(f + lane * 16 + I::PM);
+    const bf16x4 vv = *reinterpret_cast<const bf16x4*>(f + I::FACTORS + (tile & 1) * 512 + lane * 8);
     __builtin_amdgcn_sched_barrier(0);
-    // four independent sums, so that no product waits for the one before it
-    f32x4 ka = {0.f, 0.f, 0.f, 0.f}, kb = ka, oa = ka, ob = ka;
-#pragma unroll
-    for (int ks = 0; ks < DKS; ++ks) {
-      bf16x8 sh, sl;
-      split8(S[2 * ks], S[2 * ks + 1], sh, sl);
-      ka = mfma16(kt[ks][0], sh, ka);
-      oa = mfma16(qt[ks][0], sh, oa);
-      kb = mfma16(kt[ks][1], sh, kb);
-      ob = mfma16(qt[ks][1], sh, ob);
-      ka = mfma16(kt[ks][0], sl, ka);
-      oa = mfma16(qt[ks][0], sl, oa);
+    bf16x8 sh, sl;
+    split8(S[0], S[1], sh, sl);
+    f32x4 ka = mfma16(kt[0], sh, z), kb = mfma16(kt[1], sh, z);
+    f32x4 oa = mfma16(qt[0], sh, z), ob = mfma16(qt[1], sh, z);
+    ka = mfma16(kt[0], sl, ka);
+    oa = mfma16(qt[0], sl, oa);
+    output();
+    f32x4 ksum = ka + kb, osum = oa + ob;
+    if constexpr (DKS > 1) {
+      *reinterpret_cast<f32x4*>(sums + wr * 512) = ksum;
+      *reinterpret_cast<f32x4*>(sums + wr * 512 + 256) = osum;
     }
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt) S[dt] *= er[dt];
     // chunk c is read by everyone, chunk c + 1 has landed: behind its loads are those of
-    // SLOTS - 2 chunks and, once as many chunks have ended, four stores of each
+    // SLOTS - 2 chunks and the stores of SLOTS - 1
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    if (c >= SLOTS - 1) __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 2) + 4 * (SLOTS - 1)));
-    else __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 2)));
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(LPS * (SLOTS - 2) + ST * (SLOTS - 1)));
     __builtin_amdgcn_s_barrier();
-    issue(c + SLOTS);
-    factors(c + 1);  // past the end: chunk nc - 1 again
+    f32x4 kp[DKS];
+    if constexpr (DKS > 1) {
+#pragma unroll
+      for (int k = 0; k < DKS; ++k) kp[k] = *reinterpret_cast<const f32x4*>(sums + k * 512);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    char* next = f + SLOT == ring + SLOTS * SLOT ? ring : f + SLOT;
+    issue(c + SLOTS, f);
+    factors(next);  // past the end: chunk nc - 1 again
+    f = next;
+#pragma unroll
+    for (int k = 0; k < DKS; ++k)
+#pragma unroll
+      for (int i = 0; i < ST; ++i) op[k][i] = DKS == 1 ? osum[i] : sums[k * 512 + 256 + wr * ST + i];
+    sums += c & 1 ? -WAVES * DKS * 512 : WAVES * DKS * 512;
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (DKS == 2) ksum = kp[0] + kp[1];
+    if constexpr (DKS == 4) ksum = (kp[0] + kp[1]) + (kp[2] + kp[3]);
     // a 16-term product of two-term operands: [a hi | a lo] [b hi | b hi] in one, a hi b lo
-    const f32x4 xv = f32x4{bf2f(vv[0]), bf2f(vv[1]), bf2f(vv[2]), bf2f(vv[3])} - (ka + kb);
+    const f32x4 xv = f32x4{bf2f(vv[0]), bf2f(vv[1]), bf2f(vv[2]), bf2f(vv[3])} - ksum;
     const bf16x4 xh = hi4(xv), xl = lo4(xv, xh);
-    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
     const f32x4 u = mfma16(tm, cat(xh, xh), z) + mfma16k16(first4(tm), xl, z);
     const bf16x4 uh = hi4(u), ul = lo4(u, uh);
     const bf16x8 uu = cat(uh, uh);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) S[dt] = mfma16(kf[dt], uu, S[dt] * er[dt]);
-    oa = mfma16(pm, uu, oa);
-    ob = mfma16k16(first4(pm), ul, ob);
+    for (int dt = 0; dt < 2; ++dt) S[dt] = mfma16(kf[dt], uu, S[dt]);
+    pa = mfma16(pm, uu, z);
+    pb = mfma16k16(first4(pm), ul, z);
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) S[dt] = mfma16k16(first4(kf[dt]), ul, S[dt]);
-    const f32x4 o = oa + ob;
-    // every wave issues four stores (counted above); what is out of range is dropped
-    const int nt = min(CT, n - (p.first + c) * CT);
-    const unsigned long at = reinterpret_cast<unsigned long>(raw + (long)c * CT * p.ldr);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)at), hi = __builtin_amdgcn_readfirstlane((unsigned)(at >> 32));
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<float*>((unsigned long)hi << 32 | lo), (short)0,
-        __builtin_amdgcn_readfirstlane(nt * (int)p.ldr * 4), 0x00020000);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(o[i]), rs, v < V ? ((4 * g + i) * (int)p.ldr + v) * 4 : -4, 0, 0);
+    for (int dt = 0; dt < 2; ++dt) S[dt] = mfma16k16(first4(kf[dt]), ul, S[dt]);
+    so = c * step;
+    some = true;
   }
+  output();
   __builtin_amdgcn_s_waitcnt(0x0F70);  // no load may reach LDS that is another block's by then
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int d = dt * 16 + 4 * g + i;
+      const int d = wr * 32 + dt * 16 + 4 * g + i;
       if (d < D && v < p.Vp) Sg[d * p.Vp + v] = S[dt][i];
     }
 }
@@ -1644,17 +1686,29 @@ extern "C" hipError_t lsd_delta_split(const RecurParams* p, const bf16* x, long 
   if (p->s.B == 0 || p->chunks <= 0) return hipSuccess;
   if (p->D > 128 || p->V > 128 || !p->raw || !p->work) return hipErrorInvalidValue;
   // (the attribute is the current device's, of which a process may use several: set at each call)
-  const dim3 gf(p->heads, p->chunks, p->s.B), gs(p->heads * ((p->V + 16 * DELTA_WAVES - 1) / (16 * DELTA_WAVES)), p->s.B);
-#define LSD_DS(KS)                                                                                          \
-  constexpr int lds = DeltaRing<KS, DELTA_WAVES>::BYTES;                                                     \
-  const hipError_t room = hipFuncSetAttribute(                                                               \
-      reinterpret_cast<const void*>(&delta_state_kernel<KS, DELTA_WAVES>), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
-  if (room != hipSuccess) return room;                                                                       \
-  hipLaunchKernelGGL((delta_factors_kernel<KS>), gf, dim3(256), 0, st, *p, x, ldx);                           \
-  hipLaunchKernelGGL((delta_state_kernel<KS, DELTA_WAVES>), gs, dim3(64 * DELTA_WAVES), lds, st, *p);
+  // Two tiles of columns a block where one tile's blocks, of which a CU's LDS holds one, do not all
+  // run at once.  With convolution, factors and norm, 16 heads of 128 x 128, one tile against two:
+  // one sequence of 300 tokens 40 and 43 us, of 1000 86 and 97, 2 of 500 69 and 75, 3 of 500 102 and
+  // 89, 4 of 300 82 and 73, 12 of 300 206 and 178.
+  const dim3 gf(p->heads, p->chunks, p->s.B);
+  const int tiles = (p->V + 15) / 16;
+  const bool one = (long)p->heads * tiles * p->s.B <= 256;
+#define LSD_DS_W(KS, W)                                                                               \
+  {                                                                                                   \
+    constexpr int lds = DeltaRing<KS, W>::BYTES;                                                      \
+    const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_state_kernel<KS, W>), \
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, lds);     \
+    if (room != hipSuccess) return room;                                                              \
+    hipLaunchKernelGGL((delta_factors_kernel<KS>), gf, dim3(256), 0, st, *p, x, ldx);                 \
+    hipLaunchKernelGGL((delta_state_kernel<KS, W>), dim3(p->heads * ((tiles + W - 1) / W), p->s.B),   \
+                       dim3(64 * W * KS), lds, st, *p);                                               \
+  }
+#define LSD_DS(KS) \
+  if (one) LSD_DS_W(KS, 1) else LSD_DS_W(KS, 2)
   if (p->D <= 32) { LSD_DS(1) }
   else if (p->D <= 64) { LSD_DS(2) }
   else { LSD_DS(4) }
+#undef LSD_DS_W
 #undef LSD_DS
   return hipGetLastError();
 }

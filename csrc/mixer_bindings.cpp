@@ -196,8 +196,8 @@ int64_t delta_portion(int64_t D, int64_t heads, int64_t B) {
 // Factors of their own: where the blocks of the fused form, one per sequence and head, leave the chip
 // idle and the longest sequence has chunks enough to pay for two launches more and the way
 // through memory.  With the convolution, heads of 128 x 128, fused against split: 64 pairs 8 tokens
-// 36 and 38 us, 20 46 and 40; 128 pairs 20 tokens 48 and 51, 64 71 and 62; 192 pairs 64 tokens 76 and
-// 79, 100 99 and 100, 150 127 and 121, 300 217 and 208.
+// 24 and 24 us, 20 32 and 26; 128 pairs 20 tokens 34 and 33, 64 55 and 44; 192 pairs 64 tokens 58 and
+// 60, 100 85 and 81, 150 112 and 101, 300 196 and 177; 256 pairs 64 tokens 59 and 71, 300 202 and 233.
 bool delta_split(int64_t heads, int64_t B, int64_t rows) {
   const int64_t pairs = heads * B, chunks = (rows + lsd_delta_chunk() - 1) / lsd_delta_chunk();
   return pairs <= 192 && chunks >= std::max<int64_t>(2, pairs / 32);

@@ -53,6 +53,15 @@ def test_forms_agree(C, H, G, D, V, lens, starts, strong):
     assert torch.equal(a[2], b[2])
 
 
+@pytest.mark.parametrize("H,D,V,lens", [(16, 128, 128, [20, 33]), (16, 128, 128, [20, 33, 1]), (43, 64, 100, [70]), (32, 24, 20, [17] * 5)])
+def test_blocks_of_one_tile_and_of_two(C, H, D, V, lens):
+    """Tiles of 16 columns on 256 CUs: as many, and more (two a block, odd numbers of them too)."""
+    a, b = (run(C, s, lens, [0, 7, 0, 3, 0][: len(lens)], H, H, D, V, max_rows=max(lens)) for s in (0, 1))
+    assert not b[0].isnan().any()
+    assert bool(((a[0] - b[0]).abs() <= 2.0 ** -7 * (a[0].abs() + a[0].pow(2).mean().sqrt())).all())
+    assert bool(((a[1][..., :V] - b[1][..., :V]).abs() <= 1e-4 * a[1].abs().amax()).all())
+
+
 def test_long_sequences_in_portions(C):
     """256 (sequence, head) pairs: some chunks' factors fit the workspace at a time.  Sequences
     that end in the first, second and third portion, at its edge and behind cached tokens."""

@@ -9,7 +9,7 @@
 //    With two, W arrives at half the rate.  Wide tiles of up to 64 rows load W non-temporally
 //    (28672 x 4096 at 40 rows 49.5 -> 44.0 us, 4096 x 14336 23.0 -> 21.3); narrow ones, whose
 //    weights are small, and more rows are 0 to 20 % slower that way.
-//  * a block holds all of up to 48 rows; more are also divided among blocks beside each other,
+//  * a block holds all of up to 64 rows; more are also divided among blocks beside each other,
 //    which find W in L2, where that brings a CU fewer bytes.  Its width (96 to 16 columns)
 //    follows from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
 //    32-wide parts among them (WK) and are summed through LDS.  No K splits over blocks, no
@@ -190,17 +190,19 @@ static int deep_cols(int M, int N, int K, int splits, int epi) {
   }
   return best;
 }
-// More than 48 rows also in blocks of fewer rows, whose neighbours find W in L2 (48 x 96 only up to two
+// More than 64 rows also in blocks of fewer rows, whose neighbours find W in L2 (48 x 96 only up to two
 // of them: 140 rows of 11264 x 2048 24.2 us, so 25.4).  All rows in a block -> here:
-//   64 rows   2624 x 2048 8.3 -> 7.6 us (32 x 32)
 //   96 rows   3072 x 2048 12.3 -> 8.9 (48 x 32), 6464 13.2 -> 11.7 (48 x 64), 8512 14.9 -> 13.4 (48 x 80)
 //   128 rows  4800 x 1600 11.8 -> 9.4 (48 x 64), 6144 x 4096 24.9 -> 21.9 (48 x 80)
 //   256 rows  4800 x 1600 14.1 -> 11.9 (64 x 80), 11264 x 2048 gate/up 30.8 -> 27.3 (64 x 96)
-// and over 176 products of 50 to 256 rows 7 % on average; behind, by 0.2 us, 768 x 3072 in 8 slabs of
+// and over 176 products of 50 to 256 rows 7 % on average.  Each of these shapes adds up K as the
+// ones that hold all rows do, so the bits are the same.  (32 x 32 for 49 to 64 rows, 2624 x 2048 8.3 -> 7.6
+// us, does not: it halves the k-steps among two waves where 16 columns had four, and a router
+// behind it decided close calls otherwise; with four waves it is no faster.)  Behind, by 0.2 us, 768 x 3072 in 8 slabs of
 // 128 rows (4.7 us).
 static DeepShape deep_shape(int M, int N, int K, int splits, int epi) {
   DeepShape best{deep_rows(M), deep_cols(M, N, K, splits, epi)};
-  if (M <= 48) return best;
+  if (M <= 64) return best;
   auto cost = [&](DeepShape s) {
     const long blocks = (long)((N + s.cols - 1) / s.cols) * splits * ((M + s.rows - 1) / s.rows);
     return (blocks + 255) / 256 * (s.rows + s.cols);
@@ -210,13 +212,9 @@ static DeepShape deep_shape(int M, int N, int K, int splits, int epi) {
     if (epi == EPI_SILU_MUL && s.cols % 32 != 0) return;
     if (cost(s) < least) { best = s; least = cost(s); }
   };
-  if (M <= 64) {
-    offer({32, 32});
-  } else {
-    for (int cols : {32, 64, 80, 96})
-      if (cols < 96 || M <= 96) offer({48, cols});
-    for (int cols : {64, 80, 96}) offer({64, cols});
-  }
+  for (int cols : {32, 64, 80, 96})
+    if (cols < 96 || M <= 96) offer({48, cols});
+  for (int cols : {64, 80, 96}) offer({64, cols});
   return best;
 }
 
@@ -254,7 +252,6 @@ static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
     LSD_DEEP_K(true, 128, 32, 2, 2, 2, 64, 4, 0)
     return hipErrorInvalidValue;
   }
-  LSD_DEEP_K(false, 32, 32, 1, 2, 2, 64, 8, 0)
   LSD_DEEP_K(false, 48, 32, 1, 2, 2, 64, 8, 0)
   LSD_DEEP_K(false, 48, 64, 1, 4, 2, 64, 5, 0)
   LSD_DEEP_K(false, 64, 64, 4, 1, 2, 64, 5, 0)

@@ -1,4 +1,4 @@
-"""Products of 49 to 256 rows in blocks of fewer rows, at edges of rows, columns and the k-ring,
+"""Products of 50 to 256 rows, of more than 64 in blocks of fewer rows, at edges of rows, columns and the k-ring,
 against 64 bits: an fp32 sum of K products is off by (K + 2) ulp of their sizes, and a bf16 result
 by half a bf16 step more.
 """
@@ -10,7 +10,7 @@ DEV, F64 = "cuda:0", torch.float64
 BF16, GELU, SILU, F32, SLAB = 0, 1, 2, 3, 5
 
 # (rows, columns of a block): (M, N) that take them
-SHAPES = [((32, 32), 50, 2624), ((32, 32), 64, 2608), ((48, 32), 65, 3072), ((48, 32), 96, 3056), ((48, 64), 96, 6464),
+SHAPES = [((64, 32), 50, 2624), ((64, 32), 64, 2608), ((48, 32), 65, 3072), ((48, 32), 96, 3056), ((48, 64), 96, 6464),
           ((48, 64), 130, 4064), ((48, 80), 81, 8512), ((48, 80), 140, 5888), ((48, 96), 96, 11264), ((48, 96), 70, 11232),
           ((48, 64), 97, 4800), ((64, 64), 255, 4064), ((64, 64), 250, 3616), ((64, 80), 256, 4800), ((64, 80), 193, 4784),
           ((64, 96), 112, 11264), ((64, 96), 200, 5888)]
@@ -57,7 +57,7 @@ def test_products(shape, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,S", [(256, 1600, 3), (128, 768, 6), (96, 1600, 2), (60, 1312, 2), (140, 800, 5)])
+@pytest.mark.parametrize("M,N,S", [(256, 1600, 3), (128, 768, 6), (96, 1600, 2), (66, 1312, 2), (140, 800, 5)])
 def test_slabs(M, N, S):
     from llm_sharding_demo_amd import _C as C
 

@@ -52,10 +52,11 @@ hipError_t lsd_norm(float* x, const void* slab, int slab_bf16, int splits, const
                     const bf16* b, bf16* out, int T, int H, float eps, int rms, const int* rows,
                     int nrows, int Hn, float woff, hipStream_t st);
 int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits, int keys);
+int lsd_attn_decode_total(int B, int n_kv, int G, int hd, int splits, int keys);
 hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                            const int* seq_slots, const int* qpos, bf16* out, long ldo,
                            float* part_o, float* part_ml, int B, int nh, int n_kv, int hd,
-                           int max_seq, int splits, int parts, float scale_log2, hipStream_t st);
+                           int max_seq, int splits, int total, float scale_log2, hipStream_t st);
 hipError_t lsd_attn_prefill(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                             const int* tiles, int n_tiles, int rows, const int* seq_slots,
                             const int* q_start, const int* cu_q, bf16* out, long ldo, int nh,
@@ -563,18 +564,18 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   float* pop = nullptr;
   float* pmlp = nullptr;
   TORCH_CHECK(keys >= 0, "keys of the longest context");
-  const int parts = lsd_attn_decode_split(B, n_kv, (int)(nh / n_kv), hd, (int)splits,
+  const int total = lsd_attn_decode_total(B, n_kv, (int)(nh / n_kv), hd, (int)splits,
                                           (int)std::min<int64_t>(keys, kc.size(2)));
-  if (splits * parts > 1) {
-    po = torch::empty({B, nh, splits * parts, hd}, q.options().dtype(torch::kFloat32));
-    pml = torch::empty({B, nh, splits * parts, 2}, q.options().dtype(torch::kFloat32));
+  if (total > 1) {
+    po = torch::empty({B, nh, total, hd}, q.options().dtype(torch::kFloat32));
+    pml = torch::empty({B, nh, total, 2}, q.options().dtype(torch::kFloat32));
     pop = po.data_ptr<float>();
     pmlp = pml.data_ptr<float>();
   }
   const float sl2 = 1.4426950408889634f / std::sqrt((float)hd);
   check_hip(lsd_attn_decode(bptr(q), q.stride(0), bptr(kc), bptr(vc), seq_slots.data_ptr<int>(),
                             qpos.data_ptr<int>(), bptr_mut(out), out.stride(0), pop, pmlp, B, nh,
-                            n_kv, hd, kc.size(2), splits, parts, sl2, cur_stream()), "attn_decode");
+                            n_kv, hd, kc.size(2), splits, total, sl2, cur_stream()), "attn_decode");
   return out;
 }
 
@@ -800,6 +801,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("qpos"), py::arg("nh"), py::arg("splits"), py::arg("keys") = 0);
   m.def("attn_decode_split", [](int64_t B, int64_t n_kv, int64_t G, int64_t hd, int64_t splits, int64_t keys) {
     return lsd_attn_decode_split((int)B, (int)n_kv, (int)G, (int)hd, (int)splits, (int)keys); });
+  m.def("attn_decode_total", [](int64_t B, int64_t n_kv, int64_t G, int64_t hd, int64_t splits, int64_t keys) {
+    return lsd_attn_decode_total((int)B, (int)n_kv, (int)G, (int)hd, (int)splits, (int)keys); });
   m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("tiles"),
         py::arg("seq_slots"), py::arg("q_start"), py::arg("cu_q"), py::arg("nh"), py::arg("rows") = 64);
   m.def("attn_oproj", &attn_oproj);

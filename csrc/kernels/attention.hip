@@ -673,8 +673,11 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_mfma_kernel(
   bf16* vs = lds[w][1];
   const int b = item / n_kv, kvh = item % n_kv;
   const int ctx = qpos[b] + 1;
-  // split blockIdx.y of the context (long contexts: more waves than items)
-  const int per = (ctx + splits - 1) / splits;
+  // split blockIdx.y of the context (more waves than items), of whole tiles where many waves share
+  // the memory: 40 sequences of 780 keys in 4 splits of 195 29.8 us, of 224 26.8.  (Few waves wait for
+  // their own loads, which that makes larger.)  Behind the context's end a split has no keys.
+  constexpr int UNIT = SPLIT_P ? 1 : KT;
+  const int per = ((ctx + splits - 1) / splits + UNIT - 1) / UNIT * UNIT;
   const int k_lo = blockIdx.y * per, k_hi = min(ctx, k_lo + per);
   const long base = ((long)seq_slots[b] * n_kv + kvh) * (long)max_seq * HD;
   const int r = lane & 15, g = lane >> 4;
@@ -833,6 +836,7 @@ static hipError_t attn_decode_combine(const float* part_o, const float* part_ml,
                      part_o, part_ml, out, ldo, nh, splits)
 #define LSD_COMBINE_HD(HDV)                                      \
   if (splits <= 4) LSD_COMBINE(HDV, 4, 1);                       \
+  else if (splits <= 8) LSD_COMBINE(HDV, 8, 1);                  \
   else if (splits <= 64) LSD_COMBINE(HDV, 16, 1);                \
   else LSD_COMBINE(HDV, 16, 4);
     if (splits > 256) return hipErrorInvalidValue;
@@ -851,7 +855,7 @@ static bool attn_on_mfma(int G, int hd) {
 // all): few waves take short ranges.  A wave needs about 1.2 us per 32 keys; a merge, where the
 // caller's splits have none, 2.4 us and what its (sequence, head) pairs add.  32 heads over
 // 8: 1 sequence of 912 keys, 4 splits -> 16: 13.0 -> 6.9 us; 8 of 2000, 4 -> 8: 22.3 -> 17.1 (weights
-// in two terms; three add 3 %); but 40 of 780, 2 -> 4: 27.1 -> 32.0 (640 waves and more fill the chip).
+// in two terms; three add 3 %); from 640 waves on lsd_attn_decode_total sees to it.
 // One launch against two parts and their merge: 32 sequences of 20 keys 3.8 against 7.1 us, of
 // 130 8.2 against 10.4, of 260 14 against 13.2; four parts: 1 sequence of 60 keys 4.8 against
 // 5.8, of 100 7.3 against 6.0.  keys: the longest context, 0 where the caller does not know it.
@@ -869,11 +873,26 @@ extern "C" int lsd_attn_decode_split(int B, int n_kv, int G, int hd, int splits,
   return best;
 }
 
-// parts: lsd_attn_decode_split's; part_o and part_ml hold splits x parts
+// Splits that the kernel takes for a caller's `splits`.  What a launch of mixed contexts waits for
+// is the longest one's chain of tiles, so calls of 256 waves and more, which few parts leave
+// below six waves a CU, take up to 1536 waves of 128 keys and more; not from 512 items on, where a
+// merge of its own costs what shorter chains give (64 sequences of 300 keys 17.8 us in one
+// split, 19.4 in two), and no more than 16 (5 of 4000 keys: 20.9 us in 16, 22.2 in 32).  32 heads
+// over 8, mixed lengths: 40 sequences of 70 .. 1490 keys, 3 splits 31.4 us, 4 29.3; 16 of
+// 200 .. 2000, 4 -> 12 25.3 and 21.7; 48 of 150 .. 350, 1 -> 3 17.3 and 15.2; 32 heads over 16, 30 of
+// 16 .. 1000, 2 -> 6 24.9 and 18.0.
+extern "C" int lsd_attn_decode_total(int B, int n_kv, int G, int hd, int splits, int keys) {
+  const int total = splits * lsd_attn_decode_split(B, n_kv, G, hd, splits, keys);
+  const long items = (long)B * n_kv;
+  if (!attn_on_mfma(G, hd) || items * splits < g_attn_mfma_min || items < 1 || items >= 512 || keys <= 256) return total;
+  return std::max(total, (int)std::min<long>({1536 / items, (keys + 127) / 128, 16}));
+}
+
+// total: lsd_attn_decode_total's; part_o and part_ml hold as many
 extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                                       const int* seq_slots, const int* qpos, bf16* out, long ldo,
                                       float* part_o, float* part_ml, int B, int nh, int n_kv,
-                                      int hd, int max_seq, int splits, int parts, float scale_log2,
+                                      int hd, int max_seq, int splits, int total, float scale_log2,
                                       hipStream_t st) {
   if (B == 0) return hipSuccess;
   const int G = nh / n_kv;
@@ -884,11 +903,15 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
   // the weights keep all their bits, in three terms (two of 16 bits together: 7.0, 8.5 and 5.7 us)
   // (16 heads over 8, 24 sequences of 130 keys: 8.2 -> 9.4 us, where the VALU kernel is ahead; of
   // 60 and of 260 5.6 -> 5.3 and 13.8 -> 12.1)
+  // One wave a block, so that the waves spread evenly over the CUs: in blocks of four, 1024 to
+  // 2047 waves left some with twice the others' (160 sequences of 30 .. 400 keys, 1280 waves 31.6 ->
+  // 29.1 us, 130 of 100 .. 900 58.3 -> 53.0, 40 of 1000 .. 8000 in 4 splits 183 -> 138).  From 2048 on, eight a
+  // CU either way, blocks of four are up to 2 % ahead (256 of 400 .. 800: 106.4 and 108.7).
   if (attn_on_mfma(G, hd)) {
     const bool few = (long)n_items * splits < g_attn_mfma_min;
-    splits *= parts;
+    splits = total;
 #define LSD_DEC_MFMA(GV, NWV, SP)                                                                \
-  if (G == GV && few == SP && (few || n_items * splits <= 1024) == (NWV == 1)) {                 \
+  if (G == GV && few == SP && (few || n_items * splits < 2048) == (NWV == 1)) {                 \
     hipLaunchKernelGGL((attn_decode_mfma_kernel<128, GV, NWV, SP>), dim3((n_items + NWV - 1) / NWV, splits), \
                        dim3(64 * NWV), 0, st, q, ldq, kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml, \
                        n_kv, max_seq, splits, scale_log2, n_items);                              \

@@ -459,7 +459,8 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(const float* pa
 // from LDS and some ten instructions per score.  So
 //  * a wave takes two tiles of 16 queries (QT = 2) where that leaves blocks enough: each
 //    fragment read feeds both.
-//  * K and V go to LDS by DMA, a tile ahead in the other of two buffers; their 16-byte chunks
+//  * K and V go to LDS by DMA, a tile ahead in the other of two buffers, with 32-bit offsets from
+//    the tile's first key (64-bit lane addresses: 7937 tokens, 32 heads over 8, 17 us of 590 more); their 16-byte chunks
 //    are permuted within a row so that both the row reads of K and the transposing reads
 //    of V, 8 rows by 32 bytes at a time, meet every bank once.
 //  * sums are rescaled only where a query's maximum moved, and only tiles on the diagonal are
@@ -487,8 +488,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     const int* __restrict__ seq_slots, const int* __restrict__ q_start,
     const int* __restrict__ cu_q, bf16* out, long ldo, int nh, int n_kv, int max_seq,
     float scale_log2) {
-  typedef __attribute__((address_space(3))) void lds_void;
-  typedef __attribute__((address_space(1))) const void gbl_cvoid;
   constexpr int KT = 64;              // keys per tile
   constexpr int CPR = HD / 8;         // 16-B chunks per row
   constexpr int RPI = 64 / CPR;       // rows an LDS-DMA instruction brings
@@ -528,12 +527,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     lsum[t] = 0.f;
   }
   auto load_tile = [&](int kt, int buf) {
+    const long at = base + (long)kt * KT * HD;
+    const int last = kmax - 1 - kt * KT;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int row = (w * NI + i) * RPI + lane / CPR;
-      const long off = base + (long)min(kt * KT + row, kmax - 1) * HD + (((lane % CPR) ^ swz(row)) << 3);
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(kc + off), (lds_void*)(smem[buf][0] + (w * NI + i) * 512), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(vc + off), (lds_void*)(smem[buf][1] + (w * NI + i) * 512), 16, 0, 0);
+      const unsigned off = (min(row, last) * HD + (((lane % CPR) ^ swz(row)) << 3)) * 2;  // bytes
+      lds_dma16(kc + at, smem[buf][0] + (w * NI + i) * 512, off, 0);
+      lds_dma16(vc + at, smem[buf][1] + (w * NI + i) * 512, off, 0);
     }
   };
   load_tile(0, 0);

@@ -1121,7 +1121,8 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(GemmParams p, int tiles_m
 //   16128 x 4800 x 1600         215 -> 209      12000 x 11264 x 2048, SiLU     510 -> 480
 // (one DMA half a phase instead of two in every other: 1.5 % slower).  B0 of the next tile goes
 // to the registers that B1 leaves, which is why tiles are unrolled in pairs.
-// A half-tile is restaged >= 2 phases after its last read and staged 4-5 phases before it
+// A half-tile is restaged >= 2 phases after its last read, whose data is there by the end of that
+// phase (the first tile's B0 is read in front of q0, as in a q3), and staged 4-5 phases before it
 // is read; the counted waits sit one phase before the first read of what they retire.
 // Phase body: reads, stage, wait, s_barrier, 16 MFMAs as their fragments arrive, s_barrier.
 // The two wave rows run staggered by one barrier (wr = 1 takes an extra barrier up front,
@@ -1254,6 +1255,8 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
     LSD_STAMP(1)
     if (wr == 1) __builtin_amdgcn_s_barrier();  // stagger the wave rows by one barrier
     read_b(0, 0, b0);
+    __builtin_amdgcn_s_waitcnt(LGKM0);  // as at the end of a q3: the other wave row reloads B0 in its q1
+    __builtin_amdgcn_sched_barrier(0);
     int t = 0;
     for (; t + 1 < T; t += 2) {
       tile(t, 0, b0, b1);

@@ -354,7 +354,8 @@ typedef __attribute__((address_space(1))) const void gbl_cvoid;
 // lds from a wave-uniform resource at (row0, k0) with 32-bit lane offsets instead of
 // global_load_lds with 64-bit lane addresses, which take issue cycles from the products (-DLSD_GLDS_GLOBAL
 // restores the latter for A/B): 400 x 50304 x 1600 88.7 -> 82.1 us, 1000 x 6528 x 2048 36.0 -> 33.9,
-// 300 x 2048 x 7680 99.7 -> 79.8, 300 x 4800 x 1600 20.4 -> 20.0.
+// 300 x 2048 x 7680 99.7 -> 79.8, 300 x 4800 x 1600 20.4 -> 20.0.  Rows whose offsets from a tile's
+// first one pass 31 bits keep the 64-bit addresses (far_rows).
 #ifdef LSD_GLDS_GLOBAL
 constexpr bool kStageBL = false;
 #else
@@ -461,7 +462,7 @@ __device__ __forceinline__ void tiled_epilogue(const GemmParams& p, f32x4 (&acc)
   ct_store<EPI, TN, TM, 256>(p, ct, m0, n0, split);
 }
 
-template <int EPI>
+template <int EPI, bool BL = kStageBL>
 __global__ __launch_bounds__(256) void gemm_tiled_kernel(GemmParams p, int tiles_m, int tiles_n) {
   __shared__ __attribute__((aligned(16))) char smem[SMEM_TILED];  // [buf][A|W]; then C tile
   const int nwg = gridDim.x;
@@ -485,16 +486,16 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(GemmParams p, int tiles
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   if (kb < ke) {
-    stage_tile(smem, p.A, p.lda, m0, p.M - 1, kb * TBK);
-    stage_tile(smem + TILE_BYTES, p.W, p.ldw, n0, p.N - 1, kb * TBK);
+    stage_tile<TBM, BL>(smem, p.A, p.lda, m0, p.M - 1, kb * TBK);
+    stage_tile<TBN, BL>(smem + TILE_BYTES, p.W, p.ldw, n0, p.N - 1, kb * TBK);
     __syncthreads();
   }
   int cur = 0;
   for (int kt = kb; kt < ke; ++kt) {
     if (kt + 1 < ke) {
       char* nb = smem + (cur ^ 1) * 2 * TILE_BYTES;
-      stage_tile(nb, p.A, p.lda, m0, p.M - 1, (kt + 1) * TBK);
-      stage_tile(nb + TILE_BYTES, p.W, p.ldw, n0, p.N - 1, (kt + 1) * TBK);
+      stage_tile<TBM, BL>(nb, p.A, p.lda, m0, p.M - 1, (kt + 1) * TBK);
+      stage_tile<TBN, BL>(nb + TILE_BYTES, p.W, p.ldw, n0, p.N - 1, (kt + 1) * TBK);
     }
     const char* ta = smem + cur * 2 * TILE_BYTES;
     const char* tw = ta + TILE_BYTES;
@@ -1719,6 +1720,22 @@ static hipError_t launch_d256(const GemmParams& p, int kind, int* cnt, float* ws
   return bn == 128 ? launch_d256_bn<EPI, 128>(p, cnt, ws, st) : launch_d256_bn<EPI, 64>(p, cnt, ws, st);
 }
 
+// Whether a row of a 256-row tile lies 2^31 bytes or more from the tile's first one (row strides from
+// 4,194,304 elements on): the kernels of kinds 1 to 3 count in 32 bits from there, and a resource holds
+// 2^31 - 1 bytes.  Such calls, views of much wider rows, run on 128 x 128 tiles with 64-bit addresses.
+static bool far_rows(int M, int N, int K, long lda, long ldw) {
+  auto far = [&](int rows, long ld) { return rows > 1 && (256 * ld + K) * 2 >= 1L << 31; };
+  return far(M, lda) || far(N, ldw);
+}
+
+template <int EPI>
+static hipError_t launch_far(GemmParams p, hipStream_t st) {
+  if (EPI != EPI_SLAB) p.splits = 1;
+  const int tm = (p.M + TBM - 1) / TBM, tn = (p.N + TBN - 1) / TBN;
+  hipLaunchKernelGGL((gemm_tiled_kernel<EPI, false>), dim3(tm * tn * p.splits), dim3(256), 0, st, p, tm, tn);
+  return hipGetLastError();
+}
+
 template <int EPI>
 static hipError_t launch_tiled(const GemmParams& p, int* cnt, float* ws, hipStream_t st) {
   const int bm = (p.M + GBM - 1) / GBM, bn = (p.N + GBN - 1) / GBN;
@@ -1843,6 +1860,7 @@ extern "C" int lsd_gemm_ring8_tiles(int M, int N, int K, int S) {
   if (S == 1 && M > TBM && g_ring_m96 > 0 && ((M + 95) / 96) * tn64 <= g_ring_m96) return 0;
   return tm * tn64 * S <= g_tiled3_max_blocks ? tm * tn64 : 0;
 }
+extern "C" int lsd_gemm_far_rows(int M, int N, int K, long lda, long ldw) { return far_rows(M, N, K, lda, ldw); }
 extern "C" int lsd_gemm_sk_rblocks(int M, int N, int S) { return sk_rblocks(M, N, S); }
 extern "C" int lsd_gemm_sk_rows(int M, int N, int S) {  // rows per row block
   return sk_mt(M, sk_rblocks(M, N, S)) * 16;
@@ -1855,8 +1873,10 @@ extern "C" void lsd_gemm_set_sk_rows(int v) { g_sk_rows = v < 16 ? 16 : (v > 128
 extern "C" hipError_t lsd_gemm(const GemmParams* p, int epi, int kind, int* cnt, float* ws,
                                hipStream_t st) {
   if (lsd_gemm_on_deep(p->M, p->N, p->K, epi, kind, p->splits)) return lsd_gemm_deep(p, epi, st);
+  const bool far = kind && far_rows(p->M, p->N, p->K, p->lda, p->ldw);
 #define LSD_DISPATCH(E)                                                                   \
   case E:                                                                                 \
+    if (far) return launch_far<E>(*p, st);                                                \
     return kind >= 2 ? launch_d256<E>(*p, kind, cnt, ws, st)                              \
                      : (kind ? launch_tiled<E>(*p, cnt, ws, st) : launch_sk<E>(*p, cnt, ws, st));
   switch (epi) {

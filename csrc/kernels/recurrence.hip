@@ -240,19 +240,104 @@ __device__ __forceinline__ void put_two(bf16* p, f32x2 v) { *reinterpret_cast<bf
 __device__ __forceinline__ void put_four(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
 __device__ __forceinline__ void put_four(bf16* p, f32x4 v) { st4(p, pack4(v)); }
 
+// Tokens behind a sequence's first one (as many rows as sequences, of which one has several): the state
+// through memory, row by row, so that the step's own token keeps its registers (a loop around that one
+// spills: steps of 16 heads of 128 x 128 6.1 -> 6.4 us, of 160 sequences of 64 heads of 64 x 128 121 ->
+// 123; this way 6.2 and 120).
+template <typename T, bool DELTA, int LV, int NR, int NT>
+__device__ __forceinline__ void recur_more(const RecurParams& p, int h, int v0, int b, int n, float* qs, float* ks, float* gs,
+                                           float* vs, float (*red)[LV * 4]) {
+  constexpr int VB = LV * 4, DG = NT / LV, D = NR * DG, W = NT / 64;
+  const int rep = p.heads / p.groups, kh = h / rep, slot = p.s.slots[b], start = p.s.start[b];
+#pragma unroll 1
+  for (int t = 1; t < n; ++t) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // (addresses are not held through the loop)
+    const int lv = tid % LV, dg = tid / LV, col = v0 + lv * 4;
+    float* Sg = p.S + ((long)slot * p.heads + h) * D * p.V + col;
+    const long row = p.s.cu[b] + t;
+    const T* y = static_cast<const T*>(p.c.y) + row * p.c.ldy;
+    const T* low = static_cast<const T*>(p.low) + row * p.ldl;
+    __syncthreads();  // the sums of the token before are read
+#pragma unroll 1
+    for (int c = tid; c < 2 * D + VB; c += NT) {
+      const int part = c < D ? 0 : c < 2 * D ? 1 : 2, i = c - part * D;
+      const int ch = part == 0 ? p.q_ch + kh * D + i : part == 1 ? p.k_ch + kh * D + i : p.v_ch + h * p.V + v0 + i;
+      T* ring = static_cast<T*>(p.c.ring) + (long)slot * 4 * p.c.channels + ch;
+      float a = 0.f;
+#pragma unroll 1
+      for (int back = min(3, start + t); back >= 0; --back) {
+        const T* x = back <= t ? y + p.c.c0 + ch - back * p.c.ldy : ring + (long)((start + t - back) & 3) * p.c.channels;
+        a = fmaf(p.c.w[ch * 4 + 3 - back], to_f(*x), a);
+      }
+      a *= p.c.gain;
+      (part == 0 ? qs : part == 1 ? ks : vs)[i] = silu_x(p.c.bias ? a + p.c.bias[ch] : a);
+      if (part == 2 || (h % rep == 0 && v0 == 0)) ring[(long)((start + t) & 3) * p.c.channels] = y[p.c.c0 + ch];
+    }
+    const float gl = p.c.gain * to_f(y[p.gate_col + h]);
+    if constexpr (DELTA)
+      for (int d = tid; d < D; d += NT) gs[d] = expf(p.A[h] * softplus_x(p.c.gain * to_f(low[(long)h * D + d]) + p.dt_bias[(long)h * D + d]));
+    __syncthreads();
+    const f32x4 v = four(vs + lv * 4);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f}, u;
+    float iq = 1.f, ik = 1.f, a = 1.f;
+    if constexpr (DELTA) {
+      float nq = 0.f, nk = 0.f;
+#pragma unroll 1
+      for (int d = lane_id(); d < D; d += 64) {
+        nq += qs[d] * qs[d];
+        nk += ks[d] * ks[d];
+      }
+      iq = rsqrtf((float)D) / sqrtf(wave_sum(nq) + UNIT_EPS);
+      ik = 1.f / sqrtf(wave_sum(nk) + UNIT_EPS);
+      f32x4 pr = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int d = dg; d < D; d += DG) pr += four(Sg + (long)d * p.V) * gs[d] * (ks[d] * ik);
+      u = sigmoid_x(gl) * (v - column_sum<LV, W>(pr, red));
+    } else {
+      const float dt = softplus_x(gl + p.dt_bias[h]);
+      a = expf(p.A[h] * dt);
+      u = v * dt;
+    }
+#pragma unroll 1
+    for (int d = dg; d < D; d += DG) {
+      const f32x4 s = four(Sg + (long)d * p.V) * (DELTA ? gs[d] : a) + u * (ks[d] * ik);
+      *reinterpret_cast<f32x4*>(Sg + (long)d * p.V) = s;
+      o += s * (qs[d] * iq);
+    }
+    o = column_sum<LV, W>(o, red);
+    float rs = 1.f;
+    if (DELTA && !p.raw) {
+      float ss = 0.f;
+      for (int i = 0; i < 4; ++i) ss += dg == 0 ? o[i] * o[i] : 0.f;
+      rs = 1.f / sqrtf(wave_sum(ss) / p.V + p.eps);
+      if (h == p.heads - 1)
+        for (int c = p.heads * p.V + tid; c < p.out_cols; c += NT) from_f(static_cast<T*>(p.out) + row * p.ldo + c, 0.f);
+    }
+    if (dg != 0) continue;
+    T* out = static_cast<T*>(p.out) + row * p.ldo + (long)h * p.V + col;
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      if (!DELTA) from_f(out + i, (o[i] + v[i] * p.skip[h]) * silu_x(p.c.gain * to_f(y[(long)h * p.V + col + i])));
+      else if (p.raw) p.raw[row * p.ldr + (long)h * p.V + col + i] = o[i];
+      else from_f(out + i, o[i] * rs * p.norm[col + i] * sigmoid_x(p.c.gain * to_f(low[p.gate_off + (long)h * p.V + col + i])));
+    }
+  }
+}
+
 // A decode step where a block's threads hold whole rows and columns of the state (D = NR DG, V a
 // multiple of VB), four taps, and everything in fours lies on its vectors (recur_tiles).
 // The general form spends 800 vector and 500 scalar instructions a wave on addresses, masks and a
 // convolution by all threads, in 128 registers (183 for 128 x 128), and loads the gates one by one
 // behind its last sum.  Here a thread convolves two channels, all loads set out at once, as
 // vectors, and q, k and decays lie in LDS in the order in which a thread reads them; with eight rows
-// a thread at most (NT threads) 72 to 77 registers leave room for three quarters of the waves.
+// a thread at most (NT threads) 70 to 78 registers leave room for three quarters of the waves.
 // General form -> here, the state at 5.0 to 5.5 TB/s (read and written alone: 6.3):
 //   16 heads of 128 x 128  1 sequence 11.2 -> 6.0 us, 16 13.3 -> 9.5, 96 50.7 -> 40.0, 160 80.0 -> 66.4
 //   64 heads of 64 x 128   1 sequence 10.0 -> 6.9 us, 16 17.7 -> 15.0, 96 80.2 -> 75.2, 160 125 -> 121
 // (between other launches of a step, 96 sequences: 55 -> 41 and 87 -> 70).
 template <typename T, bool DELTA, int LV, int NR, int NT>
-__global__ __launch_bounds__(NT, 6) void recur_tile_kernel(RecurParams p) {
+__global__ __launch_bounds__(NT, DELTA || NT > 256 ? 6 : 7) void recur_tile_kernel(RecurParams p) {
   constexpr int VB = LV * 4, DG = NT / LV, D = NR * DG, W = NT / 64, PAIRS = (2 * D + VB) / 2;
   static_assert(PAIRS + D / 4 <= NT || !DELTA, "decays on threads of their own");
   static_assert(PAIRS < NT && D % 64 == 0 && NR % 4 == 0, "sizes");
@@ -264,8 +349,8 @@ __global__ __launch_bounds__(NT, 6) void recur_tile_kernel(RecurParams p) {
   const int nvb = p.V / VB;
   const int h = blockIdx.x / nvb, v0 = (blockIdx.x - h * nvb) * VB, b = blockIdx.y;
   const int rep = p.heads / p.groups, kh = h / rep;
-  const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b];
-  if (p.s.cu[b + 1] == r0) return;
+  const int slot = p.s.slots[b], start = p.s.start[b], r0 = p.s.cu[b], n = p.s.cu[b + 1] - r0;
+  if (n <= 0) return;
   const int lv = tid % LV, dg = tid / LV, col = v0 + lv * 4;
   float* Sg = p.S + ((long)slot * p.heads + h) * D * p.V + v0;  // (scalar; a lane adds own)
   const unsigned own = dg * p.V + lv * 4;
@@ -399,6 +484,7 @@ __global__ __launch_bounds__(NT, 6) void recur_tile_kernel(RecurParams p) {
     if (h == p.heads - 1)
       for (int c = p.heads * p.V + tid; c < p.out_cols; c += NT) from_f(static_cast<T*>(p.out) + row * p.ldo + c, 0.f);
   }
+  if (n > 1) recur_more<T, DELTA, LV, NR, NT>(p, h, v0, b, n, qs, ks, gs, vs, red);
 }
 
 // Rows of SiLU(convolution), bf16, any tap count: one block per row and 256 channels.

@@ -26,6 +26,8 @@
 #include "common.h"
 #include "moe_params.h"
 
+#include <type_traits>
+
 namespace lsd {
 
 namespace gg {
@@ -340,7 +342,8 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
 // Loads by lds_dma16 (global_load_lds before): 2260 rows over 32 experts of 2048 x 1024 and
 // 565 through a shared one of 2048 up 325 -> 295 us, down 169 -> 160; 565 x 2048 x 2048 63 -> 54;
 // 8192 x 8192 x 2048 118 -> 133 TF/s.
-template <int MODE, int MT>
+// FAR: 64-bit addresses, for rows that 32 bits do not reach (gg_f32).
+template <int MODE, int MT, bool FAR>
 __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kernel(GgParams p) {
   using namespace gg;
   constexpr int TM = 16 * MT, TN = 64, BKF = 32, SLOTS = 3;
@@ -353,27 +356,34 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
 
-  // rows from the tile's first one, gathered ones from the first of all (fit: gg_f32)
+  // bytes of rows from the tile's first one, of gathered ones from the first of all
+  typedef std::conditional_t<FAR, long, unsigned> Off;
   const long r0 = MODE == GG_UP && t.routed ? 0 : t.row0;
   const float* ab = static_cast<const float*>(t.A) + r0 * t.lda;
   const float* wb = static_cast<const float*>(t.W) + (long)t.n0 * t.ldw;
-  unsigned ao[TM / 32], wo[TN / 32];  // bytes
+  Off ao[TM / 32], wo[TN / 32];
 #pragma unroll
   for (int q = 0; q < TM / 32; ++q) {
     const int row = (w * (TM / 32) + q) * 8 + (lane >> 3);
-    ao[q] = (unsigned)((a_row<MODE>(p, t, row) - r0) * t.lda * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    ao[q] = (Off)((a_row<MODE>(p, t, row) - r0) * t.lda * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
 #pragma unroll
   for (int q = 0; q < TN / 32; ++q) {
     const int row = (w * (TN / 32) + q) * 8 + (lane >> 3);
-    wo[q] = (unsigned)(min(row, t.N - 1 - t.n0) * t.ldw * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    wo[q] = (Off)(min(row, t.N - 1 - t.n0) * t.ldw * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
+  auto dma = [&](const float* base, char* to, Off off, int k) {
+    if constexpr (FAR)
+      __builtin_amdgcn_global_load_lds((gbl_cvoid*)(reinterpret_cast<const char*>(base) + off + k), (lds_void*)to, 16, 0, 0);
+    else
+      lds_dma16(base, to, off, k);
+  };
   auto issue = [&](int kt, int slot) {
     char* b = smem + slot * SLOT_BYTES;
 #pragma unroll
-    for (int q = 0; q < TM / 32; ++q) lds_dma16(ab, b + (w * (TM / 32) + q) * 1024, ao[q], kt * BKF * 4);
+    for (int q = 0; q < TM / 32; ++q) dma(ab, b + (w * (TM / 32) + q) * 1024, ao[q], kt * BKF * 4);
 #pragma unroll
-    for (int q = 0; q < TN / 32; ++q) lds_dma16(wb, b + A_BYTES + (w * (TN / 32) + q) * 1024, wo[q], kt * BKF * 4);
+    for (int q = 0; q < TN / 32; ++q) dma(wb, b + A_BYTES + (w * (TN / 32) + q) * 1024, wo[q], kt * BKF * 4);
   };
   auto frag = [&](const char* tile, int row, int chunk) {
     return *reinterpret_cast<const f32x4*>(tile + row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4));
@@ -484,7 +494,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   }
 }
 
-// Rows without whole k-steps of 32, off 16 bytes or 4 GB apart: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
+// Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
 template <int MODE>
 __global__ __launch_bounds__(256) void group_gemm_f32_kernel(GgParams p) {
   using namespace gg;
@@ -697,32 +707,35 @@ extern "C" hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStr
 }
 
 template <int MODE, int MT>
-static hipError_t gg_f32_on(const GgParams& p, hipStream_t st) {
+static hipError_t gg_f32_on(const GgParams& p, bool far, hipStream_t st) {
   const long blocks = gg_blocks(p, MODE, 16 * MT, 64);
-  if (blocks) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  const dim3 grid((unsigned)blocks), block(256);
+  if (blocks && far) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT, true>), grid, block, 0, st, p);
+  else if (blocks) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT, false>), grid, block, 0, st, p);
   return hipGetLastError();
 }
 
 template <int MODE>
 static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
-  // the tiles' loads take whole 16 bytes and k-steps of 32, and count bytes from a tile's first
-  // row, or from the first of the rows it gathers, in 32 bits
+  // the tiles' loads take whole 16 bytes and k-steps of 32
   auto at = [](const void* x) { return reinterpret_cast<uintptr_t>(x); };
-  auto far = [](long rows, long ld, int K) { return (rows * ld + K) * 4 >= 1L << 32; };
-  if (p.K % 32 || (p.Ns > 0 && p.Ks % 32) || (at(p.A) | at(p.W) | at(p.As) | at(p.Ws)) % 16 ||
-      far(MODE == GG_UP ? p.T : 64, p.lda, p.K) || far(64, p.ldw, p.K) ||
-      (p.Ns > 0 && (far(64, p.ldas, p.Ks) || far(64, p.ldws, p.Ks)))) {
+  if (p.K % 32 || (p.Ns > 0 && p.Ks % 32) || (at(p.A) | at(p.W) | at(p.As) | at(p.Ws)) % 16) {
     const long blocks = gg_blocks(p, MODE, 64, 64);
     if (blocks) hipLaunchKernelGGL((group_gemm_f32_kernel<MODE>), dim3((unsigned)blocks), dim3(256), 0, st, p);
     return hipGetLastError();
   }
+  // and count bytes from a tile's first row, or from the first of the rows it gathers, in 32 bits
+  // where those hold them (524288 tokens of 2048 are 4 GB)
+  auto out = [](long rows, long ld, int K) { return (rows * ld + K) * 4 >= 1L << 32; };
+  const bool far = out(MODE == GG_UP ? p.T : 64, p.lda, p.K) || out(64, p.ldw, p.K) ||
+                   (p.Ns > 0 && (out(64, p.ldas, p.Ks) || out(64, p.ldws, p.Ks)));
   if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
     // half tiles where the fullest CU gets less work of them (N = K = 2048: 565 rows 67 against
     // 80 us, 200 rows 32 against 46); at the same work the whole ones (1000 rows 84 against 91)
     auto rounds = [&](int tm) { return (gg_blocks(p, MODE, tm, 64) + 255) / 256; };
-    if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, st);
+    if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, far, st);
   }
-  return gg_f32_on<MODE, 4>(p, st);
+  return gg_f32_on<MODE, 4>(p, far, st);
 }
 
 // fp32 kernels: 64-row tiles

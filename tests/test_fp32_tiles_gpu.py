@@ -85,3 +85,23 @@ def test_rows_far_apart(C, K, step, far):  # noqa: F811
     got = C.linear_fp32(*((room, w.to(DEV)) if far == "a" else (a.to(DEV), room))).cpu().to(F64)
     size = a.to(F64).abs() @ w.to(F64).abs().T
     assert bool(((got - a.to(F64) @ w.to(F64).T).abs() <= (K + 2) * ULP * size).all())
+    near = C.linear_fp32(a.to(DEV), w.to(DEV)).cpu().to(F64)
+    assert torch.equal(got, near)  # the same tiles: the same sums in the same order
+
+
+# gathered rows count from the first token: tokens that 32 bits reach, and do not
+@pytest.mark.parametrize("step", [(1 << 30) // 70 // 4 * 4 - 4, 1 << 24])
+def test_experts_of_tokens_far_apart(C, step):  # noqa: F811
+    T, top, E, K, F = 70, 2, 3, 128, 48
+    h, w, ws = rand(T, K, seed=1), rand(E, 2 * F, K, seed=2) * 0.1, rand(2 * F, K, seed=3) * 0.1
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int().to(DEV)
+    perm, tiles = C.moe_group(ids, E, 64)
+    room = torch.empty((T - 1) * step + K, device=DEV).as_strided((T, K), (step, 1))
+    room.copy_(h)
+    got = C.moe_up(room, perm, tiles, top, w.to(DEV), 0.0, 1.0, ws.to(DEV), 0.0, 64)
+    near = C.moe_up(h.to(DEV), perm, tiles, top, w.to(DEV), 0.0, 1.0, ws.to(DEV), 0.0, 64)
+    assert torch.equal(got[0], near[0]) and torch.equal(got[1], near[1])
+    y = (h.to(F64) @ ws.to(F64).T).reshape(T, F // 16, 2, 16)
+    gate, up = y[:, :, 0].reshape(T, F), y[:, :, 1].reshape(T, F)
+    want = gate * torch.sigmoid(gate) * up
+    assert float((got[1].cpu().to(F64) - want).abs().max()) < 1e-5 * float(want.abs().max())

@@ -32,7 +32,7 @@ void lsd_gemm_set_ring8_flags(int v);
 void lsd_gemm_set_ring8_pack(int v);
 void lsd_norm_set_wave_narrow_min(int v);
 void lsd_norm_set_wave_min(int v);
-int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits);
+int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits, int lanes);
 int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits);
 int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
@@ -132,7 +132,7 @@ bool slab_bf16_enabled() {
   return g_slab_bf16 != 0;
 }
 
-GemmParams base_params(const torch::Tensor& a, const torch::Tensor& w, int64_t tiled) {
+GemmParams base_params(const torch::Tensor& a, const torch::Tensor& w, int64_t tiled, int64_t lanes) {
   need(a, torch::kBFloat16, "a");
   need(w, torch::kBFloat16, "w");
   need_rows(a, "a");
@@ -144,6 +144,8 @@ GemmParams base_params(const torch::Tensor& a, const torch::Tensor& w, int64_t t
   p.M = a.size(0); p.N = w.size(0); p.K = a.size(1);
   p.splits = 1;
   p.act_scale = 1.f;
+  TORCH_CHECK(lanes >= 1, "lanes: this launch and those beside it, got ", lanes);
+  p.lanes = (int)std::min<int64_t>(lanes, 64);
   TORCH_CHECK(p.N % 16 == 0, "N must be a multiple of 16 (pad the weight), got ", p.N);
   TORCH_CHECK(tiled >= 0 && tiled <= 3, "GEMM kind must be 0 (split-K), 1 (tiled), 2 / 3 (256-row), got ", tiled);
   if (tiled >= 2)
@@ -229,8 +231,9 @@ torch::Tensor out_rows(const c10::optional<torch::Tensor>& out, int64_t M, int64
 // both with `scale` times both halves, 4 clamped gate with the limit `scale`
 torch::Tensor linear(torch::Tensor a, torch::Tensor w, c10::optional<torch::Tensor> bias,
                      int64_t act, int64_t tiled, int64_t splits,
-                     c10::optional<torch::Tensor> counters, c10::optional<torch::Tensor> into, double scale) {
-  GemmParams p = base_params(a, w, tiled);
+                     c10::optional<torch::Tensor> counters, c10::optional<torch::Tensor> into, double scale,
+                     int64_t lanes) {
+  GemmParams p = base_params(a, w, tiled, lanes);
   p.bias = opt_bias(bias, p.N);
   int epi = act == 1 ? EPI_GELU : (act >= 2 ? EPI_SILU_MUL : EPI_BF16);
   p.glu = act >= 2 ? (int)act - 2 : 0;
@@ -248,8 +251,8 @@ torch::Tensor linear(torch::Tensor a, torch::Tensor w, c10::optional<torch::Tens
 // 8-column segment, fp32 [M, N / 8] -- the sampler then reads the logits only
 // in the segments that can hold a top-k element (sample.hip)
 torch::Tensor linear_f32(torch::Tensor a, torch::Tensor w, int64_t tiled, int64_t splits,
-                         c10::optional<torch::Tensor> counters, c10::optional<torch::Tensor> segmax) {
-  GemmParams p = base_params(a, w, tiled);
+                         c10::optional<torch::Tensor> counters, c10::optional<torch::Tensor> segmax, int64_t lanes) {
+  GemmParams p = base_params(a, w, tiled, lanes);
   auto out = torch::empty({p.M, p.N}, a.options().dtype(torch::kFloat32));
   if (segmax.has_value()) {
     TORCH_CHECK(tiled != 0, "linear_f32: segment maxima need a tiled kernel");
@@ -274,8 +277,8 @@ c10::optional<torch::Tensor> linear_residual(torch::Tensor a, torch::Tensor w,
                                               c10::optional<torch::Tensor> bias, torch::Tensor x,
                                               int64_t splits, int64_t tiled,
                                               c10::optional<torch::Tensor> counters, bool defer,
-                                              c10::optional<torch::Tensor> out_slab) {
-  GemmParams p = base_params(a, w, tiled);
+                                              c10::optional<torch::Tensor> out_slab, int64_t lanes) {
+  GemmParams p = base_params(a, w, tiled, lanes);
   need(x, torch::kFloat32, "x");
   TORCH_CHECK(x.dim() == 2 && x.is_contiguous() && x.size(0) == p.M && x.size(1) == p.N,
               "residual x must be contiguous [M, N]");
@@ -314,8 +317,8 @@ torch::Tensor linear_qkv(torch::Tensor a, torch::Tensor w, c10::optional<torch::
                          torch::Tensor kc, torch::Tensor vc, torch::Tensor tslot,
                          torch::Tensor tpos, int64_t q_size, int64_t kv_size, int64_t hd,
                          c10::optional<torch::Tensor> rope, int64_t tiled, int64_t splits,
-                         c10::optional<torch::Tensor> counters) {
-  GemmParams p = base_params(a, w, tiled);
+                         c10::optional<torch::Tensor> counters, int64_t lanes) {
+  GemmParams p = base_params(a, w, tiled, lanes);
   p.bias = opt_bias(bias, p.N);
   need(kc, torch::kBFloat16, "k_cache");
   need(vc, torch::kBFloat16, "v_cache");
@@ -789,12 +792,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   lsd_register_latent(m);
   lsd_register_mixers(m);
   m.def("linear", &linear, py::arg("a"), py::arg("w"), py::arg("bias"), py::arg("act"), py::arg("tiled"),
-        py::arg("splits"), py::arg("counters"), py::arg("out") = py::none(), py::arg("scale") = 1.0);
+        py::arg("splits"), py::arg("counters"), py::arg("out") = py::none(), py::arg("scale") = 1.0,
+        py::arg("lanes") = 1);
   m.def("linear_f32", &linear_f32, py::arg("a"), py::arg("w"), py::arg("tiled"), py::arg("splits"),
-        py::arg("counters"), py::arg("segmax") = py::none());
+        py::arg("counters"), py::arg("segmax") = py::none(), py::arg("lanes") = 1);
   m.def("linear_residual", &linear_residual, py::arg("a"), py::arg("w"), py::arg("bias"), py::arg("x"),
-        py::arg("splits"), py::arg("tiled"), py::arg("counters"), py::arg("defer"), py::arg("slab") = py::none());
-  m.def("linear_qkv", &linear_qkv);
+        py::arg("splits"), py::arg("tiled"), py::arg("counters"), py::arg("defer"), py::arg("slab") = py::none(),
+        py::arg("lanes") = 1);
+  m.def("linear_qkv", &linear_qkv, py::arg("a"), py::arg("w"), py::arg("bias"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("token_slots"), py::arg("token_pos"), py::arg("q_size"), py::arg("kv_size"), py::arg("hd"), py::arg("rope"),
+        py::arg("tiled"), py::arg("splits"), py::arg("counters"), py::arg("lanes") = 1);
   m.def("embed", &embed, py::arg("ids"), py::arg("pos"), py::arg("wte"), py::arg("wpe"), py::arg("scale") = 1.0);
   m.def("norm", &norm, py::arg("x"), py::arg("slab"), py::arg("pbias"), py::arg("w"), py::arg("b"), py::arg("eps"),
         py::arg("rms"), py::arg("rows"), py::arg("want_out"), py::arg("width") = 0, py::arg("woff") = 0.0);
@@ -856,9 +863,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   // gemm_d256 (launch kind 2 / 3: all <= 256 rows in one tile, 64 / 128 columns): ring depth
   m.def("gemm_set_d256_slots", [](int64_t v) { lsd_gemm_set_d256_slots((int)v); });
   m.def("gemm_set_ring8", [](int64_t v) { lsd_gemm_set_ring8((int)v); });
-  m.def("gemm_deep_shape", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t splits) {
-    const int s = lsd_gemm_deep_shape((int)M, (int)N, (int)K, (int)epi, (int)splits);
-    return std::make_pair(s / 1024, s % 1024); });
+  m.def("gemm_deep_shape", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t splits, int64_t lanes) {
+    const int s = lsd_gemm_deep_shape((int)M, (int)N, (int)K, (int)epi, (int)splits, (int)lanes);
+    return std::make_pair(s / 1024, s % 1024); },
+        py::arg("M"), py::arg("N"), py::arg("K"), py::arg("epi"), py::arg("splits"), py::arg("lanes") = 1);
   m.def("gemm_on_deep", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t kind, int64_t splits) {
     return lsd_gemm_on_deep((int)M, (int)N, (int)K, (int)epi, (int)kind, (int)splits) != 0; });
   m.def("gemm_far_rows", [](int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {

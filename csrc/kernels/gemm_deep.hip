@@ -200,9 +200,13 @@ static int deep_cols(int M, int N, int K, int splits, int epi) {
 // us, does not: it halves the k-steps among two waves where 16 columns had four, and a router
 // behind it decided close calls otherwise; with four waves it is no faster.)  Behind, by 0.2 us, 768 x 3072 in 8 slabs of
 // 128 rows (4.7 us).
-static DeepShape deep_shape(int M, int N, int K, int splits, int epi) {
+// Beside another lane's launches the chip is full either way and what blocks take in together counts,
+// a fifth more with 64 x 80 at 256 rows than with 128 x 64.  GPT-2 XL in two lanes, all rows in a block
+// against here, tokens a second: 256 rows a lane 52.6 and 51.9 thousand, 200 48.5 and 48.6, 160 44.9 and
+// 44.2, 144 43.4 and 43.8, 128 40.0 and 41.4, 96 36.7 and 37.0.
+static DeepShape deep_shape(int M, int N, int K, int splits, int epi, int lanes) {
   DeepShape best{deep_rows(M), deep_cols(M, N, K, splits, epi)};
-  if (M <= 64) return best;
+  if (M <= 64 || (M >= 160 && lanes > 1)) return best;
   auto cost = [&](DeepShape s) {
     const long blocks = (long)((N + s.cols - 1) / s.cols) * splits * ((M + s.rows - 1) / s.rows);
     return (blocks + 255) / 256 * (s.rows + s.cols);
@@ -220,7 +224,7 @@ static DeepShape deep_shape(int M, int N, int K, int splits, int epi) {
 
 template <int EPI>
 static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
-  const DeepShape s = deep_shape(p.M, p.N, p.K, p.splits, EPI);
+  const DeepShape s = deep_shape(p.M, p.N, p.K, p.splits, EPI, p.lanes);
   const int tn = (p.N + s.cols - 1) / s.cols, mbs = (p.M + s.rows - 1) / s.rows;
 #define LSD_DEEP_K(ONE, ROWS, COLS, WM, WN, WK, BK, SLOTS, AUX)                                                       \
   if (s.rows == ROWS && s.cols == COLS) {                                                                             \
@@ -293,8 +297,8 @@ extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits) {
 }
 
 // rows * 1024 + columns of a block, for a call that is taken
-extern "C" int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits) {
-  const DeepShape s = deep_shape(M, N, K, epi == EPI_SLAB ? splits : 1, epi);
+extern "C" int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits, int lanes) {
+  const DeepShape s = deep_shape(M, N, K, epi == EPI_SLAB ? splits : 1, epi, lanes);
   return s.rows * 1024 + s.cols;
 }
 

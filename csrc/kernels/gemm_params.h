@@ -29,6 +29,8 @@ struct GemmParams {
   float* segmax; long ldseg;
   // EPI_SILU_MUL: which gated activation, and the factor of both halves or the limit (common.h gated)
   int glu; float act_scale;
+  // launches that run beside this one on other streams, itself counted (gemm_deep.hip's blocks)
+  int lanes;
 };
 
 // Small-M (M <= 8) weight-streaming GEMV with an optional fused input norm

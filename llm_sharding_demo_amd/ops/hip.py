@@ -641,7 +641,8 @@ class HipBackend(Backend):
         if self.fp32 or self._gemv_in(a, K, EPI_F32) is not None or (
                 not self._tiled(M, N) and self._resid_splits(M, N, K) == 1):
             return self._linear_f32(a, w)[None]
-        return self.C.linear_residual(a, w, None, x, self._resid_splits(M, N, K), self._tiled(M, N), self.counters, True, None)
+        return self.C.linear_residual(a, w, None, x, self._resid_splits(M, N, K), self._tiled(M, N), self.counters, True, None,
+                                      self.concurrency)
 
     # -- layers with elementwise norms (models/stage.py _token_layer) ----------------
     @staticmethod
@@ -1000,7 +1001,7 @@ class HipBackend(Backend):
         if self._gemv_in(a, w.shape[1], EPI_F32) is not None:
             return self.C.gemv(a, w, None, EPI_F32, 0, None, None, 0.0, None, None, None, None, None, 0, 0, 0, None)
         tiled, splits = self._gemm_kw(a.shape[0], w.shape[0], w.shape[1])
-        return self.C.linear_f32(a, w, tiled, splits, self.counters)
+        return self.C.linear_f32(a, w, tiled, splits, self.counters, lanes=self.concurrency)
 
     @property
     def counters(self):
@@ -1131,7 +1132,7 @@ class HipBackend(Backend):
         tiled, splits = self._gemm_kw(xn.shape[0], w.shape[0], w.shape[1])
         return self.C.linear_qkv(xn, w, b, cache_k, cache_v, meta.token_slots, meta.token_pos,
                                  mcfg.q_size, mcfg.kv_size, mcfg.head_dim, self._rope,
-                                 tiled, splits, self.counters)
+                                 tiled, splits, self.counters, self.concurrency)
 
     def attention(self, q, cache_k, cache_v, meta):
         n_kv, hd = cache_k.shape[1], cache_k.shape[3]
@@ -1165,7 +1166,7 @@ class HipBackend(Backend):
             if y is not None:
                 return self.C.silu_mul(y)
         tiled, splits = self._gemm_kw(a.shape[0], w.shape[0], w.shape[1], 2 if code == 2 else 1)
-        return self.C.linear(a, w, b, code, tiled, splits, self.counters)
+        return self.C.linear(a, w, b, code, tiled, splits, self.counters, lanes=self.concurrency)
 
     def _linear_into(self, a, w, act: str, out, scale: float):
         glu = _GLU.get(act)
@@ -1176,7 +1177,7 @@ class HipBackend(Backend):
             return self.C.gemv_into(x, w, code, nc, gw, gb, eps, out, glu or 0, scale)
         a = self.materialize(a)
         tiled, splits = self._gemm_kw(a.shape[0], w.shape[0], w.shape[1], 2 if code == 2 else 1)
-        return self.C.linear(a, w, None, code + (glu or 0), tiled, splits, self.counters, out, scale)
+        return self.C.linear(a, w, None, code + (glu or 0), tiled, splits, self.counters, out, scale, self.concurrency)
 
     def linear_residual(self, a, w, b, r: Residual, room=None) -> None:
         """x += a w^T + b; `room`: slab rows the caller owns and appends to
@@ -1198,7 +1199,7 @@ class HipBackend(Backend):
         # decode split-K: hand the S partial slabs to the next norm (which
         # reads the rows anyway) instead of a last-arriver reduce in the GEMM
         defer = bool(self.R.defer_resid) and not tiled and splits > 1
-        slab = self.C.linear_residual(a, w, b, r.x, splits, tiled, self.counters, defer, room)
+        slab = self.C.linear_residual(a, w, b, r.x, splits, tiled, self.counters, defer, room, self.concurrency)
         if slab is not None and room is None:
             r.pending.append((slab, b))
 
@@ -1224,13 +1225,13 @@ class HipBackend(Backend):
         xn = self.materialize(xn)
         tiled, splits = self.R.logits_kw(xn.shape[0], w.shape[0], w.shape[1], self.concurrency)
         if not (self.R.segmax and tiled and w.shape[0] % 8 == 0):
-            return self.C.linear_f32(xn, w, tiled, splits, self.counters)
+            return self.C.linear_f32(xn, w, tiled, splits, self.counters, lanes=self.concurrency)
         # the epilogue also writes each 8-logit segment's maximum; the sampler
         # derives its top-k threshold from them and reads only the segments
         # that reach it (attached to the logits: a slice drops it, and the
         # sampler then scans the full rows)
         seg = torch.empty(xn.shape[0], w.shape[0] // 8, dtype=torch.float32, device=xn.device)
-        out = self.C.linear_f32(xn, w, tiled, splits, self.counters, seg)
+        out = self.C.linear_f32(xn, w, tiled, splits, self.counters, seg, self.concurrency)
         out._lsd_segmax = seg
         return out
 

@@ -23,6 +23,50 @@ def test_rule(shape, M, N):
     assert _C.gemm_deep_shape(M, N, 192, BF16, 1) == shape
 
 
+# beside another lane's launches 160 rows and more stay in blocks that hold all of them
+@pytest.mark.parametrize("M,N,lanes,shape", [(256, 4800, 2, (128, 64)), (256, 4800, 1, (64, 80)), (160, 4800, 2, (96, 64)),
+                                             (159, 4800, 2, (48, 80)), (128, 4800, 2, (48, 64)), (256, 11264, 3, (128, 64)),
+                                             (64, 2624, 2, (64, 32))])
+def test_rule_with_lanes(M, N, lanes, shape):
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    assert _C.gemm_deep_shape(M, N, 192, BF16, 1, lanes) == shape
+
+
+def test_launches_know_their_lanes():
+    """Every product of a forward that shares the chip says so."""
+    pytest.importorskip("llm_sharding_demo_amd._C")
+    from llm_sharding_demo_amd.ops.hip import HipBackend, Residual
+
+    seen = []
+
+    class Calls:
+        def __getattr__(self, name):
+            def call(*args, lanes=1):
+                seen.append((name, args[SIGNATURE[name]] if len(args) > SIGNATURE[name] else lanes))
+                return torch.zeros(1)
+            return call
+
+    be = HipBackend.__new__(HipBackend)
+    be.C, be.concurrency, be.fp32, be.lane, be._counters, be.decode, be._rope = Calls(), 2, False, 0, None, True, None
+    a, w, x = torch.zeros(200, 1600).bfloat16(), torch.zeros(4800, 1600).bfloat16(), torch.zeros(200, 4800)
+
+    class Meta:
+        token_slots = token_pos = None
+        q_size, kv_size, head_dim = 1600, 1600, 64
+
+    be.linear(a, w)
+    be.linear(a, w, out=x)
+    be._linear_f32(a, w)
+    be.logits(a, w)
+    be.linear_residual(a, w, None, Residual(x))
+    be._slabs(a, w, x)
+    be.qkv_kv_append(a, w, None, None, None, Meta, Meta)
+    assert len(seen) == 7 and all(n == 2 for _, n in seen), seen
+
+
+SIGNATURE = {"linear": 9, "linear_f32": 6, "linear_residual": 9, "linear_qkv": 14}  # where lanes come by position
+
+
 def near(got, want, slack, step):
     got = got.cpu().to(F64)
     return bool(((got - want).abs() <= slack + step * want.abs()).all())
@@ -41,7 +85,9 @@ def test_products(shape, M, N, K):
     acc = a.to(F64) @ w.to(F64).T
     off = (K + 3) * 2.0 ** -24 * (a.to(F64).abs() @ w.to(F64).abs().T)
     y = acc + b.to(F64)
-    assert near(C.linear(*at, b.to(DEV), BF16, 1, 1, None), y, off + 2.0 ** -23 * y.abs(), 2.0 ** -8)
+    plain = C.linear(*at, b.to(DEV), BF16, 1, 1, None)
+    assert near(plain, y, off + 2.0 ** -23 * y.abs(), 2.0 ** -8)
+    assert torch.equal(C.linear(*at, b.to(DEV), BF16, 1, 1, None, lanes=2), plain)
     gelu = y * 0.5 * (1 + torch.tanh((2 / torch.pi) ** 0.5 * (y + 0.044715 * y ** 3)))
     assert near(C.linear(*at, b.to(DEV), GELU, 1, 1, None), gelu, 2 * off + 2.0 ** -20, 2.0 ** -8)
     assert near(C.linear_f32(*at, 1, 1, None), acc, off, 0.0)

@@ -342,8 +342,8 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
 // Loads by lds_dma16 (global_load_lds before): 2260 rows over 32 experts of 2048 x 1024 and
 // 565 through a shared one of 2048 up 325 -> 295 us, down 169 -> 160; 565 x 2048 x 2048 63 -> 54;
 // 8192 x 8192 x 2048 118 -> 133 TF/s.
-// FAR: 64-bit addresses, for rows that 32 bits do not reach (gg_f32).
-template <int MODE, int MT, bool FAR>
+// ADDR64: 64-bit addresses, for few rows and for those that 32 bits do not reach (gg_f32).
+template <int MODE, int MT, bool ADDR64>
 __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kernel(GgParams p) {
   using namespace gg;
   constexpr int TM = 16 * MT, TN = 64, BKF = 32, SLOTS = 3;
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
   const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
 
   // bytes of rows from the tile's first one, of gathered ones from the first of all
-  typedef std::conditional_t<FAR, long, unsigned> Off;
+  typedef std::conditional_t<ADDR64, long, unsigned> Off;
   const long r0 = MODE == GG_UP && t.routed ? 0 : t.row0;
   const float* ab = static_cast<const float*>(t.A) + r0 * t.lda;
   const float* wb = static_cast<const float*>(t.W) + (long)t.n0 * t.ldw;
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
     wo[q] = (Off)(min(row, t.N - 1 - t.n0) * t.ldw * 4) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
   auto dma = [&](const float* base, char* to, Off off, int k) {
-    if constexpr (FAR)
+    if constexpr (ADDR64)
       __builtin_amdgcn_global_load_lds((gbl_cvoid*)(reinterpret_cast<const char*>(base) + off + k), (lds_void*)to, 16, 0, 0);
     else
       lds_dma16(base, to, off, k);
@@ -707,10 +707,10 @@ extern "C" hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStr
 }
 
 template <int MODE, int MT>
-static hipError_t gg_f32_on(const GgParams& p, bool far, hipStream_t st) {
+static hipError_t gg_f32_on(const GgParams& p, bool addr64, hipStream_t st) {
   const long blocks = gg_blocks(p, MODE, 16 * MT, 64);
   const dim3 grid((unsigned)blocks), block(256);
-  if (blocks && far) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT, true>), grid, block, 0, st, p);
+  if (blocks && addr64) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT, true>), grid, block, 0, st, p);
   else if (blocks) hipLaunchKernelGGL((group_gemm_f32_mfma_kernel<MODE, MT, false>), grid, block, 0, st, p);
   return hipGetLastError();
 }
@@ -729,13 +729,19 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   auto out = [](long rows, long ld, int K) { return (rows * ld + K) * 4 >= 1L << 32; };
   const bool far = out(MODE == GG_UP ? p.T : 64, p.lda, p.K) || out(64, p.ldw, p.K) ||
                    (p.Ns > 0 && (out(64, p.ldas, p.Ks) || out(64, p.ldws, p.Ks)));
+  // Up to 16 rows are bound by the latency of their loads, which is less with 64-bit addresses (8 rows
+  // of 2048 x 2048 19.3 us, with offsets of 32 bits 21.2; of 1408 x 4704 40.8 and 45.7; but 32 rows of
+  // 2048 x 2048 28.3 and 27.4.  Experts, 2 of 32 and a shared one of 2048, 1024 columns down: 8
+  // tokens 18.9 and 21.6; 4 of 32 of 2048 x 1024 up: 11 tokens 99.7 and 107; 4 of 16 of 1024 x 512 up,
+  // the other way, 16.5 and 15.7).
+  const bool addr64 = far || (MODE == GG_UP || MODE == GG_DOWN ? p.T : p.M) <= 16;
   if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
     // half tiles where the fullest CU gets less work of them (N = K = 2048: 565 rows 67 against
     // 80 us, 200 rows 32 against 46); at the same work the whole ones (1000 rows 84 against 91)
     auto rounds = [&](int tm) { return (gg_blocks(p, MODE, tm, 64) + 255) / 256; };
-    if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, far, st);
+    if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, addr64, st);
   }
-  return gg_f32_on<MODE, 4>(p, far, st);
+  return gg_f32_on<MODE, 4>(p, addr64, st);
 }
 
 // fp32 kernels: 64-row tiles

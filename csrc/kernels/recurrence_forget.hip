@@ -25,7 +25,7 @@ __device__ __forceinline__ float write_gate(float z, float lower) { return (1.f 
 // holds rows dg + i * NT / LV of four columns.  Dynamic LDS: q, 1 - f [D].  The state passes
 // the caches by, as recur_seq_kernel's (a step with four such layers of 64 sequences 1366 ->
 // 1287 us, of 24 1213 -> 1177; of 1, 4 and 8 the same either way: 645, 874 and 1045).
-template <typename T, int LV, int NR, int NT = 256>
+template <typename T, int LV, int NR, int NT>
 __global__ __launch_bounds__(NT, NR > 8 ? 4 : 6) void forget_seq_kernel(ForgetParams p) {
   constexpr int VB = LV * 4, DG = NT / LV;
   extern __shared__ float dyn[];
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(NT, NR > 8 ? 4 : 6) void forget_seq_kernel(ForgetPa
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (start > 0 && live && dg + i * DG < D) 
+    if (start > 0 && live && dg + i * DG < D)
       s[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(Sg + (long)i * DG * p.Vp + own));
   }
   for (int t = 0; t < n; ++t) {
@@ -490,16 +490,14 @@ extern "C" hipError_t lsd_forget_seq(const ForgetParams* p, int vb, int f32, hip
   // -> 39.0, 160 65.8 -> 62.6) unless that takes a round more (64 sequences 23.4 -> 27.0)
   const long blocks = (long)grid.x * grid.y;
   const bool wide = (blocks + 767) / 768 <= (blocks + 1023) / 1024;
-#define LSD_FS_NT(T, LV, NR, NT) hipLaunchKernelGGL((forget_seq_kernel<T, LV, NR, NT>), grid, dim3(NT), lds, st, *p)
-#define LSD_FS(T, LV, NR)                                               \
-  if (NR > 8 && wide) LSD_FS_NT(T, LV, (NR > 8 ? NR / 2 : NR), 512);    \
-  else LSD_FS_NT(T, LV, NR, 256)
+#define LSD_FS(T, LV, NR, NT) hipLaunchKernelGGL((forget_seq_kernel<T, LV, NR, NT>), grid, dim3(NT), lds, st, *p)
 #define LSD_FS_N(T, LV)                    \
-  if (nr <= 1) { LSD_FS(T, LV, 1); }       \
-  else if (nr <= 2) { LSD_FS(T, LV, 2); }  \
-  else if (nr <= 4) { LSD_FS(T, LV, 4); }  \
-  else if (nr <= 8) { LSD_FS(T, LV, 8); }  \
-  else { LSD_FS(T, LV, 16); }
+  if (nr <= 1) LSD_FS(T, LV, 1, 256);      \
+  else if (nr <= 2) LSD_FS(T, LV, 2, 256); \
+  else if (nr <= 4) LSD_FS(T, LV, 4, 256); \
+  else if (nr <= 8) LSD_FS(T, LV, 8, 256); \
+  else if (wide) LSD_FS(T, LV, 8, 512);    \
+  else LSD_FS(T, LV, 16, 256);
 #define LSD_FS_V(T)                    \
   switch (vb) {                        \
     case 4: LSD_FS_N(T, 1) break;      \
@@ -517,7 +515,6 @@ extern "C" hipError_t lsd_forget_seq(const ForgetParams* p, int vb, int f32, hip
 #undef LSD_FS_V
 #undef LSD_FS_N
 #undef LSD_FS
-#undef LSD_FS_NT
   return hipGetLastError();
 }
 

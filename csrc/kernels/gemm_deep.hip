@@ -250,10 +250,13 @@ static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
       LSD_DEEP_K(true, 32, 16, 1, 1, 4, 128, 6, 0)
       LSD_DEEP_K(true, 64, 16, 1, 1, 4, 128, 4, 0)
     }
+    // (as many blocks of half the rows and 64 columns take in less than 96 x 32 or 128 x 32, except
+    // where rounding up the columns of each slab makes them a round more)
     LSD_DEEP_K(true, 96, 64, 2, 2, 2, 64, 4, 0)
-    LSD_DEEP_K(true, 96, 32, 2, 2, 2, 64, 5, 0)
+    if constexpr (EPI == EPI_SLAB) {
+      LSD_DEEP_K(true, 96, 32, 2, 2, 2, 64, 5, 0)
+    }
     LSD_DEEP_K(true, 128, 64, 2, 2, 2, 64, 3, 0)
-    LSD_DEEP_K(true, 128, 32, 2, 2, 2, 64, 4, 0)
     return hipErrorInvalidValue;
   }
   LSD_DEEP_K(false, 48, 32, 1, 2, 2, 64, 8, 0)

@@ -32,6 +32,17 @@ def test_rule_with_lanes(M, N, lanes, shape):
     assert _C.gemm_deep_shape(M, N, 192, BF16, 1, lanes) == shape
 
 
+def test_shapes_that_have_no_kernel():
+    """All of 65 rows and more in blocks of 32 columns: 96 rows in slabs only, 128 not at all."""
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    for M, rows in ((65, 96), (96, 96), (97, 128), (128, 128)):
+        for epi, splits in ((BF16, [1]), (SILU, [1]), (SLAB, range(1, 65))):
+            for S in splits:
+                some = {_C.gemm_deep_shape(M, N, 4096, epi, S) for N in range(32, 32768 // S + 32, 16 if epi != SILU else 32)
+                        if _C.gemm_on_deep(M, N, 4096, epi, 1, S)}
+                assert (rows, 32) not in some or (epi == SLAB and rows == 96), (M, epi, S)
+
+
 def test_launches_know_their_lanes():
     """Every product of a forward that shares the chip says so."""
     pytest.importorskip("llm_sharding_demo_amd._C")

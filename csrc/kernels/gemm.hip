@@ -612,7 +612,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(GemmParams p, int tiles_
 // BL: buffer_load ... lds from a wave-uniform resource at (row0, k0) with 32-bit lane
 // offsets instead of global_load_lds with 64-bit lane addresses (fewer issue cycles
 // per DMA instruction: prefill GEMM +6-25 %, profiles/r3_p8_buffer_lds.log).
-template <int ROWS, int NWAVES, int AUX = 0, bool BL = false>
+template <int ROWS, int NWAVES, int AUX, bool BL>
 __device__ __forceinline__ void stage_rows(char* lds_tile, const bf16* src, long ld, int row0, int row_max,
                                            int k0, int wi) {
   const int lane = lane_id();
@@ -692,7 +692,7 @@ __device__ __forceinline__ void stage_rows_packed(char* lds_tile, const bf16* sr
 // Measured and removed (round 5): a W-line L2 prefetch, one extra 4-byte-per-lane
 // LDS-DMA touch per k-step of the rows 2-6 k-steps ahead -- 7-16 % slower on every
 // GPT-2 XL shape, bench 50.1-50.5k -> 46.5-47.3k (profiles/r5_rejected_ring8_prefetch.log).
-template <int EPI, int VAR, int SLOTS, int NTW = 0, int PK = 0, bool BL = kStageBL>
+template <int EPI, int VAR, int SLOTS, int NTW = 0, int PK = 0>
 __global__ __launch_bounds__(512) void gemm_ring8_kernel(GemmParams p, int tiles_m, int tiles_n, int rot,
                                                          int* __restrict__ cnt, float* __restrict__ ws) {
   constexpr int D = SLOTS - 1, TN = 64, TM = TBM;
@@ -737,9 +737,9 @@ __global__ __launch_bounds__(512) void gemm_ring8_kernel(GemmParams p, int tiles
     int k = kt - kb + r0;
     k = kb + (k >= nk ? k - nk : k);
     if constexpr (PK & 2) stage_rows_packed<TM, LWN, 0>(b, p.A, p.M, p.K / 64, m0, p.M - 1, k, lw);
-    else stage_rows<TM, LWN, 0, BL>(b, p.A, p.lda, m0, p.M - 1, k * TBK, lw);
+    else stage_rows<TM, LWN, 0, kStageBL>(b, p.A, p.lda, m0, p.M - 1, k * TBK, lw);
     if constexpr (PK & 1) stage_rows_packed<TN, LWN, 1>(b + A_BYTES, p.W, p.N, p.K / 64, n0, p.N - 1, k, lw);
-    else stage_rows<TN, LWN, NTW ? 2 : 0, BL>(b + A_BYTES, p.W, p.ldw, n0, p.N - 1, k * TBK, lw);
+    else stage_rows<TN, LWN, NTW ? 2 : 0, kStageBL>(b + A_BYTES, p.W, p.ldw, n0, p.N - 1, k * TBK, lw);
   };
   if (loader) {
 #pragma unroll
@@ -1392,12 +1392,12 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
 //     the last-arriving split sums the S partials in split order
 //     (deterministic) and runs the fused epilogue.  A tile's splits have
 //     consecutive remapped ids, so they share an XCD (speed only).
-template <int ROWS, bool BL = kStageBL>
+template <int ROWS>
 __device__ __forceinline__ void stage8(char* lds_tile, const bf16* src, long ld, int row0, int row_max,
                                        int k0) {
   // 8 waves: ROWS / 64 wave-instructions of 1 KiB (8 rows x 128 B) each, the
   // [ROWS][64 k] image with 16-B chunks swizzled by (row >> 1) & 7 (lds_frag)
-  stage_rows<ROWS, 8, 0, BL>(lds_tile, src, ld, row0, row_max, k0, threadIdx.x >> 6);
+  stage_rows<ROWS, 8, 0, kStageBL>(lds_tile, src, ld, row0, row_max, k0, threadIdx.x >> 6);
 }
 
 template <int BN, int SLOTS>
@@ -1792,8 +1792,6 @@ static hipError_t launch_tiled(const GemmParams& p, int* cnt, float* ws, hipStre
         hipLaunchKernelGGL((gemm_ring8_kernel<EPI, 2, 3, 0, 2>), g8, b8, 0, st, p, tm, tn64, rot, cnt, ws);
       else if (g_ring8 == 2 && g_ring8_pack == 3)
         hipLaunchKernelGGL((gemm_ring8_kernel<EPI, 2, 3, 0, 3>), g8, b8, 0, st, p, tm, tn64, rot, cnt, ws);
-      else if (g_ring8 == 2 && (g_ring8_flags & 4))
-        hipLaunchKernelGGL((gemm_ring8_kernel<EPI, 2, 3, 0, 0, true>), g8, b8, 0, st, p, tm, tn64, rot, cnt, ws);
       else if (g_ring8 == 2 && (g_ring8_flags & 2))
         hipLaunchKernelGGL((gemm_ring8_kernel<EPI, 2, 3, 1>), g8, b8, 0, st, p, tm, tn64, rot, cnt, ws);
       else if (g_ring8 == 2)
@@ -1841,7 +1839,7 @@ extern "C" void lsd_gemm_set_ring_tn(int v) { g_ring_tn = (v == 64 || v == 32 ||
 extern "C" void lsd_gemm_set_ring_fill(int v) { g_ring_fill = v; }
 extern "C" void lsd_gemm_set_ring_m96(int v) { g_ring_m96 = v; }
 extern "C" void lsd_gemm_set_ring8(int v) { g_ring8 = (v == 1 || v == 2) ? v : 0; }
-extern "C" void lsd_gemm_set_ring8_flags(int v) { g_ring8_flags = v & 7; }
+extern "C" void lsd_gemm_set_ring8_flags(int v) { g_ring8_flags = v & 3; }
 extern "C" void lsd_gemm_set_ring8_pack(int v) { g_ring8_pack = v & 3; }
 extern "C" void lsd_gemm_set_d256_slots(int v) { g_d256_slots = v < 2 ? 2 : (v > 4 ? 4 : v); }
 

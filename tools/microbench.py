@@ -416,10 +416,6 @@ def stamps_p8(M=65536, N=6400, K=1600, act=1):
            "epilogue_us": q(us(t[:, 3] - t[:, 2])), "block_us": q(us(t[:, 3] - t[:, 0])),
            "span_us": round(float(us(t[:, 3].max() - t[:, 0].min())), 1),
            "sum_block_us_per_cu": round(float(us(t[:, 3] - t[:, 0]).sum()) / 256, 1)}
-    if t[:, 4].abs().sum() > 0:  # LSD_P8_PROF build: wave 0's loop cycles and where they went
-        lp = t[:, 4]
-        row.update({"loop_kcyc": q(lp / 1e3), "vmcnt_wait_frac": q(t[:, 5] / lp),
-                    "barrier1_frac": q(t[:, 6] / lp), "barrier2_frac": q(t[:, 7] / lp)})
     RESULTS.append(row)
     print(json.dumps(row), flush=True)
 
@@ -692,9 +688,6 @@ def main():
     if "p8stamps" in which:
         stamps_p8()
         stamps_p8(N=1600, K=6400, act=0)
-    if "p8prof" in which:  # LSD_P8_PROF build: loop cycles split into vmcnt waits and the two barriers
-        stamps_p8(act=0)
-        stamps_p8(M=4096, N=4096, K=4096, act=0)
     if "normwave" in which:  # prefill norms: block per row vs wave per row
         for T, H in ((8192, 1600), (32768, 1600), (65536, 1600), (8192, 4096), (32768, 768)):
             for wmin in (0, 1):

@@ -1858,6 +1858,7 @@ extern "C" int lsd_gemm_ring8_tiles(int M, int N, int K, int S) {
   if (S == 1 && M > TBM && g_ring_m96 > 0 && ((M + 95) / 96) * tn64 <= g_ring_m96) return 0;
   return tm * tn64 * S <= g_tiled3_max_blocks ? tm * tn64 : 0;
 }
+extern "C" int lsd_gemm_big_tiles(int M, int N, int K, int S) { return big_tiles(M, N, K, S); }
 extern "C" int lsd_gemm_far_rows(int M, int N, int K, long lda, long ldw) { return far_rows(M, N, K, lda, ldw); }
 extern "C" int lsd_gemm_sk_rblocks(int M, int N, int S) { return sk_rblocks(M, N, S); }
 extern "C" int lsd_gemm_sk_rows(int M, int N, int S) {  // rows per row block

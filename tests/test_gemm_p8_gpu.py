@@ -89,6 +89,7 @@ def test_more_than_a_round(C, N):
     off = (K + 3) * 2.0 ** -24 * (a.to(F64).abs() @ w.to(F64).abs().T)
     C.gemm_set_big_min(160)
     try:
+        assert C.gemm_big_tiles(M, N, K, 1) == (N > 8192)
         assert near(C.linear(a.to(DEV), w.to(DEV), None, 0, 1, 1, None), acc, off)
         x = torch.randn(M, N, generator=g)
         xd = x.to(DEV)

@@ -1,4 +1,5 @@
-"""LDS hazards of the 256 x 256 GEMM's K loop, from the order of its source.
+"""The 256 x 256 GEMM on the CPU: which launches take it, and the LDS hazards of its K loop, from the
+order of its source.
 
 The kernel's two wave rows run a barrier apart, so what one row's barrier stands for depends on
 which one the other row meets.  Here both rows' programs are written out from the statements of
@@ -111,3 +112,21 @@ def test_reads_between_loads(parts, T):
                 again = [x[2] for x in loads if x[0] == half and x[1] > tile]
                 assert not again or back < min(again), (half, tile, "loaded again before its reads have returned")
         assert sum(seen.values()) == 4 * T
+
+
+# a round of the 128 x 128 tiles is two on each of 256 CUs
+@pytest.mark.parametrize("M,N,K,S,big", [(1000, 8192, 192, 1, False), (1000, 8320, 192, 1, True), (256, 32768, 64, 1, False),
+                                         (256, 32896, 64, 1, True), (255, 65536, 64, 1, False), (1000, 8320, 160, 1, False),
+                                         (1000, 2048, 512, 4, False), (1000, 2176, 512, 4, True), (2000, 5120, 64, 1, True),
+                                         (300, 20480, 64, 1, True), (300, 20224, 64, 1, False)])
+def test_which_launches(M, N, K, S, big):
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    _C.gemm_set_big_min(160)
+    try:
+        assert _C.gemm_big_tiles(M, N, K, S) == big
+        _C.gemm_set_big_min(1 << 16)  # never
+        assert not _C.gemm_big_tiles(M, N, K, S)
+        _C.gemm_set_big_min(1)  # wherever it can
+        assert _C.gemm_big_tiles(M, N, K, S) == (M >= 256 and K % 64 == 0)
+    finally:
+        _C.gemm_set_big_min(160)

@@ -58,8 +58,9 @@ constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4
 
 // LDS-DMA of 16 bytes a lane (64 in a row of LDS) from base + off + soff, base and soff the
 // same in the whole wave.  Against global_load_lds, whose addresses are 64 bits a lane, it takes
-// fewer issue cycles beside the products of its wave: 8192 x 8192 x 2048 in fp32 119 -> 139 TF/s
-// (138 without any loads).  off + soff + 16 < 2^32; AUX: cache policy.
+// fewer issue cycles beside the products of its wave: 8192 x 8192 x 2048 in fp32 118 -> 133 TF/s.
+// Where a wave has few products its data comes later (gg_f32 in group_gemm.hip).
+// off + soff + 16 < 2^32; AUX: cache policy.
 template <int AUX = 0>
 __device__ __forceinline__ void lds_dma16(const void* base, void* lds, unsigned off, int soff) {
   typedef __attribute__((address_space(3))) void lds_void;

@@ -353,9 +353,11 @@ typedef __attribute__((address_space(1))) const void gbl_cvoid;
 // kStageBL: the 4- and 8-wave decode / tiled stagers (stage_tile, stage8) issue buffer_load ...
 // lds from a wave-uniform resource at (row0, k0) with 32-bit lane offsets instead of
 // global_load_lds with 64-bit lane addresses, which take issue cycles from the products (-DLSD_GLDS_GLOBAL
-// restores the latter for A/B): 400 x 50304 x 1600 88.7 -> 82.1 us, 1000 x 6528 x 2048 36.0 -> 33.9,
-// 300 x 2048 x 7680 99.7 -> 79.8, 300 x 4800 x 1600 20.4 -> 20.0.  Rows whose offsets from a tile's
-// first one pass 31 bits keep the 64-bit addresses (far_rows).
+// restores the latter for A/B): 128 x 128 tiles 400 x 50304 x 1600 88.7 -> 82.1 us, 1000 x 6528 x 2048
+// 36.0 -> 33.9, 818 x 11936 x 3584 78.6 -> 70.0; 256-row tiles 2 to 9 %, 909 x 3328 x 6720 69.6 -> 65.4,
+// 871 x 13152 x 3648 151 -> 142; the 8-wave ring 337 x 1664 x 7232 46.0 -> 41.0, 316 x 3712 x 7488 43.5 ->
+// 42.5, 364 x 6432 x 2304 22.7 -> 23.3.  Rows whose offsets from a tile's first one pass 31 bits keep the
+// 64-bit addresses (far_rows).
 #ifdef LSD_GLDS_GLOBAL
 constexpr bool kStageBL = false;
 #else

@@ -87,9 +87,11 @@ int g_group_rows = 8;  // row tiles per group of the expert tile order above 204
 
 void run(GgParams& p, int mode, int tm, bool f32, const char* what) {
   const int tiles_s = std::max(1, (p.T + tm - 1) / tm);
-  // An XCD takes a part of one group, so no group may have many fewer tiles than the others (565
-  // tokens in fp32, 9 tiles as 8 + 1: up 365 us, in one group 325; down 191 and 170). Groups beyond
-  // g_group_rows cost less (2000 tokens, 16 tiles as 8 + 8: up 150 us, in one group 154).
+  // Groups of like size: the places that the last one leaves empty are at most a sixteenth of all,
+  // since the XCDs share the places evenly (565 tokens in fp32, 9 tiles as 8 + 1: up 365 us, in one
+  // group 325; down 191 and 170). With many groups the last one may still be a short one: 113 tiles are
+  // 14 groups of 8 and one tile. Groups beyond g_group_rows cost less than that (2000 tokens, 16
+  // tiles as 8 + 8: up 150 us, in one group 154).
   int n = (tiles_s + g_group_rows - 1) / g_group_rows;
   auto per = [&] { return (tiles_s + n - 1) / n; };
   while (n > 1 && (per() * n - tiles_s) * 16 > tiles_s) --n;

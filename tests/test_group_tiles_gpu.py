@@ -1,4 +1,5 @@
-"""The order of expert tiles: groups of row tiles that end within one, of few and of many tokens."""
+"""The order of expert tiles: row tiles in groups whose last one is full or ends early, of few and of
+many tokens."""
 
 import pytest
 import torch

@@ -1083,7 +1083,7 @@ __global__ __launch_bounds__(64 * WAVES * DKS, 2) void delta_state_kernel(RecurP
       const int d = wr * 32 + dt * 16 + 4 * g + i;
       S[dt][i] = !fresh && d < D && v < V ? Sg[d * p.Vp + v] : 0.f;
     }
-  // (factors of more than one chunk are 256 MB at most, and outputs a quarter of that)
+  // (factors of more than one chunk are 256 MB at most, and outputs take less)
   const int pitch = (int)(p.heads * (long)I::BYTES);
   const char* items = static_cast<const char*>(p.work) + ((long)b * p.chunks * p.heads + h) * I::BYTES;
   auto issue = [&](int c, char* slot) {  // past the end the last chunk again, so that the counts hold

@@ -4,7 +4,8 @@ against the general form, which takes portions of two tokens and rows off their 
 import pytest
 import torch
 
-from .test_vizalix_gpu import BF, F32, C, DeltaCase, SsmCase, cuda, err, i32, portions  # noqa: F401
+from .test_vizalix_gpu import BF, F32, C, DeltaCase, SsmCase, err, portions  # noqa: F401
+from .test_vizalix_gpu import cuda, i32
 
 pytestmark = pytest.mark.gpu
 DTYPES = pytest.mark.parametrize("dt", [BF, F32])

@@ -17,8 +17,10 @@
 // before its first loads, so W starts without the routing, and the routing weights of a down
 // tile arrive under its products.  32 experts of 2048 x 1024 and a shared one of 2048, 4 a
 // token: 64 tokens up 58 -> 46 us (6.1 TB/s), down 37 -> 33; 16000 tokens down 587 -> 504.
-// fp32, for models served in it: MFMA 16x16x4 on fp32 operands, the same staging; VALU tiles
-// with fused multiply-adds where K has no whole steps of 32 or a row starts off 16 bytes.
+// fp32, for models served in it: three bf16 terms of every value on bf16 MFMAs; where few rows
+// leave the stream of the weights as the bound, MFMA 16x16x4 on fp32 operands with the bf16
+// kernel's staging; VALU tiles with fused multiply-adds where K has no whole steps of 32 or a
+// row starts off 16 bytes.
 //
 // A few tokens (single-stream decode): weight streaming instead of tiles, one
 // wave per output column and (token, choice), no sorting by expert; the down
@@ -333,15 +335,56 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(GgParams p) {
   }
 }
 
+// Results of a tile from its fp32 image in LDS, rows of TN + 4.
+template <int MODE, int TM, int TN, int NT = 256>
+__device__ __forceinline__ void f32_epilogue(const GgParams& p, const gg::Tile& t, const float* ct) {
+  using namespace gg;
+  constexpr int CLD = TN + 4;
+  constexpr int CPR = TN / 4;
+  for (int c = threadIdx.x; c < min(TM, t.rows) * CPR; c += NT) {
+    const int row = c / CPR, ch = (c % CPR) * 4, n = t.n0 + ch, m = t.row0 + row;
+    if (n >= t.N) continue;
+    const float* src = ct + row * CLD + ch;
+    f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    if constexpr (MODE == GG_UP) {  // gate and up rows in 16-row blocks; N % 32 == 0
+      if (ch & 16) continue;
+      const f32x4 u = *reinterpret_cast<const f32x4*>(src + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = glu_exact(v[e], u[e], t.limit, p.alpha, p.up_one);
+      *reinterpret_cast<f32x4*>(static_cast<float*>(t.out) + (long)m * t.ldo + (n >> 5) * 16 + (n & 15)) = v;
+      continue;
+    }
+    long orow = m;
+    float wt = 1.f;
+    if constexpr (MODE == GG_DOWN) {
+      if (t.routed) {
+        const int ent = p.perm[m];
+        wt = p.wts[ent];
+        orow = (long)(ent % p.top) * p.T + ent / p.top;
+      } else if (p.wts_s) {
+        wt = p.wts_s[m];
+      }
+    }
+    float* o = static_cast<float*>(t.out) + orow * t.ldo + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // single stores: rows of any width
+      if (n + e >= t.N) break;
+      if constexpr (MODE == GG_DOWN) o[e] = v[e] * wt;
+      else if constexpr (MODE == GG_ADD) o[e] += v[e];
+      else if constexpr (MODE == GG_F32) {
+        const float gt = p.gate ? 1.f / (1.f + expf(-p.gate[m * p.ldg + t.group * p.o_gs + n + e])) : 1.f;
+        o[e] = (v[e] + (p.bias ? p.bias[n + e] : 0.f)) * gt;
+      }
+      else o[e] = v[e];
+    }
+  }
+}
+
 // fp32: 16 MT x 64 tiles, 32-deep k-steps (128-byte rows, the bf16 kernel's staging and swizzle);
 // wave w owns 16 columns of all rows and leaves out the 16-row tiles that hold none, so an
 // expert's last rows cost what they are.  A lane's 16-byte fragment feeds four MFMA 16x16x4,
 // whose k-slot g stands for k = 4 g + j in both operands.
-// Bound by the matrix cores, whose fp32 rate is a sixteenth of bf16's (154 TF/s), and, where
-// experts have some tens of rows, by their weights.  64 x 128 tiles were no faster.
-// Loads by lds_dma16 (global_load_lds before): 2260 rows over 32 experts of 2048 x 1024 and
-// 565 through a shared one of 2048 up 325 -> 295 us, down 169 -> 160; 565 x 2048 x 2048 63 -> 54;
-// 8192 x 8192 x 2048 118 -> 133 TF/s.
+// For few rows, bound by the latency and the stream of the weights.
 // ADDR64: 64-bit addresses, for few rows and for those that 32 bits do not reach (gg_f32).
 template <int MODE, int MT, bool ADDR64>
 __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kernel(GgParams p) {
@@ -454,44 +497,210 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
 #pragma unroll
     for (int q = 0; q < 4; ++q) ct[(i * 16 + 4 * g + q) * CLD + w * 16 + r] = acc[0][i][q] + acc[1][i][q];
   __syncthreads();
-  constexpr int CPR = TN / 4;
-  for (int c = threadIdx.x; c < min(TM, t.rows) * CPR; c += 256) {
-    const int row = c / CPR, ch = (c % CPR) * 4, n = t.n0 + ch, m = t.row0 + row;
-    if (n >= t.N) continue;
-    const float* src = ct + row * CLD + ch;
-    f32x4 v = *reinterpret_cast<const f32x4*>(src);
-    if constexpr (MODE == GG_UP) {  // gate and up rows in 16-row blocks; N % 32 == 0
-      if (ch & 16) continue;
-      const f32x4 u = *reinterpret_cast<const f32x4*>(src + 16);
+  f32_epilogue<MODE, TM, TN>(p, t, ct);
+}
+
+// ---------------------------------------------------------------------------
+// fp32 on the bf16 matrix cores
+// ---------------------------------------------------------------------------
+// x = hi + mid + lo, each bf16: of 24 bits the first two, rounded to nearest, leave rests of 16 and 8
+// bits, so nothing is lost from 2^-110 on (below, lo is subnormal).  big: the largest |x|.  Shifts and subtractions: dot products
+// with (-1, 0) and (0, -1), which unpack and subtract at once, keep the MFMAs of other waves waiting.
+struct Split {
+  bf16x4 t[3];
+};
+__device__ __forceinline__ Split split3(f32x4 x, float& big) {
+  big = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), big);
+  big = fmaxf(fmaxf(fabsf(x[2]), fabsf(x[3])), big);
+  Split s;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = glu_exact(v[e], u[e], t.limit, p.alpha, p.up_one);
-      *reinterpret_cast<f32x4*>(static_cast<float*>(t.out) + (long)m * t.ldo + (n >> 5) * 16 + (n & 15)) = v;
-      continue;
+  for (int i = 0; i < 3; ++i) {
+    const bf16x2 a = pack2(x[0], x[1]), b = pack2(x[2], x[3]);
+    s.t[i] = __builtin_shufflevector(a, b, 0, 1, 2, 3);
+    if (i == 2) break;
+    const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+    x[0] -= __builtin_bit_cast(float, ua << 16);
+    x[1] -= __builtin_bit_cast(float, ua & 0xffff0000u);
+    x[2] -= __builtin_bit_cast(float, ub << 16);
+    x[3] -= __builtin_bit_cast(float, ub & 0xffff0000u);
+  }
+  return s;
+}
+
+// 16 MT x 64 NT tiles, 32-deep k-steps, WK parts of the k-steps on four waves each, summed in LDS.
+// Of the nine products of two split operands the six largest are summed (the others are below 2^-26 of
+// it), hi hi apart from the rest, whose sums round at 2^-8 of theirs.  A goes through registers into three
+// LDS planes, split once a block; W, whose columns no two waves share, straight into fragments.
+// Slot g of a fragment's k stands for 4 g + (0..3) and 16 + 4 g + (0..3), in both operands.
+// Off 64 bits by half and less of what fp32 MFMAs are, whose sums round every four products: K = 2048
+// 2.7e-7 and 5.7e-7 of the result, parts of K 1.3e-7 and 1.9e-7; K = 5632 4.7e-7 and 9.5e-7; SiLU of two
+// 4.2e-7 and 8.5e-7.
+// Bound by the matrix cores (six MFMAs at sixteen times the fp32 rate) and the splitting beside them
+// (22 issue cycles a value, which a tile's rows and columns share), with one block a CU by what a k-step waits for:
+// hence parts of K where blocks are few.  Against fp32 MFMAs: 565 x 2048 x 2048 59 -> 46 us, 565 x 2560 x
+// 2048 63 -> 50, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 300; 2260 rows over 32 experts of
+// 2048 x 1024 and 565 through a shared one of 2048 up 320 -> 254, down 152 -> 131.  Splitting W a k-step
+// ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
+// A tile with an operand of 2^56 or more, a sum that is not finite, or one that is not zero but below 2^-40
+// is computed again by fp32 MFMAs: terms that left the range of bf16's normal numbers matter there alone.
+template <int MODE, int MT, int NT, int WK, int D>
+__global__ __launch_bounds__(256 * WK, WK == 1 ? 2 : 1) void group_gemm_f32_split_kernel(GgParams p) {
+  using namespace gg;
+  constexpr int TM = 16 * MT, TN = 64 * NT, BKF = 32, CLD = TN + 4, PLANE = TM * 64, SLOT = 3 * PLANE, QA = (MT + 1) / 2;
+  constexpr int IMAGE = TM * CLD, SMEM = WK * (2 * SLOT > IMAGE * 4 ? 2 * SLOT : IMAGE * 4);
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
+  Tile t = locate<MODE, TM, TN>(p);
+  if (!t.live) return;
+  resolve<MODE, float>(p, t);
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int w = wave & 3, part = wave >> 2, tid = threadIdx.x & 255;
+  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
+  // this part's k-steps; the first part has as many as any
+  const int KT = t.K / BKF, most = (KT + WK - 1) / WK, first = part * most, T = max(0, min(most, KT - first));
+  // A: thread i has four k's of rows i / 8 and i / 8 + 32; W: this lane's column of each 16
+  const int ar = tid >> 3, ac = tid & 7;
+  const float* ap[QA];
+  const float* wp[NT];
+#pragma unroll
+  for (int q = 0; q < QA; ++q)
+    ap[q] = static_cast<const float*>(t.A) + a_row<MODE>(p, t, ar + 32 * q) * t.lda + first * BKF + 4 * ac;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wp[j] = static_cast<const float*>(t.W) + (long)min(t.n0 + (w * NT + j) * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
+  auto at = [&](int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4); };  // in a plane
+
+  f32x4 acc[2][MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[0][i][j] = acc[1][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float big = 0.f;
+  f32x4 ra[D][QA], rw[D][NT][2];
+  auto load = [&](int kt, f32x4 (&a)[QA], f32x4 (&b)[NT][2]) {  // (behind the last k-step: that one again)
+    const long k = (long)min(kt, T - 1) * BKF;
+#pragma unroll
+    for (int q = 0; q < QA; ++q) a[q] = *reinterpret_cast<const f32x4*>(ap[q] + k);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      b[j][0] = *reinterpret_cast<const f32x4*>(wp[j] + k);
+      b[j][1] = *reinterpret_cast<const f32x4*>(wp[j] + k + 16);
     }
-    long orow = m;
-    float wt = 1.f;
-    if constexpr (MODE == GG_DOWN) {
-      if (t.routed) {
-        const int ent = p.perm[m];
-        wt = p.wts[ent];
-        orow = (long)(ent % p.top) * p.T + ent / p.top;
-      } else if (p.wts_s) {
-        wt = p.wts_s[m];
+  };
+  char* const slots = smem + part * 2 * SLOT;
+  auto put_a = [&](int slot, const f32x4 (&a)[QA]) {  // chunk g: k's 4 g and 16 + 4 g
+    char* b = slots + slot * SLOT;
+#pragma unroll
+    for (int q = 0; q < QA; ++q) {
+      if (MT % 2 && q == QA - 1 && ar >= 16) break;
+      const Split s = split3(a[q], big);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        st4(reinterpret_cast<bf16*>(b + i * PLANE + at(ar + 32 * q, ac & 3) + (ac >> 2) * 8), s.t[i]);
+    }
+  };
+  auto steps = [&](auto L) {
+    bf16x8 wf[NT][3];
+    auto step = [&](int kt, int set) {
+      __syncthreads();  // A of k-step kt is in its slot, the other one's reads are done
+      if (WK > 1 && kt >= T) return;
+      const char* b = slots + (kt & 1) * SLOT;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const Split x = split3(rw[set][j][0], big), y = split3(rw[set][j][1], big);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) wf[j][c] = __builtin_shufflevector(x.t[c], y.t[c], 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+      load(kt + D, ra[set], rw[set]);
+#pragma unroll
+      for (int i0 = 0; i0 < L; i0 += 2) {  // two tiles at a time: independent chains
+        constexpr int ca[6] = {0, 0, 1, 1, 0, 2}, cw[6] = {0, 1, 0, 1, 2, 0};
+        bf16x8 af[2][3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int i = i0; i < min((int)L, i0 + 2); ++i)
+            af[i - i0][c] = *reinterpret_cast<const bf16x8*>(b + c * PLANE + at(i * 16 + r, g));
+#pragma unroll
+        for (int c = 0; c < 6; ++c)
+#pragma unroll
+          for (int i = i0; i < min((int)L, i0 + 2); ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+              acc[c > 0][i][j] = mfma16(af[i - i0][ca[c]], wf[j][cw[c]], acc[c > 0][i][j]);
+      }
+      put_a(~kt & 1, ra[(set + 1) % D]);
+    };
+    int kt = 0;
+    for (; kt + D <= most; kt += D)
+#pragma unroll
+      for (int d = 0; d < D; ++d) step(kt + d, d);
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+      if (kt + d < most) step(kt + d, d);
+  };
+  if (WK == 1 || T > 0) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, ra[d], rw[d]);
+    put_a(0, ra[0]);
+  }
+  count_down<MT>([&](auto ic) {
+    constexpr int l = decltype(ic)::v + 1;
+    if (MODE == GG_UP || MODE == GG_DOWN ? live == l : l == MT) steps(std::integral_constant<int, l>{});
+  });
+  bool exact = big >= 0x1p56f;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      acc[0][i][j] += acc[1][i][j];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v = fabsf(acc[0][i][j][q]);
+        exact |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
       }
     }
-    float* o = static_cast<float*>(t.out) + orow * t.ldo + n;
+  if (__syncthreads_or(exact)) {
+#pragma unroll 1
+    for (int i = 0; i < live; ++i) {
+      const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;
+      f32x4 s[NT];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {  // single stores: rows of any width
-      if (n + e >= t.N) break;
-      if constexpr (MODE == GG_DOWN) o[e] = v[e] * wt;
-      else if constexpr (MODE == GG_ADD) o[e] += v[e];
-      else if constexpr (MODE == GG_F32) {
-        const float gt = p.gate ? 1.f / (1.f + expf(-p.gate[m * p.ldg + t.group * p.o_gs + n + e])) : 1.f;
-        o[e] = (v[e] + (p.bias ? p.bias[n + e] : 0.f)) * gt;
+      for (int j = 0; j < NT; ++j) s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int k = 0; k < T * BKF; k += 16) {
+        const f32x4 av = *reinterpret_cast<const f32x4*>(a + k);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          const f32x4 wv = *reinterpret_cast<const f32x4*>(wp[j] + k);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[j], 0, 0, 0);
+        }
       }
-      else o[e] = v[e];
+#pragma unroll
+      for (int h = 0; h < MT; ++h)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+          if (h == i) acc[0][h][j] = s[j];
     }
   }
+  float* ct = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        ct[part * IMAGE + (i * 16 + 4 * g + q) * CLD + (w * NT + j) * 16 + r] = acc[0][i][j][q];
+  __syncthreads();
+  if constexpr (WK > 1) {
+    for (int c = threadIdx.x; c < IMAGE / 4; c += 256 * WK) {
+      f32x4* o = reinterpret_cast<f32x4*>(ct) + c;
+#pragma unroll
+      for (int i = 1; i < WK; ++i) *o += o[i * (IMAGE / 4)];
+    }
+    __syncthreads();
+  }
+  f32_epilogue<MODE, TM, TN, 256 * WK>(p, t, ct);
 }
 
 // Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
@@ -715,6 +924,45 @@ static hipError_t gg_f32_on(const GgParams& p, bool addr64, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int MODE, int MT, int NT, int WK, int D>
+static hipError_t gg_split_on(const GgParams& p, hipStream_t st) {
+  const long blocks = gg_blocks(p, MODE, 16 * MT, 64 * NT);
+  if (blocks)
+    hipLaunchKernelGGL((group_gemm_f32_split_kernel<MODE, MT, NT, WK, D>), dim3((unsigned)blocks), dim3(256 * WK), 0, st, p);
+  return hipGetLastError();
+}
+
+// The split kernel's tile for M rows: what its blocks take in rounds of 256, in us at K = 2048
+// (fixed part, a round) as measured over 17 .. 1500 rows of 512 .. 11264 columns.  565 rows of 2048 columns:
+// 32-row tiles 62.9 us, 48 47.3, 64 52.0, 80 40.6, 64 x 128 67.9, 96 x 128 82.8; of 2560 64.2, 49.9, 52.5,
+// 73.5, 96-row ones 43.2; 1000 of 11264 487, 367, 316, 357, 64 x 128 290, 96 x 128 265.
+struct SplitTile {
+  int rows, cols, fixed, round;
+};
+static const SplitTile SPLIT_TILES[] = {{32, 64, 1, 21}, {48, 64, 5, 25}, {64, 64, 4, 28}, {80, 64, 0, 39}, {96, 64, 0, 42},
+                                        {64, 128, 20, 45}, {96, 128, 22, 61}};
+static int split_tile(const GgParams& p) {
+  int best = 0;
+  long least = 0;
+  for (int i = 0; i < 7; ++i) {
+    const SplitTile& t = SPLIT_TILES[i];
+    const long cost = t.fixed + (gg_blocks(p, GG_F32, t.rows, t.cols) + 255) / 256 * t.round;
+    if (i == 0 || cost < least) best = i, least = cost;
+  }
+  return best;
+}
+
+// Products on split operands: experts from 20 rows a tile of the table on (2048 x 1024, 4 of 32 experts:
+// 300 tokens, 24 rows, up 194 -> 169 us, down 99 -> 92; 200, 18 rows, 158 and 168, 80 and 89, on another
+// card 182 and 169; 40, 5 rows, 121 and 126, 47 and 68).  Others with more than 16 rows, unless the few are
+// bound by the weights' stream (20 rows of 32000 x 2048 42 us and 50, of 16384 31.1 and 27.5) or K is short for the
+// splitting to hide (565 rows of 2048, K = 256 12.2 and 12.8, 512 19.2 and 17.9; of 4096, K = 512 31.4 and 32.9;
+// 100 rows of 2048, K = 512 10.6 and 11.1, 2048 28.7 and 22.9).
+static bool on_split(const GgParams& p, bool experts) {
+  if (experts) return (long)p.T * p.top >= 20L * p.n_tiles;
+  return p.K > 512 && p.M > 16 && !(p.M <= 32 && gg_blocks(p, GG_F32, 32, 64) > 256);
+}
+
 template <int MODE>
 static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   // the tiles' loads take whole 16 bytes and k-steps of 32
@@ -724,7 +972,20 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
     if (blocks) hipLaunchKernelGGL((group_gemm_f32_kernel<MODE>), dim3((unsigned)blocks), dim3(256), 0, st, p);
     return hipGetLastError();
   }
-  // and count bytes from a tile's first row, or from the first of the rows it gathers, in 32 bits
+  if (on_split(p, MODE == GG_UP || MODE == GG_DOWN)) {
+    if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
+      switch (split_tile(p)) {
+        case 0: return gg_split_on<MODE, 2, 1, 4, 2>(p, st);
+        case 1: return gg_split_on<MODE, 3, 1, 2, 3>(p, st);
+        case 2: return gg_split_on<MODE, 4, 1, 2, 2>(p, st);
+        case 3: return gg_split_on<MODE, 5, 1, 2, 2>(p, st);
+        case 4: return gg_split_on<MODE, 6, 1, 2, 2>(p, st);
+        case 6: return gg_split_on<MODE, 6, 2, 1, 2>(p, st);
+      }
+    }
+    return gg_split_on<MODE, 4, 2, 1, 2>(p, st);
+  }
+  // The others count bytes from a tile's first row, or from the first of the rows it gathers, in 32 bits
   // where those hold them (524288 tokens of 2048 are 4 GB)
   auto out = [](long rows, long ld, int K) { return (rows * ld + K) * 4 >= 1L << 32; };
   const bool far = out(MODE == GG_UP ? p.T : 64, p.lda, p.K) || out(64, p.ldw, p.K) ||
@@ -736,12 +997,19 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   // the other way, 16.5 and 15.7).
   const bool addr64 = far || (MODE == GG_UP || MODE == GG_DOWN ? p.T : p.M) <= 16;
   if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
-    // half tiles where the fullest CU gets less work of them (N = K = 2048: 565 rows 67 against
-    // 80 us, 200 rows 32 against 46); at the same work the whole ones (1000 rows 84 against 91)
+    // half tiles where the fullest CU gets less work of them (N = 2048, K = 512: 565 rows 19 us)
     auto rounds = [&](int tm) { return (gg_blocks(p, MODE, tm, 64) + 255) / 256; };
     if (rounds(32) < 2 * rounds(64)) return gg_f32_on<MODE, 2>(p, addr64, st);
   }
   return gg_f32_on<MODE, 4>(p, addr64, st);
+}
+
+// Rows and columns of the tiles of M x N fp32 results (tests)
+extern "C" void lsd_group_gemm_split_tile(int M, int N, int* rows, int* cols) {
+  GgParams p{};
+  p.M = M, p.N = N, p.groups = 1;
+  const SplitTile& t = SPLIT_TILES[split_tile(p)];
+  *rows = t.rows, *cols = t.cols;
 }
 
 // fp32 kernels: 64-row tiles

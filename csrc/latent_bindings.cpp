@@ -24,6 +24,7 @@ using lsd::RowsParams;
 extern "C" {
 hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStream_t st);
 hipError_t lsd_group_gemm_f32(const GgParams* p, int mode, hipStream_t st);
+void lsd_group_gemm_split_tile(int M, int N, int* rows, int* cols);
 hipError_t lsd_moe_gemv_up(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_moe_gemv_down(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_latent_post(const LatentPostParams* p, int f32, hipStream_t st);
@@ -622,6 +623,11 @@ void lsd_register_latent(pybind11::module& m) {
   m.def("batch_linear", &batch_linear, py::arg("a"), py::arg("w"), py::arg("tm"), py::arg("gate") = py::none());
   m.def("linear_fp32", &linear_fp32, py::arg("a"), py::arg("w"), py::arg("x") = py::none(),
         py::arg("bias") = py::none());
+  m.def("fp32_tile", [](int64_t M, int64_t N) {
+    int rows, cols;
+    lsd_group_gemm_split_tile((int)M, (int)N, &rows, &cols);
+    return std::make_pair(rows, cols);
+  });
   m.def("moe_group", &moe_group, py::arg("ids"), py::arg("experts"), py::arg("tm"));
   m.def("moe_up", &moe_up, py::arg("h"), py::arg("perm"), py::arg("tiles"), py::arg("top"), py::arg("w"),
         py::arg("limit"), py::arg("alpha"), py::arg("ws"), py::arg("limit_s"), py::arg("tm"));

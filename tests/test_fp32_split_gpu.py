@@ -1,0 +1,96 @@
+"""fp32 products as sums of three bf16 terms against 64 bits.
+
+A sum of K products in fp32 is off by at most (K + 2) ulp of the sum of the products'
+sizes, in any order (ulp: 2^-24); the products of terms that are left out are 2^-26 each.
+"""
+
+import pytest
+import torch
+
+from .test_timisun_gpu import C, rand  # noqa: F401
+
+DEV, F64, ULP = "cuda:0", torch.float64, 2.0 ** -24
+
+
+def near(got, a, w, extra=0.0):
+    want, size = a.to(F64) @ w.to(F64).T, a.to(F64).abs() @ w.to(F64).abs().T
+    return bool(((got.cpu().to(F64) - want - extra).abs() <= (a.shape[1] + 4) * ULP * size + 2 * ULP * abs(extra)).all())
+
+
+# every tile: its edges, parts of K that are empty, uneven and whole
+TILES = [(17, 40, (32, 64)), (33, 1985, (32, 64)), (33, 11264, (48, 64)), (193, 2600, (48, 64)), (500, 1985, (64, 64)),
+         (561, 2048, (80, 64)), (481, 2600, (96, 64)), (1025, 3072, (64, 128)), (561, 4160, (96, 128))]
+
+
+def test_tiles():
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    assert [_C.fp32_tile(M, N) for M, N, _ in TILES] == [t for _, _, t in TILES]
+    assert {t for _, _, t in TILES} == {(32, 64), (48, 64), (64, 64), (80, 64), (96, 64), (64, 128), (96, 128)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [544, 576, 608, 672, 928])
+@pytest.mark.parametrize("M,N,tile", TILES)
+def test_products(C, M, N, tile, K):  # noqa: F811
+    a, w, b = rand(M, K, seed=1), rand(N, K, seed=2), rand(N, seed=3)
+    got = C.linear_fp32(a.to(DEV), w.to(DEV), None, b.to(DEV))
+    want, size = a.to(F64) @ w.to(F64).T + b.to(F64), a.to(F64).abs() @ w.to(F64).abs().T + b.to(F64).abs()
+    assert bool(((got.cpu().to(F64) - want).abs() <= (K + 4) * ULP * size).all())
+
+
+# what leaves the range of bf16's normal numbers goes to fp32 MFMAs: sums as in fp32, and no other rows change
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [544, 576])
+@pytest.mark.parametrize("scale,back", [(2.0 ** -120, 2.0 ** 60), (2.0 ** 120, 2.0 ** -60), (3.4e38, 2.0 ** -100), (2.0 ** -115, 2.0 ** 100),
+                                        (2.0 ** 80, 2.0 ** -115)])
+def test_sizes(C, K, scale, back):  # noqa: F811
+    a, w = rand(70, K, seed=1).clamp(-1, 1) * scale, rand(100, K, seed=2) * back
+    assert near(C.linear_fp32(a.to(DEV), w.to(DEV)), a, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("side", ["a", "w"])
+def test_not_finite(C, side, value):  # noqa: F811
+    a, w = rand(70, 576, seed=1), rand(130, 576, seed=2)
+    (a if side == "a" else w)[40, 50] = value
+    w[3, 50] = a[5, 50] = 1.0  # no middle and low terms: infinity times them is not a number
+    want, got = a @ w.T, C.linear_fp32(a.to(DEV), w.to(DEV)).cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    ok = want.isfinite()
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    assert bool(((got - want).abs()[ok] <= 600 * ULP * 576).all())
+
+
+# 20 rows a tile of the table and more: experts on split operands, and fewer, which are not
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E", [(300, 3), (129, 5), (64, 1), (30, 9)])
+def test_experts(C, T, E):  # noqa: F811
+    H, F, top = 128, 192, min(2, E)
+    h, up, dn = rand(T, H, seed=1), rand(E, 2 * F, H, seed=2) * 0.2, rand(E, H, F, seed=3) * 0.2
+    shared_up, shared_dn = rand(2 * F, H, seed=4) * 0.2, rand(H, F, seed=5) * 0.2
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int()
+    ids[: T // 2, 0], ids[: T // 2, 1:] = 0, min(1, E - 1)  # uneven
+    wts = torch.rand(T, top)
+    order, tiles = C.moe_group(ids.to(DEV), E, 64)
+    on = T * top >= 20 * tiles.shape[0]
+    assert on == (T > 30)
+    mid, mids = C.moe_up(h.to(DEV), order, tiles, top, up.to(DEV), 0.0, 1.0, shared_up.to(DEV), 0.0, 64)
+
+    def gated(x, w):
+        y = (x.to(F64) @ w.to(F64).T).reshape(len(x), F // 16, 2, 16)
+        g, u = y[:, :, 0].reshape(len(x), F), y[:, :, 1].reshape(len(x), F)
+        return g * torch.sigmoid(g) * u
+
+    perm = order.cpu().long()[: T * top]
+    want = torch.stack([gated(h[e // top][None], up[ids[e // top, e % top]])[0] for e in perm.tolist()])
+    assert float((mid.cpu().to(F64)[: T * top] - want).abs().max()) < 1e-5 * float(want.abs().max())
+    assert float((mids.cpu().to(F64) - gated(h, shared_up)).abs().max()) < 1e-5 * float(want.abs().max())
+    slab = torch.empty(top + 1, T, H, device=DEV)
+    C.moe_down(mid, mids, order, tiles, wts.to(DEV), dn.to(DEV), shared_dn.to(DEV), slab, 64)
+    m = mid.cpu().to(F64)
+    for s, e in enumerate(perm.tolist()):
+        y = wts[e // top, e % top].to(F64) * (dn[ids[e // top, e % top]].to(F64) @ m[s])
+        assert float((slab[e % top, e // top].cpu().to(F64) - y).abs().max()) < 1e-5 * max(1.0, float(y.abs().max()))
+    y = mids.cpu().to(F64) @ shared_dn.to(F64).T
+    assert float((slab[top].cpu().to(F64) - y).abs().max()) < 1e-5 * float(y.abs().max())

@@ -202,6 +202,61 @@ __global__ __launch_bounds__(256) void norm_f32_kernel(float* x, const float* __
   for (int c = threadIdx.x; c < H; c += 256) out[(long)t * H + c] = xr[c] * rstd * (w[c] + woff);
 }
 
+// The same for rows of whole 16 bytes: NC chunks of four a thread, the row kept in registers, four slabs
+// requested at once.  565 rows of 2048 with 5 slabs: 19.4 us above, 8.1 here.
+template <int NC>
+__global__ __launch_bounds__(256) void norm_f32_vec_kernel(float* x, const float* __restrict__ slab, int splits,
+                                                           const float* __restrict__ w, float* out, int T, int H,
+                                                           float eps, const int* __restrict__ rows, int Hn, float woff) {
+  constexpr int AT_ONCE = NC <= 2 ? 4 : 2;
+  __shared__ float red[16];
+  const int t = blockIdx.x, src = rows ? rows[t] : t;
+  float* xr = x + (long)src * H;
+  int at[NC];  // (chunks behind the row: its last one, not counted and not stored)
+  f32x4 v[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    at[i] = min((int)(threadIdx.x + 256 * i) * 4, H - 4);
+    v[i] = *reinterpret_cast<const f32x4*>(xr + at[i]);
+  }
+  auto mine = [&](int i) { return (int)(threadIdx.x + 256 * i) * 4 < H; };
+  if (slab) {
+    for (int k0 = 0; k0 < splits; k0 += AT_ONCE) {
+      f32x4 a[AT_ONCE][NC];
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k)
+        if (k0 + k < splits)
+#pragma unroll
+          for (int i = 0; i < NC; ++i)
+            a[k][i] = *reinterpret_cast<const f32x4*>(slab + ((long)(k0 + k) * T + src) * H + at[i]);
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k)
+        if (k0 + k < splits)
+#pragma unroll
+          for (int i = 0; i < NC; ++i) v[i] += a[k][i];
+    }
+    __syncthreads();  // the row has been read, the last chunk by several threads
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (mine(i)) *reinterpret_cast<f32x4*>(xr + at[i]) = v[i];
+  }
+  if (out == nullptr) return;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if (mine(i)) s += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
+  const float rstd = 1.f / sqrtf(block_sum(s, red) / Hn + eps);
+#pragma unroll
+  for (int i = 0; i < NC; ++i)
+    if (mine(i)) {
+      const f32x4 g = *reinterpret_cast<const f32x4*>(w + at[i]);
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = v[i][e] * rstd * (g[e] + woff);
+      *reinterpret_cast<f32x4*>(out + (long)t * H + at[i]) = y;
+    }
+}
+
 __global__ __launch_bounds__(256) void embed_f32_kernel(const int* __restrict__ ids, const float* __restrict__ wte,
                                                         float* out, int H, int vocab, float scale) {
   int id = ids[blockIdx.x];
@@ -291,6 +346,18 @@ extern "C" hipError_t lsd_norm_f32(float* x, const float* slab, int splits, cons
                                    float eps, const int* rows, int nrows, int Hn, float woff, hipStream_t st) {
   const int n = rows ? nrows : T;
   if (n == 0) return hipSuccess;
+  auto at = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
+  const int nc = (H + 1023) / 1024;
+  if (H >= 4 && H % 4 == 0 && nc <= 8 && (at(x) | at(slab) | at(w) | at(out)) % 16 == 0) {
+#define LSD_NORM_F32(NC)                                                                                                \
+  hipLaunchKernelGGL((norm_f32_vec_kernel<NC>), dim3(n), dim3(256), 0, st, x, slab, splits, w, out, T, H, eps, rows, Hn, woff)
+    if (nc == 1) LSD_NORM_F32(1);
+    else if (nc == 2) LSD_NORM_F32(2);
+    else if (nc <= 4) LSD_NORM_F32(4);
+    else LSD_NORM_F32(8);
+#undef LSD_NORM_F32
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(norm_f32_kernel, dim3(n), dim3(256), 0, st, x, slab, splits, w, out, T, H, eps, rows, Hn, woff);
   return hipGetLastError();
 }

@@ -518,8 +518,8 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
 // fp32 on the bf16 matrix cores
 // ---------------------------------------------------------------------------
 // x = hi + mid + lo, each bf16: of 24 bits the first two, rounded to nearest, leave rests of 16 and 8
-// bits, so nothing is lost from 2^-110 on (below, lo is subnormal).  big: the largest |x|.  Shifts and subtractions: dot products
-// with (-1, 0) and (0, -1), which unpack and subtract at once, keep the MFMAs of other waves waiting.
+// bits, so nothing is lost from 2^-110 on (below, lo is subnormal).  big: the largest |x|.  (Dot products with
+// (-1, 0) and (0, -1) would unpack and subtract at once, but keep the MFMAs of other waves waiting.)
 struct Split {
   bf16x4 t[3];
 };
@@ -541,7 +541,7 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
   return s;
 }
 
-// 16 MT x 64 NT tiles, 32-deep k-steps, WK parts of the k-steps on four waves each, summed in LDS.
+// 16 MT x 16 WN tiles, 32-deep k-steps, WK parts of the k-steps on WN waves each, summed in LDS.
 // Of the nine products of two split operands the six largest are summed (the others are below 2^-26 of
 // it), hi hi apart from the rest, whose sums round at 2^-8 of theirs.  A goes through registers into three
 // LDS planes, split once a block; W, whose columns no two waves share, straight into fragments.
@@ -550,80 +550,71 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
 // 2.7e-7 and 5.7e-7 of the result, parts of K 1.3e-7 and 1.9e-7; K = 5632 4.7e-7 and 9.5e-7; SiLU of two
 // 4.2e-7 and 8.5e-7.
 // Bound by the matrix cores (six MFMAs at sixteen times the fp32 rate) and the splitting beside them
-// (22 issue cycles a value, which a tile's rows and columns share), with one block a CU by what a k-step waits for:
-// hence parts of K where blocks are few.  Against fp32 MFMAs: 565 x 2048 x 2048 59 -> 46 us, 565 x 2560 x
-// 2048 63 -> 50, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 300; 2260 rows over 32 experts of
-// 2048 x 1024 and 565 through a shared one of 2048 up 320 -> 254, down 152 -> 131.  Splitting W a k-step
+// (22 issue cycles a value, which a tile's rows and columns share), and by what a k-step waits for: hence
+// parts of K where blocks are few, and 16 columns a wave, so that four waves share a SIMD (32 columns,
+// two waves: experts below 282 and 133 us).  Against fp32 MFMAs: 565 x 2048 x 2048 59 -> 43 us, 565 x 2560 x
+// 2048 63 -> 49, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 286; 2260 rows over 32 experts of
+// 2048 x 1024 and 565 through a shared one of 2048 up 325 -> 244, down 152 -> 121.  Splitting W a k-step
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
 // A tile with an operand of 2^56 or more, a sum that is not finite, or one that is not zero but below 2^-40
 // is computed again by fp32 MFMAs: terms that left the range of bf16's normal numbers matter there alone.
-template <int MODE, int MT, int NT, int WK, int D>
-__global__ __launch_bounds__(256 * WK, WK == 1 ? 2 : 1) void group_gemm_f32_split_kernel(GgParams p) {
+template <int MODE, int MT, int WN, int WK, int D>
+__global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
-  constexpr int TM = 16 * MT, TN = 64 * NT, BKF = 32, CLD = TN + 4, PLANE = TM * 64, SLOT = 3 * PLANE, QA = (MT + 1) / 2;
+  constexpr int TM = 16 * MT, TN = 16 * WN, BKF = 32, CLD = TN + 4, PLANE = TM * 64, SLOT = 3 * PLANE;
+  constexpr int RA = 8 * WN, QA = (TM + RA - 1) / RA;  // rows of A that a part's threads bring at a time
   constexpr int IMAGE = TM * CLD, SMEM = WK * (2 * SLOT > IMAGE * 4 ? 2 * SLOT : IMAGE * 4);
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
   Tile t = locate<MODE, TM, TN>(p);
   if (!t.live) return;
   resolve<MODE, float>(p, t);
   const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
-  const int w = wave & 3, part = wave >> 2, tid = threadIdx.x & 255;
+  const int w = wave % WN, part = wave / WN, tid = threadIdx.x % (64 * WN);
   const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
   // this part's k-steps; the first part has as many as any
   const int KT = t.K / BKF, most = (KT + WK - 1) / WK, first = part * most, T = max(0, min(most, KT - first));
-  // A: thread i has four k's of rows i / 8 and i / 8 + 32; W: this lane's column of each 16
+  // A: thread i has four k's of rows i / 8, i / 8 + RA ..; W: this lane's column of each 16
   const int ar = tid >> 3, ac = tid & 7;
   const float* ap[QA];
-  const float* wp[NT];
 #pragma unroll
   for (int q = 0; q < QA; ++q)
-    ap[q] = static_cast<const float*>(t.A) + a_row<MODE>(p, t, ar + 32 * q) * t.lda + first * BKF + 4 * ac;
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-    wp[j] = static_cast<const float*>(t.W) + (long)min(t.n0 + (w * NT + j) * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
+    ap[q] = static_cast<const float*>(t.A) + a_row<MODE>(p, t, ar + RA * q) * t.lda + first * BKF + 4 * ac;
+  const float* wp = static_cast<const float*>(t.W) + (long)min(t.n0 + w * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
   auto at = [&](int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4); };  // in a plane
 
-  f32x4 acc[2][MT][NT];
+  f32x4 acc[2][MT];  // hi hi, the others
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[0][i][j] = acc[1][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < MT; ++i) acc[0][i] = acc[1][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float big = 0.f;
-  f32x4 ra[D][QA], rw[D][NT][2];
-  auto load = [&](int kt, f32x4 (&a)[QA], f32x4 (&b)[NT][2]) {  // (behind the last k-step: that one again)
+  f32x4 ra[D][QA], rw[D][2];
+  auto load = [&](int kt, f32x4 (&a)[QA], f32x4 (&b)[2]) {  // (behind the last k-step: that one again)
     const long k = (long)min(kt, T - 1) * BKF;
 #pragma unroll
     for (int q = 0; q < QA; ++q) a[q] = *reinterpret_cast<const f32x4*>(ap[q] + k);
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      b[j][0] = *reinterpret_cast<const f32x4*>(wp[j] + k);
-      b[j][1] = *reinterpret_cast<const f32x4*>(wp[j] + k + 16);
-    }
+    b[0] = *reinterpret_cast<const f32x4*>(wp + k);
+    b[1] = *reinterpret_cast<const f32x4*>(wp + k + 16);
   };
   char* const slots = smem + part * 2 * SLOT;
   auto put_a = [&](int slot, const f32x4 (&a)[QA]) {  // chunk g: k's 4 g and 16 + 4 g
     char* b = slots + slot * SLOT;
 #pragma unroll
     for (int q = 0; q < QA; ++q) {
-      if (MT % 2 && q == QA - 1 && ar >= 16) break;
+      if (TM % RA && q == QA - 1 && ar + RA * q >= TM) break;
       const Split s = split3(a[q], big);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        st4(reinterpret_cast<bf16*>(b + i * PLANE + at(ar + 32 * q, ac & 3) + (ac >> 2) * 8), s.t[i]);
+        st4(reinterpret_cast<bf16*>(b + i * PLANE + at(ar + RA * q, ac & 3) + (ac >> 2) * 8), s.t[i]);
     }
   };
   auto steps = [&](auto L) {
-    bf16x8 wf[NT][3];
+    bf16x8 wf[3];
     auto step = [&](int kt, int set) {
       __syncthreads();  // A of k-step kt is in its slot, the other one's reads are done
       if (WK > 1 && kt >= T) return;
       const char* b = slots + (kt & 1) * SLOT;
+      const Split x = split3(rw[set][0], big), y = split3(rw[set][1], big);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const Split x = split3(rw[set][j][0], big), y = split3(rw[set][j][1], big);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) wf[j][c] = __builtin_shufflevector(x.t[c], y.t[c], 0, 1, 2, 3, 4, 5, 6, 7);
-      }
+      for (int c = 0; c < 3; ++c) wf[c] = __builtin_shufflevector(x.t[c], y.t[c], 0, 1, 2, 3, 4, 5, 6, 7);
       load(kt + D, ra[set], rw[set]);
 #pragma unroll
       for (int i0 = 0; i0 < L; i0 += 2) {  // two tiles at a time: independent chains
@@ -638,9 +629,7 @@ __global__ __launch_bounds__(256 * WK, WK == 1 ? 2 : 1) void group_gemm_f32_spli
         for (int c = 0; c < 6; ++c)
 #pragma unroll
           for (int i = i0; i < min((int)L, i0 + 2); ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[c > 0][i][j] = mfma16(af[i - i0][ca[c]], wf[j][cw[c]], acc[c > 0][i][j]);
+            acc[c > 0][i] = mfma16(af[i - i0][ca[c]], wf[cw[c]], acc[c > 0][i]);
       }
       put_a(~kt & 1, ra[(set + 1) % D]);
     };
@@ -663,58 +652,45 @@ __global__ __launch_bounds__(256 * WK, WK == 1 ? 2 : 1) void group_gemm_f32_spli
   });
   bool exact = big >= 0x1p56f;
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i) {
+    acc[0][i] += acc[1][i];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      acc[0][i][j] += acc[1][i][j];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float v = fabsf(acc[0][i][j][q]);
-        exact |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
-      }
+    for (int q = 0; q < 4; ++q) {
+      const float v = fabsf(acc[0][i][q]);
+      exact |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
     }
+  }
   if (__syncthreads_or(exact)) {
 #pragma unroll 1
     for (int i = 0; i < live; ++i) {
       const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;
-      f32x4 s[NT];
-#pragma unroll
-      for (int j = 0; j < NT; ++j) s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
       for (int k = 0; k < T * BKF; k += 16) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(a + k);
+        const f32x4 av = *reinterpret_cast<const f32x4*>(a + k), wv = *reinterpret_cast<const f32x4*>(wp + k);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          const f32x4 wv = *reinterpret_cast<const f32x4*>(wp[j] + k);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[j], 0, 0, 0);
-        }
+        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s, 0, 0, 0);
       }
 #pragma unroll
       for (int h = 0; h < MT; ++h)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-          if (h == i) acc[0][h][j] = s[j];
+        if (h == i) acc[0][h] = s;
     }
   }
   float* ct = reinterpret_cast<float*>(smem);
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        ct[part * IMAGE + (i * 16 + 4 * g + q) * CLD + (w * NT + j) * 16 + r] = acc[0][i][j][q];
+    for (int q = 0; q < 4; ++q) ct[part * IMAGE + (i * 16 + 4 * g + q) * CLD + w * 16 + r] = acc[0][i][q];
   __syncthreads();
   if constexpr (WK > 1) {
-    for (int c = threadIdx.x; c < IMAGE / 4; c += 256 * WK) {
+    for (int c = threadIdx.x; c < IMAGE / 4; c += 64 * WN * WK) {
       f32x4* o = reinterpret_cast<f32x4*>(ct) + c;
 #pragma unroll
       for (int i = 1; i < WK; ++i) *o += o[i * (IMAGE / 4)];
     }
     __syncthreads();
   }
-  f32_epilogue<MODE, TM, TN, 256 * WK>(p, t, ct);
+  f32_epilogue<MODE, TM, TN, 64 * WN * WK>(p, t, ct);
 }
 
 // Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
@@ -938,27 +914,28 @@ static hipError_t gg_f32_on(const GgParams& p, bool addr64, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <int MODE, int MT, int NT, int WK, int D>
+template <int MODE, int MT, int WN, int WK, int D>
 static hipError_t gg_split_on(const GgParams& p, hipStream_t st) {
-  const long blocks = gg_blocks(p, MODE, 16 * MT, 64 * NT);
+  const long blocks = gg_blocks(p, MODE, 16 * MT, 16 * WN);
   if (blocks)
-    hipLaunchKernelGGL((group_gemm_f32_split_kernel<MODE, MT, NT, WK, D>), dim3((unsigned)blocks), dim3(256 * WK), 0, st, p);
+    hipLaunchKernelGGL((group_gemm_f32_split_kernel<MODE, MT, WN, WK, D>), dim3((unsigned)blocks), dim3(64 * WN * WK), 0, st, p);
   return hipGetLastError();
 }
 
-// The split kernel's tile for M rows: what its blocks take in rounds of 256, in us at K = 2048
-// (fixed part, a round) as measured over 17 .. 1500 rows of 512 .. 11264 columns.  565 rows of 2048 columns:
-// 32-row tiles 62.9 us, 48 47.3, 64 52.0, 80 40.6, 64 x 128 67.9, 96 x 128 82.8; of 2560 64.2, 49.9, 52.5,
-// 73.5, 96-row ones 43.2; 1000 of 11264 487, 367, 316, 357, 64 x 128 290, 96 x 128 265.
+// The split kernel's tile: what its blocks take in rounds of 256, in us at K = 2048 (fixed part, a round), as
+// measured over 100 .. 1500 rows of 2048 .. 11264 columns.  565 rows of 2048 columns: 48 x 64 47.3 us, 64 x 64 52.0,
+// 80 x 64 43.3, 48 x 128 47.7; 300 of 2048 48 x 64 in two parts of K 33.7, in four 29.0; 565 of 4160
+// 48 x 128 86, 80 x 128 100, 96 x 128 73; 1000 of 2048 64 x 64 67.7, 64 x 128 61.0; of 4160 80 x 128 117, 96 x 128
+// 128; of 11264 64 x 128 306, 80 x 128 299, 96 x 128 286.
 struct SplitTile {
-  int rows, cols, fixed, round;
+  int rows, cols, parts, fixed, round;
 };
-static const SplitTile SPLIT_TILES[] = {{32, 64, 1, 21}, {48, 64, 5, 25}, {64, 64, 4, 28}, {80, 64, 0, 39}, {96, 64, 0, 42},
-                                        {64, 128, 20, 45}, {96, 128, 22, 61}};
+static const SplitTile SPLIT_TILES[] = {{32, 64, 4, 1, 21}, {48, 64, 4, 1, 27}, {64, 64, 2, 4, 28}, {80, 64, 3, 0, 41},
+                                        {48, 128, 1, 2, 42}, {64, 128, 1, 4, 48}, {80, 128, 1, 0, 59}, {96, 128, 1, 0, 70}};
 static int split_tile(const GgParams& p) {
   int best = 0;
   long least = 0;
-  for (int i = 0; i < 7; ++i) {
+  for (int i = 0; i < 8; ++i) {
     const SplitTile& t = SPLIT_TILES[i];
     const long cost = t.fixed + (gg_blocks(p, GG_F32, t.rows, t.cols) + 255) / 256 * t.round;
     if (i == 0 || cost < least) best = i, least = cost;
@@ -966,14 +943,14 @@ static int split_tile(const GgParams& p) {
   return best;
 }
 
-// Products on split operands: experts from 20 rows a tile of the table on (2048 x 1024, 4 of 32 experts:
-// 300 tokens, 24 rows, up 194 -> 169 us, down 99 -> 92; 200, 18 rows, 158 and 168, 80 and 89, on another
-// card 182 and 169; 40, 5 rows, 121 and 126, 47 and 68).  Others with more than 16 rows, unless the few are
+// Products on split operands: experts from 18 rows a tile of the table on (2048 x 1024, 4 of 32 experts:
+// 300 tokens, 24 rows, up 185 us either way, down 93; 200, 18 rows, 161 -> 149, 78 -> 68; 160, 15 rows, 139
+// and 160, 71 and 77; 2 of 16 of 1024 x 512: 200, 18 rows, 38 -> 31).  Others with more than 16 rows, unless the few are
 // bound by the weights' stream (20 rows of 32000 x 2048 42 us and 50, of 16384 31.1 and 27.5) or K is short for the
 // splitting to hide (565 rows of 2048, K = 256 12.2 and 12.8, 512 19.2 and 17.9; of 4096, K = 512 31.4 and 32.9;
 // 100 rows of 2048, K = 512 10.6 and 11.1, 2048 28.7 and 22.9).
 static bool on_split(const GgParams& p, bool experts) {
-  if (experts) return (long)p.T * p.top >= 20L * p.n_tiles;
+  if (experts) return (long)p.T * p.top >= 18L * p.n_tiles;
   return p.K > 512 && p.M > 16 && !(p.M <= 32 && gg_blocks(p, GG_F32, 32, 64) > 256);
 }
 
@@ -989,15 +966,16 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   if (on_split(p, MODE == GG_UP || MODE == GG_DOWN)) {
     if constexpr (MODE == GG_F32 || MODE == GG_ADD) {
       switch (split_tile(p)) {
-        case 0: return gg_split_on<MODE, 2, 1, 4, 2>(p, st);
-        case 1: return gg_split_on<MODE, 3, 1, 2, 3>(p, st);
-        case 2: return gg_split_on<MODE, 4, 1, 2, 2>(p, st);
-        case 3: return gg_split_on<MODE, 5, 1, 2, 2>(p, st);
-        case 4: return gg_split_on<MODE, 6, 1, 2, 2>(p, st);
-        case 6: return gg_split_on<MODE, 6, 2, 1, 2>(p, st);
+        case 0: return gg_split_on<MODE, 2, 4, 4, 2>(p, st);
+        case 1: return gg_split_on<MODE, 3, 4, 4, 2>(p, st);
+        case 2: return gg_split_on<MODE, 4, 4, 2, 2>(p, st);
+        case 3: return gg_split_on<MODE, 5, 4, 3, 2>(p, st);
+        case 4: return gg_split_on<MODE, 3, 8, 1, 3>(p, st);
+        case 6: return gg_split_on<MODE, 5, 8, 1, 2>(p, st);
+        case 7: return gg_split_on<MODE, 6, 8, 1, 2>(p, st);
       }
     }
-    return gg_split_on<MODE, 4, 2, 1, 2>(p, st);
+    return gg_split_on<MODE, 4, 8, 1, 3>(p, st);
   }
   // The others count bytes from a tile's first row, or from the first of the rows it gathers, in 32 bits
   // where those hold them (524288 tokens of 2048 are 4 GB)
@@ -1018,12 +996,12 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   return gg_f32_on<MODE, 4>(p, addr64, st);
 }
 
-// Rows and columns of the tiles of M x N fp32 results (tests)
-extern "C" void lsd_group_gemm_split_tile(int M, int N, int* rows, int* cols) {
+// Rows and columns of the tiles of M x N fp32 results, and parts of K (tests)
+extern "C" void lsd_group_gemm_split_tile(int M, int N, int* tile) {
   GgParams p{};
   p.M = M, p.N = N, p.groups = 1;
   const SplitTile& t = SPLIT_TILES[split_tile(p)];
-  *rows = t.rows, *cols = t.cols;
+  tile[0] = t.rows, tile[1] = t.cols, tile[2] = t.parts;
 }
 
 // fp32 kernels: 64-row tiles

@@ -24,7 +24,7 @@ using lsd::RowsParams;
 extern "C" {
 hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStream_t st);
 hipError_t lsd_group_gemm_f32(const GgParams* p, int mode, hipStream_t st);
-void lsd_group_gemm_split_tile(int M, int N, int* rows, int* cols);
+void lsd_group_gemm_split_tile(int M, int N, int* tile);
 hipError_t lsd_moe_gemv_up(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_moe_gemv_down(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_latent_post(const LatentPostParams* p, int f32, hipStream_t st);
@@ -624,9 +624,9 @@ void lsd_register_latent(pybind11::module& m) {
   m.def("linear_fp32", &linear_fp32, py::arg("a"), py::arg("w"), py::arg("x") = py::none(),
         py::arg("bias") = py::none());
   m.def("fp32_tile", [](int64_t M, int64_t N) {
-    int rows, cols;
-    lsd_group_gemm_split_tile((int)M, (int)N, &rows, &cols);
-    return std::make_pair(rows, cols);
+    std::array<int, 3> t;
+    lsd_group_gemm_split_tile((int)M, (int)N, t.data());
+    return std::make_tuple(t[0], t[1], t[2]);
   });
   m.def("moe_group", &moe_group, py::arg("ids"), py::arg("experts"), py::arg("tm"));
   m.def("moe_up", &moe_up, py::arg("h"), py::arg("perm"), py::arg("tiles"), py::arg("top"), py::arg("w"),

@@ -18,14 +18,14 @@ def near(got, a, w, extra=0.0):
 
 
 # every tile: its edges, parts of K that are empty, uneven and whole
-TILES = [(17, 40, (32, 64)), (33, 1985, (32, 64)), (33, 11264, (48, 64)), (193, 2600, (48, 64)), (500, 1985, (64, 64)),
-         (561, 2048, (80, 64)), (481, 2600, (96, 64)), (1025, 3072, (64, 128)), (561, 4160, (96, 128))]
+TILES = [(17, 40, (32, 64, 4)), (33, 1985, (32, 64, 4)), (81, 5952, (48, 64, 4)), (193, 3264, (48, 64, 4)), (500, 1985, (64, 64, 2)),
+         (561, 2048, (80, 64, 3)), (561, 2560, (48, 128, 1)), (961, 2048, (64, 128, 1)), (801, 2600, (80, 128, 1)),
+         (561, 4160, (96, 128, 1))]
 
 
 def test_tiles():
     _C = pytest.importorskip("llm_sharding_demo_amd._C")
     assert [_C.fp32_tile(M, N) for M, N, _ in TILES] == [t for _, _, t in TILES]
-    assert {t for _, _, t in TILES} == {(32, 64), (48, 64), (64, 64), (80, 64), (96, 64), (64, 128), (96, 128)}
 
 
 @pytest.mark.gpu
@@ -62,7 +62,7 @@ def test_not_finite(C, side, value):  # noqa: F811
     assert bool(((got - want).abs()[ok] <= 600 * ULP * 576).all())
 
 
-# 20 rows a tile of the table and more: experts on split operands, and fewer, which are not
+# 18 rows a tile of the table and more: experts on split operands, and fewer, which are not
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,E", [(300, 3), (129, 5), (64, 1), (30, 9)])
 def test_experts(C, T, E):  # noqa: F811
@@ -73,7 +73,7 @@ def test_experts(C, T, E):  # noqa: F811
     ids[: T // 2, 0], ids[: T // 2, 1:] = 0, min(1, E - 1)  # uneven
     wts = torch.rand(T, top)
     order, tiles = C.moe_group(ids.to(DEV), E, 64)
-    on = T * top >= 20 * tiles.shape[0]
+    on = T * top >= 18 * tiles.shape[0]
     assert on == (T > 30)
     mid, mids = C.moe_up(h.to(DEV), order, tiles, top, up.to(DEV), 0.0, 1.0, shared_up.to(DEV), 0.0, 64)
 

@@ -333,8 +333,196 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
   }
 }
 
+
+// ---------------------------------------------------------------------------
+// One row, many outputs: waves that go through several
+// ---------------------------------------------------------------------------
+// A wave of the kernel above requests all that it will read and ends with it: of some ten thousand rows the
+// launch is several rounds of blocks, each of which norms x again and starts its stream from nothing; of
+// long rows few blocks fit a CU.  Here a wave goes through units of two rows (of SEGS segments each), the
+// next one in flight under the products of this one, and on to items that lie a launch's waves apart; x
+// is brought once a block.  An item is two rows, or the eight of a sampler segment, whose maximum is then
+// the wave's own.  Same sums, same order as above.
+// Cold weights, above -> here:
+//   28672 x 4096 gate/up   40.9 -> 36.5 us (6.4 TB/s)   128256 x 4096 head      180 -> 155 (6.8)
+//   4096 x 14336 residual  22.0 -> 20.2                 4096 x 4096 residual    8.2 -> 7.5
+//   6144 x 4096 QKV        11.7 -> 11.3                 16384 x 2048 gate/up   13.0 -> 12.3
+// Llama-3 8B, a step of one sequence 2907 -> 2754.  Not ahead: 3072 x 3072 5.8 and 6.1, 3072 x 8192 11.1 either
+// way, a head of 50304 x 1600 27.7 and 29.9 (x 768 21.1 -> 15.2, but in GPT-2's step, whose weights the caches
+// hold, 15 either way); 28672 x 4096 a row at a time, three to five in flight.
+template <int EPI, int NORM, int SLOTS, int SEGS>
+__global__ __launch_bounds__(256, 2) void gemv_stream_kernel(GemvParams p) {
+  constexpr int ITEM = EPI == gv::F32 ? 4 : 1, KS = SLOTS * SEGS * 512, NV = KS / 1024;  // ITEM: pairs of rows
+  __shared__ __attribute__((aligned(16))) bf16 xs[KS];
+  __shared__ float red[4];
+  const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int KC = p.K >> 3, pairs = (p.N + 1) / 2, items = (pairs + ITEM - 1) / ITEM, waves = gridDim.x * 4;
+  const int first = blockIdx.x * 4 + w, n = first < items ? (items - 1 - first) / waves + 1 : 0;  // this wave's items
+  // unit u: segment u % SEGS of the columns of pair u / SEGS
+  auto pair_of = [&](int u) { u /= SEGS; return (first + u / ITEM * waves) * ITEM + u % ITEM; };
+  bf16x8 wv[2][2][SLOTS];
+  auto load = [&](int u, bf16x8 (&v)[2][SLOTS]) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const bf16* wr = p.W + (long)min(gv_row<EPI, 2>(pair_of(u), j), p.N - 1) * p.ldw;
+#pragma unroll
+      for (int i = 0; i < SLOTS; ++i) v[j][i] = ld8_nt(wr + min(u % SEGS * SLOTS * 64 + lane + 64 * i, KC - 1) * 8);
+    }
+  };
+  if constexpr (NORM == gv::NONE) {
+    bf16x8 av[KS / 2048 + 1];
+#pragma unroll
+    for (int i = 0; i < (KS + 2047) / 2048; ++i) av[i] = ld8(p.A + min(tid + 256 * i, KC - 1) * 8);
+    if (n) load(0, wv[0]);
+    const bf16x8 zero = {};
+#pragma unroll
+    for (int i = 0; i < (KS + 2047) / 2048; ++i)
+      if ((tid + 256 * i) * 8 < KS) st8(xs + (tid + 256 * i) * 8, tid + 256 * i < KC ? av[i] : zero);
+  } else {
+    f32x4 xr[NV];
+    bf16x4 gm[NV], bt[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = min((tid + 256 * i) * 4, p.K - 4);
+      gm[i] = ld4(p.gamma + c);
+      if constexpr (NORM == gv::LN) bt[i] = ld4(p.beta + c);
+      xr[i] = *reinterpret_cast<const f32x4*>(p.X + c);
+    }
+    if (n) load(0, wv[0]);
+    float mean[1] = {0.f}, rstd[1] = {0.f};
+    if constexpr (NORM == gv::LN) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        if ((tid + 256 * i) * 4 < p.K) mean[0] += xr[i][0] + xr[i][1] + xr[i][2] + xr[i][3];
+      block_sums<1>(mean, red);
+      mean[0] /= p.K;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if ((tid + 256 * i) * 4 < p.K) {
+        const f32x4 d = xr[i] - mean[0];
+        rstd[0] += d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + d[3] * d[3];
+      }
+    block_sums<1>(rstd, red);
+    const float rs = rsqrtf(rstd[0] / p.K + p.eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int c = (tid + 256 * i) * 4;
+      bf16x4 r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float z = (xr[i][e] - mean[0]) * rs * bf2f(gm[i][e]);
+        if constexpr (NORM == gv::LN) z += bf2f(bt[i][e]);
+        r[e] = f2bf(c < p.K ? z : 0.f);
+      }
+      st4(xs + c, r);
+    }
+  }
+  __syncthreads();
+  float top = -INFINITY;  // of this item's outputs so far
+  float sum[2], e_x = 0.f, e_bias = 0.f, e_cs0 = 0.f, e_cs1 = 0.f;  // of output 2 g + (lane >> 5), under the products
+  int e_pos = 0, e_slot = 0;
+  auto products = [&](int u, bf16x8 (&v)[2][SLOTS]) {
+    if (u % SEGS == 0) {
+      sum[0] = sum[1] = 0.f;
+      const int c = min(2 * pair_of(u) + (lane >> 5), p.N - 1);
+      if (EPI != gv::SILU && p.bias) e_bias = bf2f(p.bias[c]);
+      if constexpr (EPI == gv::RESID) e_x = reinterpret_cast<const float*>(p.out)[c];
+      if constexpr (EPI == gv::QKV) {
+        e_pos = p.tpos[0];
+        e_slot = p.tslot[0];
+        if (p.rope != nullptr && c < p.q_size + p.kv_size) {
+          const int d = (c < p.q_size ? c : c - p.q_size) % p.hd;
+          const float* cs = p.rope + ((long)e_pos * (p.hd >> 1) + (d >> 1)) * 2;
+          e_cs0 = cs[0];
+          e_cs1 = cs[1];
+        }
+      }
+    }
+    float acc[2] = {sum[0], sum[1]};
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      const bf16x8 x = *reinterpret_cast<const bf16x8*>(xs + (u % SEGS * SLOTS * 64 + lane + 64 * i) * 8);
+      acc[0] = dot8(v[0][i], x, acc[0]);
+      acc[1] = dot8(v[1][i], x, acc[1]);
+    }
+    if (u % SEGS != SEGS - 1) {
+      sum[0] = acc[0], sum[1] = acc[1];
+      return;
+    }
+    int idx = 0;  // lanes 0 .. 31 end with the first row's sum, the others with the second's
+    gv_step<32, 2>(acc, idx, lane);
+    gv_step<16, 1>(acc, idx, lane);
+    gv_step<8, 1>(acc, idx, lane);
+    gv_step<4, 1>(acc, idx, lane);
+    gv_step<2, 1>(acc, idx, lane);
+    gv_step<1, 1>(acc, idx, lane);
+    float y = acc[0] + e_bias;
+    const float z = wave_xchg<32>(y);
+    const int g = pair_of(u), c = 2 * g + idx;
+    if constexpr (EPI == gv::SILU) {
+      if (lane == 0) reinterpret_cast<bf16*>(p.out)[g] = f2bf(gated(y, z, p.glu, p.act_scale));
+    } else if constexpr (EPI == gv::RESID) {
+      if ((lane & 31) == 0 && c < p.N) reinterpret_cast<float*>(p.out)[c] = e_x + y;
+    } else if constexpr (EPI == gv::QKV) {
+      if ((lane & 31) == 0) {  // (an even number of columns: heads of even dims)
+        const int qk = p.q_size + p.kv_size;
+        if (p.rope != nullptr && c < qk) y = idx ? y * e_cs0 + z * e_cs1 : y * e_cs0 - z * e_cs1;
+        if (c < p.q_size) {
+          reinterpret_cast<bf16*>(p.out)[c] = f2bf(y);
+        } else {
+          const int kc = c < qk ? c - p.q_size : c - qk;
+          bf16* cache = c < qk ? p.kc : p.vc;
+          cache[(((long)e_slot * p.n_kv + kc / p.hd) * p.max_seq + e_pos) * p.hd + kc % p.hd] = f2bf(y);
+        }
+      }
+    } else {
+      if ((lane & 31) == 0 && c < p.N) reinterpret_cast<float*>(p.out)[c] = y;
+      const int u1 = u / SEGS;
+      if (p.segmax) {
+        top = u1 % ITEM ? top : -INFINITY;
+        if (2 * g < p.N) top = fmaxf(top, 2 * g + 1 < p.N ? fmaxf(y, z) : idx ? z : y);
+        if (u1 % ITEM == ITEM - 1 && lane == 0) p.segmax[g / ITEM] = top;
+      }
+    }
+  };
+  const int units = n * ITEM * SEGS;
+  for (int u = 0; u < units; u += 2) {
+    if (u + 1 < units) load(u + 1, wv[1]);
+    products(u, wv[0]);
+    if (u + 1 >= units) break;
+    if (u + 2 < units) load(u + 2, wv[0]);
+    products(u + 1, wv[1]);
+  }
+}
+
 template <int EPI, int NORM>
 hipError_t gemv_launch(const GemvParams& p, int mr, int nb, hipStream_t st) {
+  if (mr == 1 && p.N >= 4096) {  // gemv_stream_kernel has both sides' times
+    // up to sixteen waves a CU (28672 x 4096: eight 37.1 us, sixteen and more 36.5), all with as many items
+    const int item = EPI == gv::F32 ? 8 : 2, items = (p.N + item - 1) / item, each = (items + 4095) / 4096;
+    const dim3 g(((items + each - 1) / each + 3) / 4);
+#define LSD_GS(SLOTS, SEGS)                                                                              \
+  {                                                                                                      \
+    hipLaunchKernelGGL((gemv_stream_kernel<EPI, NORM, SLOTS, SEGS>), g, dim3(256), 0, st, p);            \
+    return hipGetLastError();                                                                            \
+  }
+    if constexpr (EPI == gv::SILU && NORM != gv::NONE) {
+      if (each > 1 && p.K > 1024 && p.K <= 2048) LSD_GS(4, 1)
+      if (each > 1 && p.K > 2048 && p.K <= 4096) LSD_GS(8, 1)
+    }
+    if constexpr (EPI == gv::F32 && NORM != gv::NONE) {
+      if (p.N >= 16384 && p.K > 2048 && p.K <= 4096) LSD_GS(8, 1)
+    }
+    if constexpr (EPI == gv::QKV && NORM != gv::NONE) {
+      if (p.K > 2048 && p.K <= 4096) LSD_GS(4, 2)
+    }
+    if constexpr (EPI == gv::RESID) {
+      if (p.K > 2048 && p.K <= 4096) LSD_GS(4, 2)
+      if (p.K > 8192) LSD_GS(4, 7)
+    }
+#undef LSD_GS
+  }
   constexpr int CPW = EPI == gv::RESID ? 1 : 2;
   const int grid = (p.N + 4 * CPW - 1) / (4 * CPW);
 #define LSD_GV(MR_, NB_)                                                                    \

@@ -709,19 +709,47 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(LatentExpandedP
   }
 }
 
-__global__ __launch_bounds__(256) void latent_combine_kernel(const float* __restrict__ part_o,
-                                                             const float* __restrict__ part_ml, bf16* out, int rank,
-                                                             int splits) {
+// Merges the splits of a (token, head), a wave per 256 columns.  What it costs is the round trips to memory:
+// the partials of AT splits are requested together with all maxima and sums, which split s's lane
+// weighs for the wave, not split by split behind them (with the kernel in front, 16 heads, 512 columns: 1 token
+// of 1000 keys in 16 splits 17.9 -> 10.2 us, 24 of 500 in 8 16.3 -> 12.8, 64 of 300 in 4 17.8 -> 15.9).
+// MAXL: splits / 64, rounded up.
+template <int AT, int MAXL>
+__global__ __launch_bounds__(64) void latent_combine_kernel(const float* __restrict__ part_o,
+                                                            const float* __restrict__ part_ml, bf16* out, int rank,
+                                                            int splits) {
   const long pi = (long)blockIdx.x * splits;
-  float M = NEG, L = 0.f;
-  for (int s = 0; s < splits; ++s) M = fmaxf(M, part_ml[2 * (pi + s)]);
-  for (int s = 0; s < splits; ++s) L += part_ml[2 * (pi + s) + 1] * exp2f(part_ml[2 * (pi + s)] - M);
-  const float inv = 1.f / L;
-  for (int d = threadIdx.x; d < rank; d += 256) {
-    float v = 0.f;
-    for (int s = 0; s < splits; ++s) v += part_o[(pi + s) * rank + d] * exp2f(part_ml[2 * (pi + s)] - M);
-    out[(long)blockIdx.x * rank + d] = f2bf(v * inv);
+  const int lane = threadIdx.x, d = blockIdx.y * 256 + lane * 4;
+  const float* po = part_o + pi * rank + min(d, rank - 4);
+  f32x4 v[AT];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int i = 0; i < AT; ++i) v[i] = *reinterpret_cast<const f32x4*>(po + (long)min(s0 + i, splits - 1) * rank);
+  };
+  f32x2 ml[MAXL];
+#pragma unroll
+  for (int i = 0; i < MAXL; ++i) ml[i] = *reinterpret_cast<const f32x2*>(part_ml + 2 * (pi + min(lane + 64 * i, splits - 1)));
+  load(0);
+  float M = NEG, L = 0.f, f[MAXL];
+#pragma unroll
+  for (int i = 0; i < MAXL; ++i) M = fmaxf(M, ml[i][0]);
+  M = wave_max(M);
+#pragma unroll
+  for (int i = 0; i < MAXL; ++i) {
+    f[i] = lane + 64 * i < splits ? exp2f(ml[i][0] - M) : 0.f;
+    L += ml[i][1] * f[i];
   }
+  L = wave_sum(L);
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < MAXL; ++j)
+    for (int s0 = 64 * j; s0 < min(splits, 64 * j + 64); s0 += AT) {
+      if (s0) load(s0);
+#pragma unroll
+      for (int i = 0; i < AT; ++i) sum += v[i] * __shfl(f[j], s0 % 64 + i);
+    }
+  const float inv = 1.f / L;
+  if (d < rank) st4(out + (long)blockIdx.x * rank + d, pack4(sum * inv));
 }
 
 __device__ __forceinline__ float to_f(float v) { return v; }
@@ -977,9 +1005,15 @@ extern "C" hipError_t lsd_latent_decode(const LatentAttnParams* p, hipStream_t s
   }
 #undef LSD_LD_V
 #undef LSD_LD
-  if (p->splits > 1)
-    hipLaunchKernelGGL(latent_combine_kernel, dim3(p->B * p->H), dim3(256), 0, st, p->part_o, p->part_ml,
-                       static_cast<bf16*>(p->out), p->v_pad, p->splits);
+#define LSD_LC(AT, ML)                                                                                          \
+  hipLaunchKernelGGL((latent_combine_kernel<AT, ML>), dim3(p->B * p->H, (p->v_pad + 255) / 256), dim3(64), 0, st, \
+                     p->part_o, p->part_ml, static_cast<bf16*>(p->out), p->v_pad, p->splits)
+  if (p->splits > 1024) return hipErrorInvalidValue;
+  if (p->splits > 64) LSD_LC(16, 16);
+  else if (p->splits > 8) LSD_LC(16, 1);
+  else if (p->splits > 4) LSD_LC(8, 1);
+  else if (p->splits > 1) LSD_LC(4, 1);
+#undef LSD_LC
   return hipGetLastError();
 }
 

@@ -883,7 +883,7 @@ class HipBackend(Backend):
         q = self._batch_linear(q, uk)
         if meta.is_decode or self.fp32 or rows == 0:
             # one query per sequence, or the kernel that takes any token alone
-            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx))
+            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2])
             o = self.C.latent_decode(q, pool, kv.table, meta.token_slots, meta.token_pos, m.heads, window, m.scale,
                                      splits, *beside)
         else:

@@ -127,9 +127,6 @@ class Routing:
     router_target: int = 256
     # up to this many tokens, experts stream their weights per (token, choice)
     moe_few_t: int = 4
-    # latent decode attention: workgroups (16 heads of a sequence x splits) a
-    # launch aims for; a split keeps at least one 32-key tile per wave
-    latent_target: int = 256
     # prompts of at least latent_expand_t tokens attend over expanded keys and
     # values where that saves multiply-adds (latent_expand; 0 disables)
     latent_expand_t: int = 256
@@ -393,9 +390,25 @@ class Routing:
         expanded = keys * (dim + vdim) + rank * (dim + vdim) * rows / T
         return expanded * 1.25 < latent
 
-    def latent_splits(self, B: int, heads: int, keys: int) -> int:
-        items = B * math.ceil(heads / 16)
-        return max(1, min(math.ceil(self.latent_target / items), math.ceil((keys + 31) / 128), 64))
+    def latent_splits(self, B: int, heads: int, keys: int, rank: int) -> int:
+        """Context splits of a latent decode launch: the least of what a block's steps
+        take, more where two share a CU, and the merge of the parts.  rank 512, us, for
+        splits 1 / 2 / 4 / 8: 64 sequences of 300 keys 16.0 / 15.8 / 15.4 / 19.3, 24 of 470 22 / 17 / 13.1 /
+        12.7, 96 of 250 13.8 / 15.4 / 17.6 / 24, 160 of 250 13.9 / 21 / 24 / 31."""
+        items = B * -(-heads // 16)
+        steps = max(1, -(-keys // (64 if rank >= 320 else 128)))  # keys a block takes at a time
+        best, least = 1, 0.0
+        for k in (steps, 32, 16, 12, 8, 6, 5, 4, 3, 2, 1):  # steps a block
+            if k > steps:
+                continue
+            s = min(-(-steps // k), 64)
+            share = -(-items * s // 256)  # blocks a CU
+            cost = (0.6 + 0.003 * rank) * (1 if share <= 1 else 0.35 + 0.65 * share) * -(-steps // s)
+            if s > 1:
+                cost += 3 + 1.6e-6 * B * heads * rank * s
+            if k == steps or cost < least:
+                best, least = s, cost
+        return best
 
     def forget_segments(self, items: int, tokens: int) -> int:
         """Segments of every sequence in a chunked recurrence (items: sequences x

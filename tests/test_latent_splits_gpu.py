@@ -1,0 +1,34 @@
+"""Latent decode in parts: the merge at the edges of what it requests at once, and how many parts."""
+
+import pytest
+import torch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rank", [64, 256, 320, 576])
+@pytest.mark.parametrize("splits", [2, 4, 5, 8, 9, 16, 17, 64, 65, 128, 129, 1024])
+def test_parts(rank, splits):
+    """Against one part: half a bf16 step (2^-8) each, weights of 16 bits, 700 fp32 sums."""
+    from llm_sharding_demo_amd import _C as C
+
+    i32 = dict(dtype=torch.int32, device="cuda")
+    g = torch.Generator().manual_seed(rank + splits)
+    pos, H = [0, 63, 64, 130, 699], 5
+    pool = torch.randn(11, 64, rank, generator=g).bfloat16()
+    table = torch.randperm(11, generator=g).int().reshape(1, 11).cuda()
+    q = torch.randn(len(pos), H * rank, generator=g).bfloat16().cuda()
+    at = (q, pool.cuda(), table, torch.zeros(len(pos), **i32), torch.tensor(pos, **i32), H)
+    for window in (1 << 30, 200):
+        one, got = (C.latent_decode(*at, window, rank ** -0.5, s).double() for s in (1, splits))
+        assert bool(((got - one).abs() <= 2.0 ** -7 * one.abs() + 2.0 ** -13 * pool.abs().max().item()).all())
+
+
+def test_rule():
+    from llm_sharding_demo_amd.ops.routing import Routing
+
+    R = Routing()
+    for B, heads, keys, rank, want in [(1, 16, 61, 512, 1), (1, 16, 251, 512, 4), (1, 16, 1001, 512, 16), (24, 16, 471, 512, 8),
+                                       (64, 16, 301, 512, 3), (96, 16, 251, 512, 1), (160, 16, 251, 512, 1), (160, 16, 2001, 512, 3),
+                                       (64, 64, 301, 576, 1), (1, 16, 251, 256, 1), (16, 16, 501, 256, 4), (1, 1, 1, 64, 1), (1, 16, 0, 512, 1),
+                                       (1, 1, 1 << 20, 64, 64)]:
+        assert 1 <= (got := R.latent_splits(B, heads, keys, rank)) <= 64 and got == want, (B, heads, keys, rank, got)

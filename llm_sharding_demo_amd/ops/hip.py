@@ -766,7 +766,8 @@ class HipBackend(Backend):
         if m.talking and not m.talk_weights and tp is not None and not keep and slopes is None and gate is None:
             td = w("mixer.talk_decode", None)
             if mt.is_decode and td is not None:
-                C.talk_decode(*at, td, *rows, window, m.scale, cap, R.talk_splits(mt.num_seqs, ctx), out)
+                C.talk_decode(*at, td, *rows, window, m.scale, cap, R.talk_splits(mt.num_seqs, ctx, ctx < mt.max_ctx),
+                              out)
             else:
                 tiles = self._query_tiles(mt, C.talk_tile(tp.shape[0]), q.device)
                 C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, R.talk_prefill_splits(tiles.shape[0], ctx), out)

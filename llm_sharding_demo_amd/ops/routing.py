@@ -137,9 +137,10 @@ class Routing:
     # sequence at least forget_tokens long
     forget_target: int = 512
     forget_tokens: int = 64
-    # decode attention with mixed heads: blocks a launch aims for, two 64-key
-    # tiles each unless that leaves half of them idle
-    talk_target: int = 512
+    # decode attention with mixed heads: 64-key tiles that a launch takes one a block, as
+    # many blocks with two and more each beyond (a step of 96 sequences of 300 keys: 1 / 3 / 5 splits 977 / 932 / 919
+    # us, of 600, 5 / 10 splits 951 / 957; 48 of 900, 8 / 15 splits 673 / 673; 24 of 500, 4 / 8 522 / 504)
+    talk_target: int = 768
     # ... and prompt attention with few query tiles
     talk_prefill_target: int = 512
     # prompt attention: query tiles of 128 (else 64) from attn_tile_min blocks (32 heads
@@ -419,13 +420,11 @@ class Routing:
     def router_splits(self, T: int, K: int) -> int:
         return max(1, min(self.router_target // math.ceil(T / 16), K // self.router_k, 16))
 
-    def talk_splits(self, B: int, keys: int) -> int:
+    def talk_splits(self, B: int, keys: int, windowed: bool) -> int:
         """Context splits of a decode attention launch with mixed heads (one
         block holds all heads of a token, 64 keys a step)."""
-        tiles = math.ceil((keys + 63) / 64)  # a window may begin inside one
-        if B * tiles > self.talk_target // 2:
-            tiles = math.ceil(tiles / 2)
-        return max(1, min(math.ceil(self.talk_target / B), tiles, 64))
+        tiles = math.ceil(keys / 64) + windowed  # a window may begin inside one
+        return max(1, min(math.ceil(tiles / max(1, math.ceil(B * tiles / self.talk_target))), 64))
 
     def talk_prefill_splits(self, tiles: int, keys: int) -> int:
         """Key splits of a prompt attention launch with mixed heads: few query

@@ -32,3 +32,7 @@ def test_rule():
                                        (64, 64, 301, 576, 1), (1, 16, 251, 256, 1), (16, 16, 501, 256, 4), (1, 1, 1, 64, 1), (1, 16, 0, 512, 1),
                                        (1, 1, 1 << 20, 64, 64)]:
         assert 1 <= (got := R.latent_splits(B, heads, keys, rank)) <= 64 and got == want, (B, heads, keys, rank, got)
+    for B, keys, windowed, want in [(1, 1, False, 1), (1, 501, False, 8), (1, 1024, True, 17), (96, 301, False, 5), (96, 601, False, 5),
+                                    (48, 901, False, 15), (160, 181, False, 3), (160, 1024, True, 5), (2000, 64, False, 1),
+                                    (1, 1 << 20, False, 64)]:
+        assert R.talk_splits(B, keys, windowed) == want, (B, keys, windowed)

@@ -241,13 +241,32 @@ __device__ __forceinline__ float silu(float x) {
 // g' sigmoid(1.702 g') (u' + 1) with g' = min(g, s), u' = clamp(u, -s, s).
 enum Glu : int { GLU_SILU = 0, GLU_GELU = 1, GLU_CLAMPED = 2 };
 constexpr float GLU_ALPHA = 1.702f;
-__device__ __forceinline__ float gated(float g, float u, int glu, float s) {
-  if (glu == GLU_CLAMPED) {
+template <int GLU>
+__device__ __forceinline__ float gated(float g, float u, float s) {
+  if constexpr (GLU == GLU_CLAMPED) {
     g = fminf(g, s);
     u = fminf(fmaxf(u, -s), s);
     return g * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * GLU_ALPHA * g)) * (u + 1.f);
   }
-  return (glu == GLU_GELU ? gelu_new(s * g) : silu(s * g)) * (s * u);
+  return (GLU == GLU_GELU ? gelu_new(s * g) : silu(s * g)) * (s * u);
+}
+__device__ __forceinline__ float gated(float g, float u, int glu, float s) {
+  if (glu == GLU_CLAMPED) return gated<GLU_CLAMPED>(g, u, s);
+  return glu == GLU_GELU ? gated<GLU_GELU>(g, u, s) : gated<GLU_SILU>(g, u, s);
+}
+
+// Eight of them behind one branch: with a branch each their chains (exp2, rcp) run one behind another
+// (K = 2048, 11264 columns: 96 rows 13.7 -> 13.2 us, 500 38.5 -> 35.5, 700 46.0 -> 43.0)
+__device__ __forceinline__ bf16x8 gated8(const float (&g)[8], const float (&u)[8], int glu, float s) {
+  bf16x8 o;
+  auto all = [&](auto act) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = f2bf(gated<decltype(act)::v>(g[e], u[e], s));
+  };
+  if (glu == GLU_CLAMPED) all(Int<GLU_CLAMPED>{});
+  else if (glu == GLU_GELU) all(Int<GLU_GELU>{});
+  else all(Int<GLU_SILU>{});
+  return o;
 }
 
 // Bijective XCD-aware remap of a 1-D workgroup id (guide §5.5 T1, "XCD

@@ -157,9 +157,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
       if ((ch & 3) >= 2) continue;  // up columns: 16 to the right of their gates
       float u[8];
       eight(s + 16, u);
-      bf16x8 o;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = f2bf(gated(v[e], u[e], p.glu, p.act_scale));
+      const bf16x8 o = gated8(v, u, p.glu, p.act_scale);
       st8(reinterpret_cast<bf16*>(p.out) + (long)m * p.ldo + (n >> 5) * 16 + (n & 15), o);
     } else {
       epilogue8<EPI>(p, m, n, v, split);

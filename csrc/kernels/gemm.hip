@@ -1272,6 +1272,80 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
   // stores.  (Staged in fp32, two passes of 4-byte writes, SiLU on half of the lanes, before:
   // 12032 x 11264 x 2048 with SiLU 549 -> 485 us, bf16 525 -> 518; 16000 x 6400 x 1600 with GELU
   // 322 -> 311; 7937 x 28672 x 4096 with SiLU 1500 -> 1396.)
+  // fp32 C half-tile h (128 columns, rows of both A halves), its 16-byte chunks swizzled by the row
+  float* cf = reinterpret_cast<float*>(smem);
+  auto put = [&](int h) {
+#pragma unroll
+    for (int mi = 0; mi < 8; ++mi)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int row = (mi >> 2) * 128 + wr * 64 + (mi & 3) * 16 + r, ch = wc * 8 + j * 4 + g;
+        *reinterpret_cast<f32x4*>(cf + row * 128 + ((ch ^ ((row & 7) << 1)) << 2)) = acc[mi][h * 2 + j];
+      }
+  };
+  // x += C: 512 KB a tile, which all CUs move at about the same time.  x of a half is requested before the
+  // half in front of it is stored, and no load waits for a store (as in store_pass, a half at a time, before:
+  // from a block's last product to the next one's start 19.2 -> 14.4 us of 104 at K = 4096).
+  if constexpr (EPI == EPI_RESID) {
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        reinterpret_cast<float*>(p.out) + (long)m0 * p.ldo, 0, min(p.M - m0, 256) * (int)p.ldo * 4, 0x00020000);
+    const int ch = threadIdx.x & 31, row0 = threadIdx.x >> 5;  // 16 bytes of rows row0 + 16 i
+    const int step = 64 * (int)p.ldo;
+    // of the half's row row0; out of range behind the last row or column
+    auto first = [&](int h) {
+      const int n = n0 + h * 128 + ch * 4;
+      int v = n < p.N ? (row0 * (int)p.ldo + n) * 4 : 0x7fffffff;
+      asm volatile("" : "+v"(v));  // worked out again for the stores, not kept in 16 registers
+      return (unsigned)v;
+    };
+    bf16x4 bias[2] = {};
+    if (p.bias)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) bias[h] = *reinterpret_cast<const bf16x4*>(p.bias + min(n0 + h * 128 + ch * 4, p.N - 4));
+    f32x4 x[2][16];
+    auto load = [&](int h, int i0) {
+      const unsigned v = first(h);
+#pragma unroll
+      for (int i = i0; i < i0 + 8; ++i) x[h][i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, v + i * step, 0, 0));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto add = [&](int h, int i0) {
+      const unsigned o = first(h);
+#pragma unroll
+      for (int i = i0; i < i0 + 8; ++i) {
+        const int row = row0 + 16 * i;
+        f32x4 v = *reinterpret_cast<const f32x4*>(cf + row * 128 + ((ch ^ ((row & 7) << 1)) << 2));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += bf2f(bias[h][e]);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x[h][i] + v), rs, o + i * step, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto meet = [&] {  // every wave's LDS accesses are done (__syncthreads would wait for x and the stores)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load(0, 0);
+    load(0, 8);
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(16));  // every DMA landed before C overwrites the ring
+    meet();
+    put(0);
+    meet();
+    load(1, 0);
+    add(0, 0);
+    load(1, 8);
+    add(0, 8);
+    meet();
+    put(1);
+    meet();
+    add(1, 0);
+    add(1, 8);
+    LSD_STAMP(3)
+    return;
+  }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // every DMA landed before C overwrites the ring
   __syncthreads();
   const bool slab16 = EPI == EPI_SLAB && p.slab_bf16;
@@ -1338,26 +1412,19 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
     return;
   }
   // the others: two passes over 128-column halves (nh), the fp32 C half-tile [256][128] staged
-  float* ct = reinterpret_cast<float*>(smem);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     if (h) {  // the LDS reads of pass 0 (its stores stay in flight)
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __syncthreads();
     }
-#pragma unroll
-    for (int mi = 0; mi < 8; ++mi)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int row = (mi >> 2) * 128 + wr * 64 + (mi & 3) * 16 + r, ch = wc * 8 + j * 4 + g;
-        *reinterpret_cast<f32x4*>(ct + row * 128 + ((ch ^ ((row & 7) << 1)) << 2)) = acc[mi][h * 2 + j];
-      }
+    put(h);
     __syncthreads();
     store_pass<EPI, 256 * 16 / 512, 512>(p, 256 * 16, split, [&](int c, int& m, int& n, const float*& src) {
       const int row = c >> 4, ch = c & 15;
       m = m0 + row;
       n = n0 + h * 128 + ch * 8;
-      src = ct + row * 128 + ((ch ^ (row & 7)) << 3);
+      src = cf + row * 128 + ((ch ^ (row & 7)) << 3);
       return m < p.M && n < p.N;
     });
   }
@@ -1873,7 +1940,8 @@ extern "C" void lsd_gemm_set_sk_rows(int v) { g_sk_rows = v < 16 ? 16 : (v > 128
 extern "C" hipError_t lsd_gemm(const GemmParams* p, int epi, int kind, int* cnt, float* ws,
                                hipStream_t st) {
   if (lsd_gemm_on_deep(p->M, p->N, p->K, epi, kind, p->splits)) return lsd_gemm_deep(p, epi, st);
-  const bool far = kind && far_rows(p->M, p->N, p->K, p->lda, p->ldw);
+  const bool far = kind && (far_rows(p->M, p->N, p->K, p->lda, p->ldw) ||
+                            (kind == 1 && epi == EPI_RESID && p->ldo >= 1 << 21));  // (its rows in 256 of them likewise)
 #define LSD_DISPATCH(E)                                                                   \
   case E:                                                                                 \
     if (far) return launch_far<E>(*p, st);                                                \

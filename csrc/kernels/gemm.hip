@@ -1136,7 +1136,8 @@ constexpr int P8_SMEM = 2 * P8_BUF;    // 128 KiB (== 256 x 128 fp32 C half-tile
 // 64-bit lane addresses; VAR 0 = kind 1.
 template <int EPI, int VAR = 0>
 __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m, int tiles_n, int G) {
-  __shared__ __attribute__((aligned(16))) char smem[P8_SMEM];
+  // (QKV: and the rows' positions and slots, fetched while the products run)
+  __shared__ __attribute__((aligned(16))) char smem[P8_SMEM + (EPI == EPI_QKV ? 2048 : 0)];
   const int nwg = gridDim.x;
   const int bid = xcd_remap(blockIdx.x, nwg);
   const int per_split = tiles_m * tiles_n;
@@ -1240,6 +1241,9 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
     mma(Int<10>{}, 1, 0, bx);
   };
 
+  if constexpr (EPI == EPI_QKV)
+    __builtin_amdgcn_global_load_lds((gbl_cvoid*)((w < 4 ? p.tpos : p.tslot) + min(m0 + (w & 3) * 64 + lane, p.M - 1)),
+                                     (lds_void*)(smem + P8_SMEM + w * 256), 4, 0, 0);
   if (T > 0) {
     // prologue: tile 0 and all of tile 1 but A1, in the order of the waits
     stage(0, 0, 2);
@@ -1349,14 +1353,14 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // every DMA landed before C overwrites the ring
   __syncthreads();
   const bool slab16 = EPI == EPI_SLAB && p.slab_bf16;
-  if (EPI == EPI_BF16 || EPI == EPI_GELU || EPI == EPI_SILU_MUL || slab16) {
+  if (EPI == EPI_BF16 || EPI == EPI_GELU || EPI == EPI_SILU_MUL || EPI == EPI_QKV || slab16) {
     constexpr int WC = EPI == EPI_SILU_MUL ? 128 : 256, CH = WC / 8;  // columns and chunks of a staged row
     bf16* ct = reinterpret_cast<bf16*>(smem);
     auto put = [&](int row, int col, f32x4 v) {
       st4(ct + row * WC + (((col >> 3) ^ (row & 15)) << 3) + (col & 7), pack4(v));
     };
     bf16x4 bias[2][2] = {};
-    if constexpr (EPI == EPI_BF16 || EPI == EPI_GELU) {
+    if constexpr (EPI == EPI_BF16 || EPI == EPI_GELU || EPI == EPI_QKV) {
       if (p.bias)
 #pragma unroll
         for (int nh = 0; nh < 2; ++nh)
@@ -1366,9 +1370,25 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
             if (n < p.N) bias[nh][j] = *reinterpret_cast<const bf16x4*>(p.bias + n);
           }
     }
+    // QKV likewise (staged in fp32, two passes that asked for positions, slots and turns chunk by chunk, before:
+    // from a block's last product to its last store 8.3 -> 3.6 us of 43 at K = 1600, with turns 11.8 -> 7.0 of 102
+    // at K = 4096; 16128 x 4800 x 1600 221 -> 197 us, 7937 x 6144 x 4096 318 -> 304).
+    // This thread's chunks are rows tid / CH + 512 / CH i of chunk tid % CH
+    const int cn = n0 + (threadIdx.x % CH) * 8, qk = p.q_size + p.kv_size;
+    const int* rpos = reinterpret_cast<const int*>(smem + P8_SMEM);
+    // (cos, sin) of this lane's two adjacent (even, odd) pairs of columns, which turn together; heads of
+    // 128 columns and fewer have the same ones in both halves: requested at once, in front of the staging
+    auto turns = [&](int mi, int n) {
+      int hh, d0;
+      hd_split(p.hd, min(n, qk - 4) - (n < p.q_size ? 0 : p.q_size), hh, d0);
+      const int pos = rpos[(mi >> 2) * 128 + wr * 64 + (mi & 3) * 16 + r];
+      return *reinterpret_cast<const f32x4*>(p.rope + ((long)pos * (p.hd >> 1) + (d0 >> 1)) * 2);
+    };
+    f32x4 cs[8][2];
+    const bool halves = EPI == EPI_QKV && 128 % p.hd == 0;
     // act: the gated activation, chosen outside the loops (a branch for each value made 64 chains of exp2 and
     // rcp run one behind another: from a block's last product to its last store 6.6 -> 3.4 us, of 49 at K = 2048)
-    auto fill = [&](auto act) {
+    auto fill = [&](auto act, auto rope) {
 #pragma unroll
       for (int mi = 0; mi < 8; ++mi)
 #pragma unroll
@@ -1390,15 +1410,46 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
               if constexpr (EPI == EPI_GELU)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = gelu_new(v[q]);
+              if constexpr (decltype(rope)::v != 0) {
+                const int n = n0 + nh * 128 + wc * 32 + j * 16 + 4 * g;
+                const f32x4 t = decltype(rope)::v == 1 ? cs[mi][j] : turns(mi, n);
+                const f32x4 o = {v[0] * t[0] - v[1] * t[1], v[1] * t[0] + v[0] * t[1], v[2] * t[2] - v[3] * t[3],
+                                 v[3] * t[2] + v[2] * t[3]};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = n < qk ? o[q] : v[q];
+              }
               put(row, nh * 128 + wc * 32 + j * 16 + 4 * g, v);
             }
           }
         }
     };
-    if (EPI == EPI_SILU_MUL && p.glu == GLU_CLAMPED) fill(Int<GLU_CLAMPED>{});
-    else if (EPI == EPI_SILU_MUL && p.glu == GLU_GELU) fill(Int<GLU_GELU>{});
-    else fill(Int<GLU_SILU>{});
+    if (EPI == EPI_SILU_MUL && p.glu == GLU_CLAMPED) fill(Int<GLU_CLAMPED>{}, Int<0>{});
+    else if (EPI == EPI_SILU_MUL && p.glu == GLU_GELU) fill(Int<GLU_GELU>{}, Int<0>{});
+    else if (EPI == EPI_QKV && p.rope && n0 < qk && halves) {
+#pragma unroll
+      for (int mi = 0; mi < 8; ++mi)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) cs[mi][j] = turns(mi, n0 + wc * 32 + j * 16 + 4 * g);
+      fill(Int<GLU_SILU>{}, Int<EPI == EPI_QKV>{});
+    } else if (EPI == EPI_QKV && p.rope && n0 < qk) fill(Int<GLU_SILU>{}, Int<EPI == EPI_QKV ? 2 : 0>{});
+    else fill(Int<GLU_SILU>{}, Int<0>{});
     __syncthreads();
+    if constexpr (EPI == EPI_QKV) {
+      const int c = cn < p.q_size ? 0 : cn < qk ? cn - p.q_size : cn - qk;
+      int head, d;
+      hd_split(p.hd, c, head, d);
+      bf16* cache = (cn < qk ? p.kc : p.vc) + (long)head * p.max_seq * p.hd + d;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int row = threadIdx.x / CH + 16 * i, ch = threadIdx.x % CH, m = m0 + row;
+        if (m >= p.M || cn >= p.N) continue;
+        bf16* dst = cn < p.q_size ? reinterpret_cast<bf16*>(p.out) + (long)m * p.ldo + cn
+                                  : cache + ((long)rpos[256 + row] * p.n_kv * p.max_seq + rpos[row]) * p.hd;
+        st8(dst, ld8(ct + row * WC + ((ch ^ (row & 15)) << 3)));
+      }
+      LSD_STAMP(3)
+      return;
+    }
     bf16* out = EPI == EPI_SLAB ? reinterpret_cast<bf16*>(p.slab) + (long)split * p.M * p.N : reinterpret_cast<bf16*>(p.out);
     const long ldo = EPI == EPI_SLAB ? p.N : p.ldo;
     const int c0 = EPI == EPI_SILU_MUL ? n0 / 2 : n0, cols = EPI == EPI_SILU_MUL ? p.N / 2 : p.N;

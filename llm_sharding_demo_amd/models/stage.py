@@ -179,6 +179,7 @@ class StageModel:
         pool = self.kv.pools[self._pool_index[i if m.kv_from is None else m.kv_from]]
         h = be.rmsnorm(r, w("input_layernorm.weight"), c.norm_eps, offset=1.0, width=c.hidden)
         q, gate, routing = be.latent_project(h, w, m, spec.mlp, self.kv, pool, meta, c.norm_eps)
+        routing = be.experts_ahead(h, routing, w, spec.mlp, meta)
         o = be.latent_attention(q, gate, w, m, self.kv, pool, meta)
         be.parallel_residual(o, h, routing, w, spec.mlp, r)
 

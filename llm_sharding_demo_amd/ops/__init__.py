@@ -159,6 +159,10 @@ class ReferenceBackend(Backend):
         o = o.reshape(o.shape[0], -1)
         return o if gate is None else o * torch.sigmoid(gate)
 
+    def experts_ahead(self, h, routing, w, mlp, meta):
+        """parallel_residual's routing, the experts perhaps begun beside the attention in between."""
+        return routing
+
     def parallel_residual(self, o, h, routing, w, spec, r: Residual) -> None:
         """x += o W_o^T + experts(h): both halves of a parallel block."""
         self.linear_residual(o, w("attn.o.weight"), None, r)

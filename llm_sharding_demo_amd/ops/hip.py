@@ -191,6 +191,7 @@ class HipBackend(Backend):
         self.counters = None
         self.fp32 = False  # the stage's element type (prepare_stage)
         self._rope = None
+        self._sides = {}  # lane -> the stream beside it (experts_ahead)
         self.lane = 0  # microbatch lane (stream) currently being issued; see pipeline.py
         self.concurrency = 1  # microbatch lanes running at once (set per round by the pipeline)
 
@@ -943,6 +944,28 @@ class HipBackend(Backend):
         for heads in {l.mixer.heads for l in mcfg.layers if isinstance(l.mixer, LatentAttentionSpec)}:
             self._latent_tiles(meta, heads, 128, meta.cu_q.device)
 
+    def experts_ahead(self, h, routing, w, mlp, meta):
+        """Experts on a stream of their own while the attention of the same rows runs: in a captured decode step
+        (launches one by one would cost the host more than this gives) with the chip to itself.  A step's
+        experts wait for the memory, its attention for itself: 8 sequences of up to 1000 tokens 861 -> 770 us,
+        64 of 300 1059 -> 1018, 160 of 250 1248 -> 1185.  The rows are allocated on that stream: whatever else gets
+        them from its pool runs behind the next layer's fork, so behind this layer's norm."""
+        if mlp is None or self.fp32 or not meta.is_decode or h.shape[0] <= self.R.moe_few_t or self.concurrency > 1 \
+                or not torch.cuda.is_current_stream_capturing():
+            return routing
+        (T, H), wo = h.shape, w("attn.o.weight")
+        so = self._slab_splits(torch.empty(T, wo.shape[1], dtype=h.dtype, device="meta"), wo)
+        if not self.C.gemm_slab_bf16():
+            so = 0  # as in parallel_residual
+        if self.lane not in self._sides:
+            self._sides[self.lane] = torch.cuda.Stream(h.device)
+        side = self._sides[self.lane]
+        side.wait_stream(torch.cuda.current_stream(h.device))
+        with torch.cuda.stream(side):
+            slab = torch.empty(so + mlp.top + (mlp.shared is not None), T, H, dtype=h.dtype, device=h.device)
+            self._moe(h, *routing, w, mlp, slab[so:], None)
+        return *routing, (slab, so, side)
+
     def parallel_residual(self, o, h, routing, w, mlp, r: Residual) -> None:
         """x += o W_o^T + experts(h).  Everything that is not added in place --
         split-K partials of the out-projection, one row set per chosen expert
@@ -950,6 +973,12 @@ class HipBackend(Backend):
         wo = w("attn.o.weight")
         if mlp is None:
             self.linear_residual(o, wo, None, r)
+            return
+        if len(routing) == 3:  # experts_ahead
+            slab, so, side = routing[2]
+            self.linear_residual(o, wo, None, r, slab[:so] if so else None)
+            torch.cuda.current_stream(h.device).wait_stream(side)
+            r.pending.append((slab, None))
             return
         ids, wts = routing
         T, H = h.shape

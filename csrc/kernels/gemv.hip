@@ -30,6 +30,9 @@
 #include "gemm_params.h"
 
 namespace lsd {
+
+// y cos -+ z sin, rounded alike wherever it is inlined: a row's bits do not depend on its kernel
+__device__ __forceinline__ float turned(float y, float z, float c, float s, bool odd) { return fmaf(y, c, odd ? z * s : -(z * s)); }
 namespace gv {
 enum : int { BF16 = 0, GELU = 1, SILU = 2, F32 = 3, RESID = 4, QKV = 6 };
 enum : int { NONE = 0, LN = 1, RMS = 2 };
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
             // rope_pair_permutation makes the rotated pairs adjacent)
             const float yp = rv[(j ^ 1) * MR + m] + e_biasp;
             const int d = (n < p.q_size ? n : n - p.q_size) % p.hd;
-            y = (d & 1) ? (y * e_cs0 + yp * e_cs1) : (y * e_cs0 - yp * e_cs1);
+            y = turned(y, yp, e_cs0, e_cs1, d & 1);
           }
           if (n < p.q_size) {
             reinterpret_cast<bf16*>(p.out)[(long)m * p.ldo + n] = f2bf(y);
@@ -467,7 +470,7 @@ __global__ __launch_bounds__(256, 2) void gemv_stream_kernel(GemvParams p) {
     } else if constexpr (EPI == gv::QKV) {
       if ((lane & 31) == 0) {  // (an even number of columns: heads of even dims)
         const int qk = p.q_size + p.kv_size;
-        if (p.rope != nullptr && c < qk) y = idx ? y * e_cs0 + z * e_cs1 : y * e_cs0 - z * e_cs1;
+        if (p.rope != nullptr && c < qk) y = turned(y, z, e_cs0, e_cs1, idx);
         if (c < p.q_size) {
           reinterpret_cast<bf16*>(p.out)[c] = f2bf(y);
         } else {

@@ -1141,14 +1141,18 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
   const int nwg = gridDim.x;
   const int bid = xcd_remap(blockIdx.x, nwg);
   const int per_split = tiles_m * tiles_n;
-  const int split = bid / per_split;
+  const int KT = p.K / 64;
+  int split = 0, tile_id = bid, kb = 0, T = KT;  // K-tiles of this split
+  if (p.splits > 1) {  // (its 64-bit divisions stood in front of every tile's first load: 0.25 us of some 40)
+    split = bid / per_split;
+    tile_id = bid % per_split;
+    kb = (int)((long)KT * split / p.splits);
+    T = (int)((long)KT * (split + 1) / p.splits) - kb;
+  }
   int tm, tn;
-  tile_order(bid % per_split, tiles_m, tiles_n, G, tm, tn);
+  tile_order(tile_id, tiles_m, tiles_n, G, tm, tn);
   const int m0 = tm * 256, n0 = tn * 256;
   LSD_STAMP(0)
-  const int KT = p.K / 64;
-  const int kb = (int)((long)KT * split / p.splits);
-  const int T = (int)((long)KT * (split + 1) / p.splits) - kb;  // K-tiles of this split
 
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = w >> 2, wc = w & 3;

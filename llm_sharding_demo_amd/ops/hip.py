@@ -192,6 +192,7 @@ class HipBackend(Backend):
         self.fp32 = False  # the stage's element type (prepare_stage)
         self._rope = None
         self._sides = {}  # lane -> the stream beside it (experts_ahead)
+        self._beside = False  # whether a layer's experts run there
         self.lane = 0  # microbatch lane (stream) currently being issued; see pipeline.py
         self.concurrency = 1  # microbatch lanes running at once (set per round by the pipeline)
 
@@ -885,7 +886,8 @@ class HipBackend(Backend):
         q = self._batch_linear(q, uk)
         if meta.is_decode or self.fp32 or rows == 0:
             # one query per sequence, or the kernel that takes any token alone
-            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2])
+            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2],
+                                          self._beside)
             o = self.C.latent_decode(q, pool, kv.table, meta.token_slots, meta.token_pos, m.heads, window, m.scale,
                                      splits, *beside)
         else:
@@ -961,6 +963,7 @@ class HipBackend(Backend):
             self._sides[self.lane] = torch.cuda.Stream(h.device)
         side = self._sides[self.lane]
         side.wait_stream(torch.cuda.current_stream(h.device))
+        self._beside = True
         with torch.cuda.stream(side):
             slab = torch.empty(so + mlp.top + (mlp.shared is not None), T, H, dtype=h.dtype, device=h.device)
             self._moe(h, *routing, w, mlp, slab[so:], None)
@@ -978,6 +981,7 @@ class HipBackend(Backend):
             slab, so, side = routing[2]
             self.linear_residual(o, wo, None, r, slab[:so] if so else None)
             torch.cuda.current_stream(h.device).wait_stream(side)
+            self._beside = False
             r.pending.append((slab, None))
             return
         ids, wts = routing

@@ -391,11 +391,13 @@ class Routing:
         expanded = keys * (dim + vdim) + rank * (dim + vdim) * rows / T
         return expanded * 1.25 < latent
 
-    def latent_splits(self, B: int, heads: int, keys: int, rank: int) -> int:
+    def latent_splits(self, B: int, heads: int, keys: int, rank: int, beside: bool = False) -> int:
         """Context splits of a latent decode launch: the least of what a block's steps
         take, more where two share a CU, and the merge of the parts.  rank 512, us, for
         splits 1 / 2 / 4 / 8: 64 sequences of 300 keys 16.0 / 15.8 / 15.4 / 19.3, 24 of 470 22 / 17 / 13.1 /
-        12.7, 96 of 250 13.8 / 15.4 / 17.6 / 24, 160 of 250 13.9 / 21 / 24 / 31."""
+        12.7, 96 of 250 13.8 / 15.4 / 17.6 / 24, 160 of 250 13.9 / 21 / 24 / 31.  beside: experts run at the
+        same time, so a merge and its bytes weigh twice (a timisun-2b step, splits 1 / 2 / 4 / 8: 64 sequences of
+        300 keys 994 / 1006 / 1023 / 1048, 24 of 1024 1011 / 942 / 921 / 925, 64 of 1000 1071 / 1041 / 1053 / 1071)."""
         items = B * -(-heads // 16)
         steps = max(1, -(-keys // (64 if rank >= 320 else 128)))  # keys a block takes at a time
         best, least = 1, 0.0
@@ -406,7 +408,7 @@ class Routing:
             share = -(-items * s // 256)  # blocks a CU
             cost = (0.6 + 0.003 * rank) * (1 if share <= 1 else 0.35 + 0.65 * share) * -(-steps // s)
             if s > 1:
-                cost += 3 + 1.6e-6 * B * heads * rank * s
+                cost += (3 + 1.6e-6 * B * heads * rank * s) * (2 if beside else 1)
             if k == steps or cost < least:
                 best, least = s, cost
         return best

@@ -31,7 +31,9 @@ def test_rule():
                                        (64, 16, 301, 512, 3), (96, 16, 251, 512, 1), (160, 16, 251, 512, 1), (160, 16, 2001, 512, 3),
                                        (64, 64, 301, 576, 1), (1, 16, 251, 256, 1), (16, 16, 501, 256, 4), (1, 1, 1, 64, 1), (1, 16, 0, 512, 1),
                                        (1, 1, 1 << 20, 64, 64)]:
-        assert 1 <= (got := R.latent_splits(B, heads, keys, rank)) <= 64 and got == want, (B, heads, keys, rank, got)
+        assert R.latent_splits(B, heads, keys, rank) == want, (B, heads, keys, rank)
+    for B, keys, want in [(64, 301, 1), (24, 1024, 8), (5, 1024, 16), (64, 1001, 4), (160, 251, 1), (1, 1, 1)]:
+        assert R.latent_splits(B, 16, keys, 512, True) == want, (B, keys)
     for B, keys, windowed, want in [(1, 1, False, 1), (1, 501, False, 8), (1, 1024, True, 17), (96, 301, False, 5), (96, 601, False, 5),
                                     (48, 901, False, 15), (160, 181, False, 3), (160, 1024, True, 5), (2000, 64, False, 1),
                                     (1, 1 << 20, False, 64)]:

@@ -1417,8 +1417,9 @@ __global__ __launch_bounds__(512) void gemm_p8_kernel(GemmParams p, int tiles_m,
               if constexpr (decltype(rope)::v != 0) {
                 const int n = n0 + nh * 128 + wc * 32 + j * 16 + 4 * g;
                 const f32x4 t = decltype(rope)::v == 1 ? cs[mi][j] : turns(mi, n);
-                const f32x4 o = {v[0] * t[0] - v[1] * t[1], v[1] * t[0] + v[0] * t[1], v[2] * t[2] - v[3] * t[3],
-                                 v[3] * t[2] + v[2] * t[3]};
+                float o[4] = {v[0], v[1], v[2], v[3]};
+                turn_pair(o[0], o[1], t[0], t[1]);
+                turn_pair(o[2], o[3], t[2], t[3]);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = n < qk ? o[q] : v[q];
               }

@@ -123,6 +123,14 @@ __device__ __forceinline__ void epilogue4(const GemmParams& p, int row0, int n, 
   }
 }
 
+// (a, b) turned by (cos, sin) = (c, s).  Which product is fused is said here, and alike for every tile: left to the
+// compiler, a row's queries and keys differed in their last bits with the kernel that its launch took.
+__device__ __forceinline__ void turn_pair(float& a, float& b, float c, float s) {
+  const float t = fmaf(a, c, -(b * s));
+  b = fmaf(a, s, b * c);
+  a = t;
+}
+
 // Row-contiguous epilogue of 8 consecutive columns [n, n+8) of row m (the
 // tiled kernel's LDS-transposed output): every store is one 16-byte vector.
 // n % 8 == 0; bias / out / x / caches are 16-byte aligned (host-checked).
@@ -228,12 +236,7 @@ __device__ __forceinline__ void epi8_post(const GemmParams& p, int m, int n, con
       for (int h = 0; h < 2; ++h) {
         const f32x4 t = h ? e.cs1 : e.cs0;  // (cos, sin) of pairs d0/2 + 2h, d0/2 + 2h + 1
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const float c = t[2 * q], sn = t[2 * q + 1];
-          const float a = y[4 * h + 2 * q], b = y[4 * h + 2 * q + 1];
-          y[4 * h + 2 * q] = a * c - b * sn;
-          y[4 * h + 2 * q + 1] = b * c + a * sn;
-        }
+        for (int q = 0; q < 2; ++q) turn_pair(y[4 * h + 2 * q], y[4 * h + 2 * q + 1], t[2 * q], t[2 * q + 1]);
       }
     }
     bf16x8 o;

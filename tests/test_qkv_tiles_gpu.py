@@ -47,3 +47,34 @@ def test_qkv(M, rope, heads, kv, hd, kind):
     for t in (kc, vc):  # nothing else is written
         t[slot.long(), :, pos.long()] = 0
         assert int(t.count_nonzero()) == 0
+
+
+@pytest.mark.parametrize("M,kind,big", [(1000, 2, None), (1000, 3, None), (2000, 1, None), (2000, 1, 0), (2000, 1, 1), (2000, 1, 4)])
+@pytest.mark.parametrize("heads,kv,hd", [(6, 2, 128), (3, 1, 256), (7, 2, 96)])
+def test_turns_are_rounded_alike(M, kind, big, heads, kv, hd):
+    """Sums of small whole numbers are exact, so a turned pair is a cos - (b sin), a sin + (b cos) to the bit, each
+    bracket rounded by itself: the same from every kernel of tiles (kind 1: 256 x 256, 128 x 128 with big None)."""
+    from llm_sharding_demo_amd import _C as C
+
+    K, N, seq = 128, (heads + 2 * kv) * hd, 64
+    g = torch.Generator(device=DEV).manual_seed(M + hd)
+    a, w = (torch.randint(-9, 10, s, generator=g, device=DEV).bfloat16() for s in ((M, K), (N, K)))
+    kc, vc = (torch.zeros(M, kv, seq, hd, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    slot, pos = torch.arange(M, device=DEV).int(), (torch.arange(M, device=DEV) * 7 % seq).int()
+    angle = torch.rand(seq, hd // 2, generator=g, device=DEV) * 6.3
+    table = torch.stack([angle.cos(), angle.sin()], -1).contiguous()
+    C.gemm_set_big_min(1 << 30 if big is None else 1)
+    C.gemm_set_big_kind(4 if big is None else big)
+    try:
+        assert kind != 1 or C.gemm_big_tiles(M, N, K, 1) == (big is not None)
+        q = C.linear_qkv(a, w, None, kc, vc, slot, pos, heads * hd, kv * hd, hd, table, kind, 1,
+                         torch.zeros(1 << 16, dtype=torch.int32, device=DEV))
+    finally:
+        C.gemm_set_big_kind(4)
+        C.gemm_set_big_min(160)
+    y = (a.cpu().to(F64) @ w.cpu().to(F64).T)[:, : (heads + kv) * hd].reshape(M, heads + kv, hd // 2, 2)
+    c, s = (table.cpu()[pos.cpu().long()].to(F64)[:, None, :, i] for i in (0, 1))
+    x, z = y[..., 0], y[..., 1]
+    want = torch.stack([x * c - (z * s).float(), x * s + (z * c).float()], -1).float().bfloat16().reshape(M, -1)
+    got = torch.cat([q.cpu(), kc.cpu()[slot.cpu().long(), :, pos.cpu().long()].reshape(M, -1)], 1)
+    assert torch.equal(got, want)

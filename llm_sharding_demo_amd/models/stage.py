@@ -180,7 +180,7 @@ class StageModel:
         h = be.rmsnorm(r, w("input_layernorm.weight"), c.norm_eps, offset=1.0, width=c.hidden)
         q, gate, routing = be.latent_project(h, w, m, spec.mlp, self.kv, pool, meta, c.norm_eps)
         routing = be.experts_ahead(h, routing, w, spec.mlp, meta)
-        o = be.latent_attention(q, gate, w, m, self.kv, pool, meta)
+        o = be.latent_attention(q, gate, w, m, self.kv, pool, meta, spec.mlp)
         be.parallel_residual(o, h, routing, w, spec.mlp, r)
 
     # Vizalix: mixer and feed-forward of the same residual, each behind a norm

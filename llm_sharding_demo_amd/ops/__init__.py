@@ -150,7 +150,8 @@ class ReferenceBackend(Backend):
             routing = ref.route(z, w("mlp.correction"), mlp.top)
         return q, gate, routing
 
-    def latent_attention(self, q, gate, w, m, kv, pool, meta):
+    def latent_attention(self, q, gate, w, m, kv, pool, meta, mlp=None):
+        """mlp: the experts that read the same rows."""
         sink = w("attn.sink").float() if m.sink else None
         o = torch.cat([ref.latent_attention(q[s], pool, kv.table, mt.seq_slots, mt.q_start, mt.cu_q, m.scale, m.window,
                                             m.kv_rank, sink) for s, mt in self._parts(meta)])

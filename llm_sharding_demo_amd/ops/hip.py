@@ -192,7 +192,6 @@ class HipBackend(Backend):
         self.fp32 = False  # the stage's element type (prepare_stage)
         self._rope = None
         self._sides = {}  # lane -> the stream beside it (experts_ahead)
-        self._beside = False  # whether a layer's experts run there
         self.lane = 0  # microbatch lane (stream) currently being issued; see pipeline.py
         self.concurrency = 1  # microbatch lanes running at once (set per round by the pipeline)
 
@@ -869,11 +868,13 @@ class HipBackend(Backend):
                 q = self.C.latent_post(q, m.heads * dp, True, self.fp32, None, 0, None, eps, None, *where, None, 0, **turn)[0]
         return (y if keep else q), (y[:, nq: nq + ng] if m.gate else None), (ids, wts)
 
-    def latent_attention(self, q, gate, w, m, kv, pool, meta):
-        o = [self._latent_part(q[s], None if gate is None else gate[s], w, m, kv, pool, mt) for s, mt in self._parts(meta)]
+    def latent_attention(self, q, gate, w, m, kv, pool, meta, mlp=None):
+        at = w, m, kv, pool
+        ahead = self._may_run_ahead(q.shape[0], mlp, meta)
+        o = [self._latent_part(q[s], None if gate is None else gate[s], *at, mt, ahead) for s, mt in self._parts(meta)]
         return o[0] if len(o) == 1 else torch.cat(o)  # mixed step: each part its own kernel
 
-    def _latent_part(self, q, gate, w, m, kv, pool, meta):
+    def _latent_part(self, q, gate, w, m, kv, pool, meta, ahead):
         window = m.window or 1 << 30
         beside = (m.kv_rank, w("attn.sink") if m.sink else None)
         uk, uv = w("attn.uk.weight"), w("attn.uv.weight")
@@ -886,8 +887,7 @@ class HipBackend(Backend):
         q = self._batch_linear(q, uk)
         if meta.is_decode or self.fp32 or rows == 0:
             # one query per sequence, or the kernel that takes any token alone
-            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2],
-                                          self._beside)
+            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2], ahead)
             o = self.C.latent_decode(q, pool, kv.table, meta.token_slots, meta.token_pos, m.heads, window, m.scale,
                                      splits, *beside)
         else:
@@ -946,14 +946,21 @@ class HipBackend(Backend):
         for heads in {l.mixer.heads for l in mcfg.layers if isinstance(l.mixer, LatentAttentionSpec)}:
             self._latent_tiles(meta, heads, 128, meta.cu_q.device)
 
+    def _may_run_ahead(self, rows: int, mlp, meta) -> bool:
+        """Whether a captured step of these rows begins its experts ahead of the attention where no other lane is at
+        work.  What the attention does differently then (latent_splits) hangs on this alone, so an eager
+        step, a captured one and one beside another lane add up alike."""
+        return mlp is not None and not self.fp32 and meta.is_decode and rows > self.R.moe_few_t
+
     def experts_ahead(self, h, routing, w, mlp, meta):
         """Experts on a stream of their own while the attention of the same rows runs: in a captured decode step
-        (launches one by one would cost the host more than this gives) with the chip to itself.  A step's
+        (launches one by one would cost the host more than this gives) beside no other lane.  A step's
         experts wait for the memory, its attention for itself: 8 sequences of up to 1000 tokens 861 -> 770 us,
-        64 of 300 1059 -> 1018, 160 of 250 1248 -> 1185.  The rows are allocated on that stream: whatever else gets
-        them from its pool runs behind the next layer's fork, so behind this layer's norm."""
-        if mlp is None or self.fp32 or not meta.is_decode or h.shape[0] <= self.R.moe_few_t or self.concurrency > 1 \
-                or not torch.cuda.is_current_stream_capturing():
+        64 of 300 1059 -> 1018, 160 of 250 1248 -> 1185; two stages on one GPU, 4 groups of 16 sequences, 64 tokens
+        203 -> 200 ms.  The rows are allocated on that stream: whatever else gets them from its pool runs behind the
+        next layer's fork, so behind this layer's norm."""
+        rows = h.shape[0]
+        if not self._may_run_ahead(rows, mlp, meta) or self.concurrency > 1 or not torch.cuda.is_current_stream_capturing():
             return routing
         (T, H), wo = h.shape, w("attn.o.weight")
         so = self._slab_splits(torch.empty(T, wo.shape[1], dtype=h.dtype, device="meta"), wo)
@@ -963,7 +970,6 @@ class HipBackend(Backend):
             self._sides[self.lane] = torch.cuda.Stream(h.device)
         side = self._sides[self.lane]
         side.wait_stream(torch.cuda.current_stream(h.device))
-        self._beside = True
         with torch.cuda.stream(side):
             slab = torch.empty(so + mlp.top + (mlp.shared is not None), T, H, dtype=h.dtype, device=h.device)
             self._moe(h, *routing, w, mlp, slab[so:], None)
@@ -981,7 +987,6 @@ class HipBackend(Backend):
             slab, so, side = routing[2]
             self.linear_residual(o, wo, None, r, slab[:so] if so else None)
             torch.cuda.current_stream(h.device).wait_stream(side)
-            self._beside = False
             r.pending.append((slab, None))
             return
         ids, wts = routing

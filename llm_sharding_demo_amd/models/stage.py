@@ -183,6 +183,12 @@ class StageModel:
         o = be.latent_attention(q, gate, w, m, self.kv, pool, meta, spec.mlp)
         be.parallel_residual(o, h, routing, w, spec.mlp, r)
 
+    def runs_ahead(self, rows: int) -> bool:
+        """Whether a decode step of `rows` rows captured now has launches beside one another that one
+        captured beside another lane has not."""
+        return (self.cfg.arch == "timisun" and any(self.cfg.layers[i].mlp is not None for i in self.layers)
+                and self.backend.runs_ahead(rows))
+
     # Vizalix: mixer and feed-forward of the same residual, each behind a norm
     # with one number for a gain -- applied after the projections that follow,
     # so both read the same normed rows

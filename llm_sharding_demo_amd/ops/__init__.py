@@ -164,6 +164,10 @@ class ReferenceBackend(Backend):
         """parallel_residual's routing, the experts perhaps begun beside the attention in between."""
         return routing
 
+    def runs_ahead(self, rows: int) -> bool:
+        """Whether experts_ahead begins the experts of a captured step of `rows` rows, as things are."""
+        return False
+
     def parallel_residual(self, o, h, routing, w, spec, r: Residual) -> None:
         """x += o W_o^T + experts(h): both halves of a parallel block."""
         self.linear_residual(o, w("attn.o.weight"), None, r)

@@ -952,6 +952,9 @@ class HipBackend(Backend):
         step, a captured one and one beside another lane add up alike."""
         return mlp is not None and not self.fp32 and meta.is_decode and rows > self.R.moe_few_t
 
+    def runs_ahead(self, rows: int) -> bool:
+        return not self.fp32 and rows > self.R.moe_few_t and self.concurrency == 1
+
     def experts_ahead(self, h, routing, w, mlp, meta):
         """Experts on a stream of their own while the attention of the same rows runs: in a captured decode step
         (launches one by one would cost the host more than this gives) beside no other lane.  A step's
@@ -960,7 +963,7 @@ class HipBackend(Backend):
         203 -> 200 ms.  The rows are allocated on that stream: whatever else gets them from its pool runs behind the
         next layer's fork, so behind this layer's norm."""
         rows = h.shape[0]
-        if not self._may_run_ahead(rows, mlp, meta) or self.concurrency > 1 or not torch.cuda.is_current_stream_capturing():
+        if not (self._may_run_ahead(rows, mlp, meta) and self.runs_ahead(rows) and torch.cuda.is_current_stream_capturing()):
             return routing
         (T, H), wo = h.shape, w("attn.o.weight")
         so = self._slab_splits(torch.empty(T, wo.shape[1], dtype=h.dtype, device="meta"), wo)

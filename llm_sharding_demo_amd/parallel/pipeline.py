@@ -410,6 +410,10 @@ class StageWorker(racecheck.Shared):
         return (self.graph_io and self.use_graphs and gp.kind != "fwd_b" and gp.b > 0
                 and not gp.chunks and self.P > 1)
 
+    def _graph_key(self, gp: GroupPlan, io: bool) -> tuple:
+        """What a captured decode step depends on: its sizes, its transfers, and what it overlaps alone only."""
+        return gp.b, gp.ctxb, io, self.stage.runs_ahead(gp.b)
+
     def on_lane(self, g: int):
         if not self.lanes:
             return contextlib.nullcontext()
@@ -605,7 +609,7 @@ class StageWorker(racecheck.Shared):
             if self.P > 1 and not io:
                 return False
             gs = self.groups[gp.g]
-            key = (gp.b, gp.ctxb, io)
+            key = self._graph_key(gp, io)
             ent = gs.graphs.get(key)
             if ent is None:
                 return False
@@ -1237,7 +1241,7 @@ class StageWorker(racecheck.Shared):
         slot[2] = True
 
     def _decode(self, gp: GroupPlan, gs: GroupState, inp: torch.Tensor, io: bool = False) -> torch.Tensor:
-        key = (gp.b, gp.ctxb, io)
+        key = self._graph_key(gp, io)
         lane = self.lane_of(gp.g)
 
         def body():

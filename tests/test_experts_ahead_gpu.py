@@ -79,3 +79,23 @@ def test_parts_are_those_of_eager_steps(seqs, tmp_path):
     assert eng.stages[0].backend._sides and bool(spies[1].slabs) == (seqs > 8)  # (up to 8 rows are added by a GEMV)
     parts = [set(s.parts) for s in spies]
     assert parts[0] == parts[1] and max(p for _, p in parts[0]) > 1
+
+
+def test_graphs_of_two_lanes(tmp_path):
+    """Steps with the chip to themselves and steps beside another lane have graphs of their own, also of one size."""
+    from llm_sharding_demo_amd.config import SamplingParams
+
+    path = str(tmp_path)
+    cfg = wide_model(path, heads=4, rank=192)
+    room = dict(max_batch=16, max_seq_len=192, kv_tokens=192 * 16, num_microbatches=2)
+    prompts = [ids_of(20 + i, cfg["vocab"], i) for i in range(16)]
+    sps = [SamplingParams(temperature=0.8, top_k=20, seed=5, max_new_tokens=n) for n in (60, 20)]
+    eager, eng = make_engine(path, "bf16", use_graphs=False, **room), make_engine(path, "bf16", **room)
+    for order in ([0] * 8 + [1] * 8, [0, 1] * 8):
+        args = prompts, [sps[i] for i in order]
+        want = eager.generate_ids(*args)
+        for _ in range(2):
+            assert eng.generate_ids(*args) == want
+    keys = [k for gs in eng.workers[0].groups.values() for k in gs.graphs]
+    alone = {k[:3] for k in keys if k[3]}
+    assert alone & {k[:3] for k in keys if not k[3]}

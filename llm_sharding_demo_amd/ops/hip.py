@@ -969,10 +969,11 @@ class HipBackend(Backend):
         so = self._slab_splits(torch.empty(T, wo.shape[1], dtype=h.dtype, device="meta"), wo)
         if not self.C.gemm_slab_bf16():
             so = 0  # as in parallel_residual
-        if self.lane not in self._sides:
-            self._sides[self.lane] = torch.cuda.Stream(h.device)
-        side = self._sides[self.lane]
-        side.wait_stream(torch.cuda.current_stream(h.device))
+        cur = torch.cuda.current_stream(h.device)
+        side = self._sides.get(self.lane)
+        while side is None or side == cur:  # (streams come round in a pool, the capturing one too)
+            side = self._sides[self.lane] = torch.cuda.Stream(h.device)
+        side.wait_stream(cur)
         with torch.cuda.stream(side):
             slab = torch.empty(so + mlp.top + (mlp.shared is not None), T, H, dtype=h.dtype, device=h.device)
             self._moe(h, *routing, w, mlp, slab[so:], None)

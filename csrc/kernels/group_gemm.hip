@@ -557,7 +557,8 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
 // 2048 x 1024 and 565 through a shared one of 2048 up 325 -> 244, down 152 -> 121.  Splitting W a k-step
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
 // A tile with an operand of 2^56 or more, a sum that is not finite, or one that is not zero but below 2^-40
-// is computed again by fp32 MFMAs: terms that left the range of bf16's normal numbers matter there alone.
+// is computed again by fp32 MFMAs, in the order of the kernel above: terms that left the range of bf16's normal
+// numbers matter there alone.
 template <int MODE, int MT, int WN, int WK, int D>
 __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
@@ -664,16 +665,18 @@ __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_
 #pragma unroll 1
     for (int i = 0; i < live; ++i) {
       const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;
-      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll 1
-      for (int k = 0; k < T * BKF; k += 16) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(a + k), wv = *reinterpret_cast<const f32x4*>(wp + k);
+      for (int k = 0; k < T * BKF; k += BKF)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s, 0, 0, 0);
-      }
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 av = *reinterpret_cast<const f32x4*>(a + k + 16 * h), wv = *reinterpret_cast<const f32x4*>(wp + k + 16 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[h], 0, 0, 0);
+        }
 #pragma unroll
       for (int h = 0; h < MT; ++h)
-        if (h == i) acc[0][h] = s;
+        if (h == i) acc[0][h] = s[0] + s[1];
     }
   }
   float* ct = reinterpret_cast<float*>(smem);

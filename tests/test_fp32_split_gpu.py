@@ -94,3 +94,20 @@ def test_experts(C, T, E):  # noqa: F811
         assert float((slab[e % top, e // top].cpu().to(F64) - y).abs().max()) < 1e-5 * max(1.0, float(y.abs().max()))
     y = mids.cpu().to(F64) @ shared_dn.to(F64).T
     assert float((slab[top].cpu().to(F64) - y).abs().max()) < 1e-5 * float(y.abs().max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,tile", [(193, 3264, (48, 64, 4)), (961, 2048, (64, 128, 1)), (561, 4160, (96, 128, 1))])
+def test_recomputed_sums(C, M, N, tile):  # noqa: F811
+    """A tile with a value past the terms' range is summed as few rows are, by fp32 MFMAs in two chains: to the bit where
+    a block has all of K."""
+    a, w = rand(M, 576, seed=1), rand(N, 576, seed=2)
+    assert C.fp32_tile(M, N) == tile
+    few = C.linear_fp32(a[:16].to(DEV), w.to(DEV)).cpu()
+    a[9, 3] = 2.0 ** 60
+    got = C.linear_fp32(a.to(DEV), w.to(DEV)).cpu()[:16]
+    got[9] = few[9]
+    if tile[2] == 1:
+        assert torch.equal(got, few)
+    else:
+        assert bool(((got - few).abs() <= 580 * ULP * (a[:16].abs() @ w.abs().T)).all())

@@ -556,9 +556,9 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
 // 2048 63 -> 49, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 286; 2260 rows over 32 experts of
 // 2048 x 1024 and 565 through a shared one of 2048 up 325 -> 244, down 152 -> 121.  Splitting W a k-step
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
-// A tile with an operand of 2^56 or more, a sum that is not finite, or one that is not zero but below 2^-40
-// is computed again by fp32 MFMAs, in the order of the kernel above: terms that left the range of bf16's normal
-// numbers matter there alone.
+// Terms behind bf16's numbers are lost: of an operand, 2^-134 at most.  Where that may count the tile is computed
+// again by fp32 MFMAs, in the order of the kernel above: an operand of 2^56 or more, a sum that is not finite, one
+// below 2^-40, zeros among them unless their column of W is zero (padding).
 template <int MODE, int MT, int WN, int WK, int D>
 __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
@@ -658,10 +658,31 @@ __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float v = fabsf(acc[0][i][q]);
-      exact |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
+      exact |= !(v < INFINITY) || (v < 0x1p-40f && (MODE == GG_F32 || MODE == GG_ADD || i < live));
     }
   }
-  if (__syncthreads_or(exact)) {
+  exact = __syncthreads_or(exact);
+  if (exact) {  // for zeros alone only where the column of W has values
+    int mine = 0, some = big >= 0x1p56f;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v = fabsf(acc[0][i][q]);
+        mine |= v == 0.f && i < live;
+        some |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
+      }
+    mine |= __shfl_xor(mine, 16);
+    mine |= __shfl_xor(mine, 32);
+    if (mine)
+#pragma unroll 4
+      for (int k = 0; k < T * BKF; k += 16) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(wp + k);
+        some |= v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f;
+      }
+    exact = __syncthreads_or(some);
+  }
+  if (exact) {
 #pragma unroll 1
     for (int i = 0; i < live; ++i) {
       const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;

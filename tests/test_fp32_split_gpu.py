@@ -111,3 +111,16 @@ def test_recomputed_sums(C, M, N, tile):  # noqa: F811
         assert torch.equal(got, few)
     else:
         assert bool(((got - few).abs() <= 580 * ULP * (a[:16].abs() @ w.abs().T)).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(70, 100), (300, 2048), (561, 2560)])
+def test_operands_behind_the_terms(C, M, N):  # noqa: F811
+    """Operands without a bf16 term, in rows of their own: the sums are zero until they are computed again; columns
+    of zeros stay zeros."""
+    a, w = rand(M, 576, seed=1).clamp(-1, 1), rand(N, 576, seed=2) * 2.0 ** 50
+    a[::3] *= 2.0 ** -140
+    w[5:90:7] = 0
+    assert int(a[::3].count_nonzero()) > 100 and float(a[::3].abs().max()) < 2.0 ** -134
+    got = C.linear_fp32(a.to(DEV), w.to(DEV))
+    assert near(got, a, w) and int(got[:, 5:90:7].count_nonzero()) == 0 and int(got[::3, :5].count_nonzero()) > 0

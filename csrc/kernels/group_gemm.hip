@@ -969,13 +969,35 @@ static int split_tile(const GgParams& p) {
 
 // Products on split operands: experts from 18 rows a tile of the table on (2048 x 1024, 4 of 32 experts:
 // 300 tokens, 24 rows, up 185 us either way, down 93; 200, 18 rows, 161 -> 149, 78 -> 68; 160, 15 rows, 139
-// and 160, 71 and 77; 2 of 16 of 1024 x 512: 200, 18 rows, 38 -> 31).  Others with more than 16 rows, unless the few are
+// and 160, 71 and 77; 2 of 16 of 1024 x 512: 200, 18 rows, 38 -> 31), short K from 28 (1024 x 512, 4 of 32: 200 tokens,
+// 18 rows, K = 128 10.8 and 14.2, 256 15.7 and 19.0, 384 24.0 either way, 512 28.1 and 26.6; 565, 34 rows, 128 18.7
+// and 15.9), where the fp32 tiles, half as wide, are one a CU and more (2 of 8, 200 tokens, 224 tiles: K = 128 7.1 and
+// 9.9, 512 14.4 and 17.6, 1536 35.5 and 41.4; 2 of 8 of 256 x 128, 1000 tokens, 9.2 and 11.9; 2 of 8 of 2048 x 1024, 120
+// tokens, 256 tiles, 67 and 51).
+// Others with more than 16 rows, unless the few are
 // bound by the weights' stream (20 rows of 32000 x 2048 42 us and 50, of 16384 31.1 and 27.5) or K is short for the
 // splitting to hide (565 rows of 2048, K = 256 12.2 and 12.8, 512 19.2 and 17.9; of 4096, K = 512 31.4 and 32.9;
-// 100 rows of 2048, K = 512 10.6 and 11.1, 2048 28.7 and 22.9).
-static bool on_split(const GgParams& p, bool experts) {
-  if (experts) return (long)p.T * p.top >= 18L * p.n_tiles;
-  return p.K > 512 && p.M > 16 && !(p.M <= 32 && gg_blocks(p, GG_F32, 32, 64) > 256);
+// 100 rows of 2048, K = 512 10.6 and 11.1, 2048 28.7 and 22.9), up to 768 where the fp32 tiles fill the chip once (24 rows:
+// K = 640, N = 6144 11.3 and 11.0, 11264 12.1 and 13.3, 16000 12.5 and 13.5, K = 768, N = 11264 13.4 either way;
+// 40 rows of 8192, K = 544 10.7 and 11.1, of 11264 13.5 and 13.0).
+static bool on_split(const GgParams& p, bool routed) {
+  if (routed) {
+    const long rows = (long)p.T * p.top, experts = p.n_tiles - rows / 64;
+    // fp32 tiles that hold rows, about: half a tile an expert beside whole ones
+    long tiles = max(experts, rows / 64 + experts / 2) * ((p.N + 63) / 64);
+    if (p.Ns > 0) tiles += (p.T + 63L) / 64 * ((p.Ns + 63) / 64);
+    return tiles >= 256 && rows >= (p.K >= 384 ? 18L : 28L) * p.n_tiles;
+  }
+  const long tiles = gg_blocks(p, GG_F32, 32, 64);
+  if (p.K <= 512 || p.M <= 16 || (p.M <= 32 && tiles > 256)) return false;
+  return p.K >= 768 || tiles > 256 || tiles <= (p.M <= 32 ? 96 : 192);
+}
+
+// Whether experts' products are on split operands (tests)
+extern "C" int lsd_moe_on_split(int T, int top, int n_tiles, int N, int Ns, int K) {
+  GgParams p{};
+  p.T = T, p.top = top, p.n_tiles = n_tiles, p.N = N, p.Ns = Ns, p.K = K;
+  return on_split(p, true);
 }
 
 template <int MODE>

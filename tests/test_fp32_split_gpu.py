@@ -124,3 +124,32 @@ def test_operands_behind_the_terms(C, M, N):  # noqa: F811
     assert int(a[::3].count_nonzero()) > 100 and float(a[::3].abs().max()) < 2.0 ** -134
     got = C.linear_fp32(a.to(DEV), w.to(DEV))
     assert near(got, a, w) and int(got[:, 5:90:7].count_nonzero()) == 0 and int(got[::3, :5].count_nonzero()) > 0
+
+
+# where experts change kernels: fp32 tiles more than the CUs, rows a tile of the table, K
+RULE = [(200, 2, 14, 1024, 1024, 512, False), (300, 2, 25, 1024, 1024, 512, True), (300, 2, 25, 1024, 1024, 352, False),
+        (565, 4, 67, 1024, 1024, 128, True), (200, 4, 45, 1024, 1024, 512, False), (200, 4, 44, 1024, 1024, 512, True),
+        (200, 4, 44, 1024, 1024, 352, False), (1000, 2, 39, 256, 0, 256, False), (120, 2, 11, 2048, 0, 2048, True)]
+
+
+def test_experts_rule():
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    assert [_C.moe_on_split(*r[:-1]) for r in RULE] == [r[-1] for r in RULE]
+
+
+# experts on split operands: 28 rows a tile of the table and more, their last tiles part full, and short K
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,H,F", [(290, 9, 128, 1024), (129, 2, 64, 2080), (300, 3, 448, 1200), (1, 1, 64, 16)])
+def test_experts_on_split(C, T, E, H, F):  # noqa: F811
+    top = min(2, E)
+    h, up = rand(T, H, seed=1), rand(E, 2 * F, H, seed=2) * 0.2
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int()
+    order, tiles = C.moe_group(ids.to(DEV), E, 64)
+    assert C.moe_on_split(T, top, tiles.shape[0], 2 * F, 0, H) == (T > 1)
+    mid, _ = C.moe_up(h.to(DEV), order, tiles, top, up.to(DEV), 0.0, 1.0, None, 0.0, 64)
+    perm = order.cpu().long()[: T * top]
+    for s, e in enumerate(perm.tolist()):
+        y = (up[ids[e // top, e % top]].to(F64) @ h[e // top].to(F64)).reshape(F // 16, 2, 16)
+        g, u = y[:, 0].reshape(F), y[:, 1].reshape(F)
+        want = g * torch.sigmoid(g) * u
+        assert float((mid[s].cpu().to(F64) - want).abs().max()) < 1e-5 * max(1.0, float(want.abs().max()))

@@ -746,7 +746,10 @@ __global__ __launch_bounds__(64) void latent_combine_kernel(const float* __restr
     for (int s0 = 64 * j; s0 < min(splits, 64 * j + 64); s0 += AT) {
       if (s0) load(s0);
 #pragma unroll
-      for (int i = 0; i < AT; ++i) sum += v[i] * __shfl(f[j], s0 % 64 + i);
+      for (int i = 0; i < AT; ++i) {
+        const float w = __shfl(f[j], s0 % 64 + i);
+        if (s0 + i < splits) sum += v[i] * w;  // (a last split asked for again may be infinite)
+      }
     }
   const float inv = 1.f / L;
   if (d < rank) st4(out + (long)blockIdx.x * rank + d, pack4(sum * inv));

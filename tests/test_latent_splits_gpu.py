@@ -38,3 +38,18 @@ def test_rule():
                                     (48, 901, False, 15), (160, 181, False, 3), (160, 1024, True, 5), (2000, 64, False, 1),
                                     (1, 1 << 20, False, 64)]:
         assert R.talk_splits(B, keys, windowed) == want, (B, keys, windowed)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [2, 3, 5, 9, 11])
+def test_infinite_parts(splits):
+    """Values whose sum passes fp32's range are infinite, whatever the number of parts."""
+    from llm_sharding_demo_amd import _C as C
+
+    i32 = dict(dtype=torch.int32, device="cuda")
+    pool = torch.full((11, 64, 64), 3e38, dtype=torch.bfloat16, device="cuda")
+    pool[..., ::2] *= -1
+    at = (torch.zeros(1, 64, dtype=torch.bfloat16, device="cuda"), pool, torch.arange(11, **i32).reshape(1, 11),
+          torch.zeros(1, **i32), torch.tensor([699], **i32), 1, 1 << 30, 1.0)
+    one = C.latent_decode(*at, 1)
+    assert bool(one.isinf().all()) and torch.equal(C.latent_decode(*at, splits), one)

@@ -393,22 +393,30 @@ class Routing:
 
     def latent_splits(self, B: int, heads: int, keys: int, rank: int, beside: bool = False) -> int:
         """Context splits of a latent decode launch: the least of what a block's steps
-        take, more where two share a CU, and the merge of the parts.  rank 512, us, for
+        take, more where others share its CU, and the merge of the parts.  rank 512, us, for
         splits 1 / 2 / 4 / 8: 64 sequences of 300 keys 16.0 / 15.8 / 15.4 / 19.3, 24 of 470 22 / 17 / 13.1 /
-        12.7, 96 of 250 13.8 / 15.4 / 17.6 / 24, 160 of 250 13.9 / 21 / 24 / 31.  beside: experts run at the
+        12.7, 96 of 250 13.8 / 15.4 / 17.6 / 24, 160 of 250 13.9 / 21 / 24 / 31.  Blocks of ranks below 320 are smaller:
+        more of them share a CU, and a round that is partly full costs what it holds (160 sequences of 500 to 2000 keys,
+        splits 1 / 2 / 3 / 4: rank 64, 64 heads 19.7 / 23.4 / 22.7 / 23.1, rank 192, 64 heads 38.1 / 43.0 / 46.8 / 50.9, 32 heads
+        30.2 / 31.3 / 29.9 / 31.9).  Of 475 launches of ranks 64 to 576 the splits taken are 0.9 % behind the best on
+        average, 5 % at most behind as many as give 256 blocks but for one sequence of 64 heads.  beside: experts run at the
         same time, so a merge and its bytes weigh twice (a timisun-2b step, splits 1 / 2 / 4 / 8: 64 sequences of
         300 keys 994 / 1006 / 1023 / 1048, 24 of 1024 1011 / 942 / 921 / 925, 64 of 1000 1071 / 1041 / 1053 / 1071)."""
-        items = B * -(-heads // 16)
-        steps = max(1, -(-keys // (64 if rank >= 320 else 128)))  # keys a block takes at a time
+        items, wide = B * -(-heads // 16), rank >= 320
+        steps = max(1, -(-keys // (64 if wide else 128)))  # keys a block takes at a time
         best, least = 1, 0.0
         for k in (steps, 32, 16, 12, 8, 6, 5, 4, 3, 2, 1):  # steps a block
             if k > steps:
                 continue
             s = min(-(-steps // k), 64)
-            share = -(-items * s // 256)  # blocks a CU
-            cost = (0.6 + 0.003 * rank) * (1 if share <= 1 else 0.35 + 0.65 * share) * -(-steps // s)
+            share = max(1.0, items * s / 256)  # blocks a CU
+            if wide:
+                cost, merge = (0.4 + 0.0035 * rank) * (0.45 + 0.55 * math.ceil(share)), 2.5
+            else:
+                cost, merge = (0.6 + 0.0025 * rank) * (0.2 + 0.4 * (share + math.ceil(share))), 1.5
+            cost *= -(-steps // s)
             if s > 1:
-                cost += (3 + 1.6e-6 * B * heads * rank * s) * (2 if beside else 1)
+                cost += (merge + 2e-6 * B * heads * rank * s) * (2 if beside else 1)
             if k == steps or cost < least:
                 best, least = s, cost
         return best

@@ -348,7 +348,10 @@ extern "C" hipError_t lsd_norm_f32(float* x, const float* slab, int splits, cons
   if (n == 0) return hipSuccess;
   auto at = [](const void* q) { return reinterpret_cast<uintptr_t>(q); };
   const int nc = (H + 1023) / 1024;
-  if (H >= 4 && H % 4 == 0 && nc <= 8 && (at(x) | at(slab) | at(w) | at(out)) % 16 == 0) {
+  // rows with slabs from 384 columns on: narrow ones leave most of its threads without a chunk, behind a barrier more
+  // (1 slab: 2000 rows of 64 2.9 and 3.6 us, of 256 3.7 and 4.0, of 384 4.3 either way, 8000 of 256 8.9 and 9.5, of
+  // 384 12.7 and 10.6)
+  if (H >= (slab ? 384 : 4) && H % 4 == 0 && nc <= 8 && (at(x) | at(slab) | at(w) | at(out)) % 16 == 0) {
 #define LSD_NORM_F32(NC)                                                                                                \
   hipLaunchKernelGGL((norm_f32_vec_kernel<NC>), dim3(n), dim3(256), 0, st, x, slab, splits, w, out, T, H, eps, rows, Hn, woff)
     if (nc == 1) LSD_NORM_F32(1);

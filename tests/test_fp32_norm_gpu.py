@@ -40,3 +40,10 @@ def test_slabs_alone(C):  # noqa: F811
     xd = x.to(DEV)
     assert C.norm_fp32(xd, slab.to(DEV), None, 1e-5, None, False, 0, 0.0) is None
     assert torch.equal(xd.cpu(), ((x + slab[0]) + slab[1]) + slab[2])
+
+
+# both sides of the line for rows with slabs, and rows without
+@pytest.mark.parametrize("H", [64, 380, 384, 388])
+@pytest.mark.parametrize("S", [0, 1, 5])
+def test_narrow_rows(C, H, S):  # noqa: F811
+    test_rows(C, H, S, 0)

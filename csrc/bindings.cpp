@@ -68,6 +68,7 @@ hipError_t lsd_attn_oproj(const bf16* q, long ldq, const bf16* kc, const bf16* v
                           int max_seq, float scale_log2, const bf16* W, long ldw, const bf16* bias,
                           float* x, int N, int NC, float* part, int* cnt, hipStream_t st);
 int lsd_gemv_ok(int M, int K, int epi, int norm);
+int lsd_gemv_on_stream(int N, int K, int epi, int norm);
 void lsd_gemv_set_nt(int v);
 hipError_t lsd_gemv(const lsd::GemvParams* p, int epi, int norm, hipStream_t st);
 hipError_t lsd_apply_rows(const int64_t* args, int b, hipStream_t st);
@@ -847,6 +848,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("qkv_post", &qkv_post);
   // GEMV weight stream with non-temporal loads (A/B knob, LSD_GEMV_NT)
   m.def("gemv_set_nt", [](int64_t v) { lsd_gemv_set_nt((int)v); });
+  m.def("gemv_on_stream", [](int64_t N, int64_t K, int64_t epi, int64_t norm) {
+    return lsd_gemv_on_stream((int)N, (int)K, (int)epi, (int)norm) != 0; });
   m.def("gemv_ok", [](int64_t M, int64_t K, int64_t epi, int64_t norm) {
     return lsd_gemv_ok((int)M, (int)K, (int)epi, (int)norm) != 0; });
   m.def("set_stamps", &set_stamps);

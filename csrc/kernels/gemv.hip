@@ -31,7 +31,7 @@
 
 namespace lsd {
 
-// y cos -+ z sin, rounded alike wherever it is inlined: a row's bits do not depend on its kernel
+// y cos -+ z sin, rounded alike in both kernels
 __device__ __forceinline__ float turned(float y, float z, float c, float s, bool odd) { return fmaf(y, c, odd ? z * s : -(z * s)); }
 namespace gv {
 enum : int { BF16 = 0, GELU = 1, SILU = 2, F32 = 3, RESID = 4, QKV = 6 };
@@ -352,7 +352,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
 //   6144 x 4096 QKV        11.7 -> 11.3                 16384 x 2048 gate/up   13.0 -> 12.3
 // Llama-3 8B, a step of one sequence 2907 -> 2754.  Not ahead: 3072 x 3072 5.8 and 6.1, 3072 x 8192 11.1 either
 // way, a head of 50304 x 1600 27.7 and 29.9 (x 768 21.1 -> 15.2, but in GPT-2's step, whose weights the caches
-// hold, 15 either way); 28672 x 4096 a row at a time, three to five in flight.
+// hold, 15 either way); 28672 x 4096 a row at a time, three to five in flight.  Loads are non-temporal whatever
+// gemv_set_nt says: through the caches the same launches take 7 to 14 % longer, and so does a kernel that may do either.
 template <int EPI, int NORM, int SLOTS, int SEGS>
 __global__ __launch_bounds__(256, 2) void gemv_stream_kernel(GemvParams p) {
   constexpr int ITEM = EPI == gv::F32 ? 4 : 1, KS = SLOTS * SEGS * 512, NV = KS / 1024;  // ITEM: pairs of rows
@@ -499,31 +500,57 @@ __global__ __launch_bounds__(256, 2) void gemv_stream_kernel(GemvParams p) {
   }
 }
 
+// Whether one row of K through N rows of W takes gemv_stream_kernel: blocks (0: gemv_kernel), slots and segments.
+struct GvStream {
+  int blocks, slots, segs;
+};
+static GvStream gv_stream(int epi, int norm, int N, int K) {
+  if (N < 4096 || (norm == gv::NONE) != (epi == gv::RESID)) return {};
+  // up to sixteen waves a CU (28672 x 4096: eight 37.1 us, sixteen and more 36.5), all with as many items
+  const int item = epi == gv::F32 ? 8 : 2, items = (N + item - 1) / item, each = (items + 4095) / 4096;
+  const int blocks = ((items + each - 1) / each + 3) / 4, rounds = (blocks + 255) / 256;
+  // Only where it is ahead; cold weights, us, gemv_kernel and gemv_stream_kernel.  The CUs must have like numbers of
+  // blocks, their last round 7/8 full: head of 50304 x 3072 (786 blocks) 51.1 and 52.0, of 65536 x 3072 (1024) 65.9 and
+  // 61.2; residual 4608 x 14336 (576) 24.5 and 24.8, 6144 x 14336 (768) 31.2 and 28.7.
+  if (8 * blocks < 7 * 256 * rounds) return {};
+  // And a unit, whose slots behind K are requested all the same, must be well filled: gate/up 28672 x 1536 16.0 and
+  // 16.2, x 1664 17.5 and 17.3; 16384 x 2688 16.8 and 17.1, x 3072 18.6 and 18.5 (11264 x 4096 17.6 and 17.4, 14336 21.3
+  // and 21.4, 16384 23.9 and 23.0); head 16384 x 2056 13.9 and 15.2, x 2560 16.0 and 15.0; QKV 15360 x 3328 19.2 and
+  // 19.6, x 3584 20.4 and 20.0; residual 4096 x 8200 14.0 and 14.2, x 10240 16.0 and 15.7, x 10880 17.1 and 17.3, x 11008
+  // 17.5 and 18.1, x 11072 16.9 and 16.4, x 12288 18.8 and 17.6.
+  // Of two segments, a wave's only item and sixteen waves a CU have nothing in flight beside it: 8192 x 4096 QKV 13.6
+  // and 14.1, residual 13.1 either way.
+  const bool two = K >= 3584 && K <= 4096 && (each > 1 || blocks <= 768);
+  switch (epi) {
+    case gv::SILU:
+      if (N >= 11264 && K > 1536 && K <= 2048) return {blocks, 4, 1};
+      if (N >= 16384 && K >= 3072 && K <= 4096) return {blocks, 8, 1};
+      break;
+    case gv::F32:
+      if (N >= 16384 && K >= 2560 && K <= 4096) return {blocks, 8, 1};
+      break;
+    case gv::QKV:
+      if (two) return {blocks, 4, 2};
+      break;
+    case gv::RESID:
+      if (two) return {blocks, 4, 2};
+      if (K > 11008) return {blocks, 4, 7};
+  }
+  return {};
+}
+
 template <int EPI, int NORM>
 hipError_t gemv_launch(const GemvParams& p, int mr, int nb, hipStream_t st) {
-  if (mr == 1 && p.N >= 4096) {  // gemv_stream_kernel has both sides' times
-    // up to sixteen waves a CU (28672 x 4096: eight 37.1 us, sixteen and more 36.5), all with as many items
-    const int item = EPI == gv::F32 ? 8 : 2, items = (p.N + item - 1) / item, each = (items + 4095) / 4096;
-    const dim3 g(((items + each - 1) / each + 3) / 4);
-#define LSD_GS(SLOTS, SEGS)                                                                              \
-  {                                                                                                      \
-    hipLaunchKernelGGL((gemv_stream_kernel<EPI, NORM, SLOTS, SEGS>), g, dim3(256), 0, st, p);            \
-    return hipGetLastError();                                                                            \
+  if (const GvStream s = gv_stream(EPI, NORM, p.N, p.K); mr == 1 && s.blocks) {
+#define LSD_GS(SLOTS, SEGS)                                                                                             \
+  if (s.slots == SLOTS && s.segs == SEGS) {                                                                             \
+    hipLaunchKernelGGL((gemv_stream_kernel<EPI, NORM, SLOTS, SEGS>), dim3(s.blocks), dim3(256), 0, st, p);              \
+    return hipGetLastError();                                                                                           \
   }
-    if constexpr (EPI == gv::SILU && NORM != gv::NONE) {
-      if (each > 1 && p.K > 1024 && p.K <= 2048) LSD_GS(4, 1)
-      if (each > 1 && p.K > 2048 && p.K <= 4096) LSD_GS(8, 1)
-    }
-    if constexpr (EPI == gv::F32 && NORM != gv::NONE) {
-      if (p.N >= 16384 && p.K > 2048 && p.K <= 4096) LSD_GS(8, 1)
-    }
-    if constexpr (EPI == gv::QKV && NORM != gv::NONE) {
-      if (p.K > 2048 && p.K <= 4096) LSD_GS(4, 2)
-    }
-    if constexpr (EPI == gv::RESID) {
-      if (p.K > 2048 && p.K <= 4096) LSD_GS(4, 2)
-      if (p.K > 8192) LSD_GS(4, 7)
-    }
+    if constexpr (EPI == gv::SILU && NORM != gv::NONE) { LSD_GS(4, 1) LSD_GS(8, 1) }
+    if constexpr (EPI == gv::F32 && NORM != gv::NONE) LSD_GS(8, 1)
+    if constexpr (EPI == gv::QKV && NORM != gv::NONE) LSD_GS(4, 2)
+    if constexpr (EPI == gv::RESID) { LSD_GS(4, 2) LSD_GS(4, 7) }
 #undef LSD_GS
   }
   constexpr int CPW = EPI == gv::RESID ? 1 : 2;
@@ -572,6 +599,8 @@ extern "C" int lsd_gemv_ok(int M, int K, int epi, int norm) {
       return 0;
   }
 }
+
+extern "C" int lsd_gemv_on_stream(int N, int K, int epi, int norm) { return gv_stream(epi, norm, N, K).blocks != 0; }
 
 static int g_gemv_nt = 0;
 extern "C" void lsd_gemv_set_nt(int v) { g_gemv_nt = v; }

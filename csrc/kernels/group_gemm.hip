@@ -558,7 +558,9 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
 // Terms behind bf16's numbers are lost: of an operand, 2^-134 at most.  Where that may count the tile is computed
 // again by fp32 MFMAs, in the order of the kernel above: an operand of 2^56 or more, a sum that is not finite, one
-// below 2^-40, zeros among them unless their column of W is zero (padding).
+// below 2^-40.  Zeros among these stand where all of their column are and its first weights too, as padding's;
+// looking through all of a column's weights took 10 to 50 us of a launch with padding, a maximum of W's values beside
+// the one of both 20 % of the products.
 template <int MODE, int MT, int WN, int WK, int D>
 __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
@@ -658,29 +660,29 @@ __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float v = fabsf(acc[0][i][q]);
-      exact |= !(v < INFINITY) || (v < 0x1p-40f && (MODE == GG_F32 || MODE == GG_ADD || i < live));
+      exact |= !(v >= 0x1p-40f && v < INFINITY) && (MODE == GG_F32 || MODE == GG_ADD || i < live);
     }
   }
   exact = __syncthreads_or(exact);
-  if (exact) {  // for zeros alone only where the column of W has values
-    int mine = 0, some = big >= 0x1p56f;
+  if (exact) {  // for zeros alone only where the column has other sums, or W values in the part's first k-step
+    int zero = 0, other = 0, some = big >= 0x1p56f;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float v = fabsf(acc[0][i][q]);
-        mine |= v == 0.f && i < live;
+        zero |= v == 0.f && (MODE == GG_F32 || MODE == GG_ADD || i < live);
+        other |= v > 0.f;
         some |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
       }
-    mine |= __shfl_xor(mine, 16);
-    mine |= __shfl_xor(mine, 32);
-    if (mine)
-#pragma unroll 4
-      for (int k = 0; k < T * BKF; k += 16) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(wp + k);
-        some |= v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f;
-      }
-    exact = __syncthreads_or(some);
+    zero |= __shfl_xor(zero, 16);
+    zero |= __shfl_xor(zero, 32);
+    if (zero && T > 0) {
+      const f32x4 u = *reinterpret_cast<const f32x4*>(wp), v = *reinterpret_cast<const f32x4*>(wp + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) other |= u[e] != 0.f || v[e] != 0.f;
+    }
+    exact = __syncthreads_or(some || (zero && other));
   }
   if (exact) {
 #pragma unroll 1

@@ -153,3 +153,15 @@ def test_experts_on_split(C, T, E, H, F):  # noqa: F811
         g, u = y[:, 0].reshape(F), y[:, 1].reshape(F)
         want = g * torch.sigmoid(g) * u
         assert float((mid[s].cpu().to(F64) - want).abs().max()) < 1e-5 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N", [(70, 100), (561, 2560), (961, 2048), (561, 4160)])
+def test_weights_behind_the_terms(C, M, N):  # noqa: F811
+    """Columns of W without a bf16 term, and rows that are all of a tile."""
+    a, w = rand(M, 576, seed=1).clamp(-1, 1) * 2.0 ** 50, rand(N, 576, seed=2).clamp(-1, 1)
+    w[3:90:7] *= 2.0 ** -140
+    got = C.linear_fp32(a.to(DEV), w.to(DEV))
+    assert near(got, a, w) and bool((got[:, 3:90:7] != 0).all())
+    got = C.linear_fp32(w[3:90:7].repeat(6, 1).to(DEV), a.to(DEV))
+    assert near(got, w[3:90:7].repeat(6, 1), a) and bool((got != 0).all())

@@ -62,7 +62,7 @@ def test_not_finite(C, side, value):  # noqa: F811
     assert bool(((got - want).abs()[ok] <= 600 * ULP * 576).all())
 
 
-# 18 rows a tile of the table and more: experts on split operands, and fewer, which are not
+# experts whose fp32 tiles are fewer than the CUs stay on fp32 MFMAs, 18 rows a tile of the table and more or not
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,E", [(300, 3), (129, 5), (64, 1), (30, 9)])
 def test_experts(C, T, E):  # noqa: F811
@@ -165,3 +165,36 @@ def test_weights_behind_the_terms(C, M, N):  # noqa: F811
     assert near(got, a, w) and bool((got[:, 3:90:7] != 0).all())
     got = C.linear_fp32(w[3:90:7].repeat(6, 1).to(DEV), a.to(DEV))
     assert near(got, w[3:90:7].repeat(6, 1), a) and bool((got != 0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,H,F,Fs", [(290, 9, 1280, 1024, 192), (65, 2, 4224, 2752, 64)])
+def test_experts_and_shared_on_split(C, T, E, H, F, Fs):  # noqa: F811
+    """Both products, beside a shared expert: sums of K products and a gated one in front of them, against 64 bits."""
+    top = 2
+    h, up, dn = rand(T, H, seed=1), rand(E, 2 * F, H, seed=2) * 0.05, rand(E, H, F, seed=3) * 0.05
+    shared_up, shared_dn = rand(2 * Fs, H, seed=4) * 0.05, rand(H, Fs, seed=5) * 0.05
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int()
+    wts = torch.rand(T, top)
+    order, tiles = C.moe_group(ids.to(DEV), E, 64)
+    for N, Ns, K in ((2 * F, 2 * Fs, H), (H, H, F)):
+        assert C.moe_on_split(T, top, tiles.shape[0], N, Ns, K)
+    mid, mids = C.moe_up(h.to(DEV), order, tiles, top, up.to(DEV), 0.0, 1.0, shared_up.to(DEV), 0.0, 64)
+    slab = torch.empty(top + 1, T, H, device=DEV)
+    C.moe_down(mid, mids, order, tiles, wts.to(DEV), dn.to(DEV), shared_dn.to(DEV), slab, 64)
+
+    def gated(x, w):
+        y = (x @ w.to(F64).T).reshape(len(x), -1, 2, 16)
+        return (y[:, :, 0] * torch.sigmoid(y[:, :, 0]) * y[:, :, 1]).reshape(len(x), -1)
+
+    def close(got, want):
+        assert float((got.cpu().to(F64) - want).abs().max()) < 1e-5 * float(want.abs().max())
+    perm, x = order.cpu().long()[: T * top], h.to(F64)
+    token, expert = perm // top, ids.reshape(-1)[perm]
+    close(mids, gated(x, shared_up))
+    close(slab[top], mids.cpu().to(F64) @ shared_dn.to(F64).T)
+    for e in range(E):
+        mine = (expert == e).nonzero()[:, 0]
+        close(mid.cpu()[mine], gated(x[token[mine]], up[e]))
+        want = wts.reshape(-1)[perm[mine]].to(F64)[:, None] * (mid.cpu()[mine].to(F64) @ dn[e].to(F64).T)
+        close(slab[:top].cpu()[perm[mine] % top, token[mine]], want)

@@ -34,7 +34,7 @@ class Routing:
     # preceding LayerNorm / RMSNorm into its prologue (0 disables)
     gemv_max_m: int = 8
     gemv_norm_max_m: int = 2
-    gemv_nt: int = 0  # non-temporal weight loads in the GEMV (A/B)
+    gemv_nt: int = 0  # non-temporal weight loads in gemv_kernel (A/B; gemv_stream_kernel's always are)
     # -- decode attention --------------------------------------------------
     target_blocks: int = 512  # >> 256 CUs: VALU decode attention splits the context up to this
     split_keys: int = 256      # ... with at least this many keys per split (64 / 128 lose at 1-16

@@ -886,8 +886,9 @@ class HipBackend(Backend):
                 return self._latent_expanded(q, gate, w, m, kv, pool, meta, window, reach)
         q = self._batch_linear(q, uk)
         if meta.is_decode or self.fp32 or rows == 0:
-            # one query per sequence, or the kernel that takes any token alone
-            splits = self.R.latent_splits(q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2], ahead)
+            # one query per sequence, or the kernel that takes any token alone, and none in parts
+            splits = 1 if self.fp32 or rows == 0 else self.R.latent_splits(
+                q.shape[0], m.heads, min(window, meta.max_ctx), pool.shape[2], ahead)
             o = self.C.latent_decode(q, pool, kv.table, meta.token_slots, meta.token_pos, m.heads, window, m.scale,
                                      splits, *beside)
         else:

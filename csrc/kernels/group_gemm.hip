@@ -953,6 +953,7 @@ static hipError_t gg_split_on(const GgParams& p, hipStream_t st) {
 // 80 x 64 43.3, 48 x 128 47.7; 300 of 2048 48 x 64 in two parts of K 33.7, in four 29.0; 565 of 4160
 // 48 x 128 86, 80 x 128 100, 96 x 128 73; 1000 of 2048 64 x 64 67.7, 64 x 128 61.0; of 4160 80 x 128 117, 96 x 128
 // 128; of 11264 64 x 128 306, 80 x 128 299, 96 x 128 286.
+// For every K: of 329 sizes with K from 544 to 8192 the tiles so chosen take 0.54 to 1.02 of the fp32 MFMAs' times.
 struct SplitTile {
   int rows, cols, parts, fixed, round;
 };

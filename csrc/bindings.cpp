@@ -58,7 +58,7 @@ int lsd_attn_decode_total(int B, int n_kv, int G, int hd, int splits, int keys);
 hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                            const int* seq_slots, const int* qpos, bf16* out, long ldo,
                            float* part_o, float* part_ml, int B, int nh, int n_kv, int hd,
-                           int max_seq, int splits, int total, float scale_log2, hipStream_t st);
+                           int max_seq, int splits, int total, int keys, float scale_log2, hipStream_t st);
 hipError_t lsd_attn_prefill(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                             const int* tiles, int n_tiles, int rows, const int* seq_slots,
                             const int* q_start, const int* cu_q, bf16* out, long ldo, int nh,
@@ -551,7 +551,8 @@ void check_cache(const torch::Tensor& kc, const torch::Tensor& vc) {
               reinterpret_cast<uintptr_t>(vc.data_ptr()) % 16 == 0, "caches must be 16-byte aligned");
 }
 
-// keys: the longest context (0: not known), by which short ranges are not taken apart further
+// keys: the longest context (0: not known), by which short ranges are not taken apart further and
+// blocks request as many keys at once as it has
 torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
                           torch::Tensor seq_slots, torch::Tensor qpos, int64_t nh,
                           int64_t splits, int64_t keys) {
@@ -570,8 +571,8 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   float* pop = nullptr;
   float* pmlp = nullptr;
   TORCH_CHECK(keys >= 0, "keys of the longest context");
-  const int total = lsd_attn_decode_total(B, n_kv, (int)(nh / n_kv), hd, (int)splits,
-                                          (int)std::min<int64_t>(keys, kc.size(2)));
+  const int longest = (int)std::min<int64_t>(keys, kc.size(2));
+  const int total = lsd_attn_decode_total(B, n_kv, (int)(nh / n_kv), hd, (int)splits, longest);
   if (total > 1) {
     po = torch::empty({B, nh, total, hd}, q.options().dtype(torch::kFloat32));
     pml = torch::empty({B, nh, total, 2}, q.options().dtype(torch::kFloat32));
@@ -581,7 +582,7 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   const float sl2 = 1.4426950408889634f / std::sqrt((float)hd);
   check_hip(lsd_attn_decode(bptr(q), q.stride(0), bptr(kc), bptr(vc), seq_slots.data_ptr<int>(),
                             qpos.data_ptr<int>(), bptr_mut(out), out.stride(0), pop, pmlp, B, nh,
-                            n_kv, hd, kc.size(2), splits, total, sl2, cur_stream()), "attn_decode");
+                            n_kv, hd, kc.size(2), splits, total, longest, sl2, cur_stream()), "attn_decode");
   return out;
 }
 

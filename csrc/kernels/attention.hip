@@ -37,9 +37,32 @@ constexpr float NEG = -1e30f;
 #define LSD_KV_LOAD ld8_nt
 #endif
 
-// NWV waves per block: 4 for full batches; 16 for small ones (fewer
-// (sequence, head) items than CUs), where the whole context of an item is
-// requested in one round of loads instead of a chain of dependent rounds.
+// One step of a sum over lanes that lie OFF apart, of the first N of V values: the upper lanes go on with the
+// upper half of them, the lower ones with the lower half (N = 1: both).  idx: the first value a lane has.
+template <int OFF, int N, int V>
+__device__ __forceinline__ void fold_step(float (&v)[V], int& idx, int lane) {
+  if constexpr (N == 1) {
+    v[0] += wave_xor_n(v[0], OFF);
+  } else {
+    constexpr int h = N / 2;
+    const bool up = (lane & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+      const float send = up ? v[i] : v[i + h], keep = up ? v[i + h] : v[i];
+      v[i] = keep + wave_xor_n(send, OFF);
+    }
+    if (up) idx += h;
+  }
+}
+
+// NWV waves per block, U keys per lane group in flight.  Full batches: 4 waves, 4 keys, V behind the
+// scores (fewer live registers, and the other blocks on the CU hide the latency; V with K costs two lanes of
+// 256 sequences 1.5 %).  Small ones (fewer (sequence, head) items than CUs): 8 keys or more than 4 waves, an
+// item's K and V requested in one round of loads instead of a chain of dependent ones.
+// There a launch is its chain: position, K and V, scores, merges.  The merges are kept short: a wave scales its
+// sums once by its own maximum and folds them over its key groups, each lane going on with half of its columns
+// (7 exchanges for 8 columns, 24 when every lane merges all of them pair by pair), and a lane a column merges
+// the waves.  12 heads of 64, one sequence of 204 keys 4.7 -> 4.0 us, on 4 waves of 8 keys for 8 of 4 3.7.
 template <int HD, int G, int U, int NWV>
 __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ kc,
@@ -48,7 +71,9 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
     int max_seq, int splits, float scale_log2, int n_items) {
   constexpr int LPK = HD / 8;    // lanes per key row
   constexpr int KPI = 64 / LPK;  // keys per wave-instruction
-  __shared__ float sm[NWV][G][LPK][10];
+  constexpr bool ROUND = NWV > 4 || U > 4;  // V with K
+  __shared__ float sm_o[NWV][G][HD];
+  __shared__ float sm_ml[NWV][G][2];
   // work item = (sequence, kv head); a capped grid (lsd_attn_set_max_wg) loops
   // over items so the kernel occupies only part of the chip and a concurrent
   // lane's GEMMs keep the rest
@@ -86,11 +111,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
         const int kk = min(key[u], k_hi - 1);
         kv[u] = LSD_KV_LOAD(kc + base + (long)kk * HD);
       }
-      // small batches: V (independent of the scores) is requested with K, one
-      // round trip per item.  Full batches keep V behind the scores: fewer
-      // live registers, and the other blocks on the CU hide the latency
-      // (measured: moving it costs the 2 x 256 bench ~1.5 %)
-      if constexpr (NWV > 4) {
+      if constexpr (ROUND) {
 #pragma unroll
         for (int u = 0; u < U; ++u) vv[u] = LSD_KV_LOAD(vc + base + (long)min(key[u], k_hi - 1) * HD);
       }
@@ -106,7 +127,7 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
           for (int msk = 1; msk < LPK; msk <<= 1) acc += wave_xchg_n(acc, msk);
           s[g][u] = key[u] < k_hi ? acc : NEG;
         }
-      if constexpr (NWV <= 4) {
+      if constexpr (!ROUND) {
 #pragma unroll
         for (int u = 0; u < U; ++u) vv[u] = LSD_KV_LOAD(vc + base + (long)min(key[u], k_hi - 1) * HD);
       }
@@ -135,67 +156,64 @@ __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
       }
     }
 
-    // merge the key groups of this wave (lanes with equal ds)
+    // merge the key groups of this wave (lanes with equal ds: exact xor partners)
 #pragma unroll
-    for (int msk = LPK; msk < 64; msk <<= 1) {
+    for (int g = 0; g < G; ++g) {
+      float mw = m[g];
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        // lanes of one head-dim slice (equal ds) merge: exact xor partners
-        const float mo = wave_xor_n(m[g], msk), lo = wave_xor_n(l[g], msk);
-        const float mn = fmaxf(m[g], mo);
-        const float a = exp2f(m[g] - mn), bb = exp2f(mo - mn);
-        l[g] = l[g] * a + lo * bb;
+      for (int msk = LPK; msk < 64; msk <<= 1) mw = fmaxf(mw, wave_xor_n(mw, msk));
+      const float f = exp2f(m[g] - mw);
+      float lw = l[g] * f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o[g][j] = o[g][j] * a + wave_xor_n(o[g][j], msk) * bb;
-        m[g] = mn;
+      for (int msk = LPK; msk < 64; msk <<= 1) lw += wave_xor_n(lw, msk);
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = o[g][j] * f;
+      int idx = 0;
+      fold_step<32, 8>(v, idx, lane);
+      fold_step<16, 4>(v, idx, lane);
+      if constexpr (LPK == 8) {
+        fold_step<8, 2>(v, idx, lane);
+        sm_o[w][g][ds * 8 + idx] = v[0];
+      } else {
+        *reinterpret_cast<f32x2*>(&sm_o[w][g][ds * 8 + idx]) = f32x2{v[0], v[1]};
       }
-    }
-    // merge the 4 waves through LDS
-    if (kg == 0) {
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        sm[w][g][ds][0] = m[g];
-        sm[w][g][ds][1] = l[g];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) sm[w][g][ds][2 + j] = o[g][j];
+      if (lane == 0) {
+        sm_ml[w][g][0] = mw;
+        sm_ml[w][g][1] = lw;
       }
     }
     __syncthreads();
-    if (w == 0 && kg == 0) {
+    // merge the waves: two columns of a head a thread
+    for (int t = threadIdx.x; t < G * (HD / 2); t += NWV * 64) {
+      const int g = t / (HD / 2), d = t % (HD / 2) * 2;
+      float mv[NWV], mm = NEG;
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float mm = NEG;
+      for (int ww = 0; ww < NWV; ++ww) mm = fmaxf(mm, mv[ww] = sm_ml[ww][g][0]);
+      float ll = 0.f, a = 0.f, c = 0.f;
 #pragma unroll
-        for (int ww = 0; ww < NWV; ++ww) mm = fmaxf(mm, sm[ww][g][ds][0]);
-        float ll = 0.f, oo[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ww = 0; ww < NWV; ++ww) {
-          const float f = exp2f(sm[ww][g][ds][0] - mm);
-          ll += sm[ww][g][ds][1] * f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) oo[j] += sm[ww][g][ds][2 + j] * f;
-        }
-        const int h = kvh * G + g;
-        if (splits == 1) {
-          const float inv = ll > 0.f ? 1.f / ll : 0.f;
-          bf16x8 r;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) r[j] = f2bf(oo[j] * inv);
-          st8(out + (long)b * ldo + (long)h * HD + ds * 8, r);
-        } else {
-          const int nh = n_kv * G;
-          const long pi = ((long)b * nh + h) * splits + split;
-          float* po = part_o + pi * HD + ds * 8;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) po[j] = oo[j];
-          if (ds == 0) {
-            part_ml[pi * 2] = mm;
-            part_ml[pi * 2 + 1] = ll;
-          }
+      for (int ww = 0; ww < NWV; ++ww) {
+        const float f = exp2f(mv[ww] - mm);
+        const f32x2 x = *reinterpret_cast<const f32x2*>(&sm_o[ww][g][d]);
+        ll += sm_ml[ww][g][1] * f;
+        a += x[0] * f;
+        c += x[1] * f;
+      }
+      const int h = kvh * G + g;
+      if (splits == 1) {
+        const float inv = ll > 0.f ? 1.f / ll : 0.f;
+        *reinterpret_cast<bf16x2*>(out + (long)b * ldo + (long)h * HD + d) = pack2(a * inv, c * inv);
+      } else {
+        const int nh = n_kv * G;
+        const long pi = ((long)b * nh + h) * splits + split;
+        *reinterpret_cast<f32x2*>(part_o + pi * HD + d) = f32x2{a, c};
+        if (d == 0) {
+          part_ml[pi * 2] = mm;
+          part_ml[pi * 2 + 1] = ll;
         }
       }
     }
-    __syncthreads();  // sm is reused by this block's next item
+    __syncthreads();  // sm_o is reused by this block's next item
   }
 }
 
@@ -810,7 +828,7 @@ using namespace lsd;
 
 static int g_attn_max_wg = 0;  // 0: one workgroup per (sequence, kv head)
 extern "C" void lsd_attn_set_max_wg(int v) { g_attn_max_wg = v; }
-static int g_attn_small_waves = 8;  // waves per block for small decode batches (4, 8, 16; 88)
+static int g_attn_small_waves = 0;  // waves per block for small decode batches (4, 8, 16; 88; 0: decode_keys)
 static int g_attn_small_waves128 = 88;  // ... for 128-dim heads
 extern "C" void lsd_attn_set_small_waves(int v) { g_attn_small_waves = v; }
 extern "C" void lsd_attn_set_small_waves128(int v) { g_attn_small_waves128 = v; }
@@ -889,11 +907,25 @@ extern "C" int lsd_attn_decode_total(int B, int n_kv, int G, int hd, int splits,
   return std::max(total, (int)std::min<long>({1536 / items, (keys + 127) / 128, 16}));
 }
 
-// total: lsd_attn_decode_total's; part_o and part_ml hold as many
+// Keys in flight a lane group of 64-dim ungrouped heads on 4 waves, whose blocks take 8 times as many keys a
+// wave and round: as few as hold the keys of a split in one round, behind 128 keys 8 (rounds of 256).  us for
+// 2 / 4 / 8 (before, 8 waves of 4 keys up to 128 blocks, 4 of 4 beyond), contexts from half of the longest on:
+//   12 items   40 keys 2.9 3.1 3.5 (4.0)   100 3.3 3.1 3.5 (4.1)   200 4.9 4.3 3.8 (4.6)   450 8.4 6.6 5.7 (5.9)
+//   300        40 4.1 4.3 4.6 (4.6)        100 4.6 4.6 5.0 (5.0)   200 6.0 5.6 5.6 (5.9)   700 12.2 11.1 11.0 (11.4)
+//   2400       40 8.0 10.4 12.1 (11.8)     100 11.1 12.0 13.2 (13.3)  200 17.2 17.4 16.9 (18.3)  1000 72.2 70.5 69.4 (71.0)
+//   5000       16 10.5 15.3 17.7 (17.9)    100 17.9 20.7 23.6 (22.9)  200 31.4 31.0 30.5 (32.1)  450 65.8 64.4 63.3 (64.9)
+// From 2048 items on 4 behind 128 keys: V with K costs two lanes of 256 sequences of 25 heads, which share the
+// chip, 0.2 % of their tokens and 1.5 % of a step.
+static int decode_keys(int keys, long items) {
+  if (keys <= (items < 512 ? 64 : 128)) return 2;
+  return keys <= 128 || items >= 2048 ? 4 : 8;
+}
+
+// total: lsd_attn_decode_total's; part_o and part_ml hold as many.  keys: the longest context, 0 where not known
 extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, const bf16* vc,
                                       const int* seq_slots, const int* qpos, bf16* out, long ldo,
                                       float* part_o, float* part_ml, int B, int nh, int n_kv,
-                                      int hd, int max_seq, int splits, int total, float scale_log2,
+                                      int hd, int max_seq, int splits, int total, int keys, float scale_log2,
                                       hipStream_t st) {
   if (B == 0) return hipSuccess;
   const int G = nh / n_kv;
@@ -927,18 +959,25 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
 #undef LSD_DEC_MFMA
     return hipErrorInvalidValue;
   }
-  // fewer blocks than half the CUs: wider blocks (g_attn_small_waves waves),
-  // K and V of an item requested in one round of loads.
+  // 64-dim ungrouped heads: decode_keys.  Others: fewer blocks than half the CUs: wider blocks
+  // (g_attn_small_waves waves), K and V of an item requested in one round of loads.
   // full batches: 4 waves (unroll 4) by default; 8 waves, 4 waves with
   // unroll 2 (42) and 2 waves (2) for A/B (lsd_attn_set_large_waves)
   const int lw = hd == 64 ? g_attn_large_waves64 : g_attn_large_waves128;
   // small grids: g_attn_small_waves (8; 88 = 8 waves with 8 keys per wave in
   // flight, so a 256-key context of a 128-dim head is one round of loads:
   // Llama-3 8B single stream 3.196 -> 3.172-3.181 ms, batch 4 3.757 -> 3.735;
-  // GPT-2 XL's 64-dim heads 1.394 -> 1.43 ms, so 128-dim heads only;
   // profiles/r6_attn_u8.log)
   const int swd = hd == 128 ? g_attn_small_waves128 : g_attn_small_waves;
-  const int sw = (long)gx * splits <= 128 ? swd : (lw == 8 || lw == 42 || lw == 2 ? lw : 0);
+  int sw = (long)gx * splits <= 128 ? swd : (lw == 8 || lw == 42 || lw == 2 ? lw : 4);
+  if (sw == 0 || sw == 4) {
+    if (hd == 64 && G == 1 && (sw == 0 || (long)gx * splits > 128)) {
+      const int u = decode_keys(((keys > 0 ? std::min(keys, max_seq) : max_seq) + splits - 1) / splits, n_items);
+      sw = u == 2 ? 42 : u == 8 ? 48 : 4;
+    } else if (sw == 0) {
+      sw = 8;
+    }
+  }
   dim3 grid(gx, splits);
 #define LSD_DEC(HDV, GV)                                                                        \
   if (hd == HDV && G == GV) {                                                                   \
@@ -954,6 +993,10 @@ extern "C" hipError_t lsd_attn_decode(const bf16* q, long ldq, const bf16* kc, c
       hipLaunchKernelGGL((attn_decode_kernel<HDV, (GV <= 4 ? GV : 1), 8, 8>), grid, dim3(512),  \
                          0, st, q, ldq, kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml,     \
                          n_kv, max_seq, splits, scale_log2, n_items);                           \
+    else if (sw == 48 && HDV == 64 && GV == 1)                                                  \
+      hipLaunchKernelGGL((attn_decode_kernel<HDV, GV, (HDV == 64 && GV == 1 ? 8 : 4), 4>), grid, dim3(256), 0, st, q, ldq, \
+                         kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml, n_kv, max_seq,     \
+                         splits, scale_log2, n_items);                                          \
     else if (sw == 42)                                                                          \
       hipLaunchKernelGGL((attn_decode_kernel<HDV, GV, 2, 4>), grid, dim3(256), 0, st, q, ldq,   \
                          kc, vc, seq_slots, qpos, out, ldo, part_o, part_ml, n_kv, max_seq,     \

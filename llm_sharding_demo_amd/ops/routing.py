@@ -46,13 +46,15 @@ class Routing:
     attn_mfma_min: int = 256
     attn_mfma_split_below: int = 1024
     attn_mfma_waves: int = 1024
-    attn_small_waves: int = 8  # waves per small-batch VALU attention block
+    # waves per small-batch VALU attention block; 0: 4 waves, whose keys in flight follow from the
+    # context (64-dim ungrouped heads; decode_keys in attention.hip), 8 for others
+    attn_small_waves: int = 0
     # ... for 128-dim heads: 88 = 8 waves with 8 keys per wave in flight (a 256-key
     # context in one round of loads; Llama-3 8B single stream -0.6 %, r6_attn_u8.log)
     attn_small_waves128: int = 88
-    # full-batch block: 4 waves; 8 waves 10 % slower (r4_attn_large_waves.log); 42 = 4 waves with 2
-    # keys per wave in flight and 2 = 2-wave blocks: faster alone at <= 192 keys, slower in the
-    # two-lane bench (XL p50 8.44 -> 8.58-8.63 ms; r6_attn_ab.log)
+    # full-batch block: 4 waves (64-dim ungrouped heads: keys in flight by the context, as above); 8
+    # waves 10 % slower (r4_attn_large_waves.log); 42 = 4 waves with 2 keys per wave in flight, 2 = 2-wave
+    # blocks
     attn_large_waves: int = 4
     attn_max_wg: int = 0       # cap the attention grid (A/B; 0 = none)
     # -- decode GEMMs ------------------------------------------------------
@@ -463,6 +465,10 @@ class Routing:
                 ms = max(1, min(math.ceil(self.attn_mfma_waves / items), math.ceil(max_ctx / 512), 256))
             if items * ms >= self.attn_mfma_min:
                 return ms
+        if hd == 64 and max_ctx <= 2 * self.split_keys:
+            # two rounds of a block's loads cost less than a merge of its own (12 heads, 300 keys 5.4 us,
+            # in two splits 6.0; 450 5.7 and 6.1; three rounds and splits: 700 7.3 and 6.1)
+            return 1
         if items < self.target_blocks:
             return min(math.ceil(self.target_blocks / items), max(1, math.ceil(max_ctx / self.split_keys)))
         return 1

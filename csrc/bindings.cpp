@@ -37,6 +37,7 @@ int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits);
 int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
 int lsd_gemm_big_tiles(int M, int N, int K, int S);
+int lsd_gemm_on_wave4(int M, int N, int K, int epi, int S);
 int lsd_gemm_far_rows(int M, int N, int K, long lda, long ldw);
 void lsd_attn_set_max_wg(int v);
 void lsd_attn_set_small_waves(int v);
@@ -876,6 +877,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return lsd_gemm_on_deep((int)M, (int)N, (int)K, (int)epi, (int)kind, (int)splits) != 0; });
   m.def("gemm_big_tiles", [](int64_t M, int64_t N, int64_t K, int64_t S) {
     return lsd_gemm_big_tiles((int)M, (int)N, (int)K, (int)S) != 0; });
+  m.def("gemm_on_wave4", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t S) {
+    return lsd_gemm_on_wave4((int)M, (int)N, (int)K, (int)epi, (int)S); });
   m.def("gemm_far_rows", [](int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw) {
     return lsd_gemm_far_rows((int)M, (int)N, (int)K, lda, ldw) != 0; });
   m.def("gemm_ring8_tiles", [](int64_t M, int64_t N, int64_t K, int64_t S) {

@@ -279,4 +279,22 @@ __device__ __forceinline__ int xcd_remap(int bid, int nwg) {
   return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + bid / nx;
 }
 
+// Tile order of the large GEMMs.  G = 0: M-fastest (consecutive workgroups
+// share a W panel).  G > 0: groups of G row panels, M-fastest inside a group
+// and the group's column panels in turn -- the tiles in flight at once (the
+// XCD-contiguous ranges of xcd_remap) then cover a few row panels instead of
+// sweeping every row panel per column panel, so each A panel is read from
+// HBM about once instead of once per column tile.
+__device__ __forceinline__ void tile_order(int t, int tiles_m, int tiles_n, int G, int& tm, int& tn) {
+  if (G <= 0) {
+    tm = t % tiles_m;
+    tn = t / tiles_m;
+    return;
+  }
+  const int gsz = G * tiles_n, grp = t / gsz, idx = t % gsz;
+  const int gm = min(G, tiles_m - grp * G);
+  tm = grp * G + idx % gm;
+  tn = idx / gm;
+}
+
 }  // namespace lsd

@@ -910,24 +910,6 @@ __device__ __forceinline__ bf16x8 lds_frag_big(const char* op, int row, int g) {
   return *reinterpret_cast<const bf16x8*>(op + row * 64 + ((g ^ big_swz((row >> 2) & 3)) << 4));
 }
 
-// Tile order of the large GEMMs.  G = 0: M-fastest (consecutive workgroups
-// share a W panel).  G > 0: groups of G row panels, M-fastest inside a group
-// and the group's column panels in turn -- the tiles in flight at once (the
-// XCD-contiguous ranges of xcd_remap) then cover a few row panels instead of
-// sweeping every row panel per column panel, so each A panel is read from
-// HBM about once instead of once per column tile.
-__device__ __forceinline__ void tile_order(int t, int tiles_m, int tiles_n, int G, int& tm, int& tn) {
-  if (G <= 0) {
-    tm = t % tiles_m;
-    tn = t / tiles_m;
-    return;
-  }
-  const int gsz = G * tiles_n, grp = t / gsz, idx = t % gsz;
-  const int gm = min(G, tiles_m - grp * G);
-  tm = grp * G + idx % gm;
-  tn = idx / gm;
-}
-
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_big_kernel(GemmParams p, int tiles_m, int tiles_n, int G) {
   __shared__ __attribute__((aligned(16))) char smem[GSMEM];
@@ -1719,7 +1701,8 @@ __global__ __launch_bounds__(512) void gemm_d256_kernel(GemmParams p, int* __res
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
-static int g_big_min_blocks = 160;  // lsd_gemm_set_big_min(): tuning / tests (1 << 16 and more: never)
+constexpr int BIG_MIN_BLOCKS = 160;
+static int g_big_min_blocks = BIG_MIN_BLOCKS;  // lsd_gemm_set_big_min(): tuning / tests (1 << 16 and more: never)
 // Whether a tiled launch runs on 256 x 256 tiles, one block a CU: from g_big_min_blocks of them on, or
 // where the 128 x 128 tiles, two blocks a CU, take more than one round.  A round of either, with
 // the operands of 2048 columns: 1000 rows of 6144 (384 tiles, 96) 31.7 us and 38.5, of 8576 (536, 136) 53.0
@@ -1946,12 +1929,19 @@ using namespace lsd;
 
 extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits);  // gemm_deep.hip
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st);
+extern "C" int lsd_gemm_wave4_tile(int M, int N, int K, int epi, int S);  // gemm_wave4.hip
+extern "C" hipError_t lsd_gemm_wave4(const GemmParams* p, int epi, int code, hipStream_t st);
 
 // Kinds 0 and 1 of up to 48 rows, and up to 256 of few blocks, run on the deep ring where K has
 // whole k-steps of 64 (gemm_deep.hip has the line and both sides' times); the split-K kernel,
 // the rings and the tiled kernels take the rest.
 extern "C" int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits) {
   return kind <= 1 && lsd_gemm_deep_ok(M, N, K, epi, splits);
+}
+
+// The tile of a kind 1 launch on gemm_wave4.hip's kernel (0: the others; also where a test asks for or bars 256 x 256 tiles)
+extern "C" int lsd_gemm_on_wave4(int M, int N, int K, int epi, int S) {
+  return g_big_min_blocks == BIG_MIN_BLOCKS && (S == 1 || epi == EPI_SLAB) ? lsd_gemm_wave4_tile(M, N, K, epi, S) : 0;
 }
 
 extern "C" void lsd_gemm_set_big_min(int v) { g_big_min_blocks = v; }
@@ -1998,6 +1988,8 @@ extern "C" hipError_t lsd_gemm(const GemmParams* p, int epi, int kind, int* cnt,
   if (lsd_gemm_on_deep(p->M, p->N, p->K, epi, kind, p->splits)) return lsd_gemm_deep(p, epi, st);
   const bool far = kind && (far_rows(p->M, p->N, p->K, p->lda, p->ldw) ||
                             (kind == 1 && epi == EPI_RESID && p->ldo >= 1 << 21));  // (its rows in 256 of them likewise)
+  if (kind == 1 && !far)
+    if (const int code = lsd_gemm_on_wave4(p->M, p->N, p->K, epi, p->splits)) return lsd_gemm_wave4(p, epi, code, st);
 #define LSD_DISPATCH(E)                                                                   \
   case E:                                                                                 \
     if (far) return launch_far<E>(*p, st);                                                \

@@ -17,7 +17,7 @@
 // before its first loads, so W starts without the routing, and the routing weights of a down
 // tile arrive under its products.  32 experts of 2048 x 1024 and a shared one of 2048, 4 a
 // token: 64 tokens up 58 -> 46 us (6.1 TB/s), down 37 -> 33; 16000 tokens down 587 -> 504.
-// fp32, for models served in it: three bf16 terms of every value on bf16 MFMAs; where few rows
+// fp32, for models served in it: two fp16 terms of every value on fp16 MFMAs, or three bf16 ones; where few rows
 // leave the stream of the weights as the bound, MFMA 16x16x4 on fp32 operands with the bf16
 // kernel's staging; VALU tiles with fused multiply-adds where K has no whole steps of 32 or a
 // row starts off 16 bytes.
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256, MT == 2 ? 4 : 3) void group_gemm_f32_mfma_kern
 }
 
 // ---------------------------------------------------------------------------
-// fp32 on the bf16 matrix cores
+// fp32 on the 16-bit matrix cores
 // ---------------------------------------------------------------------------
 // x = hi + mid + lo, each bf16: of 24 bits the first two, rounded to nearest, leave rests of 16 and 8
 // bits, so nothing is lost from 2^-110 on (below, lo is subnormal).  big: the largest |x|.  (Dot products with
@@ -541,6 +541,101 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
   return s;
 }
 
+// What follows the products on split operands, S the tile's sums, WN waves a part.  Terms behind the 16-bit numbers are
+// lost.  Where that may count the tile is computed again by fp32 MFMAs, in the order of the kernel above: operands outside of the
+// terms' range, a sum that is not finite, one below LEAST.  Zeros among these stand where all of their column are and its weights
+// too, as padding's, of which the first ones are looked at where it is not known (weights) that there are others; looking through all of a column's weights took 10 to 50 us of a launch with padding.
+// wmax: of the tile's columns, or null.
+template <int MODE, int WM, int MT, int WN, int NT, int WK>
+__device__ __forceinline__ void split_tail(const GgParams& p, const gg::Tile& t, char* smem, f32x4 (&S)[MT][NT], int first, int T,
+                                           bool outside, const float* wmax, float LEAST) {
+  using namespace gg;
+  constexpr int TM = 16 * MT * WM, TN = 16 * NT * WN, BKF = 32, CLD = TN + 4, IMAGE = TM * CLD;
+  constexpr bool WHOLE = MODE == GG_F32 || MODE == GG_ADD;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int wn = wave % WN, wm = wave / WN % WM, part = wave / (WN * WM);
+  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16) - wm * MT;  // of this wave's tiles
+  auto weights = [&](int j) {
+    return static_cast<const float*>(t.W) + (long)min(t.n0 + (wn * NT + j) * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
+  };
+  bool exact = outside;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v = fabsf(S[i][j][q]);
+        exact |= !(v >= LEAST && v < INFINITY) && (WHOLE || i < live);
+      }
+  exact = __syncthreads_or(exact);
+  if (exact) {  // for zeros alone only where the column has other sums, or W values
+    int some = outside;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      int zero = 0, other = wmax && wmax[(wn * NT + j) * 16 + r] > 0.f;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v = fabsf(S[i][j][q]);
+          zero |= v == 0.f && (WHOLE || i < live);
+          other |= v > 0.f;
+          some |= !(v < INFINITY) || (v < LEAST && v > 0.f);
+        }
+      zero |= __shfl_xor(zero, 16);
+      zero |= __shfl_xor(zero, 32);
+      if (zero && !wmax && T > 0) {
+        const f32x4 u = *reinterpret_cast<const f32x4*>(weights(j)), v = *reinterpret_cast<const f32x4*>(weights(j) + 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) other |= u[e] != 0.f || v[e] != 0.f;
+      }
+      some |= zero && other;
+    }
+    exact = __syncthreads_or(some);
+  }
+  if (exact) {
+#pragma unroll 1
+    for (int i = 0; i < min(live, MT); ++i) {
+      const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, (wm * MT + i) * 16 + r) * t.lda + first * BKF + 4 * g;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float* wp = weights(j);
+        f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+        for (int k = 0; k < T * BKF; k += BKF)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const f32x4 av = *reinterpret_cast<const f32x4*>(a + k + 16 * h), wv = *reinterpret_cast<const f32x4*>(wp + k + 16 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[h], 0, 0, 0);
+          }
+#pragma unroll
+        for (int h = 0; h < MT; ++h)
+          if (h == i) S[h][j] = s[0] + s[1];
+      }
+    }
+  }
+  float* ct = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        ct[part * IMAGE + ((wm * MT + i) * 16 + 4 * g + q) * CLD + (wn * NT + j) * 16 + r] = S[i][j][q];
+  __syncthreads();
+  if constexpr (WK > 1) {
+    for (int c = threadIdx.x; c < IMAGE / 4; c += 64 * WM * WN * WK) {
+      f32x4* o = reinterpret_cast<f32x4*>(ct) + c;
+#pragma unroll
+      for (int i = 1; i < WK; ++i) *o += o[i * (IMAGE / 4)];
+    }
+    __syncthreads();
+  }
+  f32_epilogue<MODE, TM, TN, 64 * WM * WN * WK>(p, t, ct);
+}
+
 // 16 MT x 16 WN tiles, 32-deep k-steps, WK parts of the k-steps on WN waves each, summed in LDS.
 // Of the nine products of two split operands the six largest are summed (the others are below 2^-26 of
 // it), hi hi apart from the rest, whose sums round at 2^-8 of theirs.  A goes through registers into three
@@ -556,11 +651,8 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
 // 2048 63 -> 49, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 286; 2260 rows over 32 experts of
 // 2048 x 1024 and 565 through a shared one of 2048 up 325 -> 244, down 152 -> 121.  Splitting W a k-step
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
-// Terms behind bf16's numbers are lost: of an operand, 2^-134 at most.  Where that may count the tile is computed
-// again by fp32 MFMAs, in the order of the kernel above: an operand of 2^56 or more, a sum that is not finite, one
-// below 2^-40.  Zeros among these stand where all of their column are and its first weights too, as padding's;
-// looking through all of a column's weights took 10 to 50 us of a launch with padding, a maximum of W's values beside
-// the one of both 20 % of the products.
+// Behind bf16's numbers 2^-134 of an operand is lost at most; computed again from an operand of 2^56 or a sum below
+// 2^-40 on.  (A maximum of W's values beside the one of both took 20 % of the products.)
 template <int MODE, int MT, int WN, int WK, int D>
 __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
@@ -653,70 +745,183 @@ __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_
     constexpr int l = decltype(ic)::v + 1;
     if (MODE == GG_UP || MODE == GG_DOWN ? live == l : l == MT) steps(std::integral_constant<int, l>{});
   });
-  bool exact = big >= 0x1p56f;
+  f32x4 sum[MT][1];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    acc[0][i] += acc[1][i];
+  for (int i = 0; i < MT; ++i) sum[i][0] = acc[0][i] + acc[1][i];
+  split_tail<MODE, 1, MT, WN, 1, WK>(p, t, smem, sum, first, T, big >= 0x1p56f, nullptr, 0x1p-40f);
+}
+
+// Long sums, on two fp16 terms: scale x = hi + lo / 2048, both rounded to nearest, 22 bits of x and more (4e-8 of it off
+// on average), hi infinite from 65520 / scale on, x off by up to 2^-36 / scale instead below 2^-14 / scale.
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+constexpr float LO = 2048.f, SCALE_A = 4.f, SCALE_W = 256.f;
+constexpr float LEAST_A = 0x1p-11f / SCALE_A, LEAST_W = 0x1p-11f / SCALE_W;
+__device__ __forceinline__ void split2(f32x4 x, float scale, f16x4& hi, f16x4& lo, float& most) {
+  most = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), most);
+  most = fmaxf(fmaxf(fabsf(x[2]), fabsf(x[3])), most);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float v = fabsf(acc[0][i][q]);
-      exact |= !(v >= 0x1p-40f && v < INFINITY) && (MODE == GG_F32 || MODE == GG_ADD || i < live);
-    }
+  for (int e = 0; e < 4; ++e) hi[e] = (_Float16)__builtin_fmaf(x[e], scale, 0.f);
+  asm("" : "+v"(hi));  // (pairs as they are: otherwise every second one is converted again for its rest)
+#pragma unroll
+  for (int e = 0; e < 4; ++e) lo[e] = (_Float16)__builtin_fmaf(__builtin_fmaf(x[e], scale, -(float)hi[e]), LO, 0.f);
+}
+
+template <int N, class F>
+__device__ __forceinline__ void count_up(F f) {  // f(0) .. f(N - 1)
+  if constexpr (N > 0) {
+    count_up<N - 1>(f);
+    f(Int<N - 1>{});
   }
-  exact = __syncthreads_or(exact);
-  if (exact) {  // for zeros alone only where the column has other sums, or W values in the part's first k-step
-    int zero = 0, other = 0, some = big >= 0x1p56f;
+}
+
+// 16 MT WM x 16 NT WN tiles with half of the kernel above's products: hi hi, in two chains, and hi lo + lo hi.  A value takes 4
+// operations to split instead of 6, which go on for the next k-step between this one's MFMAs; PF k-steps are loaded ahead of that.
+// The two chains make up for what the terms leave out: off 64 bits by (before) K = 1024 1.65e-7 (1.94e-7) of the result, K = 2048
+// 2.2e-7 (2.7e-7), in two parts 1.73e-7 (1.94e-7), in three 1.49e-7 (1.50e-7), K = 5632 3.5e-7 (4.7e-7), SiLU of two, K = 2048
+// 3.4e-7 (4.3e-7); with one chain 2.2e-7 at K = 1024.  Shorter ones are left to the kernel above: K = 544 1.38e-7 (1.30e-7).
+// Bound by what a CU takes in.  W goes through LDS like A, in whole lines: loaded straight into fragments (16 rows of 64 bytes
+// an instruction), 1000 x 11264 x 2048 on 64 x 128 took 230 us, without the splitting 216, without the MFMAs 200, without both 203,
+// without loads behind the first ones 136; through LDS 208 to 225, and 176 on 128 x 128.  Waves of 32 x 32 read least from LDS.
+// Against the kernel above: 500 x 1985 x 2048 40.3 -> 31.3 us, 565 x 2048 41.2 -> 31.5, 961 x 2048 58.3 -> 45.6, 565 x 4160 75 -> 48,
+// 1000 x 11264 258 -> 176, 565 x 2624 51 -> 43; 2260 rows over 32 experts of 2048 x 1024 and 565 through a shared one of 2048 up
+// 259 -> 201, down 126 -> 106, 5600 and 1400 rows 452 -> 356 and 245 -> 190.  For experts 96 rows a tile, the few rows behind
+// a full one with it, were behind, with their registers at two waves a SIMD (up 472, down 240 with the most rows).
+// Rows of A or columns of W whose largest value is too small for terms of 22 bits, and what split_tail names: computed again.
+template <int MODE, int WM, int MT, int WN, int NT, int WK, int PF, int OCC>
+__global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_kernel(GgParams p) {
+  using namespace gg;
+  constexpr int TM = 16 * MT * WM, TN = 16 * NT * WN, BKF = 32, CLD = TN + 4, PLANE = (TM + TN) * 64, SLOT = 2 * PLANE;
+  constexpr int RQ = 8 * WM * WN, QA = (TM + RQ - 1) / RQ, QW = TN / RQ;  // rows that a part's threads bring at a time
+  constexpr int IMAGE = TM * CLD, SMEM = WK * (2 * SLOT > IMAGE * 4 ? 2 * SLOT : IMAGE * 4);
+  static_assert(TN % RQ == 0, "whole passes over W");
+  __shared__ __attribute__((aligned(16))) char smem[SMEM];
+  __shared__ float wmax[WK * TN];
+  Tile t = locate<MODE, TM, TN>(p);
+  if (!t.live) return;
+  resolve<MODE, float>(p, t);
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int wn = wave % WN, wm = wave / WN % WM, part = wave / (WN * WM), tid = threadIdx.x % (64 * WM * WN);
+  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16) - wm * MT;  // of this wave's tiles
+  // this part's k-steps; the first part has as many as any
+  const int KT = t.K / BKF, most = (KT + WK - 1) / WK, first = part * most, T = max(0, min(most, KT - first));
+  // thread i brings four k's of rows i / 8, i / 8 + RQ .. of W and of A: whole lines
+  const int row = tid >> 3, ac = tid & 7;
+  constexpr int UNITS = QW + QA;
+  const float* src[UNITS];
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u)
+    src[u] = (u < QW ? static_cast<const float*>(t.W) + (long)min(t.n0 + row + RQ * u, t.N - 1) * t.ldw
+                     : static_cast<const float*>(t.A) + a_row<MODE>(p, t, row + RQ * (u - QW)) * t.lda) + first * BKF + 4 * ac;
+  auto at = [&](int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4); };  // in a plane: W's rows, A's
+
+  f32x4 acc[3][MT][NT];  // hi hi of even and of odd k-steps, 2048 times the others
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float v = fabsf(acc[0][i][q]);
-        zero |= v == 0.f && (MODE == GG_F32 || MODE == GG_ADD || i < live);
-        other |= v > 0.f;
-        some |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
+      for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float largest[UNITS] = {};
+  f32x4 raw[PF][UNITS];
+  char* const slots = smem + part * 2 * SLOT;
+  auto load = [&](int u, int kt, int ring) {  // (behind the last k-step: that one again)
+    raw[ring][u] = *reinterpret_cast<const f32x4*>(src[u] + (long)min(kt, T - 1) * BKF);
+  };
+  char* const put = slots + at(row, ac & 3) + (ac >> 2) * 8;  // chunk g: k's 4 g and 16 + 4 g (RQ rows on: the same chunk)
+  auto part_up = [&](int u, int ring, int slot) {
+    if (TM % RQ && u == UNITS - 1 && row + RQ * (QA - 1) >= TM) return;
+    f16x4 hi, lo;
+    split2(raw[ring][u], u < QW ? SCALE_W : SCALE_A, hi, lo, largest[u]);
+    char* b = put + slot * SLOT + (u < QW ? RQ * u : TN + RQ * (u - QW)) * 64;
+    *reinterpret_cast<u32x2*>(b) = __builtin_bit_cast(u32x2, hi);
+    *reinterpret_cast<u32x2*>(b + PLANE) = __builtin_bit_cast(u32x2, lo);
+  };
+  auto steps = [&](auto L) {
+    auto step = [&](int kt, auto unroll) {
+      constexpr int U = decltype(unroll)::v, S = U & 1, R = (U + 1) % PF, GROUPS = L < 2 ? 1 : (L + 1) / 2;
+      __syncthreads();  // k-step kt is in its slot, the other one's reads are done
+      if (WK > 1 && kt >= T) return;
+      const char* b = slots + S * SLOT;
+      f16x8 wf[NT][2];
+      if constexpr (L > 0) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) wf[j][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at((wn * NT + j) * 16 + r, g));
       }
-    zero |= __shfl_xor(zero, 16);
-    zero |= __shfl_xor(zero, 32);
-    if (zero && T > 0) {
-      const f32x4 u = *reinterpret_cast<const f32x4*>(wp), v = *reinterpret_cast<const f32x4*>(wp + 16);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) other |= u[e] != 0.f || v[e] != 0.f;
-    }
-    exact = __syncthreads_or(some || (zero && other));
-  }
-  if (exact) {
-#pragma unroll 1
-    for (int i = 0; i < live; ++i) {
-      const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;
-      f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 1
-      for (int k = 0; k < T * BKF; k += BKF)
+      for (int i0 = 0; i0 < 2 * GROUPS; i0 += 2) {
+        f16x8 af[2][2];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const f32x4 av = *reinterpret_cast<const f32x4*>(a + k + 16 * h), wv = *reinterpret_cast<const f32x4*>(wp + k + 16 * h);
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[h], 0, 0, 0);
+          for (int i = i0; i < min((int)L, i0 + 2); ++i)
+            af[i - i0][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at(TN + (wm * MT + i) * 16 + r, g));
+#pragma unroll
+        for (int u = i0 / 2 * UNITS / GROUPS; u < (i0 / 2 + 1) * UNITS / GROUPS; ++u) {
+          part_up(u, R, S ^ 1);
+          load(u, kt + 1 + PF, R);
         }
 #pragma unroll
-      for (int h = 0; h < MT; ++h)
-        if (h == i) acc[0][h] = s[0] + s[1];
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int i = i0; i < min((int)L, i0 + 2); ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+              f32x4& s = acc[c ? 2 : S][i][j];
+              s = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i - i0][c >> 1], wf[j][c & 1], s, 0, 0, 0);
+            }
+      }
+      // an MFMA, a part of the splitting, and so on; a pair of tiles' reads in front of its first
+      if constexpr (L > 0) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT, 0);
+#pragma unroll
+        for (int i = 0; i < 3 * L * NT; ++i) {
+          if (i % (6 * NT) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, (UNITS * 16 + 3 * L * NT - 1) / (3 * L * NT), 0);
+        }
+      }
+    };
+    int kt = 0;
+    for (; kt + 2 <= most; kt += 2) count_up<2>([&](auto u) { step(kt + decltype(u)::v, u); });
+    if (kt < most) step(kt, Int<0>{});
+  };
+  if (WK == 1 || T > 0) {
+#pragma unroll
+    for (int d = 0; d < PF; ++d)
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) load(u, d, d);
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      part_up(u, 0, 0);
+      load(u, PF, 0);
     }
   }
-  float* ct = reinterpret_cast<float*>(smem);
+  if constexpr (MODE == GG_UP || MODE == GG_DOWN) {
+    count_up<MT + 1>([&](auto ic) {
+      constexpr int l = decltype(ic)::v;
+      if (min(max(live, 0), MT) == l) steps(std::integral_constant<int, l>{});
+    });
+  } else {
+    steps(std::integral_constant<int, MT>{});
+  }
+  bool small = false;
+#pragma unroll
+  for (int u = 0; u < UNITS; ++u) {  // of a row's eight threads
+    float& m = largest[u];
+#pragma unroll
+    for (int d = 1; d < 8; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+    small |= m > 0.f && m < (u < QW ? LEAST_W : LEAST_A);
+    if (u < QW && ac == 0) wmax[part * TN + row + RQ * u] = m;
+  }
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) ct[part * IMAGE + (i * 16 + 4 * g + q) * CLD + w * 16 + r] = acc[0][i][q];
-  __syncthreads();
-  if constexpr (WK > 1) {
-    for (int c = threadIdx.x; c < IMAGE / 4; c += 64 * WN * WK) {
-      f32x4* o = reinterpret_cast<f32x4*>(ct) + c;
-#pragma unroll
-      for (int i = 1; i < WK; ++i) *o += o[i * (IMAGE / 4)];
-    }
-    __syncthreads();
-  }
-  f32_epilogue<MODE, TM, TN, 64 * WN * WK>(p, t, ct);
+    for (int j = 0; j < NT; ++j)
+      acc[0][i][j] = (acc[0][i][j] + acc[1][i][j] + acc[2][i][j] * (1.f / LO)) * (1.f / (SCALE_A * SCALE_W));
+  split_tail<MODE, WM, MT, WN, NT, WK>(p, t, smem, acc[0], first, T, small, wmax + part * TN, 0x1p-36f);
 }
 
 // Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.
@@ -948,7 +1153,16 @@ static hipError_t gg_split_on(const GgParams& p, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The split kernel's tile: what its blocks take in rounds of 256, in us at K = 2048 (fixed part, a round), as
+template <int MODE, int WM, int MT, int WN, int NT, int WK, int PF, int OCC>
+static hipError_t gg_half_on(const GgParams& p, hipStream_t st) {
+  const long blocks = gg_blocks(p, MODE, 16 * MT * WM, 16 * NT * WN);
+  if (blocks)
+    hipLaunchKernelGGL((group_gemm_f32_half_kernel<MODE, WM, MT, WN, NT, WK, PF, OCC>), dim3((unsigned)blocks),
+                       dim3(64 * WM * WN * WK), 0, st, p);
+  return hipGetLastError();
+}
+
+// The split kernels' tiles: what their blocks take in rounds of 256, in us at K = 2048 (fixed part, a round), as
 // measured over 100 .. 1500 rows of 2048 .. 11264 columns.  565 rows of 2048 columns: 48 x 64 47.3 us, 64 x 64 52.0,
 // 80 x 64 43.3, 48 x 128 47.7; 300 of 2048 48 x 64 in two parts of K 33.7, in four 29.0; 565 of 4160
 // 48 x 128 86, 80 x 128 100, 96 x 128 73; 1000 of 2048 64 x 64 67.7, 64 x 128 61.0; of 4160 80 x 128 117, 96 x 128
@@ -959,11 +1173,18 @@ struct SplitTile {
 };
 static const SplitTile SPLIT_TILES[] = {{32, 64, 4, 1, 21}, {48, 64, 4, 1, 27}, {64, 64, 2, 4, 28}, {80, 64, 3, 0, 41},
                                         {48, 128, 1, 2, 42}, {64, 128, 1, 4, 48}, {80, 128, 1, 0, 59}, {96, 128, 1, 0, 70}};
-static int split_tile(const GgParams& p) {
+// Two fp16 terms: K of 1024 and more, of which a part has 682 (the kernel has both errors), in no fewer parts than three
+// terms would take (sums of 1024 in one part are 1.7e-7 off, in three on three terms 1.1e-7), where that is ahead: 100 rows
+// of 2048 on 64 x 64 27.2 us, on three terms and 32 x 64 22.8.  48 x 128 never is: 565 rows of 2560 44.8, on 64 x 128 39.8.
+static const SplitTile HALF_TILES[] = {{64, 64, 2, 6, 22}, {80, 64, 3, 3, 29}, {64, 128, 1, 8, 34}, {96, 128, 1, 0, 49}, {128, 128, 1, 0, 57}};
+static bool half_terms(int K, int parts) { return K >= 1024 && K >= 682 * parts; }
+static int split_tile(const GgParams& p) {  // of SPLIT_TILES, or behind them
   int best = 0;
   long least = 0;
-  for (int i = 0; i < 8; ++i) {
-    const SplitTile& t = SPLIT_TILES[i];
+  for (int i = 0, parts = 0; i < 13; ++i) {
+    const SplitTile& t = i < 8 ? SPLIT_TILES[i] : HALF_TILES[i - 8];
+    if (i == 8) parts = SPLIT_TILES[best].parts;
+    if (i >= 8 && (t.parts < parts || !half_terms(p.K, t.parts))) continue;
     const long cost = t.fixed + (gg_blocks(p, GG_F32, t.rows, t.cols) + 255) / 256 * t.round;
     if (i == 0 || cost < least) best = i, least = cost;
   }
@@ -1022,7 +1243,14 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
         case 4: return gg_split_on<MODE, 3, 8, 1, 3>(p, st);
         case 6: return gg_split_on<MODE, 5, 8, 1, 2>(p, st);
         case 7: return gg_split_on<MODE, 6, 8, 1, 2>(p, st);
+        case 8: return gg_half_on<MODE, 2, 2, 2, 2, 2, 1, 4>(p, st);
+        case 9: return gg_half_on<MODE, 1, 5, 4, 1, 3, 1, 3>(p, st);
+        case 10: return gg_half_on<MODE, 2, 2, 4, 2, 1, 1, 4>(p, st);
+        case 11: return gg_half_on<MODE, 2, 3, 4, 2, 1, 2, 2>(p, st);
+        case 12: return gg_half_on<MODE, 2, 4, 4, 2, 1, 2, 2>(p, st);
       }
+    } else if (half_terms(min(p.K, p.Ns > 0 ? p.Ks : p.K), 1)) {
+      return gg_half_on<MODE, 2, 2, 4, 2, 1, 2, 4>(p, st);
     }
     return gg_split_on<MODE, 4, 8, 1, 3>(p, st);
   }
@@ -1045,11 +1273,12 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
   return gg_f32_on<MODE, 4>(p, addr64, st);
 }
 
-// Rows and columns of the tiles of M x N fp32 results, and parts of K (tests)
-extern "C" void lsd_group_gemm_split_tile(int M, int N, int* tile) {
+// Rows and columns of the tiles of M x N fp32 results of K products (0: few), and parts of K (tests)
+extern "C" void lsd_group_gemm_split_tile(int M, int N, int K, int* tile) {
   GgParams p{};
-  p.M = M, p.N = N, p.groups = 1;
-  const SplitTile& t = SPLIT_TILES[split_tile(p)];
+  p.M = M, p.N = N, p.K = K, p.groups = 1;
+  const int i = split_tile(p);
+  const SplitTile& t = i < 8 ? SPLIT_TILES[i] : HALF_TILES[i - 8];
   tile[0] = t.rows, tile[1] = t.cols, tile[2] = t.parts;
 }
 

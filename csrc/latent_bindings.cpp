@@ -24,7 +24,7 @@ using lsd::RowsParams;
 extern "C" {
 hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStream_t st);
 hipError_t lsd_group_gemm_f32(const GgParams* p, int mode, hipStream_t st);
-void lsd_group_gemm_split_tile(int M, int N, int* tile);
+void lsd_group_gemm_split_tile(int M, int N, int K, int* tile);
 int lsd_moe_on_split(int T, int top, int n_tiles, int N, int Ns, int K);
 hipError_t lsd_moe_gemv_up(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_moe_gemv_down(const MoeGemvParams* p, hipStream_t st);
@@ -624,11 +624,11 @@ void lsd_register_latent(pybind11::module& m) {
   m.def("batch_linear", &batch_linear, py::arg("a"), py::arg("w"), py::arg("tm"), py::arg("gate") = py::none());
   m.def("linear_fp32", &linear_fp32, py::arg("a"), py::arg("w"), py::arg("x") = py::none(),
         py::arg("bias") = py::none());
-  m.def("fp32_tile", [](int64_t M, int64_t N) {
+  m.def("fp32_tile", [](int64_t M, int64_t N, int64_t K) {
     std::array<int, 3> t;
-    lsd_group_gemm_split_tile((int)M, (int)N, t.data());
+    lsd_group_gemm_split_tile((int)M, (int)N, (int)K, t.data());
     return std::make_tuple(t[0], t[1], t[2]);
-  });
+  }, py::arg("M"), py::arg("N"), py::arg("K") = 0);
   m.def("moe_on_split", [](int64_t T, int64_t top, int64_t n_tiles, int64_t N, int64_t Ns, int64_t K) {
     return lsd_moe_on_split((int)T, (int)top, (int)n_tiles, (int)N, (int)Ns, (int)K) != 0; });
   m.def("moe_group", &moe_group, py::arg("ids"), py::arg("experts"), py::arg("tm"));

@@ -1,0 +1,127 @@
+"""fp32 products on two fp16 terms against 64 bits.
+
+A sum of K products in fp32 is off by at most (K + 2) ulp of the sum of the products' sizes, in any order (ulp:
+2^-24); terms of 22 bits leave 2^-22 of each product, four ulp, and their low ones' product 2^-22 more.
+"""
+
+import pytest
+import torch
+
+from .test_timisun_gpu import C, rand  # noqa: F401
+
+DEV, F64, ULP = "cuda:0", torch.float64, 2.0 ** -24
+
+
+def near(got, a, w):
+    want, size = a.to(F64) @ w.to(F64).T, a.to(F64).abs() @ w.to(F64).abs().T
+    return bool(((got.cpu().to(F64) - want).abs() <= (a.shape[1] + 14) * ULP * size).all())
+
+
+# every tile: its edges, parts of K that are even and uneven
+TILES = [(500, 1985, 1376, (64, 64, 2)), (449, 2048, 2080, (64, 64, 2)), (561, 2048, 2048, (80, 64, 3)), (565, 2000, 2144, (80, 64, 3)),
+         (961, 2048, 1024, (64, 128, 1)), (513, 2600, 1056, (64, 128, 1)), (561, 4160, 1024, (96, 128, 1)),
+         (222, 11264, 1088, (128, 128, 1))]
+
+
+def test_tiles():
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    assert [_C.fp32_tile(M, N, K) for M, N, K, _ in TILES] == [t for *_, t in TILES]
+    # short K and sums that would be in fewer parts stay on three terms
+    assert _C.fp32_tile(961, 2100, 992) == _C.fp32_tile(961, 2100) and _C.fp32_tile(100, 2048, 2048) == (32, 64, 4)
+    assert _C.fp32_tile(300, 2048, 2048) == (48, 64, 4) and _C.fp32_tile(565, 2048, 1024) == (80, 64, 3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile", TILES)
+def test_products(C, M, N, K, tile):  # noqa: F811
+    a, w, b = rand(M, K, seed=1), rand(N, K, seed=2) * 0.02, rand(N, seed=3)
+    got = C.linear_fp32(a.to(DEV), w.to(DEV)).cpu()
+    assert near(got, a, w)
+    want = a.to(F64) @ w.to(F64).T
+    # not behind three bf16 terms, whose sums are 1.3e-7 to 2e-7 of the result off here
+    assert float((got.to(F64) - want).norm() / want.norm()) < 2e-7
+    x = rand(M, N, seed=4)
+    y = x.to(DEV).clone()
+    C.linear_fp32(a.to(DEV), w.to(DEV), y)
+    assert float((y.cpu().to(F64) - x.to(F64) - want).abs().max()) < (K + 14) * ULP * float((a.abs() @ w.abs().T).max())
+    assert torch.equal(C.linear_fp32(a.to(DEV), w.to(DEV), None, b.to(DEV)).cpu(), got + b)
+
+
+# rows and columns that leave the terms' range, alone and beside others, are computed again
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile", [TILES[0], TILES[2], TILES[4], TILES[6], TILES[7]])
+@pytest.mark.parametrize("scale", [2.0 ** -140, 2.0 ** -40, 2.0 ** -16, 2.0 ** 13, 2.0 ** 60])
+def test_sizes(C, M, N, K, tile, scale):  # noqa: F811
+    a, w = rand(M, K, seed=1).clamp(-1, 1), rand(N, K, seed=2).clamp(-1, 1) * 0.02
+    a[5:100:30] *= scale
+    big = w * (2.0 ** 50 if scale < 2.0 ** -100 else 1.0)
+    assert near(C.linear_fp32(a.to(DEV), big.to(DEV)), a, big)
+    w[3:90:29] *= scale
+    w[7] = 0
+    a[5:100:30] = rand(4, K, seed=3) * (2.0 ** 50 if scale < 2.0 ** -100 else 1.0)
+    got = C.linear_fp32(a.to(DEV), w.to(DEV))
+    rows = slice(5, 100, 30) if scale < 2.0 ** -100 else slice(None)  # (products of the others are below fp32's numbers)
+    assert near(got[rows], a[rows], w) and int(got[:, 7].count_nonzero()) == 0
+
+
+@pytest.mark.gpu
+def test_lone_small_values(C):  # noqa: F811
+    """Small values of a row beside which the weights are zeros: sums of their own size."""
+    M, N, K, _ = TILES[4]
+    a, w = rand(M, K, seed=1), torch.zeros(N, K)
+    a[:, 100], w[:, 100] = 2.0 ** -45, 1.0
+    got = C.linear_fp32(a.to(DEV), w.to(DEV))
+    assert near(got, a, w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 65504.0, -3e38])
+@pytest.mark.parametrize("side", ["a", "w"])
+def test_not_finite(C, side, value):  # noqa: F811
+    M, N, K, _ = TILES[0]
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2)
+    (a if side == "a" else w)[40, 50] = value
+    w[3, 50] = a[5, 50] = 0.5
+    want, got = a @ w.T, C.linear_fp32(a.to(DEV), w.to(DEV)).cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    size = a.nan_to_num(0, 0, 0).abs() @ w.nan_to_num(0, 0, 0).abs().T
+    assert bool(((got - want).abs()[ok] <= 2 * (K + 14) * ULP * size[ok]).all())
+
+
+# experts of 1024 columns and more: full and part full tiles, beside a shared expert
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,H,F,Fs", [(290, 3, 1024, 1088, 1024), (150, 2, 1056, 1024, 0)])
+def test_experts(C, T, E, H, F, Fs):  # noqa: F811
+    H = (H + 63) // 64 * 64
+    h, up, dn = rand(T, H, seed=1), rand(E, 2 * F, H, seed=2) * 0.05, rand(E, H, F, seed=3) * 0.05
+    top = 2
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int()
+    ids[: T // 3, 0], ids[: T // 3, 1] = 0, 1
+    wts = torch.rand(T, top)
+    shared_up, shared_dn = (rand(2 * Fs, H, seed=4) * 0.05, rand(H, Fs, seed=5) * 0.05) if Fs else (None, None)
+    order, tiles = C.moe_group(ids.to(DEV), E, 64)
+    for N, Ns, K in ((2 * F, 2 * Fs, H), (H, H if Fs else 0, F)):
+        assert C.moe_on_split(T, top, tiles.shape[0], N, Ns, K) or K < 2 * F
+    dev = lambda t: None if t is None else t.to(DEV)  # noqa: E731
+    mid, mids = C.moe_up(h.to(DEV), order, tiles, top, up.to(DEV), 0.0, 1.0, dev(shared_up), 0.0, 64)
+    slab = torch.empty(top + bool(Fs), T, H, device=DEV)
+    C.moe_down(mid, mids if Fs else None, order, tiles, wts.to(DEV), dn.to(DEV), dev(shared_dn), slab, 64)
+
+    def gated(x, w):
+        y = (x @ w.to(F64).T).reshape(len(x), -1, 2, 16)
+        return (y[:, :, 0] * torch.sigmoid(y[:, :, 0]) * y[:, :, 1]).reshape(len(x), -1)
+
+    def close(got, want):  # sums of some thousand products: 1e-6 of the largest, and twice in front of a gate
+        assert float((got.cpu().to(F64) - want).abs().max()) < 4e-6 * float(want.abs().max())
+    perm, x = order.cpu().long()[: T * top], h.to(F64)
+    token, expert = perm // top, ids.reshape(-1)[perm]
+    if Fs:
+        close(mids, gated(x, shared_up))
+        close(slab[top], mids.cpu().to(F64) @ shared_dn.to(F64).T)
+    for e in range(E):
+        mine = (expert == e).nonzero()[:, 0]
+        close(mid.cpu()[mine], gated(x[token[mine]], up[e]))
+        want = wts.reshape(-1)[perm[mine]].to(F64)[:, None] * (mid.cpu()[mine].to(F64) @ dn[e].to(F64).T)
+        close(slab[:top].cpu()[perm[mine] % top, token[mine]], want)

@@ -9,14 +9,17 @@
 //    With two, W arrives at half the rate.  Wide tiles of up to 64 rows load W non-temporally
 //    (28672 x 4096 at 40 rows 49.5 -> 44.0 us, 4096 x 14336 23.0 -> 21.3); narrow ones, whose
 //    weights are small, and more rows are 0 to 20 % slower that way.
+//  * rows of W that lie powers of two apart: blocks that walk through K together stand at the same place of
+//    all of them, and where they all start at once W arrives at 4.9 to 5.5 TB/s.  Each column tile then starts its sums
+//    elsewhere (deep_turn): 16384 x 4096 of 24 rows 25.9 -> 21.9 us, 32000 x 2048 26.3 -> 23.1, 11264 x 2048 11.2 -> 10.6.
 //  * a block holds all of up to 64 rows; more are also divided among blocks beside each other,
-//    which find W in L2, where that brings a CU fewer bytes.  Its width (96 to 16 columns)
+//    which find W in L2, where that brings a CU fewer bytes.  Its width (128 to 16 columns)
 //    follows from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
 //    32-wide parts among them (WK) and are summed through LDS.  No K splits over blocks, no
 //    tickets and no workspace, except where the caller takes the partial sums as slabs.
 //
 // Alone, cold weights, before (split-K with the weights in registers; 128 x 64 ring) -> now:
-//   28672 x 4096 gate/up, 40 rows   65.9 -> 44.0 us     4096 x 14336 slabs, 40 rows  28.8 -> 21.3
+//   28672 x 4096 gate/up, 40 rows   65.9 -> 37.8 us     4096 x 14336 slabs, 40 rows  28.8 -> 21.3
 //   6144 x 4096 QKV, 40 rows        18.7 -> 14.4        4096 x 4096 slabs, 40 rows   15.0 -> 8.7
 //   6144 x 2048, 24 rows            12.2 -> 7.6         2624 x 2048 fp32, 64 rows    13.1 -> 7.5
 //   11264 x 2048 gate/up, 96 rows   19.8 -> 16.8        4800 x 1600 QKV, 128 rows    13.6 -> 9.4
@@ -34,8 +37,9 @@ constexpr int NT_LOAD = 2;  // cache policy of an LDS-DMA: non-temporal
 // k-step of BK; SLOTS k-steps in LDS; AUX: cache policy of W; ONE: a block holds all rows (a row
 // block found at run time, by a division, costs 0.3 us a launch: 40 rows of GPT-2 XL 2274 -> 2211 us
 // a step without).
+// turn: a column tile starts its sums at another k than its neighbours.
 template <int WM, int WN, int WK, int MTW, int NTW, int BK, int SLOTS, int AUX, int EPI, bool ONE>
-__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams p, int tiles_n, int row_blocks) {
+__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams p, int tiles_n, int row_blocks, int turn) {
   constexpr int WAVES = WM * WN * WK, BM = 16 * WM * MTW, BN = 16 * WN * NTW;
   constexpr int RB = BK * 2, CPR = RB / 16, RPI = 64 / CPR;  // bytes and 16-byte chunks of a row, rows per instruction
   constexpr int A_BYTES = BM * RB, SLOT = (BM + BN) * RB;
@@ -73,7 +77,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_deep_kernel(GemmParams
     dstw[q] = A_BYTES + ins * 1024;
     srcw[q] = p.W + (long)min(n0 + row, p.N - 1) * p.ldw + (((lane % CPR) ^ swz(row)) << 3);
   }
+  const int from = (nb * 5 & 31) & turn;  // (turn: 31, of at least 32 k-steps, or 0)
   auto issue = [&](int kt, int slot) {
+    kt += from;
+    kt = kt >= KT ? kt - KT : kt;
 #pragma unroll
     for (int q = 0; q < LW; ++q)
       __builtin_amdgcn_global_load_lds((gbl_cvoid*)(srcw[q] + (long)kt * BK), (lds_void*)(smem + slot * SLOT + dstw[q]),
@@ -194,7 +201,7 @@ static int deep_cols(int M, int N, int K, int splits, int epi) {
 //   128 rows  4800 x 1600 11.8 -> 9.4 (48 x 64), 6144 x 4096 24.9 -> 21.9 (48 x 80)
 //   256 rows  4800 x 1600 14.1 -> 11.9 (64 x 80), 11264 x 2048 gate/up 30.8 -> 27.3 (64 x 96)
 // and over 176 products of 50 to 256 rows 7 % on average.  Each of these shapes adds up K as the
-// ones that hold all rows do, so the bits are the same.  (32 x 32 for 49 to 64 rows, 2624 x 2048 8.3 -> 7.6
+// ones that hold all rows do, so the bits are the same, where column tiles all start at the first k.  (32 x 32 for 49 to 64 rows, 2624 x 2048 8.3 -> 7.6
 // us, does not: it halves the k-steps among two waves where 16 columns had four, and a router
 // behind it decided close calls otherwise; with four waves it is no faster.)  Behind, by 0.2 us, 768 x 3072 in 8 slabs of
 // 128 rows (4.7 us).
@@ -202,9 +209,13 @@ static int deep_cols(int M, int N, int K, int splits, int epi) {
 // a fifth more with 64 x 80 at 256 rows than with 128 x 64.  GPT-2 XL in two lanes, all rows in a block
 // against here, tokens a second: 256 rows a lane 52.6 and 51.9 thousand, 200 48.5 and 48.6, 160 44.9 and
 // 44.2, 144 43.4 and 43.8, 128 40.0 and 41.4, 96 36.7 and 37.0.
+// Up to 128 rows also 128 columns, which take in A half as often (us on 64 columns -> 128, both where deep_turn lets them start
+// elsewhere): 28672 x 4096, 16 / 32 / 48 / 64 rows 38.7 39.8 42.6 47.1 -> 36.2 36.8 37.8 39.1; 32000 x 2048, 48 rows 24.9 -> 24.1, 96
+// 33.6 -> 28.8, 128 36.3 -> 30.5; 128256 x 4096, 48 rows 190 -> 174; 50304 x 1600, 48 rows 36.1 -> 32.2; but 40960 x 1600, where they
+// cost more, 27.5 and 30.0.
 static DeepShape deep_shape(int M, int N, int K, int splits, int epi, int lanes) {
   DeepShape best{deep_rows(M), deep_cols(M, N, K, splits, epi)};
-  if (M <= 64 || (M >= 160 && lanes > 1)) return best;
+  if (M >= 160 && lanes > 1) return best;
   auto cost = [&](DeepShape s) {
     const long blocks = (long)((N + s.cols - 1) / s.cols) * splits * ((M + s.rows - 1) / s.rows);
     return (blocks + 255) / 256 * (s.rows + s.cols);
@@ -214,20 +225,30 @@ static DeepShape deep_shape(int M, int N, int K, int splits, int epi, int lanes)
     if (epi == EPI_SILU_MUL && s.cols % 32 != 0) return;
     if (cost(s) < least) { best = s; least = cost(s); }
   };
+  if (M <= 128 && (epi == EPI_SILU_MUL || epi == EPI_F32 || epi == EPI_BF16 || epi == EPI_GELU)) offer({best.rows, 128});
+  if (M <= 64) return best;
   for (int cols : {32, 64, 80, 96})
     if (cols < 96 || M <= 96) offer({48, cols});
   for (int cols : {64, 80, 96}) offer({64, cols});
   return best;
 }
 
+// Column tiles start at places of K of their own where W's rows lie whole 4 KB apart and all blocks, two a CU, start
+// at once.  Later ones are out of step by themselves (128256 x 4096, 48 rows of 128 columns 174 us, turned 190), as are rows of other
+// strides (K = 1600, 768: up to 4 % slower turned), and 32 columns gain too little (6144 x 4096 14.3 and 14.9).
+static bool deep_turn(const GemmParams& p, long blocks, int cols) {
+  return p.splits == 1 && p.K >= 2048 && p.K % 2048 == 0 && p.ldw % 2048 == 0 && cols >= 64 && blocks <= 512;
+}
+
 template <int EPI>
 static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
   const DeepShape s = deep_shape(p.M, p.N, p.K, p.splits, EPI, p.lanes);
   const int tn = (p.N + s.cols - 1) / s.cols, mbs = (p.M + s.rows - 1) / s.rows;
+  const int turn = deep_turn(p, (long)tn * mbs, s.cols) ? 31 : 0;
 #define LSD_DEEP_K(ONE, ROWS, COLS, WM, WN, WK, BK, SLOTS, AUX)                                                       \
   if (s.rows == ROWS && s.cols == COLS) {                                                                             \
     hipLaunchKernelGGL((gemm_deep_kernel<WM, WN, WK, ROWS / (16 * WM), COLS / (16 * WN), BK, SLOTS, AUX, EPI, ONE>),  \
-                       dim3((unsigned)(tn * p.splits * mbs)), dim3(64 * WM * WN * WK), 0, st, p, tn, mbs);            \
+                       dim3((unsigned)(tn * p.splits * mbs)), dim3(64 * WM * WN * WK), 0, st, p, tn, mbs, turn);            \
     return hipGetLastError();                                                                                         \
   }
   // slots: two blocks per CU
@@ -236,6 +257,14 @@ static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
     LSD_DEEP_K(true, 48, 32, 1, 2, 2, 64, 8, 0)
     if constexpr (EPI != EPI_SILU_MUL) {
       LSD_DEEP_K(true, 48, 16, 1, 1, 4, 128, 5, 0)
+    }
+    if constexpr (EPI == EPI_SILU_MUL || EPI == EPI_F32 || EPI == EPI_BF16 || EPI == EPI_GELU) {
+      LSD_DEEP_K(true, 16, 128, 1, 4, 1, 64, 3, NT_LOAD)
+      LSD_DEEP_K(true, 32, 128, 1, 4, 1, 64, 3, NT_LOAD)
+      LSD_DEEP_K(true, 48, 128, 1, 4, 1, 64, 3, NT_LOAD)
+      LSD_DEEP_K(true, 64, 128, 1, 4, 1, 64, 3, NT_LOAD)
+      LSD_DEEP_K(true, 96, 128, 2, 4, 1, 64, 4, 0)
+      LSD_DEEP_K(true, 128, 128, 2, 4, 1, 64, 4, 0)
     }
     LSD_DEEP_K(true, 16, 64, 1, 4, 1, 64, 8, NT_LOAD)
     LSD_DEEP_K(true, 32, 64, 1, 4, 1, 64, 6, NT_LOAD)

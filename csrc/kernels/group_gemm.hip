@@ -822,11 +822,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Experts: each column tile starts its sums at another k than its neighbours and than the next expert, so that blocks under way
+  // together do not stand at the same place of rows that lie powers of two apart (the sizes above: up 204 -> 195 us, down
+  // 112 -> 101; 300 tokens 146 -> 131 and 82 -> 75, 1400 359 -> 351 and 196 -> 186; others up to 10 % faster and slower)
+  const int from = (MODE == GG_UP || MODE == GG_DOWN) && T > 0 ? (t.n0 / TN * 11 + t.group * 7) % T : 0;
   float largest[UNITS] = {};
   f32x4 raw[PF][UNITS];
   char* const slots = smem + part * 2 * SLOT;
   auto load = [&](int u, int kt, int ring) {  // (behind the last k-step: that one again)
-    raw[ring][u] = *reinterpret_cast<const f32x4*>(src[u] + (long)min(kt, T - 1) * BKF);
+    const int k = min(kt, T - 1) + from;
+    raw[ring][u] = *reinterpret_cast<const f32x4*>(src[u] + (long)(k >= T ? k - T : k) * BKF);
   };
   char* const put = slots + at(row, ac & 3) + (ac >> 2) * 8;  // chunk g: k's 4 g and 16 + 4 g (RQ rows on: the same chunk)
   auto part_up = [&](int u, int ring, int slot) {

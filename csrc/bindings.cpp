@@ -38,6 +38,7 @@ int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
 int lsd_gemm_big_tiles(int M, int N, int K, int S);
 int lsd_gemm_on_wave4(int M, int N, int K, int epi, int S);
+int lsd_gemm_prompt_slabs(int M, int N, int K, int S);
 int lsd_gemm_far_rows(int M, int N, int K, long lda, long ldw);
 void lsd_attn_set_max_wg(int v);
 void lsd_attn_set_small_waves(int v);
@@ -873,6 +874,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const int s = lsd_gemm_deep_shape((int)M, (int)N, (int)K, (int)epi, (int)splits, (int)lanes);
     return std::make_pair(s / 1024, s % 1024); },
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("epi"), py::arg("splits"), py::arg("lanes") = 1);
+  m.def("gemm_prompt_slabs", [](int64_t M, int64_t N, int64_t K, int64_t S) {
+    return lsd_gemm_prompt_slabs((int)M, (int)N, (int)K, (int)S); });
   m.def("gemm_on_deep", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t kind, int64_t splits) {
     return lsd_gemm_on_deep((int)M, (int)N, (int)K, (int)epi, (int)kind, (int)splits) != 0; });
   m.def("gemm_big_tiles", [](int64_t M, int64_t N, int64_t K, int64_t S) {

@@ -366,6 +366,20 @@ static int wave4_tile(int M, int N, int K, int S) {
   return best;
 }
 
+// What a launch takes that writes S slabs, and the norm that adds them up (1/1000 us): the tiles' times above, 128 x 64 ones where
+// they are up to one a CU, and each slab written and read.  Fitted to 264 residual projections of 260 to 3000 rows (N 768 to 4096, K 768
+// to 14336) in 2 to 8 slabs with their norm, weights from HBM: the number so chosen is 0.6 % behind the best on average.
+static long slabs_cost(int M, int N, int K, int S) {
+  long c = 5500 + 570L * (K / 64) / S;
+  if ((long)((M + 127) / 128) * ((N + 63) / 64) * S > 256) {
+    c = wave4_cost(M, N, K, S, 4, 4, 1, 6320, 11770, 1072, 0);
+#define LSD_WAVE4(MI, NJ, SLOTS, B, F, R, C1, C2) c = std::min(c, wave4_cost(M, N, K, S, MI, NJ, B, F, R, C1, C2));
+    LSD_WAVE4_TILES(LSD_WAVE4)
+#undef LSD_WAVE4
+  }
+  return c + S * (150 + (long)M * N * 11 / 10000);
+}
+
 template <int EPI>
 static hipError_t wave4_launch(const GemmParams& p, int code, hipStream_t st) {
 #define LSD_WAVE4(MI, NJ, S, B, F, R, C1, C2)                                                                     \
@@ -382,6 +396,21 @@ static hipError_t wave4_launch(const GemmParams& p, int code, hipStream_t st) {
 }  // namespace lsd
 
 using namespace lsd;
+
+// Slabs of a prompt's residual projection whose rule leaves S > 1: 2 to 8, or S.  Against the rule's, which knows 128 x 64 and
+// 256 x 256 tiles, 6 % less on average with their norm: 1000 x 768 x 768 in 6 14.9 us, in 3 11.8; 700 x 768 x 1024 in 8 14.1, in 4 11.6;
+// 260 x 1600 x 1600 in 7 13.3, in 5 11.2; 333 x 4096 x 4096 in 3 25.2, in 4 23.0.  Prompts of GPT-2, 360 tokens 676 -> 610 us, GPT-2 medium,
+// 720 1676 -> 1608, GPT-2 XL, 750 4874 -> 4788.
+extern "C" int lsd_gemm_prompt_slabs(int M, int N, int K, int S) {
+  if (S <= 1 || M <= 256 || K % 64 != 0 || K < 256) return S;
+  int best = 0;
+  long least = 0;
+  for (int s = 2; s <= 8 && s <= K / 128; ++s) {
+    const long c = slabs_cost(M, N, K, s);
+    if (best == 0 || c < least) { best = s; least = c; }
+  }
+  return S <= 8 || slabs_cost(M, N, K, S) >= least ? best : S;
+}
 
 extern "C" int lsd_gemm_wave4_tile(int M, int N, int K, int epi, int S) { return epi == EPI_F32 ? 0 : wave4_tile(M, N, K, S); }
 

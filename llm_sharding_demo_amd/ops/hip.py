@@ -640,9 +640,9 @@ class HipBackend(Backend):
         """a w^T as slabs [S, T, H] (their sum); x: rows of the same shape."""
         (M, K), N = a.shape, w.shape[0]
         if self.fp32 or self._gemv_in(a, K, EPI_F32) is not None or (
-                not self._tiled(M, N) and self._resid_splits(M, N, K) == 1):
+                not self._tiled(M, N) and self._launch_splits(M, N, K) == 1):
             return self._linear_f32(a, w)[None]
-        return self.C.linear_residual(a, w, None, x, self._resid_splits(M, N, K), self._tiled(M, N), self.counters, True, None,
+        return self.C.linear_residual(a, w, None, x, self._launch_splits(M, N, K), self._tiled(M, N), self.counters, True, None,
                                       self.concurrency)
 
     # -- layers with elementwise norms (models/stage.py _token_layer) ----------------
@@ -1035,7 +1035,7 @@ class HipBackend(Backend):
         if self.fp32 or self._gemv_in(a, K, EPI_RESID) is not None or self._tiled(M, N) or not self.R.defer_resid \
                 or (self.R.blaslt_resid(M, K, self._decode) and a.is_contiguous()):
             return 0
-        s = self._resid_splits(M, N, K)
+        s = self._launch_splits(M, N, K)
         return s if s > 1 else 0
 
     def _linear_f32(self, a, w):
@@ -1080,6 +1080,12 @@ class HipBackend(Backend):
                 plans.clear()
             plans[key] = S
         return S
+
+    def _launch_splits(self, M: int, N: int, K: int) -> int:
+        """K splits a residual projection is launched with: the rule's, and the slabs of
+        prompts that leave some by what their tiles take."""
+        S = self._resid_splits(M, N, K)
+        return S if S <= 1 or self._decode or M <= 256 else self.C.gemm_prompt_slabs(M, N, K, S)
 
     @classmethod
     def decode_attn_splits(cls, B: int, nh: int, n_kv: int, hd: int, max_ctx: int) -> int:
@@ -1238,7 +1244,7 @@ class HipBackend(Backend):
         if self.R.blaslt_resid(M, K, self._decode) and a.is_contiguous() \
                 and self.C.blaslt_residual(a, w, b, r.x, self.lane):
             return
-        splits = self._resid_splits(M, N, K)
+        splits = self._launch_splits(M, N, K)
         tiled = self._tiled(M, N)
         # decode split-K: hand the S partial slabs to the next norm (which
         # reads the rows anyway) instead of a last-arriver reduce in the GEMM

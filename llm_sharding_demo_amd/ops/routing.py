@@ -268,7 +268,8 @@ class Routing:
 
     def residual_splits(self, M: int, N: int, K: int, decode: bool = True, lanes: int = 1) -> int:
         """K splits a residual projection is launched with: the rule above, and
-        what the kernels behind it make of slabs."""
+        what the kernels behind it make of slabs.  Prompts' slabs of more than 256
+        rows are reckoned once more at their launch (lsd_gemm_prompt_slabs in gemm_wave4.hip)."""
         S = self.resid_splits(M, N, K, decode, lanes)
         if not decode:
             S = self.prompt_slabs(M, N, K, S)

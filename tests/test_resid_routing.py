@@ -110,3 +110,29 @@ def test_delta_rule_splits_by_length():
                                     (16, 8, 20, False), (16, 8, 64, True), (16, 12, 64, False), (16, 12, 100, True),
                                     (16, 13, 4000, False), (16, 1, 0, False)]:
         assert _C.delta_split(heads, seqs, rows) == want, (heads, seqs, rows)
+
+
+def test_slabs_of_prompts_at_their_launch():
+    """By what tiles and norm take: 2 to 8 where the rule leaves some, and nothing else is changed."""
+    import pytest
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+    from llm_sharding_demo_amd.ops.hip import HipBackend
+
+    for M, N, K, S, want in [(1000, 2048, 5632, 8, 2), (1000, 2048, 2048, 2, 2), (500, 2048, 2048, 4, 4), (260, 1600, 1600, 7, 5), (700, 768, 1024, 8, 4),
+                             (257, 768, 256, 4, 2), (260, 768, 4096, 15, 8), (3000, 2048, 5632, 1, 1), (256, 2048, 5632, 8, 8),
+                             (1000, 2048, 96, 2, 2), (1000, 2048, 5600, 3, 3), (257, 768, 192, 3, 3)]:
+        assert _C.gemm_prompt_slabs(M, N, K, S) == want, (M, N, K)
+    for M in (257, 300, 700, 2000, 20000):
+        for N in (16, 768, 2048, 4096):
+            for K in (256, 768, 2048, 14336):
+                assert 2 <= _C.gemm_prompt_slabs(M, N, K, 5) <= min(8, K // 128)
+    b = HipBackend.__new__(HipBackend)
+    b.C = _C
+    b.decode = False
+    assert b._launch_splits(1000, 2048, 5632) == 2 and b._resid_splits(1000, 2048, 5632) == 8
+    assert b._launch_splits(65536, 1600, 6400) == 1
+    b.decode = True
+    assert b._launch_splits(512, 4096, 14336) == b._resid_splits(512, 4096, 14336) == 8

@@ -145,7 +145,10 @@ __device__ __forceinline__ void transpose_groups(u32x4 (&x)[4]) {
 // into its own four (row 4 g of the product is head g, so lane (r, g) ends with
 // all keys of query r, head g) -> barrier -> softmax in the lane, weights
 // transposed between lane groups and registers, second product per head.  Few
-// queries: the keys are split over blockIdx.y, partial outputs combined after.
+// queries: the keys are split over blockIdx.y, partial outputs combined after.  A 32-key tile takes a block some
+// 7 us, one behind the other, and a split 131 KB of partial outputs with 16 heads of 128; so splits are as short as
+// two blocks a CU allow, and as long for every tile of queries (p.per): in as many for each as for the longest, tiles
+// with few keys wrote as much (1000 tokens, 7 splits each 73 us, up to 11 of three key tiles 58).
 template <int DKS, int VT, int HP>
 __global__ __launch_bounds__(HP == 32 ? 512 : 256, HP == 32 ? 1 : 2) void talk_prefill_kernel(TalkParams p) {
   constexpr int TK = 32, HW = HP / 4, NW = HW > 4 ? HW : 4, QG = NW / HW;
@@ -153,7 +156,8 @@ __global__ __launch_bounds__(HP == 32 ? 512 : 256, HP == 32 ? 1 : 2) void talk_p
   constexpr int PLANE = TK * 16 * PITCH;
   __shared__ __attribute__((aligned(16))) _Float16 ss[QG * 2 * PLANE];
   __shared__ __attribute__((aligned(16))) bf16 vst[NW][TK * VLD];
-  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  // parts of the longest tiles, side by side, are spread over the XCDs
+  const int tile = p.splits > 1 ? blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
   const int seq = p.tiles[2 * tile], off = p.tiles[2 * tile + 1];
   const int cu = p.s.cu[seq], qlen = p.s.cu[seq + 1] - cu, st = p.s.start[seq];
   const int* table = p.table + (long)p.s.slots[seq] * p.tw;
@@ -186,9 +190,18 @@ __global__ __launch_bounds__(HP == 32 ? 512 : 256, HP == 32 ? 1 : 2) void talk_p
   const int lo = first_key(st + off, p.window), hi = st + min(off + QG * 16, qlen);
   int kt0 = lo / TK, kt1 = (hi + TK - 1) / TK;
   if (p.splits > 1) {
-    const int per = (kt1 - kt0 + p.splits - 1) / p.splits;
+    const int per = max(p.per, (kt1 - kt0 + p.splits - 1) / p.splits);
     kt0 += blockIdx.y * per;
     kt1 = min(kt1, kt0 + per);
+    if (kt0 >= kt1) {  // no keys: a sum of zero, no outputs (the combine ends in front of it)
+      const int h = hw * 4 + g;
+      if (h < H && qi < qlen) {
+        const long pi = ((long)(cu + qi) * H + h) * p.splits + blockIdx.y;
+        p.part_ml[2 * pi] = NEG;
+        p.part_ml[2 * pi + 1] = 0.f;
+      }
+      return;
+    }
   }
   // 64 columns of the tile's V rows, 16 bytes per lane and 8 rows
   bf16x8 vr[4];
@@ -612,16 +625,22 @@ __global__ __launch_bounds__(64) void talk_combine_kernel(TalkParams p) {
     L += l[i] * w;
   }
   const float inv = 1.f / wave_sum(L), gate = head_gate<bf16>(p, b, h);
+  int parts = 0;  // up to the last one that has a key: those behind it may hold no outputs
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const unsigned long long some = __ballot(l[i] != 0.f);
+    if (some) parts = 64 * i + 64 - __clzll(some);
+  }
   __syncthreads();
   bf16* out = static_cast<bf16*>(p.out) + (long)b * p.ldo;
   for (int d = lane; d < p.vdim; d += 64) {
     float v = 0.f;
-    for (int s = 0; s < p.splits; s += RUN) {
+    for (int s = 0; s < parts; s += RUN) {
       float x[RUN];
 #pragma unroll
-      for (int i = 0; i < RUN; ++i) x[i] = p.part_o[(pi + min(s + i, p.splits - 1)) * p.vdim + d];
+      for (int i = 0; i < RUN; ++i) x[i] = p.part_o[(pi + min(s + i, parts - 1)) * p.vdim + d];
 #pragma unroll
-      for (int i = 0; i < RUN; ++i) v += x[i] * ws[s + i];
+      for (int i = 0; i < RUN; ++i) v += s + i < parts ? x[i] * ws[s + i] : 0.f;
     }
     out[h * p.vdim + d] = f2bf(v * inv * gate);
   }

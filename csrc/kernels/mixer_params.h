@@ -105,6 +105,7 @@ struct TalkParams {
   SeqParams s;
   // decode, splits > 1
   float* part_o; float* part_ml; int splits;
+  int per;                             // talk_prefill: key tiles of a split at least
 };
 
 // Behind the in-projection y [rows][H dim | G dim | G vdim]: short convolution,

@@ -520,9 +520,10 @@ void partials(TalkParams& p, int64_t splits, const Tensor& q, Tensor& po, Tensor
   p.part_o = po.data_ptr<float>(); p.part_ml = pml.data_ptr<float>();
 }
 
-// packed ragged queries; tiles [n, 2] = (sequence, first query) of talk_tile(hp) queries
+// packed ragged queries; tiles [n, 2] = (sequence, first query) of talk_tile(hp) queries.  keys: the longest
+// context (0: not known), whose splits' length is every tile's
 void talk_prefill(Tensor q, Tensor k, Tensor v, Tensor table, Tensor frag, Tensor tiles, Tensor slots, Tensor start,
-                  Tensor cu, int64_t window, double scale, double cap, int64_t splits, Tensor out) {
+                  Tensor cu, int64_t window, double scale, double cap, int64_t splits, Tensor out, int64_t keys) {
   TalkParams p = talk_base(q, k, v, table, c10::nullopt, window, scale, cap, out, {0, c10::nullopt, c10::nullopt});
   const int hp = frag_of(p, q, frag);
   Tensor po, pml;
@@ -530,6 +531,8 @@ void talk_prefill(Tensor q, Tensor k, Tensor v, Tensor table, Tensor frag, Tenso
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 2, "tiles must be [n, 2]");
   p.tiles = iptr(tiles, 0, "tiles"); p.n_tiles = tiles.size(0);
   p.s = seqs(slots, start, cu);
+  const int64_t seen = std::min<int64_t>(std::max<int64_t>(keys, 0), (int64_t)p.window + lsd_talk_tile(hp) + 31);
+  p.per = (int)(((seen + 31) / 32 + splits - 1) / splits);
   check_hip(lsd_talk_prefill(&p, hp, cur_stream()), "talk_prefill");
 }
 
@@ -774,7 +777,7 @@ void lsd_register_mixers(pybind11::module& m) {
   m.def("talk_tile", [](int64_t hp) { return lsd_talk_tile((int)hp); });
   m.def("talk_prefill", &talk_prefill, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("table"), py::arg("frag"),
         py::arg("tiles"), py::arg("slots"), py::arg("start"), py::arg("cu"), py::arg("window"), py::arg("scale"),
-        py::arg("cap"), py::arg("splits"), py::arg("out"));
+        py::arg("cap"), py::arg("splits"), py::arg("out"), py::arg("keys") = 0);
   m.def("talk_decode", &talk_decode, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("table"), py::arg("frag"),
         py::arg("slots"), py::arg("pos"), py::arg("window"), py::arg("scale"), py::arg("cap"), py::arg("splits"),
         py::arg("out"));

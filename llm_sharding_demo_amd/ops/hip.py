@@ -770,8 +770,13 @@ class HipBackend(Backend):
                 C.talk_decode(*at, td, *rows, window, m.scale, cap, R.talk_splits(mt.num_seqs, ctx, ctx < mt.max_ctx),
                               out)
             else:
-                tiles = self._query_tiles(mt, C.talk_tile(tp.shape[0]), q.device)
-                C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, R.talk_prefill_splits(tiles.shape[0], ctx), out)
+                hp = tp.shape[0]
+                tiles = self._query_tiles(mt, C.talk_tile(hp), q.device)
+                if mt.is_decode or mt.host_starts is None:
+                    splits = R.talk_prefill_splits(tiles.shape[0], ctx)
+                else:  # (32 heads: one block a CU)
+                    splits = R.talk_prefill_parts(mt.host_qlens, mt.host_starts, window, C.talk_tile(hp), 490 if hp < 32 else 245)
+                C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, splits, out, mt.max_ctx)
             return
         mfma = not self.fp32 and m.softcap is None and C.paged_ok(dp, vp)
         if mfma and m.talking and m.talk_weights and tp is not None:

@@ -444,6 +444,28 @@ class Routing:
         tiles over long contexts, at least four 32-key tiles each."""
         return max(1, min(self.talk_prefill_target // max(1, tiles), keys // 128, 16))
 
+    def talk_prefill_parts(self, qlens, starts, window: int, rows: int, blocks: int = 490) -> int:
+        """Key splits of a prompt attention launch with capped mixed scores, in which a tile of
+        `rows` queries takes as many of them as it has keys for (attention_talk.hip): as
+        short as leave `blocks` blocks, a little less than two a CU.  us with the combine, 16
+        heads of 128, splits by tiles alone -> here: 1000 tokens 73 -> 58, 500 61 -> 37, 4 x 250 67 -> 37, 100
+        31 -> 19, 1500 97 -> 80, 1000 and 400 86 -> 72; a split more or less than two a CU
+        takes 1000 72, 1500 102."""
+        tiles, keys, longest = 0, 0.0, 0
+        for n, first in zip(qlens, starts):
+            t, lo, hi = math.ceil(n / rows), first + min(n, rows), first + n
+            if hi <= window:
+                mean = (lo + hi) / 2
+            elif lo >= window:
+                mean = window
+            else:
+                mean = ((window - lo) * (window + lo) / 2 + (hi - window) * window) / (hi - lo)
+            tiles, keys, longest = tiles + t, keys + t * (mean / 32 + 0.5), max(longest, min(hi, window + rows + 31))
+        room = blocks - tiles / 2  # (a tile's last split is half full on average)
+        if room <= 0 or longest == 0:
+            return 1
+        return max(1, min(math.ceil(math.ceil(longest / 32) / max(1, math.ceil(keys / room))), 16))
+
     def paged_splits(self, items: int, keys: int) -> int:
         """Context splits of decode attention, a wave per (token, K / V head)."""
         return max(1, min(math.ceil(self.paged_waves / items), math.ceil(keys / self.paged_split_keys), 64))

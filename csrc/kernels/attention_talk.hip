@@ -603,11 +603,18 @@ __global__ __launch_bounds__(256, 2) void talk_decode_kernel(TalkParams p) {
     for (int c = H * vdim + threadIdx.x; c < p.out_cols; c += 256) static_cast<bf16*>(p.out)[(long)b * p.ldo + c] = f2bf(0.f);
 }
 
-// One wave per (query, head); the last head's also clears the pad columns.
-__global__ __launch_bounds__(64) void talk_combine_kernel(TalkParams p) {
-  constexpr int RUN = 8;  // splits whose rows are loaded together
+// One (query, head) a block; the last head's also clears the pad columns.  A wave reads RUN splits at a time, one
+// wait after the other, which is all the time it takes where rows are few: with more than RUN splits NW waves take a
+// part each (50 splits, 64 blocks: 8.25 us with one wave, 4.5 with four).  SOME: splits behind the last one with a
+// key hold no outputs and are not read; that end is known only after the sums, so others do not ask for it (11.6 us in that launch).
+constexpr int COMBINE_RUN = 8;
+template <int NW, bool SOME>
+__global__ __launch_bounds__(64 * NW) void talk_combine_kernel(TalkParams p) {
+  constexpr int RUN = COMBINE_RUN;
   __shared__ float ws[256];
-  const int b = blockIdx.x / p.H, h = blockIdx.x % p.H, lane = threadIdx.x;
+  __shared__ float2 sums[NW][64];
+  const int b = blockIdx.x / p.H, h = blockIdx.x % p.H, lane = threadIdx.x & 63;
+  const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long pi = (long)blockIdx.x * p.splits;
   float m[4], l[4], M = NEG, L = 0.f;
 #pragma unroll
@@ -620,32 +627,52 @@ __global__ __launch_bounds__(64) void talk_combine_kernel(TalkParams p) {
   M = wave_max(M);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float w = lane + 64 * i < p.splits ? exp2f(m[i] - M) : 0.f;
-    ws[lane + 64 * i] = w;
-    L += l[i] * w;
+    const float e = lane + 64 * i < p.splits ? exp2f(m[i] - M) : 0.f;
+    if (i % NW == w) ws[lane + 64 * i] = e;
+    L += l[i] * e;
   }
   const float inv = 1.f / wave_sum(L), gate = head_gate<bf16>(p, b, h);
-  int parts = 0;  // up to the last one that has a key: those behind it may hold no outputs
+  int parts = p.splits;
+  if (SOME) {
+    parts = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned long long some = __ballot(l[i] != 0.f);
-    if (some) parts = 64 * i + 64 - __clzll(some);
-  }
-  __syncthreads();
-  bf16* out = static_cast<bf16*>(p.out) + (long)b * p.ldo;
-  for (int d = lane; d < p.vdim; d += 64) {
-    float v = 0.f;
-    for (int s = 0; s < parts; s += RUN) {
-      float x[RUN];
-#pragma unroll
-      for (int i = 0; i < RUN; ++i) x[i] = p.part_o[(pi + min(s + i, parts - 1)) * p.vdim + d];
-#pragma unroll
-      for (int i = 0; i < RUN; ++i) v += s + i < parts ? x[i] * ws[s + i] : 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const unsigned long long some = __ballot(l[i] != 0.f);
+      if (some) parts = 64 * i + 64 - __clzll(some);
     }
-    out[h * p.vdim + d] = f2bf(v * inv * gate);
+  }
+  const int own = (parts + NW - 1) / NW, s0 = w * own, s1 = min(s0 + own, parts);
+  __syncthreads();
+  bf16* out = static_cast<bf16*>(p.out) + (long)b * p.ldo + h * p.vdim;
+  const int d = 2 * lane;  // (at most 128 columns, an even number)
+  float2 v = {0.f, 0.f};
+  if (d < p.vdim)
+    for (int s = s0; s < s1; s += RUN) {
+      float2 x[RUN];
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) x[i] = *reinterpret_cast<const float2*>(p.part_o + (pi + min(s + i, s1 - 1)) * p.vdim + d);
+#pragma unroll
+      for (int i = 0; i < RUN; ++i) {
+        const float e = s + i < s1 ? ws[s + i] : 0.f;
+        v.x += x[i].x * e;
+        v.y += x[i].y * e;
+      }
+    }
+  if (NW > 1) {
+    sums[w][lane] = v;
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      v.x += sums[i][lane].x;
+      v.y += sums[i][lane].y;
+    }
+  }
+  if (w == 0 && d < p.vdim) {
+    out[d] = f2bf(v.x * inv * gate);
+    out[d + 1] = f2bf(v.y * inv * gate);
   }
   if (h == p.H - 1)
-    for (int c = p.H * p.vdim + lane; c < p.out_cols; c += 64) out[c] = f2bf(0.f);
+    for (int c = p.H * p.vdim + threadIdx.x; c < p.out_cols; c += 64 * NW) static_cast<bf16*>(p.out)[(long)b * p.ldo + c] = f2bf(0.f);
 }
 
 }  // namespace
@@ -668,11 +695,17 @@ extern "C" int lsd_talk_tile(int hp) { return hp == 8 ? 32 : 16; }  // queries o
   else if (p->vdim <= 64) hipLaunchKernelGGL((KERNEL<4, 4, __VA_ARGS__>), GRID, dim3(NT), 0, st, *p);             \
   else hipLaunchKernelGGL((KERNEL<4, 8, __VA_ARGS__>), GRID, dim3(NT), 0, st, *p);
 
-extern "C" hipError_t lsd_attention_combine(const TalkParams* p, hipStream_t st) {
+// some: splits behind a query's last key hold no outputs
+hipError_t combine(const TalkParams* p, bool some, hipStream_t st) {
   if (p->T == 0) return hipSuccess;
-  hipLaunchKernelGGL(talk_combine_kernel, dim3(p->T * p->H), dim3(64), 0, st, *p);
+  const dim3 grid(p->T * p->H);
+  if (some) hipLaunchKernelGGL((talk_combine_kernel<1, true>), grid, dim3(64), 0, st, *p);
+  else if (p->splits > COMBINE_RUN) hipLaunchKernelGGL((talk_combine_kernel<4, false>), grid, dim3(256), 0, st, *p);
+  else hipLaunchKernelGGL((talk_combine_kernel<1, false>), grid, dim3(64), 0, st, *p);
   return hipGetLastError();
 }
+
+extern "C" hipError_t lsd_attention_combine(const TalkParams* p, hipStream_t st) { return combine(p, false, st); }
 
 extern "C" hipError_t lsd_talk_prefill(const TalkParams* p, int hp, hipStream_t st) {
   if (p->n_tiles == 0) return hipSuccess;
@@ -684,7 +717,7 @@ extern "C" hipError_t lsd_talk_prefill(const TalkParams* p, int hp, hipStream_t 
     case 32: LSD_TK_V(talk_prefill_kernel, grid, 512, 32) break;
     default: return hipErrorInvalidValue;
   }
-  if (p->splits > 1) return lsd_attention_combine(p, st);
+  if (p->splits > 1) return combine(p, true, st);
   return hipGetLastError();
 }
 

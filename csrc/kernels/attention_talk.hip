@@ -606,7 +606,8 @@ __global__ __launch_bounds__(256, 2) void talk_decode_kernel(TalkParams p) {
 // One (query, head) a block; the last head's also clears the pad columns.  A wave reads RUN splits at a time, one
 // wait after the other, which is all the time it takes where rows are few: with more than RUN splits NW waves take a
 // part each (50 splits, 64 blocks: 8.25 us with one wave, 4.5 with four).  SOME: splits behind the last one with a
-// key hold no outputs and are not read; that end is known only after the sums, so others do not ask for it (11.6 us in that launch).
+// key hold no outputs and are not read; that end is known only after the sums, so others do not ask for it (11.6 us in
+// that launch).
 constexpr int COMBINE_RUN = 8;
 template <int NW, bool SOME>
 __global__ __launch_bounds__(64 * NW) void talk_combine_kernel(TalkParams p) {

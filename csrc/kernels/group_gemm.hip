@@ -541,99 +541,88 @@ __device__ __forceinline__ Split split3(f32x4 x, float& big) {
   return s;
 }
 
-// What follows the products on split operands, S the tile's sums, WN waves a part.  Terms behind the 16-bit numbers are
-// lost.  Where that may count the tile is computed again by fp32 MFMAs, in the order of the kernel above: operands outside of the
-// terms' range, a sum that is not finite, one below LEAST.  Zeros among these stand where all of their column are and its weights
-// too, as padding's, of which the first ones are looked at where it is not known (weights) that there are others; looking through all of a column's weights took 10 to 50 us of a launch with padding.
-// wmax: of the tile's columns, or null.
-template <int MODE, int WM, int MT, int WN, int NT, int WK>
-__device__ __forceinline__ void split_tail(const GgParams& p, const gg::Tile& t, char* smem, f32x4 (&S)[MT][NT], int first, int T,
-                                           bool outside, const float* wmax, float LEAST) {
-  using namespace gg;
-  constexpr int TM = 16 * MT * WM, TN = 16 * NT * WN, BKF = 32, CLD = TN + 4, IMAGE = TM * CLD;
-  constexpr bool WHOLE = MODE == GG_F32 || MODE == GG_ADD;
-  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
-  const int wn = wave % WN, wm = wave / WN % WM, part = wave / (WN * WM);
-  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16) - wm * MT;  // of this wave's tiles
-  auto weights = [&](int j) {
-    return static_cast<const float*>(t.W) + (long)min(t.n0 + (wn * NT + j) * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
-  };
-  bool exact = outside;
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float v = fabsf(S[i][j][q]);
-        exact |= !(v >= LEAST && v < INFINITY) && (WHOLE || i < live);
-      }
-  exact = __syncthreads_or(exact);
-  if (exact) {  // for zeros alone only where the column has other sums, or W values
-    int some = outside;
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      int zero = 0, other = wmax && wmax[(wn * NT + j) * 16 + r] > 0.f;
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float v = fabsf(S[i][j][q]);
-          zero |= v == 0.f && (WHOLE || i < live);
-          other |= v > 0.f;
-          some |= !(v < INFINITY) || (v < LEAST && v > 0.f);
-        }
-      zero |= __shfl_xor(zero, 16);
-      zero |= __shfl_xor(zero, 32);
-      if (zero && !wmax && T > 0) {
-        const f32x4 u = *reinterpret_cast<const f32x4*>(weights(j)), v = *reinterpret_cast<const f32x4*>(weights(j) + 16);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) other |= u[e] != 0.f || v[e] != 0.f;
-      }
-      some |= zero && other;
-    }
-    exact = __syncthreads_or(some);
-  }
-  if (exact) {
-#pragma unroll 1
-    for (int i = 0; i < min(live, MT); ++i) {
-      const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, (wm * MT + i) * 16 + r) * t.lda + first * BKF + 4 * g;
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const float* wp = weights(j);
-        f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll 1
-        for (int k = 0; k < T * BKF; k += BKF)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const f32x4 av = *reinterpret_cast<const f32x4*>(a + k + 16 * h), wv = *reinterpret_cast<const f32x4*>(wp + k + 16 * h);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[h], 0, 0, 0);
-          }
-#pragma unroll
-        for (int h = 0; h < MT; ++h)
-          if (h == i) S[h][j] = s[0] + s[1];
-      }
-    }
-  }
-  float* ct = reinterpret_cast<float*>(smem);
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        ct[part * IMAGE + ((wm * MT + i) * 16 + 4 * g + q) * CLD + (wn * NT + j) * 16 + r] = S[i][j][q];
+// The parts' images of a tile are whole in LDS: their sum, and the results.  WAVES a part.
+template <int MODE, int TM, int TN, int WAVES, int WK>
+__device__ __forceinline__ void parts_out(const GgParams& p, const gg::Tile& t, float* ct) {
+  constexpr int IMAGE = TM * (TN + 4);
   __syncthreads();
   if constexpr (WK > 1) {
-    for (int c = threadIdx.x; c < IMAGE / 4; c += 64 * WM * WN * WK) {
+    for (int c = threadIdx.x; c < IMAGE / 4; c += 64 * WAVES * WK) {
       f32x4* o = reinterpret_cast<f32x4*>(ct) + c;
 #pragma unroll
       for (int i = 1; i < WK; ++i) *o += o[i * (IMAGE / 4)];
     }
     __syncthreads();
   }
-  f32_epilogue<MODE, TM, TN, 64 * WM * WN * WK>(p, t, ct);
+  f32_epilogue<MODE, TM, TN, 64 * WAVES * WK>(p, t, ct);
+}
+
+// What follows the products on three terms, S the tile's sums.  Terms behind bf16's numbers are lost: of an operand, 2^-134 at
+// most.  Where that may count the tile is computed again by fp32 MFMAs, in the order of the kernel above: an operand of 2^56 or
+// more (outside), a sum that is not finite, one below 2^-40.  Zeros among these stand where all of their column are and its first
+// weights too, as padding's; looking through all of a column's weights took 10 to 50 us of a launch with padding.
+template <int MODE, int MT, int WN, int WK>
+__device__ __forceinline__ void split_tail(const GgParams& p, const gg::Tile& t, char* smem, f32x4 (&S)[MT], int first, int T, bool outside) {
+  using namespace gg;
+  constexpr int TM = 16 * MT, TN = 16 * WN, BKF = 32, CLD = TN + 4, IMAGE = TM * CLD;
+  constexpr bool WHOLE = MODE == GG_F32 || MODE == GG_ADD;
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int w = wave % WN, part = wave / WN;
+  const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16);
+  const float* wp = static_cast<const float*>(t.W) + (long)min(t.n0 + w * 16 + r, t.N - 1) * t.ldw + first * BKF + 4 * g;
+  bool exact = outside;
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = fabsf(S[i][q]);
+      exact |= !(v >= 0x1p-40f && v < INFINITY) && (WHOLE || i < live);
+    }
+  exact = __syncthreads_or(exact);
+  if (exact) {  // for zeros alone only where the column has other sums, or W values in the part's first k-step
+    int zero = 0, other = 0, some = outside;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v = fabsf(S[i][q]);
+        zero |= v == 0.f && (WHOLE || i < live);
+        other |= v > 0.f;
+        some |= !(v < INFINITY) || (v < 0x1p-40f && v > 0.f);
+      }
+    zero |= __shfl_xor(zero, 16);
+    zero |= __shfl_xor(zero, 32);
+    if (zero && T > 0) {
+      const f32x4 u = *reinterpret_cast<const f32x4*>(wp), v = *reinterpret_cast<const f32x4*>(wp + 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) other |= u[e] != 0.f || v[e] != 0.f;
+    }
+    exact = __syncthreads_or(some || (zero && other));
+  }
+  if (exact) {
+#pragma unroll 1
+    for (int i = 0; i < live; ++i) {
+      const float* a = static_cast<const float*>(t.A) + a_row<MODE>(p, t, i * 16 + r) * t.lda + first * BKF + 4 * g;
+      f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 1
+      for (int k = 0; k < T * BKF; k += BKF)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 av = *reinterpret_cast<const f32x4*>(a + k + 16 * h), wv = *reinterpret_cast<const f32x4*>(wp + k + 16 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], wv[e], s[h], 0, 0, 0);
+        }
+#pragma unroll
+      for (int h = 0; h < MT; ++h)
+        if (h == i) S[h] = s[0] + s[1];
+    }
+  }
+  float* ct = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ct[part * IMAGE + (i * 16 + 4 * g + q) * CLD + w * 16 + r] = S[i][q];
+  parts_out<MODE, TM, TN, WN, WK>(p, t, ct);
 }
 
 // 16 MT x 16 WN tiles, 32-deep k-steps, WK parts of the k-steps on WN waves each, summed in LDS.
@@ -651,8 +640,7 @@ __device__ __forceinline__ void split_tail(const GgParams& p, const gg::Tile& t,
 // 2048 63 -> 49, 100 x 2048 x 2048 29 -> 23, 1000 x 11264 x 2048 390 -> 286; 2260 rows over 32 experts of
 // 2048 x 1024 and 565 through a shared one of 2048 up 325 -> 244, down 152 -> 121.  Splitting W a k-step
 // ahead, beside the MFMAs, gives nothing: MFMAs and splitting take turns to issue.
-// Behind bf16's numbers 2^-134 of an operand is lost at most; computed again from an operand of 2^56 or a sum below
-// 2^-40 on.  (A maximum of W's values beside the one of both took 20 % of the products.)
+// (A maximum of W's values beside the one of both took 20 % of the products.)
 template <int MODE, int MT, int WN, int WK, int D>
 __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_split_kernel(GgParams p) {
   using namespace gg;
@@ -745,18 +733,16 @@ __global__ __launch_bounds__(64 * WN * WK, WN == 8 ? 4 : 1) void group_gemm_f32_
     constexpr int l = decltype(ic)::v + 1;
     if (MODE == GG_UP || MODE == GG_DOWN ? live == l : l == MT) steps(std::integral_constant<int, l>{});
   });
-  f32x4 sum[MT][1];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) sum[i][0] = acc[0][i] + acc[1][i];
-  split_tail<MODE, 1, MT, WN, 1, WK>(p, t, smem, sum, first, T, big >= 0x1p56f, nullptr, 0x1p-40f);
+  for (int i = 0; i < MT; ++i) acc[0][i] += acc[1][i];
+  split_tail<MODE, MT, WN, WK>(p, t, smem, acc[0], first, T, big >= 0x1p56f);
 }
 
-// Long sums, on two fp16 terms: scale x = hi + lo / 2048, both rounded to nearest, 22 bits of x and more (4e-8 of it off
-// on average), hi infinite from 65520 / scale on, x off by up to 2^-36 / scale instead below 2^-14 / scale.
+// Long sums, on two fp16 terms: scale x = hi + lo / 2048, both rounded to nearest: off by up to 2^-24 of x or, below
+// 2^-12 / scale, 2^-36 / scale, hi infinite from 65520 / scale on.  most: the largest |x|.
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 constexpr float LO = 2048.f, SCALE_A = 4.f, SCALE_W = 256.f;
-constexpr float LEAST_A = 0x1p-11f / SCALE_A, LEAST_W = 0x1p-11f / SCALE_W;
 __device__ __forceinline__ void split2(f32x4 x, float scale, f16x4& hi, f16x4& lo, float& most) {
   most = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), most);
   most = fmaxf(fmaxf(fabsf(x[2]), fabsf(x[3])), most);
@@ -775,6 +761,61 @@ __device__ __forceinline__ void count_up(F f) {  // f(0) .. f(N - 1)
   }
 }
 
+// Sums of one 16 x 16 tile by fp32 MFMAs; a, w: this lane's row and column at its k's.  AHEAD k-steps' loads are on their way.
+__device__ __forceinline__ f32x4 fp32_sums(const float* a, const float* w, int steps) {
+  constexpr int AHEAD = 4;
+  f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, av[AHEAD][2], wv[AHEAD][2];
+  auto load = [&](int k, int at) {  // (behind the last one that one again)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      av[at][h] = *reinterpret_cast<const f32x4*>(a + min(k, steps - 1) * 32 + 16 * h);
+      wv[at][h] = *reinterpret_cast<const f32x4*>(w + min(k, steps - 1) * 32 + 16 * h);
+    }
+  };
+  auto add = [&](int at) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[at][h][e], wv[at][h][e], s[h], 0, 0, 0);
+  };
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) load(k, k);
+  int k0 = 0;
+#pragma unroll 1
+  for (; k0 + AHEAD <= steps; k0 += AHEAD)  // (whole groups: a way out between would have every load waited for)
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      add(k);
+      __builtin_amdgcn_sched_barrier(0);
+      load(k0 + k + AHEAD, k);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+  for (int k = 0; k < AHEAD - 1; ++k)
+    if (k0 + k < steps) add(k);
+  return s[0] + s[1];
+}
+
+// Sums of n products, n a multiple of 4, of a row and of C columns by a wave.
+template <int C>
+__device__ __forceinline__ void fp32_row(const float* a, const float* const (&w)[C], int n, float (&out)[C]) {
+  const int at = 4 * lane_id();
+  f32x4 s[C] = {};
+#pragma unroll 4
+  for (int k = 0; k < n; k += 256)
+    if (k + at < n) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(a + k + at);
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const f32x4 y = *reinterpret_cast<const f32x4*>(w[c] + k + at);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[c][e] = __builtin_fmaf(x[e], y[e], s[c][e]);
+      }
+    }
+#pragma unroll
+  for (int c = 0; c < C; ++c) out[c] = wave_sum((s[c][0] + s[c][1]) + (s[c][2] + s[c][3]));
+}
+
 // 16 MT WM x 16 NT WN tiles with half of the kernel above's products: hi hi, in two chains, and hi lo + lo hi.  A value takes 4
 // operations to split instead of 6, which go on for the next k-step between this one's MFMAs; PF k-steps are loaded ahead of that.
 // The two chains make up for what the terms leave out: off 64 bits by (before) K = 1024 1.65e-7 (1.94e-7) of the result, K = 2048
@@ -787,7 +828,15 @@ __device__ __forceinline__ void count_up(F f) {  // f(0) .. f(N - 1)
 // 1000 x 11264 258 -> 176, 565 x 2624 51 -> 43; 2260 rows over 32 experts of 2048 x 1024 and 565 through a shared one of 2048 up
 // 259 -> 201, down 126 -> 106, 5600 and 1400 rows 452 -> 356 and 245 -> 190.  For experts 96 rows a tile, the few rows behind
 // a full one with it, were behind, with their registers at two waves a SIMD (up 472, down 240 with the most rows).
-// Rows of A or columns of W whose largest value is too small for terms of 22 bits, and what split_tail names: computed again.
+//
+// The terms leave out at most 3 2^-24 of the sizes of the products, and 2^-38 and half as much again a product with a small value of
+// A, 2^-44 with one of W: of K products 1.5 K (2^-38 of the column's largest weight + 2^-44 of the row's largest value).  Of a sum
+// of 2^-13 of the one and 2^-19 of the other and more that is 3 K / 4 of its 2^-24.
+// Where the sizes of a sum's two chains are together less than that it is computed again from the operands, and where it is not
+// finite: by itself where a 16 x 16 tile has such sums in up to ROWS rows, by fp32 MFMAs where in more.  (By the size of the sum
+// alone, every tenth tile of normal operands would have one, 3 us of a launch.)  A row or a column of zeros has zeros.
+// 961 x 2048 x 2048, us: normal operands 47 (three bf16 terms 58), a value of 20000 85 (58), one in every tenth row 147, in every
+// row 272 (58); rows of 2^-8 47.
 template <int MODE, int WM, int MT, int WN, int NT, int WK, int PF, int OCC>
 __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_kernel(GgParams p) {
   using namespace gg;
@@ -797,6 +846,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
   static_assert(TN % RQ == 0, "whole passes over W");
   __shared__ __attribute__((aligned(16))) char smem[SMEM];
   __shared__ float wmax[WK * TN];
+  __shared__ __attribute__((aligned(16))) float amax[WK * TM];
   Tile t = locate<MODE, TM, TN>(p);
   if (!t.live) return;
   resolve<MODE, float>(p, t);
@@ -912,21 +962,102 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
   } else {
     steps(std::integral_constant<int, MT>{});
   }
-  bool small = false;
 #pragma unroll
   for (int u = 0; u < UNITS; ++u) {  // of a row's eight threads
     float& m = largest[u];
 #pragma unroll
     for (int d = 1; d < 8; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
-    small |= m > 0.f && m < (u < QW ? LEAST_W : LEAST_A);
-    if (u < QW && ac == 0) wmax[part * TN + row + RQ * u] = m;
+    const int at = row + RQ * (u < QW ? u : u - QW);
+    if (ac == 0 && u < QW) wmax[part * TN + at] = m;
+    if (ac == 0 && u >= QW && at < TM) amax[part * TM + at] = m;
   }
+  __syncthreads();  // (and every wave has read its last k-step: sums take its place)
+  constexpr int ROWS = 3;
+  float* const ct = reinterpret_cast<float*>(smem) + part * IMAGE;
+  constexpr float UNIT = 1.f / (SCALE_A * SCALE_W);
+  float least = INFINITY, odd = 0.f, line = 0x1p-34f;  // of this lane's sums: the smallest size; zero where all are finite; the line's most
 #pragma unroll
-  for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i) {
+    const f32x4 av = *reinterpret_cast<const f32x4*>(amax + part * TM + (wm * MT + i) * 16 + 4 * g);
+    line = fmaxf(fmaxf(fmaxf(av[0], av[1]), fmaxf(av[2], av[3])) * 0x1p-18f, line);
 #pragma unroll
-    for (int j = 0; j < NT; ++j)
-      acc[0][i][j] = (acc[0][i][j] + acc[1][i][j] + acc[2][i][j] * (1.f / LO)) * (1.f / (SCALE_A * SCALE_W));
-  split_tail<MODE, WM, MT, WN, NT, WK>(p, t, smem, acc[0], first, T, small, wmax + part * TN, 0x1p-36f);
+    for (int j = 0; j < NT; ++j) {
+      line = fmaxf(wmax[part * TN + (wn * NT + j) * 16 + r] * 0x1p-12f, line);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float c0 = acc[0][i][j][q], c1 = acc[1][i][j][q], s = (c0 + c1 + acc[2][i][j][q] * (1.f / LO)) * UNIT;
+        least = fminf(least, fabsf(c0) + fabsf(c1));
+        odd = __builtin_fmaf(s, 0.f, odd);
+        ct[((wm * MT + i) * 16 + 4 * g + q) * CLD + (wn * NT + j) * 16 + r] = acc[2][i][j][q] = s;
+      }
+    }
+  }
+  unsigned again = 0;  // row 4 g + q of tile (i, j), column r: bit (i NT + j) 4 + q where it is computed again
+  if (__ballot(least * UNIT < line || odd != 0.f) != 0) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const f32x4 av = *reinterpret_cast<const f32x4*>(amax + part * TM + (wm * MT + i) * 16 + 4 * g);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const float wv = wmax[part * TN + (wn * NT + j) * 16 + r];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool few = (fabsf(acc[0][i][j][q]) + fabsf(acc[1][i][j][q])) * UNIT < fmaxf(wv * 0x1p-13f + av[q] * 0x1p-19f, 0x1p-34f);
+          const bool out = (wm * MT + i) * 16 + 4 * g + q < t.rows && t.n0 + (wn * NT + j) * 16 + r < t.N;
+          again |= (unsigned)(out && ((few && wv > 0.f && av[q] > 0.f) || !(fabsf(acc[2][i][j][q]) < INFINITY))) << ((i * NT + j) * 4 + q);
+        }
+      }
+    }
+  }
+  if (__ballot(again != 0) != 0 && T > 0) {
+    const float* const A = static_cast<const float*>(t.A) + first * BKF;
+    const float* const W = static_cast<const float*>(t.W) + first * BKF;
+#pragma unroll 1
+    for (int f = 0; f < MT * NT; ++f) {
+      const int r0 = (wm * MT + f / NT) * 16, c0 = (wn * NT + f % NT) * 16;
+      unsigned long long row[4];  // columns to be summed, of 16 bits for each of the rows q, 4 + q, 8 + q, 12 + q
+      int rows = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        row[q] = __ballot(again >> (4 * f + q) & 1);
+#pragma unroll
+        for (int h = 0; h < 64; h += 16) rows += (row[q] >> h & 0xffff) != 0;
+      }
+      if (rows > ROWS) {
+        const f32x4 s = fp32_sums(A + a_row<MODE>(p, t, r0 + r) * t.lda + 4 * g, W + (long)min(t.n0 + c0 + r, t.N - 1) * t.ldw + 4 * g, T);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ct[(r0 + 4 * g + q) * CLD + c0 + r] = s[q];
+        continue;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll 1
+        while (row[q]) {  // a column, or four of a row, the last ones the same
+          const int h = __builtin_ctzll(row[q]) >> 4, at = r0 + 4 * h + q;
+          const float* ar = A + a_row<MODE>(p, t, at) * t.lda;
+          auto some = [&](auto count) {
+            constexpr int C = decltype(count)::v;
+            int col[C];
+            const float* w[C];
+            float s[C];
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+              const unsigned left = row[q] >> 16 * h & 0xffff;
+              col[c] = left ? __builtin_ctz(left) : col[0];
+              if (left) row[q] &= row[q] - 1;
+              w[c] = W + (long)(t.n0 + c0 + col[c]) * t.ldw;
+            }
+            fp32_row<C>(ar, w, T * BKF, s);
+            if (lane == 0)
+#pragma unroll
+              for (int c = 0; c < C; ++c) ct[at * CLD + c0 + col[c]] = s[c];
+          };
+          if (__builtin_popcountll(row[q] >> 16 * h & 0xffff) > 1) some(Int<4>{});
+          else some(Int<1>{});
+        }
+    }
+  }
+  parts_out<MODE, TM, TN, WM * WN, WK>(p, t, reinterpret_cast<float*>(smem));
 }
 
 // Rows without whole k-steps of 32 or off 16 bytes: 64 x 64 tiles, 4 x 4 outputs per thread, 16-deep k-steps.

@@ -1,7 +1,8 @@
 """fp32 products on two fp16 terms against 64 bits.
 
 A sum of K products in fp32 is off by at most (K + 2) ulp of the sum of the products' sizes, in any order (ulp:
-2^-24); terms of 22 bits leave 2^-22 of each product, four ulp, and their low ones' product 2^-22 more.
+2^-24); the terms leave out three ulp of each product.  Of values too small for them they leave out more, 3 K / 4 ulp of the
+sizes at most where such sums are not computed again; an fp32 MFMA adds 32 products in a few roundings, so sums stay in K + 14.
 """
 
 import pytest
@@ -72,6 +73,55 @@ def test_lone_small_values(C):  # noqa: F811
     a[:, 100], w[:, 100] = 2.0 ** -45, 1.0
     got = C.linear_fp32(a.to(DEV), w.to(DEV))
     assert near(got, a, w)
+
+
+# 2^-16 and 2^-22 are where terms of A and of W begin to keep fewer than 22 bits
+SMALL = torch.tensor([m * 2.0 ** -e for e in range(12, 46) for m in (1.7, 1.05, 1.3)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile", TILES)
+def test_lone_products(C, M, N, K, tile):  # noqa: F811
+    """Values far below the others of their row of A or column of W, whose partners are zeros but for one or for few:
+    their sums are of their own size, and as near as any."""
+    n = len(SMALL)
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2) * 0.02
+    a[:n, 100] = SMALL
+    for column, partner in ((7, 1.0), (33, -2.0 ** -6), (60, 128.0), (1980, 0.3)):
+        w[column] = 0
+        w[column, 100] = partner
+    w[200: 200 + n, K - 5] = SMALL * 2.0 ** -6
+    for row, partner in ((110, 8192.0), (111, 1.0), (200, -0.01)):
+        a[row] = 0
+        a[row, K - 5] = partner
+    for row, e in ((120, 20), (150, 26), (180, 34)):  # many such products
+        a[row, : K // 2] *= 2.0 ** -e
+    w[61, K // 2:] = 0
+    got = C.linear_fp32(a.to(DEV), w.to(DEV))
+    assert near(got, a, w)
+
+
+@pytest.mark.gpu
+def test_lone_products_of_experts(C):  # noqa: F811
+    """The same of one expert's and a shared expert's down product, beside an expert with few rows."""
+    T, H, F, n = 200, 2176, 1024, len(SMALL)
+    mid, mids, dn = rand(T, F, seed=1), rand(T, F, seed=2), rand(2, H, F, seed=3) * 0.02
+    shared = rand(H, F, seed=4) * 0.02
+    ids = (torch.arange(T)[:, None] >= T - 3).int()  # the last three tokens to the second expert
+    order, tiles = C.moe_group(ids.to(DEV), 2, 64)
+    assert C.moe_on_split(T, 1, tiles.shape[0], H, H, F)
+    for x in (mid, mids):
+        x[:n, 100] = SMALL
+        x[110], x[110, F - 5] = 0, 8192.0
+    for w in (dn[0], shared):
+        w[7], w[7, 100] = 0, 1.0
+        w[60], w[60, 100] = 0, 128.0
+        w[100: 100 + n, F - 5] = SMALL * 2.0 ** -6
+    slab = torch.empty(2, T, H, device=DEV)
+    C.moe_down(mid.to(DEV), mids.to(DEV), order, tiles, torch.ones(T, 1).to(DEV), dn.to(DEV), shared.to(DEV), slab, 64)
+    at = order.cpu().long()[:T]
+    assert near(slab[1], mids, shared)
+    assert near(slab[0][at[: T - 3].to(DEV)], mid[: T - 3], dn[0]) and near(slab[0][at[T - 3:].to(DEV)], mid[T - 3:], dn[1])
 
 
 @pytest.mark.gpu

@@ -450,7 +450,10 @@ class Routing:
         short as leave `blocks` blocks, a little less than two a CU.  us with the combine, 16
         heads of 128, splits by tiles alone -> here: 1000 tokens 73 -> 58, 500 61 -> 37, 4 x 250 67 -> 37, 100
         31 -> 19, 1500 97 -> 80, 1000 and 400 86 -> 72; a split more or less than two a CU
-        takes 1000 72, 1500 102."""
+        takes 1000 72, 1500 102.
+        Every token has partial outputs in every split: no more of them than prompts of one length
+        come to, twice `rows` a block (128 MB with 16 heads of 128; without this bound 800 tokens'
+        prompts of 16 and one such chunk at position 30000 took 1.7 GB a layer)."""
         tiles, keys, longest = 0, 0.0, 0
         for n, first in zip(qlens, starts):
             t, lo, hi = math.ceil(n / rows), first + min(n, rows), first + n
@@ -464,7 +467,8 @@ class Routing:
         room = blocks - tiles / 2  # (a tile's last split is half full on average)
         if room <= 0 or longest == 0:
             return 1
-        return max(1, min(math.ceil(math.ceil(longest / 32) / max(1, math.ceil(keys / room))), 16))
+        splits = min(math.ceil(math.ceil(longest / 32) / max(1, math.ceil(keys / room))), 16)
+        return max(1, min(splits, int(2 * blocks * rows / sum(qlens))))
 
     def paged_splits(self, items: int, keys: int) -> int:
         """Context splits of decode attention, a wave per (token, K / V head)."""

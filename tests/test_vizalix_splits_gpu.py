@@ -17,6 +17,11 @@ def test_rule():
                                         ([1500], [0], 1024, 7), ([4000], [0], 1024, 2), ([20000], [0], 1024, 1), ([16], [7000], 1 << 30, 16),
                                         ([0, 5], [3, 0], 64, 1), ([0], [0], 64, 1)]:
         assert r.talk_prefill_parts(qlens, starts, window, 16) == want, (qlens, starts)
+    # partial outputs of every token and split: as many as equal prompts have, not more where one is longer than the others
+    for qlens, starts, window, want in [([16] * 800 + [16], [0] * 800 + [30000], 1 << 30, 1), ([16] * 500 + [16], [0] * 500 + [8000], 1024, 1),
+                                        ([16] * 100 + [1000], [0] * 101, 1024, 6), ([1] * 300 + [16], [0] * 300 + [8000], 1024, 16)]:
+        got = r.talk_prefill_parts(qlens, starts, window, 16)
+        assert got == want and (got == 1 or got * sum(qlens) <= 2 * 490 * 16), (len(qlens), got)
 
 
 @pytest.mark.gpu

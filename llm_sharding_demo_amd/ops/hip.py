@@ -772,11 +772,11 @@ class HipBackend(Backend):
             else:
                 hp = tp.shape[0]
                 tiles = self._query_tiles(mt, C.talk_tile(hp), q.device)
-                if mt.is_decode or mt.host_starts is None:
-                    splits = R.talk_prefill_splits(tiles.shape[0], ctx)
-                else:  # (32 heads: one block a CU)
-                    splits = R.talk_prefill_parts(mt.host_qlens, mt.host_starts, window, C.talk_tile(hp), 490 if hp < 32 else 245)
-                C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, splits, out, mt.max_ctx)
+                if mt.is_decode or mt.host_starts is None:  # (a replay's chunks start elsewhere: a split's length is each tile's own)
+                    splits, keys = R.talk_prefill_splits(tiles.shape[0], ctx), 0
+                else:
+                    splits, keys = R.talk_prefill_parts(mt.host_qlens, mt.host_starts, window, C.talk_tile(hp), 490 if hp < 32 else 245), mt.max_ctx
+                C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, splits, out, keys)
             return
         mfma = not self.fp32 and m.softcap is None and C.paged_ok(dp, vp)
         if mfma and m.talking and m.talk_weights and tp is not None:

@@ -775,7 +775,7 @@ class HipBackend(Backend):
                 if mt.is_decode or mt.host_starts is None:  # (a replay's chunks start elsewhere: a split's length is each tile's own)
                     splits, keys = R.talk_prefill_splits(tiles.shape[0], ctx), 0
                 else:
-                    splits, keys = R.talk_prefill_parts(mt.host_qlens, mt.host_starts, window, C.talk_tile(hp), 490 if hp < 32 else 245), mt.max_ctx
+                    splits, keys = self._talk_parts(mt, window, C.talk_tile(hp), 490 if hp < 32 else 245), mt.max_ctx
                 C.talk_prefill(*at, tp, tiles, *seqs, window, m.scale, cap, splits, out, keys)
             return
         mfma = not self.fp32 and m.softcap is None and C.paged_ok(dp, vp)
@@ -812,6 +812,14 @@ class HipBackend(Backend):
             rows = 128 if blocks >= self.R.attn_tile_min else 64
             kept = meta._tiles = heads, prefill_tiles(meta, rows).to(device), rows
         return kept[1:]
+
+    def _talk_parts(self, meta, window: int, rows: int, blocks: int) -> int:
+        """Splits of a prompt launch with capped mixed scores, kept on the batch: every layer asks."""
+        cache = meta.__dict__.setdefault("_talk_parts", {})
+        key = (window, rows, blocks)
+        if key not in cache:
+            cache[key] = self.R.talk_prefill_parts(meta.host_qlens, meta.host_starts, window, rows, blocks)
+        return cache[key]
 
     @staticmethod
     def _query_tiles(meta, rows: int, device):

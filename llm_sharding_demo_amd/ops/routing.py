@@ -454,6 +454,9 @@ class Routing:
         Every token has partial outputs in every split: no more of them than prompts of one length
         come to, twice `rows` a block (128 MB with 16 heads of 128; without this bound 800 tokens'
         prompts of 16 and one such chunk at position 30000 took 1.7 GB a layer)."""
+        most = int(2 * blocks * rows / max(1, sum(qlens)))
+        if most <= 1:
+            return 1
         tiles, keys, longest = 0, 0.0, 0
         for n, first in zip(qlens, starts):
             t, lo, hi = math.ceil(n / rows), first + min(n, rows), first + n
@@ -467,8 +470,7 @@ class Routing:
         room = blocks - tiles / 2  # (a tile's last split is half full on average)
         if room <= 0 or longest == 0:
             return 1
-        splits = min(math.ceil(math.ceil(longest / 32) / max(1, math.ceil(keys / room))), 16)
-        return max(1, min(splits, int(2 * blocks * rows / sum(qlens))))
+        return max(1, min(math.ceil(math.ceil(longest / 32) / max(1, math.ceil(keys / room))), 16, most))
 
     def paged_splits(self, items: int, keys: int) -> int:
         """Context splits of decode attention, a wave per (token, K / V head)."""

@@ -38,6 +38,19 @@ def layer(meta, calls, heads=16):
                  SimpleNamespace(table=None), meta, None, None)
 
 
+def test_splits_are_reckoned_once_a_batch(monkeypatch):
+    from llm_sharding_demo_amd.ops.hip import HipBackend
+    from llm_sharding_demo_amd.runtime.batch import BatchMeta
+
+    asked, calls, rule = [], [], HipBackend.R.talk_prefill_parts
+    monkeypatch.setattr(type(HipBackend.R), "talk_prefill_parts", lambda self, *a: asked.append(a) or rule(*a))
+    for first in (0, 400):
+        meta = BatchMeta.build([0, 1], [0, first], [500, 100], "cpu")
+        for _ in range(3):
+            layer(meta, calls)
+    assert len(asked) == 2 and len(set(calls)) == 1 and len(calls) == 6
+
+
 def test_splits_of_a_captured_chunk():
     """Its replays start elsewhere: splits by tiles, each as long as its tile's keys over them, not as the captured context's."""
     from llm_sharding_demo_amd.runtime.batch import BatchMeta

@@ -761,10 +761,12 @@ __device__ __forceinline__ void count_up(F f) {  // f(0) .. f(N - 1)
   }
 }
 
-// Sums of one 16 x 16 tile by fp32 MFMAs; a, w: this lane's row and column at its k's.  AHEAD k-steps' loads are on their way.
+// Sums of one 16 x 16 tile by fp32 MFMAs, in eight chains, or they would be further off than three bf16 terms' (a value of 20000 in
+// every row, K = 2048, two chains 7.9e-7 of the result, eight 4.0e-7, three terms 4.05e-7); a, w: this lane's row and column at its k's.  AHEAD k-steps' loads are
+// on their way.
 __device__ __forceinline__ f32x4 fp32_sums(const float* a, const float* w, int steps) {
   constexpr int AHEAD = 4;
-  f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, av[AHEAD][2], wv[AHEAD][2];
+  f32x4 s[2][4] = {}, av[AHEAD][2], wv[AHEAD][2];
   auto load = [&](int k, int at) {  // (behind the last one that one again)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -776,7 +778,7 @@ __device__ __forceinline__ f32x4 fp32_sums(const float* a, const float* w, int s
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) s[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[at][h][e], wv[at][h][e], s[h], 0, 0, 0);
+      for (int h = 0; h < 2; ++h) s[h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[at][h][e], wv[at][h][e], s[h][e], 0, 0, 0);
   };
 #pragma unroll
   for (int k = 0; k < AHEAD; ++k) load(k, k);
@@ -793,7 +795,7 @@ __device__ __forceinline__ f32x4 fp32_sums(const float* a, const float* w, int s
 #pragma unroll
   for (int k = 0; k < AHEAD - 1; ++k)
     if (k0 + k < steps) add(k);
-  return s[0] + s[1];
+  return ((s[0][0] + s[0][1]) + (s[0][2] + s[0][3])) + ((s[1][0] + s[1][1]) + (s[1][2] + s[1][3]));
 }
 
 // Sums of n products, n a multiple of 4, of a row and of C columns by a wave.
@@ -821,6 +823,8 @@ __device__ __forceinline__ void fp32_row(const float* a, const float* const (&w)
 // The two chains make up for what the terms leave out: off 64 bits by (before) K = 1024 1.65e-7 (1.94e-7) of the result, K = 2048
 // 2.2e-7 (2.7e-7), in two parts 1.73e-7 (1.94e-7), in three 1.49e-7 (1.50e-7), K = 5632 3.5e-7 (4.7e-7), SiLU of two, K = 2048
 // 3.4e-7 (4.3e-7); with one chain 2.2e-7 at K = 1024.  Shorter ones are left to the kernel above: K = 544 1.38e-7 (1.30e-7).
+// Not so where sums round less than the terms: rows without negative values, K = 1024 1.7e-7 (1.4e-7), K = 2048 2.2e-7 (2.15e-7), in
+// three parts 1.5e-7 (1.2e-7), K = 5632 3.5e-7 (3.9e-7); columns of 2 % of the weights, K = 2048 1.1e-7 (0.5e-7); a lone product 2^-23 at most (none).
 // Bound by what a CU takes in.  W goes through LDS like A, in whole lines: loaded straight into fragments (16 rows of 64 bytes
 // an instruction), 1000 x 11264 x 2048 on 64 x 128 took 230 us, without the splitting 216, without the MFMAs 200, without both 203,
 // without loads behind the first ones 136; through LDS 208 to 225, and 176 on 128 x 128.  Waves of 32 x 32 read least from LDS.

@@ -125,6 +125,19 @@ def test_lone_products_of_experts(C):  # noqa: F811
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,tile", [TILES[2], TILES[4]])
+@pytest.mark.parametrize("rows", [slice(None), slice(None, None, 40)])
+def test_large_values(C, M, N, K, tile, rows):  # noqa: F811
+    """Rows that the terms cannot hold are summed again, as near to 64 bits as on three bf16 terms (2.4e-7 and 2.9e-7 of
+    the result; by fp32 MFMAs in two chains, as few rows are, 4.6e-7 and 5.5e-7)."""
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2) * 0.02
+    a[rows, 50] = 20000.0
+    got, want = C.linear_fp32(a.to(DEV), w.to(DEV)).cpu().to(F64), a.to(F64) @ w.to(F64).T
+    assert near(got, a, w)
+    assert float((got - want)[rows].norm() / want[rows].norm()) < 3.5e-7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 65504.0, -3e38])
 @pytest.mark.parametrize("side", ["a", "w"])
 def test_not_finite(C, side, value):  # noqa: F811

@@ -761,8 +761,8 @@ __device__ __forceinline__ void count_up(F f) {  // f(0) .. f(N - 1)
   }
 }
 
-// Sums of one 16 x 16 tile by fp32 MFMAs, in eight chains, or they would be further off than three bf16 terms' (a value of 20000 in
-// every row, K = 2048, two chains 7.9e-7 of the result, eight 4.0e-7, three terms 4.05e-7); a, w: this lane's row and column at its k's.  AHEAD k-steps' loads are
+// Sums of one 16 x 16 tile by fp32 MFMAs, in eight chains, or they would be further off than three bf16 terms' (two chains 7.9e-7 of
+// the result, K = 2048, eight 4.0e-7, three terms 4.05e-7); a, w: this lane's row and column at its k's.  AHEAD k-steps' loads are
 // on their way.
 __device__ __forceinline__ f32x4 fp32_sums(const float* a, const float* w, int steps) {
   constexpr int AHEAD = 4;
@@ -839,8 +839,10 @@ __device__ __forceinline__ void fp32_row(const float* a, const float* const (&w)
 // Where the sizes of a sum's two chains are together less than that it is computed again from the operands, and where it is not
 // finite: by itself where a 16 x 16 tile has such sums in up to ROWS rows, by fp32 MFMAs where in more.  (By the size of the sum
 // alone, every tenth tile of normal operands would have one, 3 us of a launch.)  A row or a column of zeros has zeros.
-// 961 x 2048 x 2048, us: normal operands 47 (three bf16 terms 58), a value of 20000 85 (58), one in every tenth row 147, in every
-// row 272 (58); rows of 2^-8 47.
+// Before that a tile with a value of 16376 in A or 256 in W is summed once more with powers of two for scales that hold its
+// largest values, up to 2^60; what is small beside them is lost sooner, and the line above moves with it.
+// 961 x 2048 x 2048, us: normal operands 47 (three bf16 terms 58), a value of 20000 79 (58), one in every tenth row 87, in every
+// row 81 (58; by fp32 MFMAs alone 272); rows of 2^-8 48.
 template <int MODE, int WM, int MT, int WN, int NT, int WK, int PF, int OCC>
 __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_kernel(GgParams p) {
   using namespace gg;
@@ -859,137 +861,163 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
   const int live = __builtin_amdgcn_readfirstlane((t.rows + 15) / 16) - wm * MT;  // of this wave's tiles
   // this part's k-steps; the first part has as many as any
   const int KT = t.K / BKF, most = (KT + WK - 1) / WK, first = part * most, T = max(0, min(most, KT - first));
-  // thread i brings four k's of rows i / 8, i / 8 + RQ .. of W and of A: whole lines
-  const int row = tid >> 3, ac = tid & 7;
   constexpr int UNITS = QW + QA;
-  const float* src[UNITS];
-#pragma unroll
-  for (int u = 0; u < UNITS; ++u)
-    src[u] = (u < QW ? static_cast<const float*>(t.W) + (long)min(t.n0 + row + RQ * u, t.N - 1) * t.ldw
-                     : static_cast<const float*>(t.A) + a_row<MODE>(p, t, row + RQ * (u - QW)) * t.lda) + first * BKF + 4 * ac;
-  auto at = [&](int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4); };  // in a plane: W's rows, A's
-
   f32x4 acc[3][MT][NT];  // hi hi of even and of odd k-steps, 2048 times the others
+  // All products with these scales; whether a value is beyond the terms'.  (mine: the thread, as addresses of its own: kept in
+  // registers for another pass, they would have the loops' spilled)
+  auto products = [&](float sa, float sw, int mine) {
+    const int lane = mine & 63, r = lane & 15, g = lane >> 4;
+    // thread i brings four k's of rows i / 8, i / 8 + RQ .. of W and of A: whole lines
+    const int row = mine >> 3, ac = mine & 7;
+    const float* src[UNITS];
 #pragma unroll
-  for (int c = 0; c < 3; ++c)
+    for (int u = 0; u < UNITS; ++u)
+      src[u] = (u < QW ? static_cast<const float*>(t.W) + (long)min(t.n0 + row + RQ * u, t.N - 1) * t.ldw
+                       : static_cast<const float*>(t.A) + a_row<MODE>(p, t, row + RQ * (u - QW)) * t.lda) + first * BKF + 4 * ac;
+    auto at = [&](int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4); };  // in a plane: W's rows, A's
+
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+    for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Experts: each column tile starts its sums at another k than its neighbours and than the next expert, so that blocks under way
-  // together do not stand at the same place of rows that lie powers of two apart (the sizes above: up 204 -> 195 us, down
-  // 112 -> 101; 300 tokens 146 -> 131 and 82 -> 75, 1400 359 -> 351 and 196 -> 186; others up to 10 % faster and slower)
-  const int from = (MODE == GG_UP || MODE == GG_DOWN) && T > 0 ? (t.n0 / TN * 11 + t.group * 7) % T : 0;
-  float largest[UNITS] = {};
-  f32x4 raw[PF][UNITS];
-  char* const slots = smem + part * 2 * SLOT;
-  auto load = [&](int u, int kt, int ring) {  // (behind the last k-step: that one again)
-    const int k = min(kt, T - 1) + from;
-    raw[ring][u] = *reinterpret_cast<const f32x4*>(src[u] + (long)(k >= T ? k - T : k) * BKF);
-  };
-  char* const put = slots + at(row, ac & 3) + (ac >> 2) * 8;  // chunk g: k's 4 g and 16 + 4 g (RQ rows on: the same chunk)
-  auto part_up = [&](int u, int ring, int slot) {
-    if (TM % RQ && u == UNITS - 1 && row + RQ * (QA - 1) >= TM) return;
-    f16x4 hi, lo;
-    split2(raw[ring][u], u < QW ? SCALE_W : SCALE_A, hi, lo, largest[u]);
-    char* b = put + slot * SLOT + (u < QW ? RQ * u : TN + RQ * (u - QW)) * 64;
-    *reinterpret_cast<u32x2*>(b) = __builtin_bit_cast(u32x2, hi);
-    *reinterpret_cast<u32x2*>(b + PLANE) = __builtin_bit_cast(u32x2, lo);
-  };
-  auto steps = [&](auto L) {
-    auto step = [&](int kt, auto unroll) {
-      constexpr int U = decltype(unroll)::v, S = U & 1, R = (U + 1) % PF, GROUPS = L < 2 ? 1 : (L + 1) / 2;
-      __syncthreads();  // k-step kt is in its slot, the other one's reads are done
-      if (WK > 1 && kt >= T) return;
-      const char* b = slots + S * SLOT;
-      f16x8 wf[NT][2];
-      if constexpr (L > 0) {
+      for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-          for (int c = 0; c < 2; ++c) wf[j][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at((wn * NT + j) * 16 + r, g));
-      }
-#pragma unroll
-      for (int i0 = 0; i0 < 2 * GROUPS; i0 += 2) {
-        f16x8 af[2][2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-          for (int i = i0; i < min((int)L, i0 + 2); ++i)
-            af[i - i0][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at(TN + (wm * MT + i) * 16 + r, g));
-#pragma unroll
-        for (int u = i0 / 2 * UNITS / GROUPS; u < (i0 / 2 + 1) * UNITS / GROUPS; ++u) {
-          part_up(u, R, S ^ 1);
-          load(u, kt + 1 + PF, R);
-        }
-#pragma unroll
-        for (int c = 0; c < 3; ++c)
-#pragma unroll
-          for (int i = i0; i < min((int)L, i0 + 2); ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-              f32x4& s = acc[c ? 2 : S][i][j];
-              s = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i - i0][c >> 1], wf[j][c & 1], s, 0, 0, 0);
-            }
-      }
-      // an MFMA, a part of the splitting, and so on; a pair of tiles' reads in front of its first
-      if constexpr (L > 0) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT, 0);
-#pragma unroll
-        for (int i = 0; i < 3 * L * NT; ++i) {
-          if (i % (6 * NT) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x2, (UNITS * 16 + 3 * L * NT - 1) / (3 * L * NT), 0);
-        }
-      }
+        for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Experts: each column tile starts its sums at another k than its neighbours and than the next expert, so that blocks under way
+    // together do not stand at the same place of rows that lie powers of two apart (the sizes above: up 204 -> 195 us, down
+    // 112 -> 101; 300 tokens 146 -> 131 and 82 -> 75, 1400 359 -> 351 and 196 -> 186; others up to 10 % faster and slower)
+    const int from = (MODE == GG_UP || MODE == GG_DOWN) && T > 0 ? (t.n0 / TN * 11 + t.group * 7) % T : 0;
+    float largest[UNITS] = {};
+    f32x4 raw[PF][UNITS];
+    char* const slots = smem + part * 2 * SLOT;
+    auto load = [&](int u, int kt, int ring) {  // (behind the last k-step: that one again)
+      const int k = min(kt, T - 1) + from;
+      raw[ring][u] = *reinterpret_cast<const f32x4*>(src[u] + (long)(k >= T ? k - T : k) * BKF);
     };
-    int kt = 0;
-    for (; kt + 2 <= most; kt += 2) count_up<2>([&](auto u) { step(kt + decltype(u)::v, u); });
-    if (kt < most) step(kt, Int<0>{});
+    char* const put = slots + at(row, ac & 3) + (ac >> 2) * 8;  // chunk g: k's 4 g and 16 + 4 g (RQ rows on: the same chunk)
+    auto part_up = [&](int u, int ring, int slot) {
+      if (TM % RQ && u == UNITS - 1 && row + RQ * (QA - 1) >= TM) return;
+      f16x4 hi, lo;
+      split2(raw[ring][u], u < QW ? sw : sa, hi, lo, largest[u]);
+      char* b = put + slot * SLOT + (u < QW ? RQ * u : TN + RQ * (u - QW)) * 64;
+      *reinterpret_cast<u32x2*>(b) = __builtin_bit_cast(u32x2, hi);
+      *reinterpret_cast<u32x2*>(b + PLANE) = __builtin_bit_cast(u32x2, lo);
+    };
+    auto steps = [&](auto L) {
+      auto step = [&](int kt, auto unroll) {
+        constexpr int U = decltype(unroll)::v, S = U & 1, R = (U + 1) % PF, GROUPS = L < 2 ? 1 : (L + 1) / 2;
+        __syncthreads();  // k-step kt is in its slot, the other one's reads are done
+        if (WK > 1 && kt >= T) return;
+        const char* b = slots + S * SLOT;
+        f16x8 wf[NT][2];
+        if constexpr (L > 0) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) wf[j][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at((wn * NT + j) * 16 + r, g));
+        }
+#pragma unroll
+        for (int i0 = 0; i0 < 2 * GROUPS; i0 += 2) {
+          f16x8 af[2][2];
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int i = i0; i < min((int)L, i0 + 2); ++i)
+              af[i - i0][c] = *reinterpret_cast<const f16x8*>(b + c * PLANE + at(TN + (wm * MT + i) * 16 + r, g));
+#pragma unroll
+          for (int u = i0 / 2 * UNITS / GROUPS; u < (i0 / 2 + 1) * UNITS / GROUPS; ++u) {
+            part_up(u, R, S ^ 1);
+            load(u, kt + 1 + PF, R);
+          }
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = i0; i < min((int)L, i0 + 2); ++i)
+#pragma unroll
+              for (int j = 0; j < NT; ++j) {
+                f32x4& s = acc[c ? 2 : S][i][j];
+                s = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i - i0][c >> 1], wf[j][c & 1], s, 0, 0, 0);
+              }
+        }
+        // an MFMA, a part of the splitting, and so on; a pair of tiles' reads in front of its first
+        if constexpr (L > 0) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 2 * NT, 0);
+#pragma unroll
+          for (int i = 0; i < 3 * L * NT; ++i) {
+            if (i % (6 * NT) == 0) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, (UNITS * 16 + 3 * L * NT - 1) / (3 * L * NT), 0);
+          }
+        }
+      };
+      int kt = 0;
+      for (; kt + 2 <= most; kt += 2) count_up<2>([&](auto u) { step(kt + decltype(u)::v, u); });
+      if (kt < most) step(kt, Int<0>{});
+    };
+    if (WK == 1 || T > 0) {
+#pragma unroll
+      for (int d = 0; d < PF; ++d)
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) load(u, d, d);
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) {
+        part_up(u, 0, 0);
+        load(u, PF, 0);
+      }
+    }
+    if constexpr (MODE == GG_UP || MODE == GG_DOWN) {
+      count_up<MT + 1>([&](auto ic) {
+        constexpr int l = decltype(ic)::v;
+        if (min(max(live, 0), MT) == l) steps(std::integral_constant<int, l>{});
+      });
+    } else {
+      steps(std::integral_constant<int, MT>{});
+    }
+    bool over = false;
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {  // of a row's eight threads
+      float& m = largest[u];
+#pragma unroll
+      for (int d = 1; d < 8; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+      over |= !(m * (u < QW ? sw : sa) < 65504.f);
+      const int at = row + RQ * (u < QW ? u : u - QW);
+      if (ac == 0 && u < QW) wmax[part * TN + at] = m;
+      if (ac == 0 && u >= QW && at < TM) amax[part * TM + at] = m;
+    }
+    return __syncthreads_or(over);  // (and every wave has read its last k-step)
   };
-  if (WK == 1 || T > 0) {
-#pragma unroll
-    for (int d = 0; d < PF; ++d)
-#pragma unroll
-      for (int u = 0; u < UNITS; ++u) load(u, d, d);
-#pragma unroll
-    for (int u = 0; u < UNITS; ++u) {
-      part_up(u, 0, 0);
-      load(u, PF, 0);
+  float ua = 1.f / SCALE_A, uw = 1.f / SCALE_W;  // of the products' sums (powers of two)
+  if (products(SCALE_A, SCALE_W, tid)) {  // once more with scales that hold the largest values
+    float most_a = 0.f, most_w = 0.f;
+    for (int c = lane; c < WK * TM; c += 64) most_a = fmaxf(most_a, amax[c]);
+    for (int c = lane; c < WK * TN; c += 64) most_w = fmaxf(most_w, wmax[c]);
+    most_a = wave_max(most_a);
+    most_w = wave_max(most_w);
+    if (most_a < 0x1p60f && most_w < 0x1p60f) {
+      auto fit = [](float most, float unit) {  // most / unit below 2^15, or as it was
+        const float to = __builtin_bit_cast(float, (__builtin_bit_cast(unsigned, most) >> 23) - 14 << 23);
+        return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, most < 65504.f * unit ? unit : to)));
+      };
+      ua = fit(most_a, ua);
+      uw = fit(most_w, uw);
+      int mine = tid;
+      asm volatile("" : "+v"(mine));
+      products(1.f / ua, 1.f / uw, mine);
     }
   }
-  if constexpr (MODE == GG_UP || MODE == GG_DOWN) {
-    count_up<MT + 1>([&](auto ic) {
-      constexpr int l = decltype(ic)::v;
-      if (min(max(live, 0), MT) == l) steps(std::integral_constant<int, l>{});
-    });
-  } else {
-    steps(std::integral_constant<int, MT>{});
-  }
-#pragma unroll
-  for (int u = 0; u < UNITS; ++u) {  // of a row's eight threads
-    float& m = largest[u];
-#pragma unroll
-    for (int d = 1; d < 8; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
-    const int at = row + RQ * (u < QW ? u : u - QW);
-    if (ac == 0 && u < QW) wmax[part * TN + at] = m;
-    if (ac == 0 && u >= QW && at < TM) amax[part * TM + at] = m;
-  }
-  __syncthreads();  // (and every wave has read its last k-step: sums take its place)
   constexpr int ROWS = 3;
   float* const ct = reinterpret_cast<float*>(smem) + part * IMAGE;
-  constexpr float UNIT = 1.f / (SCALE_A * SCALE_W);
-  float least = INFINITY, odd = 0.f, line = 0x1p-34f;  // of this lane's sums: the smallest size; zero where all are finite; the line's most
+  const float unit = ua * uw;
+  float least = INFINITY, odd = 0.f, line = 0x1p-24f * unit;  // of this lane's sums: the smallest size; zero where all are finite; the line's most
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
     const f32x4 av = *reinterpret_cast<const f32x4*>(amax + part * TM + (wm * MT + i) * 16 + 4 * g);
-    line = fmaxf(fmaxf(fmaxf(av[0], av[1]), fmaxf(av[2], av[3])) * 0x1p-18f, line);
+    line = fmaxf(fmaxf(fmaxf(av[0], av[1]), fmaxf(av[2], av[3])) * (uw * 0x1p-10f), line);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      line = fmaxf(wmax[part * TN + (wn * NT + j) * 16 + r] * 0x1p-12f, line);
+      line = fmaxf(wmax[part * TN + (wn * NT + j) * 16 + r] * (ua * 0x1p-10f), line);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float c0 = acc[0][i][j][q], c1 = acc[1][i][j][q], s = (c0 + c1 + acc[2][i][j][q] * (1.f / LO)) * UNIT;
+        const float c0 = acc[0][i][j][q], c1 = acc[1][i][j][q], s = (c0 + c1 + acc[2][i][j][q] * (1.f / LO)) * unit;
         least = fminf(least, fabsf(c0) + fabsf(c1));
         odd = __builtin_fmaf(s, 0.f, odd);
         ct[((wm * MT + i) * 16 + 4 * g + q) * CLD + (wn * NT + j) * 16 + r] = acc[2][i][j][q] = s;
@@ -997,7 +1025,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
     }
   }
   unsigned again = 0;  // row 4 g + q of tile (i, j), column r: bit (i NT + j) 4 + q where it is computed again
-  if (__ballot(least * UNIT < line || odd != 0.f) != 0) {
+  if (__ballot(least * unit < line || odd != 0.f) != 0) {
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
       const f32x4 av = *reinterpret_cast<const f32x4*>(amax + part * TM + (wm * MT + i) * 16 + 4 * g);
@@ -1006,7 +1034,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
         const float wv = wmax[part * TN + (wn * NT + j) * 16 + r];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const bool few = (fabsf(acc[0][i][j][q]) + fabsf(acc[1][i][j][q])) * UNIT < fmaxf(wv * 0x1p-13f + av[q] * 0x1p-19f, 0x1p-34f);
+          const bool few = (fabsf(acc[0][i][j][q]) + fabsf(acc[1][i][j][q])) * unit < fmaxf((wv * ua + av[q] * uw) * 0x1p-11f, 0x1p-24f * unit);
           const bool out = (wm * MT + i) * 16 + 4 * g + q < t.rows && t.n0 + (wn * NT + j) * 16 + r < t.N;
           again |= (unsigned)(out && ((few && wv > 0.f && av[q] > 0.f) || !(fabsf(acc[2][i][j][q]) < INFINITY))) << ((i * NT + j) * 4 + q);
         }

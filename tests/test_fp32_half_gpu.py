@@ -94,6 +94,8 @@ def test_lone_products(C, M, N, K, tile):  # noqa: F811
     for row, partner in ((110, 8192.0), (111, 1.0), (200, -0.01)):
         a[row] = 0
         a[row, K - 5] = partner
+    a[20, 300], a[70, 301], w[210, 302], w[290, 303] = 20000.0, 2.0 ** 40, 300.0, 2.0 ** 30  # (beside them lost sooner)
+    w[[7, 33, 60, 1980], 300:304] = 0
     for row, e in ((120, 20), (150, 26), (180, 34)):  # many such products
         a[row, : K // 2] *= 2.0 ** -e
     w[61, K // 2:] = 0
@@ -127,14 +129,18 @@ def test_lone_products_of_experts(C):  # noqa: F811
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,tile", [TILES[2], TILES[4]])
 @pytest.mark.parametrize("rows", [slice(None), slice(None, None, 40)])
-def test_large_values(C, M, N, K, tile, rows):  # noqa: F811
-    """Rows that the terms cannot hold are summed again, as near to 64 bits as on three bf16 terms (2.4e-7 and 2.9e-7 of
-    the result; by fp32 MFMAs in two chains, as few rows are, 4.6e-7 and 5.5e-7)."""
+@pytest.mark.parametrize("value,weight", [(20000.0, 0.0), (16376.0, 0.0), (3e9, 0.0), (2.0 ** 59, 0.0), (2.0 ** 70, 0.0), (20000.0, 300.0), (2.0 ** 50, 2.0 ** 50)])
+def test_large_values(C, M, N, K, tile, rows, value, weight):  # noqa: F811
+    """Rows that the terms cannot hold are summed again with other scales, or by fp32 MFMAs behind 2^60, as near to 64 bits as on three
+    bf16 terms (a value of 20000 2.4e-7 and 2.9e-7 of the result; by fp32 MFMAs in two chains, as few rows are, 4.6e-7 and 5.5e-7)."""
     a, w = rand(M, K, seed=1), rand(N, K, seed=2) * 0.02
-    a[rows, 50] = 20000.0
+    a[rows, 50] = value
+    if weight:
+        w[::3, K - 2] = weight
     got, want = C.linear_fp32(a.to(DEV), w.to(DEV)).cpu().to(F64), a.to(F64) @ w.to(F64).T
     assert near(got, a, w)
-    assert float((got - want)[rows].norm() / want[rows].norm()) < 3.5e-7
+    if not weight:  # (with it products of a few large values, which round less)
+        assert float((got - want)[rows].norm() / want[rows].norm()) < 3.5e-7
 
 
 @pytest.mark.gpu

@@ -882,10 +882,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[c][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // Experts: each column tile starts its sums at another k than its neighbours and than the next expert, so that blocks under way
-    // together do not stand at the same place of rows that lie powers of two apart (the sizes above: up 204 -> 195 us, down
-    // 112 -> 101; 300 tokens 146 -> 131 and 82 -> 75, 1400 359 -> 351 and 196 -> 186; others up to 10 % faster and slower)
-    const int from = (MODE == GG_UP || MODE == GG_DOWN) && T > 0 ? (t.n0 / TN * 11 + t.group * 7) % T : 0;
+    const int from = (MODE == GG_UP || MODE == GG_DOWN) && p.turn && T > 0 ? (t.n0 / TN * 11 + t.group * 7) % T : 0;
     float largest[UNITS] = {};
     f32x4 raw[PF][UNITS];
     char* const slots = smem + part * 2 * SLOT;
@@ -1385,11 +1382,31 @@ static bool on_split(const GgParams& p, bool routed) {
   return p.K >= 768 || tiles > 256 || tiles <= (p.M <= 32 ? 96 : 192);
 }
 
+// Whether each column tile of experts on two terms starts its sums at another k than its neighbours and than the next expert: blocks
+// under way together otherwise stand at the same place of rows of W that lie whole 4 KB apart.  Up to 96 rows an expert, whose
+// W is read about once; long sums only where all blocks start at once.  us with, without, 32 experts, 4 a token:
+//   2048 x 1024 (K = 2048 up, 1024 down)   200 tokens 106 115, 58 70   300 110 120, 61 73   500 150 160, 84 91   700 169 168, 89 94
+//   2048 x 2048   200 204 203, 106 120   500 268 277, 153 167   4096 x 1024 (more blocks)   240 209 205, 115 132   400 222 213, 125 144
+//   16 experts, 2 a token, 4096 x 1024, one round   200 127 147, 58 72   500 151 157, 83 88
+// 175 rows an expert 2048 x 1024 368 and 362, 190 and 189; other strides, 2048 x 1088, 8 experts of 2560 x 2560, 1600 x 1600, 300 to
+// 1400 tokens: 1 to 3 % slower so.
+static bool moe_turned(const GgParams& p) {
+  const long rows = (long)p.T * p.top, experts = p.n_tiles - rows / 64;
+  if (p.K % 1024 != 0 || rows > 96 * experts) return false;
+  return p.K <= 2048 || experts * ((p.N + 127) / 128) + (p.Ns > 0 ? (p.T + 63L) / 64 * ((p.Ns + 127) / 128) : 0) <= 256;
+}
+
 // Whether experts' products are on split operands (tests)
 extern "C" int lsd_moe_on_split(int T, int top, int n_tiles, int N, int Ns, int K) {
   GgParams p{};
   p.T = T, p.top = top, p.n_tiles = n_tiles, p.N = N, p.Ns = Ns, p.K = K;
   return on_split(p, true);
+}
+
+extern "C" int lsd_moe_turned(int T, int top, int n_tiles, int N, int Ns, int K) {
+  GgParams p{};
+  p.T = T, p.top = top, p.n_tiles = n_tiles, p.N = N, p.Ns = Ns, p.K = K;
+  return moe_turned(p);
 }
 
 template <int MODE>
@@ -1418,7 +1435,9 @@ static hipError_t gg_f32(const GgParams& p, hipStream_t st) {
         case 12: return gg_half_on<MODE, 2, 4, 4, 2, 1, 2, 2>(p, st);
       }
     } else if (half_terms(min(p.K, p.Ns > 0 ? p.Ks : p.K), 1)) {
-      return gg_half_on<MODE, 2, 2, 4, 2, 1, 2, 4>(p, st);
+      GgParams q = p;
+      q.turn = moe_turned(p);
+      return gg_half_on<MODE, 2, 2, 4, 2, 1, 2, 4>(q, st);
     }
     return gg_split_on<MODE, 4, 8, 1, 3>(p, st);
   }

@@ -36,6 +36,7 @@ struct GgParams {
   const float* wts_s;             // GG_DOWN: its weight per token, or null (1)
   const float* gate; long ldg;    // GG_BATCH / GG_F32: out *= sigmoid(gate[m][o_gs g + n]), or null
   int gr, gr_s;                   // row tiles per group of the tile order (experts, shared)
+  int turn;                       // fp32 experts: column tiles start their sums at places of K of their own
 };
 
 // Experts of a few tokens (weight streaming): see moe_gemv_*_kernel.

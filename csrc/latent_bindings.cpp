@@ -26,6 +26,7 @@ hipError_t lsd_group_gemm(const GgParams* p, int mode, int tm, hipStream_t st);
 hipError_t lsd_group_gemm_f32(const GgParams* p, int mode, hipStream_t st);
 void lsd_group_gemm_split_tile(int M, int N, int K, int* tile);
 int lsd_moe_on_split(int T, int top, int n_tiles, int N, int Ns, int K);
+int lsd_moe_turned(int T, int top, int n_tiles, int N, int Ns, int K);
 hipError_t lsd_moe_gemv_up(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_moe_gemv_down(const MoeGemvParams* p, hipStream_t st);
 hipError_t lsd_latent_post(const LatentPostParams* p, int f32, hipStream_t st);
@@ -631,6 +632,8 @@ void lsd_register_latent(pybind11::module& m) {
   }, py::arg("M"), py::arg("N"), py::arg("K") = 0);
   m.def("moe_on_split", [](int64_t T, int64_t top, int64_t n_tiles, int64_t N, int64_t Ns, int64_t K) {
     return lsd_moe_on_split((int)T, (int)top, (int)n_tiles, (int)N, (int)Ns, (int)K) != 0; });
+  m.def("moe_turned", [](int64_t T, int64_t top, int64_t n_tiles, int64_t N, int64_t Ns, int64_t K) {
+    return lsd_moe_turned((int)T, (int)top, (int)n_tiles, (int)N, (int)Ns, (int)K) != 0; });
   m.def("moe_group", &moe_group, py::arg("ids"), py::arg("experts"), py::arg("tm"));
   m.def("moe_up", &moe_up, py::arg("h"), py::arg("perm"), py::arg("tiles"), py::arg("top"), py::arg("w"),
         py::arg("limit"), py::arg("alpha"), py::arg("ws"), py::arg("limit_s"), py::arg("tm"));

@@ -159,9 +159,21 @@ def test_not_finite(C, side, value):  # noqa: F811
     assert bool(((got - want).abs()[ok] <= 2 * (K + 14) * ULP * size[ok]).all())
 
 
-# experts of 1024 columns and more: full and part full tiles, beside a shared expert
+# where column tiles start their sums elsewhere: tokens, choices, tiles of the table, columns, the shared expert's, K
+TURNED = [(300, 4, 50, 2048, 4096, 2048, True), (300, 4, 50, 2048, 2048, 1024, True), (700, 4, 75, 2048, 0, 1024, True),
+          (800, 4, 82, 2048, 0, 1024, False), (300, 4, 50, 2176, 4224, 2112, False), (300, 4, 50, 2048, 2048, 1088, False),
+          (300, 2, 17, 5120, 0, 2560, False), (300, 4, 50, 2048, 0, 4096, False), (300, 2, 25, 2048, 0, 4096, True),
+          (300, 2, 25, 2048, 2048, 4096, False), (300, 2, 25, 2048, 0, 3072, True)]
+
+
+def test_turned():
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    assert [_C.moe_turned(*r[:-1]) for r in TURNED] == [r[-1] for r in TURNED]
+
+
+# experts of 1024 columns and more: full and part full tiles, beside a shared expert; the third ones turned
 @pytest.mark.gpu
-@pytest.mark.parametrize("T,E,H,F,Fs", [(290, 3, 1024, 1088, 1024), (150, 2, 1056, 1024, 0)])
+@pytest.mark.parametrize("T,E,H,F,Fs", [(290, 3, 1024, 1088, 1024), (150, 2, 1056, 1024, 0), (290, 9, 1024, 1088, 1024), (150, 8, 3072, 1024, 0)])
 def test_experts(C, T, E, H, F, Fs):  # noqa: F811
     H = (H + 63) // 64 * 64
     h, up, dn = rand(T, H, seed=1), rand(E, 2 * F, H, seed=2) * 0.05, rand(E, H, F, seed=3) * 0.05

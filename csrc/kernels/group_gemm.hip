@@ -840,7 +840,8 @@ __device__ __forceinline__ void fp32_row(const float* a, const float* const (&w)
 // finite: by itself where a 16 x 16 tile has such sums in up to ROWS rows, by fp32 MFMAs where in more.  (By the size of the sum
 // alone, every tenth tile of normal operands would have one, 3 us of a launch.)  A row or a column of zeros has zeros.
 // Before that a tile with a value of 16376 in A or 256 in W is summed once more with powers of two for scales that hold its
-// largest values, up to 2^60; what is small beside them is lost sooner, and the line above moves with it.
+// largest values, up to 2^60; what is small beside them is lost sooner, and the line above moves with it.  Not one of experts, whose
+// registers are all taken (down products of 700 rows 80 -> 87 us, others up to 2 % faster and slower with the code for it).
 // 961 x 2048 x 2048, us: normal operands 47 (three bf16 terms 58), a value of 20000 79 (58), one in every tenth row 87, in every
 // row 81 (58; by fp32 MFMAs alone 272); rows of 2^-8 48.
 template <int MODE, int WM, int MT, int WN, int NT, int WK, int PF, int OCC>
@@ -983,7 +984,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, OCC) void group_gemm_f32_half_ke
     return __syncthreads_or(over);  // (and every wave has read its last k-step)
   };
   float ua = 1.f / SCALE_A, uw = 1.f / SCALE_W;  // of the products' sums (powers of two)
-  if (products(SCALE_A, SCALE_W, tid)) {  // once more with scales that hold the largest values
+  if (products(SCALE_A, SCALE_W, tid) && MODE != GG_UP && MODE != GG_DOWN) {  // once more with scales that hold the largest values
     float most_a = 0.f, most_w = 0.f;
     for (int c = lane; c < WK * TM; c += 64) most_a = fmaxf(most_a, amax[c]);
     for (int c = lane; c < WK * TN; c += 64) most_w = fmaxf(most_w, wmax[c]);

@@ -33,6 +33,7 @@ void lsd_gemm_set_ring8_pack(int v);
 void lsd_norm_set_wave_narrow_min(int v);
 void lsd_norm_set_wave_min(int v);
 int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits, int lanes);
+int lsd_gemm_deep_turned(int M, int N, int K, long ldw, int epi, int splits);
 int lsd_gemm_on_deep(int M, int N, int K, int epi, int kind, int splits);
 int lsd_gemm_d256_bn(int kind, int M, int N, int K);
 int lsd_gemm_ring8_tiles(int M, int N, int K, int S);
@@ -874,6 +875,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     const int s = lsd_gemm_deep_shape((int)M, (int)N, (int)K, (int)epi, (int)splits, (int)lanes);
     return std::make_pair(s / 1024, s % 1024); },
         py::arg("M"), py::arg("N"), py::arg("K"), py::arg("epi"), py::arg("splits"), py::arg("lanes") = 1);
+  m.def("gemm_deep_turned", [](int64_t M, int64_t N, int64_t K, int64_t ldw, int64_t epi, int64_t splits) {
+    return lsd_gemm_deep_turned((int)M, (int)N, (int)K, ldw, (int)epi, (int)splits) != 0; });
   m.def("gemm_prompt_slabs", [](int64_t M, int64_t N, int64_t K, int64_t S) {
     return lsd_gemm_prompt_slabs((int)M, (int)N, (int)K, (int)S); });
   m.def("gemm_on_deep", [](int64_t M, int64_t N, int64_t K, int64_t epi, int64_t kind, int64_t splits) {

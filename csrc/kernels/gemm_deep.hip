@@ -11,7 +11,7 @@
 //    weights are small, and more rows are 0 to 20 % slower that way.
 //  * rows of W that lie powers of two apart: blocks that walk through K together stand at the same place of
 //    all of them, and where they all start at once W arrives at 4.9 to 5.5 TB/s.  Each column tile then starts its sums
-//    elsewhere (deep_turn): 16384 x 4096 of 24 rows 25.9 -> 21.9 us, 32000 x 2048 26.3 -> 23.1, 11264 x 2048 11.2 -> 10.6.
+//    elsewhere (deep_turn): 16384 x 4096 of 24 rows 25.9 -> 21.9 us, 32000 x 2048 26.3 -> 23.5, 11264 x 2048 11.2 -> 10.6.
 //  * a block holds all of up to 64 rows; more are also divided among blocks beside each other,
 //    which find W in L2, where that brings a CU fewer bytes.  Its width (128 to 16 columns)
 //    follows from the columns: narrow outputs take narrow tiles, whose waves split the k-step's
@@ -233,25 +233,25 @@ static DeepShape deep_shape(int M, int N, int K, int splits, int epi, int lanes)
   return best;
 }
 
-// Column tiles start at places of K of their own where W's rows lie whole 4 KB apart and all blocks, two a CU, start
-// at once.  Later ones are out of step by themselves (128256 x 4096, 48 rows of 128 columns 174 us, turned 190), as are rows of other
+// Column tiles start at places of K of their own where W's rows lie whole 4 KB apart and all blocks start at once: two a CU
+// (96 x 128 and 128 x 128 ones, one a CU, are never more than 256: lsd_gemm_deep_ok).  Later ones are out of step by themselves (128256 x 4096, 48 rows of 128 columns 174 us, turned 190), as are rows of other
 // strides (K = 1600, 768: up to 4 % slower turned), and 32 columns gain too little (6144 x 4096 14.3 and 14.9).
-static bool deep_turn(const GemmParams& p, long blocks, int cols) {
-  return p.splits == 1 && p.K >= 2048 && p.K % 2048 == 0 && p.ldw % 2048 == 0 && cols >= 64 && blocks <= 512;
+static bool deep_turn(int splits, int K, long ldw, long blocks, int cols) {
+  return splits == 1 && K >= 2048 && K % 2048 == 0 && ldw % 2048 == 0 && cols >= 64 && blocks <= 512;
 }
 
 template <int EPI>
 static hipError_t deep_launch(const GemmParams& p, hipStream_t st) {
   const DeepShape s = deep_shape(p.M, p.N, p.K, p.splits, EPI, p.lanes);
   const int tn = (p.N + s.cols - 1) / s.cols, mbs = (p.M + s.rows - 1) / s.rows;
-  const int turn = deep_turn(p, (long)tn * mbs, s.cols) ? 31 : 0;
+  const int turn = deep_turn(p.splits, p.K, p.ldw, (long)tn * mbs, s.cols) ? 31 : 0;
 #define LSD_DEEP_K(ONE, ROWS, COLS, WM, WN, WK, BK, SLOTS, AUX)                                                       \
   if (s.rows == ROWS && s.cols == COLS) {                                                                             \
     hipLaunchKernelGGL((gemm_deep_kernel<WM, WN, WK, ROWS / (16 * WM), COLS / (16 * WN), BK, SLOTS, AUX, EPI, ONE>),  \
                        dim3((unsigned)(tn * p.splits * mbs)), dim3(64 * WM * WN * WK), 0, st, p, tn, mbs, turn);            \
     return hipGetLastError();                                                                                         \
   }
-  // slots: two blocks per CU
+  // slots: two blocks per CU, of 96 and 128 rows by 128 columns one
   if (mbs == 1) {
     LSD_DEEP_K(true, 48, 64, 1, 4, 1, 64, 5, NT_LOAD)
     LSD_DEEP_K(true, 48, 32, 1, 2, 2, 64, 8, 0)
@@ -330,6 +330,12 @@ extern "C" int lsd_gemm_deep_ok(int M, int N, int K, int epi, int splits) {
 extern "C" int lsd_gemm_deep_shape(int M, int N, int K, int epi, int splits, int lanes) {
   const DeepShape s = deep_shape(M, N, K, epi == EPI_SLAB ? splits : 1, epi, lanes);
   return s.rows * 1024 + s.cols;
+}
+
+// Whether its column tiles start at places of K of their own (tests)
+extern "C" int lsd_gemm_deep_turned(int M, int N, int K, long ldw, int epi, int splits) {
+  const DeepShape s = deep_shape(M, N, K, splits, epi, 1);
+  return deep_turn(splits, K, ldw, (long)((N + s.cols - 1) / s.cols) * ((M + s.rows - 1) / s.rows), s.cols);
 }
 
 extern "C" hipError_t lsd_gemm_deep(const GemmParams* p, int epi, hipStream_t st) {

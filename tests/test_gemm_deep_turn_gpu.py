@@ -47,13 +47,33 @@ def test_products(C, shape, M, N, K):  # noqa: F811
         assert near(C.linear(ad, wd, None, SILU, 1, 1, None), gate / (1 + torch.exp(-gate)) * up, both)
 
 
+def test_turned():
+    """Rows whole 4 KB apart, all blocks under way at once, blocks of 64 columns and more."""
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    for shape, M, N, K in WIDE:
+        assert _C.gemm_deep_turned(M, N, K, K, F32, 1) == (K in (2048, 4096))
+    for M, N, K, ldw in ((20, 16384, 2112, 4096), (20, 16384, 2048, 2112), (20, 128256, 4096, 4096), (20, 6144, 4096, 4096)):
+        assert not _C.gemm_deep_turned(M, N, K, ldw, F32, 1)
+    assert _C.gemm_deep_turned(20, 16384, 2048, 4096, F32, 1) and not _C.gemm_deep_turned(20, 16384, 2048, 2048, 5, 2)
+
+
+def test_wide_blocks_all_start_at_once():
+    """Blocks of 96 and 128 rows by 128 columns, one of which a CU holds: never more than CUs."""
+    _C = pytest.importorskip("llm_sharding_demo_amd._C")
+    for M in range(65, 129):
+        for N in range(32, 70000, 32 * 13):
+            if _C.gemm_on_deep(M, N, 2048, F32, 1, 1) and _C.gemm_deep_shape(M, N, 2048, F32, 1)[1] == 128:
+                assert (N + 127) // 128 <= 256
+
+
 @pytest.mark.gpu
-def test_rows_of_w_in_a_wider_tensor(C):  # noqa: F811
-    """Rows 4 KB apart of which fewer k's are taken, and whole rows at another stride: not turned, the same results."""
+@pytest.mark.parametrize("k,stride", [(2112, 4096), (2048, 4096), (2048, 2112), (2048, 2048)])
+def test_rows_of_w_in_a_wider_tensor(C, k, stride):  # noqa: F811
+    """Rows 4 KB apart of which fewer k's are taken, turned where those are whole 4 KB too, and rows at another stride."""
     g = torch.Generator().manual_seed(5)
-    a, w = torch.randn(20, 4096, generator=g).bfloat16(), (torch.randn(16384, 4096, generator=g) / 64).bfloat16().to(DEV)
-    for k in (2112, 2048):
-        ak, wk = a[:, :k].contiguous().to(DEV), w[:, :k]
-        want = (ak.to(F64) @ wk.to(F64).T).cpu()
-        off = (k + 3) * 2.0 ** -24 * (ak.to(F64).abs() @ wk.to(F64).abs().T).cpu()
-        assert bool(((C.linear_f32(ak, wk, 1, 1, None).cpu().to(F64) - want).abs() <= off).all())
+    a, w = torch.randn(20, k, generator=g).bfloat16(), (torch.randn(16384, stride, generator=g) / 64).bfloat16().to(DEV)
+    assert C.gemm_deep_turned(20, 16384, k, stride, F32, 1) == (k == 2048 and stride != 2112)
+    ak, wk = a.to(DEV), w[:, :k]
+    want = (ak.to(F64) @ wk.to(F64).T).cpu()
+    off = (k + 3) * 2.0 ** -24 * (ak.to(F64).abs() @ wk.to(F64).abs().T).cpu()
+    assert bool(((C.linear_f32(ak, wk, 1, 1, None).cpu().to(F64) - want).abs() <= off).all())

@@ -269,13 +269,43 @@ class Routing:
     def residual_splits(self, M: int, N: int, K: int, decode: bool = True, lanes: int = 1) -> int:
         """K splits a residual projection is launched with: the rule above, and
         what the kernels behind it make of slabs.  Prompts' slabs of more than 256
-        rows are reckoned once more at their launch (lsd_gemm_prompt_slabs in gemm_wave4.hip)."""
+        rows are reckoned once more at their launch (launch_slabs)."""
         S = self.resid_splits(M, N, K, decode, lanes)
         if not decode:
             S = self.prompt_slabs(M, N, K, S)
         if self.tiled(M, N) or self.defer_resid:
             S = self.slab_splits(M, N, K, S)
         return S
+
+    # gemm_wave4.hip's tiles in rows and columns of 64, blocks a CU, and what a launch takes in 1/1000 us: fixed, a
+    # round, a round's K-tile with one block a CU, with two; the last one is the 256 x 256 kernel
+    _WAVE4 = ((2, 2, 2, 4850, 2580, 496, 835), (3, 2, 2, 5890, 3770, 544, 1089), (3, 3, 1, 6640, 7540, 705, 0),
+              (4, 2, 2, 6400, 4390, 791, 1358), (4, 3, 1, 7500, 10750, 849, 0), (3, 4, 1, 7460, 10050, 867, 0),
+              (4, 4, 1, 6320, 11770, 1072, 0))
+
+    @classmethod
+    def launch_slabs(cls, M: int, N: int, K: int, S: int) -> int:
+        """Slabs that a prompt's residual projection is launched with where the rule leaves S
+        (mirrors lsd_gemm_prompt_slabs() in gemm_wave4.hip)."""
+        if S <= 1 or M <= 256 or K % 64 or K < 256:
+            return S
+
+        def cost(s):
+            if -(-M // 128) * -(-N // 64) * s <= 256:
+                least = 5500 + 570 * (K // 64) // s
+            else:
+                least = None
+                for mi, nj, bpc, fixed, a_round, one, two in cls._WAVE4:
+                    tiles, cap = -(-M // (64 * mi)) * -(-N // (64 * nj)) * s, 256 * bpc
+                    rounds = -(-tiles // cap)
+                    last = tiles - cap * (rounds - 1)
+                    k = (rounds - 1) * (two if bpc == 2 else one) + (two if bpc == 2 and last > 256 else one)
+                    c = fixed + a_round * (rounds - 1) + K // 64 * k // s
+                    least = c if least is None else min(least, c)
+            return least + s * (150 + M * N * 11 // 10000)
+
+        best = min(range(2, min(8, K // 128) + 1), key=cost)
+        return best if S <= 8 or cost(S) >= cost(best) else S
 
     @staticmethod
     def on_deep(M: int, N: int, K: int, splits: int = 1, pairs: bool = False) -> bool:
@@ -526,6 +556,8 @@ def route_table(model: str, rows, routing: Routing | None = None) -> dict:
                     route = "gemv"
                 elif kind == "resid":
                     s = r.residual_splits(M, N, K, decode, lanes)
+                    if not decode:
+                        s = r.launch_slabs(M, N, K, s)
                     t = r.tiled(M, N)
                     slabs = s if t or r.defer_resid else 1
                     route = f"{'tiled' if t else 'splitk-slab' if r.defer_resid and s > 1 else 'splitk'}/s{s}"

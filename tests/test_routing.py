@@ -78,6 +78,19 @@ def test_deep_ring_rule_is_the_kernels():
                     assert Routing.on_deep(*at, S) == _C.gemm_on_deep(*at, EPI_SLAB, 0, S), (at, S)
 
 
+def test_slabs_rule_is_the_launchs():
+    """The table's copy of the rule against the launch's."""
+    try:
+        from llm_sharding_demo_amd import _C
+    except Exception as e:  # pragma: no cover - extension not built here
+        pytest.skip(f"_C not importable: {e}")
+    for M in (1, 256, 257, 300, 512, 777, 1000, 2048, 4097, 20000, 65536):
+        for N in (16, 768, 1600, 2048, 4096, 5120):
+            for K in (64, 96, 192, 256, 320, 768, 1600, 5600, 6400, 14336):
+                for S in (1, 2, 3, 8, 11, 15):
+                    assert Routing.launch_slabs(M, N, K, S) == _C.gemm_prompt_slabs(M, N, K, S), (M, N, K, S)
+
+
 def test_routing_env_override():
     r = Routing.from_env("ring8=0, sk_target=256")
     assert r.ring8 == 0 and r.sk_target == 256 and r.tiled3_max == Routing().tiled3_max

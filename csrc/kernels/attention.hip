@@ -61,8 +61,8 @@ __device__ __forceinline__ void fold_step(float (&v)[V], int& idx, int lane) {
 // item's K and V requested in one round of loads instead of a chain of dependent ones.
 // There a launch is its chain: position, K and V, scores, merges.  The merges are kept short: a wave scales its
 // sums once by its own maximum and folds them over its key groups, each lane going on with half of its columns
-// (7 exchanges for 8 columns, 24 when every lane merges all of them pair by pair), and a lane a column merges
-// the waves.  12 heads of 64, one sequence of 204 keys 4.7 -> 4.0 us, on 4 waves of 8 keys for 8 of 4 3.7.
+// (7 exchanges for 8 columns, 24 when every lane merges all of them pair by pair), and a thread for two columns
+// merges the waves.  12 heads of 64, one sequence of 204 keys 4.7 -> 4.0 us, on 4 waves of 8 keys for 8 of 4 3.7.
 template <int HD, int G, int U, int NWV>
 __global__ __launch_bounds__(NWV * 64) void attn_decode_kernel(
     const bf16* __restrict__ q, long ldq, const bf16* __restrict__ kc,

@@ -310,7 +310,8 @@ using namespace lsd;
 // 1 .. 256 rows, whole k-steps; gate / up pairs lie in one tile.  splits > 1 only as slabs:
 // the other epilogues run unsplit, whatever the caller asked for.  More than 48 rows only up to
 // two blocks a CU (49 .. 64 rows two and a half): behind that the 128 x 128 tiles, which read A half
-// as often, are as fast or faster.  Vocabulary-wide, deep ring against those tiles:
+// as often, are as fast or faster.  Vocabulary-wide, deep ring in blocks of 64 columns against those tiles (deep_shape has what 128
+// columns give up to 48 rows; more rows have not been timed on them where they are not taken):
 //   50304 x 1600  64 rows 40.3 against 37.0 us, 96 50 against 41, 128 56 against 44 (48 rows 38 and 37)
 //   128256 x 4096  64 rows 220 against 203, 128 260 against 208 (40 rows both 190)
 //   40960 x 1600  64 rows 31.5 against 35, 80 36 against 37, 128 44 against 42

@@ -526,7 +526,10 @@ class Routing:
                 return ms
         if hd == 64 and max_ctx <= 2 * self.split_keys:
             # two rounds of a block's loads cost less than a merge of its own (12 heads, 300 keys 5.4 us,
-            # in two splits 6.0; 450 5.7 and 6.1; three rounds and splits: 700 7.3 and 6.1)
+            # in two splits 6.0; 450 5.7 and 6.1; three rounds and splits: 700 7.3 and 6.1; up to 400 items, 280 to
+            # 512 keys 0.3 to 2 us less, and grouped heads likewise or within 2 %: 32 over 8, one sequence of
+            # 280 7.3 and 8.5, 512 8.55 and 8.40, 16 over 8 5.8 and 6.6; behind by up to a tenth where 256
+            # blocks and more have over 350: 32 sequences, 12 heads, 450 8.7 and 8.0, 16 over 8, 400 9.2 and 8.3)
             return 1
         if items < self.target_blocks:
             return min(math.ceil(self.target_blocks / items), max(1, math.ceil(max_ctx / self.split_keys)))

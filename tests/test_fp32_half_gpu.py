@@ -127,9 +127,10 @@ def test_lone_products_of_experts(C):  # noqa: F811
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,tile", [TILES[2], TILES[4]])
-@pytest.mark.parametrize("rows", [slice(None), slice(None, None, 40)])
-@pytest.mark.parametrize("value,weight", [(20000.0, 0.0), (16376.0, 0.0), (3e9, 0.0), (2.0 ** 59, 0.0), (2.0 ** 70, 0.0), (20000.0, 300.0), (2.0 ** 50, 2.0 ** 50)])
+@pytest.mark.parametrize("M,N,K,tile,rows,value,weight", [
+    *((*case, slice(None, None, step), value, weight) for case in (TILES[2], TILES[4]) for step in (1, 40) for value, weight in (
+        (16376.0, 0.0), (3e9, 0.0), (2.0 ** 59, 0.0), (2.0 ** 70, 0.0), (20000.0, 300.0), (2.0 ** 50, 2.0 ** 50))),
+    *((*case, slice(None, None, step), 20000.0, 0.0) for case in TILES for step in (1, 40))])
 def test_large_values(C, M, N, K, tile, rows, value, weight):  # noqa: F811
     """Rows that the terms cannot hold are summed again with other scales, or by fp32 MFMAs behind 2^60, as near to 64 bits as on three
     bf16 terms (a value of 20000 2.4e-7 and 2.9e-7 of the result; by fp32 MFMAs in two chains, as few rows are, 4.6e-7 and 5.5e-7)."""
